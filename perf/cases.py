@@ -309,14 +309,17 @@ def _load_records(s, seed):
 
 
 def _crowd_records(case, seed, blas):
-    """Instances of small spheres over a field, each with its own rotation, size and place."""
+    """Instances of small spheres over a field: places and sizes of the crowd's own, and this frame's turn and
+    step of each (up to one sphere's width from where the structure was built)."""
     n = case["instances"]
-    rng = scenes.Rng(seed * 31 + 7)
+    home = scenes.Rng(7)
     side = math.sqrt(n)
+    pos = home.uniform(2 * n, -side, side).reshape(-1, 2)
+    scl = home.uniform(n, 0.4, 0.9)
+    y = home.uniform(n, 0.0, 4.0)
+    rng = scenes.Rng(seed * 31 + 8)
     ang = rng.uniform(n, 0.0, 2.0 * math.pi)
-    pos = rng.uniform(2 * n, -side, side).reshape(-1, 2)
-    scl = rng.uniform(n, 0.4, 0.9)
-    y = rng.uniform(n, 0.0, 4.0)
+    pos = pos + rng.uniform(2 * n, -0.7, 0.7).reshape(-1, 2)
     c, s = np.cos(ang) * scl, np.sin(ang) * scl
     rec = np.zeros(n, dtype=abi.INSTANCE_DTYPE)
     m = np.zeros((n, 3, 4))

@@ -7,51 +7,20 @@
 //   AccelerationStructure::clone        src/util_structs.rs:359-405
 // with a linear BVH (Karras 2012): primitive boxes and centres, 30-bit Morton
 // codes, a stable LSD radix sort written here (LDS digit ranking with wave
-// ballots), the radix-tree split search and a bottom-up box merge with
-// atomic arrival counters, then a top-down collapse of the binary tree into
-// 4-wide nodes, one breadth-first level per launch (node numbers from a
-// prefix sum, so they do not depend on scheduling), and the slot boxes of
-// the wide nodes from the deepest level up. The blobs are bit-identical to
-// the host oracle's: every box operation is an exact min/max or a fixed FP32
-// sequence.
+// ballots), the radix-tree split search, bottom-up boxes with the treelet
+// passes and a top-down collapse into 4-wide nodes (build_tree.hpp). Up to
+// kSmallBuild primitives go from their inputs to the binary tree in one
+// workgroup. The blobs are bit-identical to the host oracle's: every box
+// operation is an exact min/max or a fixed FP32 sequence.
 #include <algorithm>
 #include <cstring>
 #include <vector>
 
+#include "build_tree.hpp"
 #include "rtg_device.hpp"
 #include "rtg_internal.hpp"
 
 namespace rtg {
-
-// min/max of box planes as selects: the first operand wins ties, so that
-// +0/-0 resolve the same way on every device.
-__device__ inline float mins(float a, float b) { return b < a ? b : a; }
-__device__ inline float maxs(float a, float b) { return b > a ? b : a; }
-__device__ inline Box box_union(const Box& a, const Box& b) {
-    Box r;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        r.lo[k] = mins(a.lo[k], b.lo[k]);
-        r.hi[k] = maxs(a.hi[k], b.hi[k]);
-    }
-    return r;
-}
-__device__ inline Box box_empty() {
-    Box b;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        b.lo[k] = __builtin_inff();
-        b.hi[k] = -__builtin_inff();
-    }
-    return b;
-}
-
-// Order-preserving map of float to uint (for atomic min/max of centres).
-__device__ inline uint32_t f2ord(float f) {
-    uint32_t u = __float_as_uint(f);
-    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-}
-__device__ inline float ord2f(uint32_t o) { return __uint_as_float((o & 0x80000000u) ? (o & 0x7fffffffu) : ~o); }
 
 __device__ inline float centre(const Box& b, int a) { return (b.lo[a] + b.hi[a]) * 0.5f + 0.0f; }
 
@@ -94,12 +63,6 @@ __device__ inline Box ref_box(const Node* nodes, uint32_t c, const Box* leaf_box
         return b;
     }
     return node_box(nodes[c]);
-}
-
-// Surface area of a box (half of it: the collapse only compares areas).
-__device__ inline float box_area(const Box& b) {
-    float ex = b.hi[0] - b.lo[0], ey = b.hi[1] - b.lo[1], ez = b.hi[2] - b.lo[2];
-    return (ex * ey + ey * ez) + ez * ex;
 }
 
 // Block-wide reduction of centre bounds, then one atomic per block and axis.
@@ -147,11 +110,66 @@ __global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t v) {
         p[i] = v;
 }
 
-__global__ void k_init_bounds(uint32_t* cb) {
-    if (threadIdx.x < 3) {
-        cb[threadIdx.x] = 0xffffffffu;
-        cb[3 + threadIdx.x] = 0u;
+// Words a build clears before its kernels: the centre bounds (cb[0..2] the
+// least, cb[3..5] the largest, cb[6] whether a box plane is NaN) and the
+// tiers' counters (tier_words per treelet pass, then a list of node 0 alone
+// and its length). The geometry descriptors of a few geometries come with
+// the launch.
+constexpr int kTierWords = 4;  // bottom roots, middle roots, list space of the middle and of the top tier
+constexpr int kTierCounters = kTierWords * kTreeletRounds + 2;
+constexpr int kTopRoot = kTierWords * kTreeletRounds, kTopCount = kTopRoot + 1;
+constexpr uint32_t kGeomArgs = 8;
+struct GeomArgs {
+    GeomDesc g[kGeomArgs];
+};
+__global__ __launch_bounds__(64) void k_build_init(uint32_t* cb, uint32_t* tiers, GeomArgs args, uint32_t ngeom,
+                                                   GeomDesc* geoms) {
+    const uint32_t t = threadIdx.x;
+    if (t < 7) cb[t] = t < 3 ? 0xffffffffu : 0u;
+    if (t < kTierCounters) tiers[t] = t == kTopCount ? 1u : 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < kGeomArgs; ++k)
+        if (k == t && k < ngeom) geoms[k] = args.g[k];
+}
+
+// Record and box of triangle i.
+__device__ inline void make_tri(const GeomDesc* geoms, uint32_t ngeom, uint32_t i, TriRec& r, Box& b,
+                                uint32_t* status) {
+    uint32_t lo = 0, hi = ngeom;  // last geometry with first_tri <= i
+    while (hi - lo > 1) {
+        uint32_t mid = (lo + hi) >> 1;
+        if (geoms[mid].first_tri <= i) lo = mid;
+        else hi = mid;
     }
+    const GeomDesc g = geoms[lo];
+    uint32_t t = i - g.first_tri;
+    uint32_t i0 = g.indices[3ull * t], i1 = g.indices[3ull * t + 1], i2 = g.indices[3ull * t + 2];
+    if (i0 > g.max_vertex || i1 > g.max_vertex || i2 > g.max_vertex) {
+        atomicOr(status, (uint32_t)kStatusBadIndex);
+        i0 = i1 = i2 = 0;
+    }
+    const float* a = reinterpret_cast<const float*>(g.vertices + (uint64_t)i0 * g.stride);
+    const float* bb = reinterpret_cast<const float*>(g.vertices + (uint64_t)i1 * g.stride);
+    const float* cc = reinterpret_cast<const float*>(g.vertices + (uint64_t)i2 * g.stride);
+    float A[3] = {a[0], a[1], a[2]}, B[3] = {bb[0], bb[1], bb[2]}, Cv[3] = {cc[0], cc[1], cc[2]};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        r.v0[k] = A[k];
+        r.v1[k] = B[k];
+        r.v2[k] = Cv[k];
+        b.lo[k] = mins(mins(A[k], B[k]), Cv[k]);
+        b.hi[k] = maxs(maxs(A[k], B[k]), Cv[k]);
+    }
+    r.prim = t;
+    r.geom = lo | ((g.flags & RTG_GEOMETRY_OPAQUE) ? 0u : kNonOpaqueBit);
+    r.pad = 0;
+}
+
+__device__ inline bool box_has_nan(const Box& b) {
+    bool nan = false;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) nan = nan || b.lo[k] != b.lo[k] || b.hi[k] != b.hi[k];
+    return nan;
 }
 
 // Triangle records, primitive boxes, centre bounds.
@@ -161,38 +179,12 @@ __global__ __launch_bounds__(256) void k_tri_setup(const GeomDesc* geoms, uint32
     float c[3] = {0, 0, 0};
     bool valid[3] = {false, false, false};
     if (i < ntri) {
-        uint32_t lo = 0, hi = ngeom;  // last geometry with first_tri <= i
-        while (hi - lo > 1) {
-            uint32_t mid = (lo + hi) >> 1;
-            if (geoms[mid].first_tri <= i) lo = mid;
-            else hi = mid;
-        }
-        const GeomDesc g = geoms[lo];
-        uint32_t t = i - g.first_tri;
-        uint32_t i0 = g.indices[3ull * t], i1 = g.indices[3ull * t + 1], i2 = g.indices[3ull * t + 2];
         TriRec r;
         Box b;
-        if (i0 > g.max_vertex || i1 > g.max_vertex || i2 > g.max_vertex) {
-            atomicOr(status, (uint32_t)kStatusBadIndex);
-            i0 = i1 = i2 = 0;
-        }
-        const float* a = reinterpret_cast<const float*>(g.vertices + (uint64_t)i0 * g.stride);
-        const float* bb = reinterpret_cast<const float*>(g.vertices + (uint64_t)i1 * g.stride);
-        const float* cc = reinterpret_cast<const float*>(g.vertices + (uint64_t)i2 * g.stride);
-        float A[3] = {a[0], a[1], a[2]}, B[3] = {bb[0], bb[1], bb[2]}, Cv[3] = {cc[0], cc[1], cc[2]};
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            r.v0[k] = A[k];
-            r.v1[k] = B[k];
-            r.v2[k] = Cv[k];
-            b.lo[k] = mins(mins(A[k], B[k]), Cv[k]);
-            b.hi[k] = maxs(maxs(A[k], B[k]), Cv[k]);
-        }
-        r.prim = t;
-        r.geom = lo | ((g.flags & RTG_GEOMETRY_OPAQUE) ? 0u : kNonOpaqueBit);
-        r.pad = 0;
+        make_tri(geoms, ngeom, i, r, b, status);
         tris[i] = r;
         boxes[i] = b;
+        if (box_has_nan(b)) atomicOr(&cb[6], 1u);
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             c[k] = centre(b, k);
@@ -254,6 +246,15 @@ __device__ inline const AsHeader* checked_blas(const rtg_instance& in, const uin
     return reinterpret_cast<const AsHeader*>(a);
 }
 
+// Leaf record and world box of instance i.
+__device__ inline void make_inst(const rtg_instance* inst, uint32_t i, const uint64_t* reg, uint32_t nreg, InstRec& r,
+                                 Box& b, uint32_t* status) {
+    rtg_instance in = inst[i];
+    const AsHeader* bh = checked_blas(in, reg, nreg, status);
+    b = instance_world_box(in, bh);
+    fill_inst_rec(r, in, i, bh ? in.acceleration_structure_reference : 0);
+}
+
 __global__ __launch_bounds__(256) void k_inst_setup(const rtg_instance* inst, uint32_t n, const uint64_t* reg,
                                                     uint32_t nreg, InstRec* recs, Box* boxes, uint32_t* cb,
                                                     uint32_t* status) {
@@ -261,11 +262,9 @@ __global__ __launch_bounds__(256) void k_inst_setup(const rtg_instance* inst, ui
     float c[3] = {0, 0, 0};
     bool valid[3] = {false, false, false};
     if (i < n) {
-        rtg_instance in = inst[i];
-        const AsHeader* bh = checked_blas(in, reg, nreg, status);
-        Box b = instance_world_box(in, bh);
         InstRec r;
-        fill_inst_rec(r, in, i, bh ? in.acceleration_structure_reference : 0);
+        Box b;
+        make_inst(inst, i, reg, nreg, r, b, status);
         recs[i] = r;
         boxes[i] = b;
 #pragma unroll
@@ -292,20 +291,25 @@ __device__ inline uint32_t quantize10(float c, float lo, float hi) {
     return (uint32_t)q;
 }
 
-__global__ __launch_bounds__(256) void k_morton(const Box* boxes, uint32_t n, const uint32_t* cb, uint32_t* keys,
-                                                uint32_t* vals) {
-    uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    float lo[3], hi[3];
+__device__ inline void bounds_from_words(const uint32_t* cb, float lo[3], float hi[3]) {
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         lo[a] = cb[a] == 0xffffffffu ? __builtin_inff() : ord2f(cb[a]);
         hi[a] = cb[3 + a] == 0u ? -__builtin_inff() : ord2f(cb[3 + a]);
     }
-    Box b = boxes[i];
-    uint32_t k = (spread3(quantize10(centre(b, 0), lo[0], hi[0])) << 2) |
-                 (spread3(quantize10(centre(b, 1), lo[1], hi[1])) << 1) | spread3(quantize10(centre(b, 2), lo[2], hi[2]));
-    keys[i] = k;
+}
+__device__ inline uint32_t morton(const Box& b, const float lo[3], const float hi[3]) {
+    return (spread3(quantize10(centre(b, 0), lo[0], hi[0])) << 2) |
+           (spread3(quantize10(centre(b, 1), lo[1], hi[1])) << 1) | spread3(quantize10(centre(b, 2), lo[2], hi[2]));
+}
+
+__global__ __launch_bounds__(256) void k_morton(const Box* boxes, uint32_t n, const uint32_t* cb, uint32_t* keys,
+                                                uint32_t* vals) {
+    uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    float lo[3], hi[3];
+    bounds_from_words(cb, lo, hi);
+    keys[i] = morton(boxes[i], lo, hi);
     vals[i] = i;
 }
 
@@ -327,41 +331,44 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_hist(const uint32_t* keys, ui
         if (i < n) atomicAdd(&h[(keys[i] >> shift) & 0xffu], 1u);
     }
     __syncthreads();
-    hist[threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
+    hist[(size_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
 }
 
-// Exclusive scan of m entries in one block of 1024 threads.
-__global__ __launch_bounds__(1024) void k_scan_exclusive(uint32_t* data, uint32_t m) {
-    __shared__ uint32_t part[1024];
-    uint32_t chunk = (m + 1023) / 1024;
-    uint32_t b = threadIdx.x * chunk, e = min(m, b + chunk);
-    uint32_t s = 0;
-    for (uint32_t i = b; i < e; ++i) s += data[i];
-    part[threadIdx.x] = s;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        uint32_t v = threadIdx.x >= (uint32_t)off ? part[threadIdx.x - off] : 0u;
-        __syncthreads();
-        part[threadIdx.x] += v;
-        __syncthreads();
+// Exclusive scan of each digit's counts over the tiles (one workgroup per
+// digit) and the digits' totals.
+__global__ __launch_bounds__(256) void k_rs_scan(uint32_t* hist, uint32_t ntiles, uint32_t* totals) {
+    __shared__ uint32_t part[4];
+    uint32_t* row = hist + (size_t)blockIdx.x * ntiles;
+    uint32_t run = 0;
+    for (uint32_t b = 0; b < ntiles; b += 256) {
+        const uint32_t i = b + threadIdx.x;
+        const uint32_t v = i < ntiles ? row[i] : 0u;
+        uint32_t total;
+        const uint32_t incl = block_scan<256>(v, part, total);
+        if (i < ntiles) row[i] = run + incl - v;
+        run += total;
     }
-    uint32_t run = part[threadIdx.x] - s;
-    for (uint32_t i = b; i < e; ++i) {
-        uint32_t v = data[i];
-        data[i] = run;
-        run += v;
-    }
+    if (threadIdx.x == 0) totals[blockIdx.x] = run;
 }
 
 __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const uint32_t* kin, const uint32_t* vin, uint32_t* kout,
                                                            uint32_t* vout, uint32_t n, int shift,
-                                                           const uint32_t* offsets, uint32_t ntiles) {
+                                                           const uint32_t* offsets, uint32_t ntiles,
+                                                           const uint32_t* totals) {
     constexpr int kWaves = kRsThreads / 64;
+    static_assert(kRsThreads == 256, "a thread per digit");
+    __shared__ uint32_t part[kWaves];
     __shared__ uint32_t base_off[256];
     __shared__ uint32_t running[256];
     __shared__ uint32_t wave_cnt[kWaves][256];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    base_off[threadIdx.x] = offsets[threadIdx.x * ntiles + blockIdx.x];
+    {
+        // first position of each digit: the totals of the digits below it
+        const uint32_t mine = totals[threadIdx.x];
+        uint32_t all;
+        base_off[threadIdx.x] =
+            block_scan<256>(mine, part, all) - mine + offsets[(size_t)threadIdx.x * ntiles + blockIdx.x];
+    }
     running[threadIdx.x] = 0;
     for (int k = 0; k < kWaves; ++k) wave_cnt[k][threadIdx.x] = 0;
     __syncthreads();
@@ -415,10 +422,9 @@ __device__ inline int delta(const uint32_t* keys, int n, int i, int j) {
     return __clz((int)(a ^ b));
 }
 
-__global__ __launch_bounds__(256) void k_karras(const uint32_t* keys, int n, uint32_t* left, uint32_t* right,
-                                                uint32_t* parent, uint32_t* rfirst, uint32_t* rcount) {
-    int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n - 1) return;
+// Internal node i of the radix tree over sorted codes: its children's
+// references, primitive counts, and its own count.
+__device__ inline uint32_t radix_node(const uint32_t* keys, int n, int i, uint32_t child[2], uint32_t count[2]) {
     int d = (delta(keys, n, i, i + 1) - delta(keys, n, i, i - 1)) >= 0 ? 1 : -1;
     int dmin = delta(keys, n, i, i - d);
     int lmax = 2;
@@ -436,246 +442,238 @@ __global__ __launch_bounds__(256) void k_karras(const uint32_t* keys, int n, uin
     } while (t > 1);
     int gamma = i + s * d + (d < 0 ? d : 0);
     int lo = min(i, j), hi = max(i, j);
-    uint32_t lc = (lo == gamma) ? (kLeafBit | (uint32_t)gamma) : (uint32_t)gamma;
-    uint32_t rc = (hi == gamma + 1) ? (kLeafBit | (uint32_t)(gamma + 1)) : (uint32_t)(gamma + 1);
-    left[i] = lc;
-    right[i] = rc;
-    rfirst[i] = (uint32_t)lo;
-    rcount[i] = (uint32_t)(hi - lo + 1);
-    // parent array: internal nodes at [0, n-1), leaves at [n-1, 2n-1)
-    parent[(lc & kLeafBit) ? (n - 1) + (lc & kFirstMask) : lc] = (uint32_t)i;
-    parent[(rc & kLeafBit) ? (n - 1) + (rc & kFirstMask) : rc] = (uint32_t)i;
-    if (i == 0) parent[0] = 0xffffffffu;
+    child[0] = (lo == gamma) ? (kLeafBit | (uint32_t)gamma) : (uint32_t)gamma;
+    child[1] = (hi == gamma + 1) ? (kLeafBit | (uint32_t)(gamma + 1)) : (uint32_t)(gamma + 1);
+    count[0] = (uint32_t)(gamma - lo + 1);
+    count[1] = (uint32_t)(hi - gamma);
+    return (uint32_t)(hi - lo + 1);
 }
 
-// Depth of every internal node of the binary tree (the root has depth 0),
-// by walking its parent chain; the largest depth is folded into *max_depth.
-__global__ __launch_bounds__(256) void k_node_depth(int n, const uint32_t* parent, uint32_t* depth,
-                                                    uint32_t* max_depth) {
+// The radix tree, the leaf boxes in sorted order and the first pass's tiers.
+__global__ __launch_bounds__(256) void k_karras(const uint32_t* keys, int n, const uint32_t* order, const Box* boxes,
+                                                Box* lbox, BinNode* bin, uint32_t* rcount, uint32_t* low,
+                                                uint32_t* mid, uint32_t* counts) {
     int i = blockIdx.x * 256 + threadIdx.x;
-    uint32_t d = 0;
-    if (i < n - 1) {
-        for (uint32_t p = parent[i]; p != 0xffffffffu; p = parent[p]) ++d;
-        depth[i] = d;
-    }
-    for (int off = 32; off > 0; off >>= 1) d = max(d, (uint32_t)__shfl_xor((int)d, off));
-    if ((threadIdx.x & 63) == 0 && d) atomicMax(max_depth, d);
-}
-
-// Boxes and surface areas of the internal nodes at depth `d` (the deeper
-// ones are done).
-__global__ __launch_bounds__(256) void k_boxes_level(uint32_t d, const uint32_t* depth, const Box* boxes,
-                                                     const uint32_t* order, int n, const uint32_t* left,
-                                                     const uint32_t* right, Box* ibox, float* area) {
-    int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n - 1 || depth[i] != d) return;
-    uint32_t c[2] = {left[i], right[i]};
-    Box cbx[2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) cbx[s] = (c[s] & kLeafBit) ? boxes[order[c[s] & kFirstMask]] : ibox[c[s]];
-    Box u = box_union(cbx[0], cbx[1]);
-    ibox[i] = u;
-    area[i] = box_area(u);
-}
-
-// ---------------------------------------------------------------------------
-// Treelet restructuring (Karras & Aila 2013, HPG, "Fast Parallel
-// Construction of High-Quality Bounding Volume Hierarchies", section 4) of
-// the binary tree, for single-primitive leaves. The treelet of internal node
-// r: r's two children, then, while fewer than kTreeletLeaves, the treelet
-// leaf with the largest area that is an internal node replaced by its left
-// child in place and its right child appended. Its topology becomes the one
-// that minimises the summed surface area of its internal nodes (SAH cost with
-// fixed leaves), by dynamic programming over subsets of treelet leaves:
-// cost(S) = area(S) + min over partitions (P, S\P), P holding S's lowest
-// leaf, of cost(P) + cost(S\P); partitions tried in decreasing order of P,
-// the first minimum kept. New internal nodes reuse the treelet's numbers:
-// r for the whole set, then the expanded nodes in expansion order, handed
-// out as subsets are split from a stack (P's subtree first). A node is
-// processed after its whole subtree (arrival counters), so the result does
-// not depend on thread timing.
-// ---------------------------------------------------------------------------
-constexpr int kTreeletLeaves = 7;
-constexpr int kTreeletRounds = 5;  // passes with RTG_BUILD_PREFER_FAST_TRACE
-
-__device__ inline Box bin_box(const Box* boxes, const uint32_t* order, const Box* ibox, uint32_t c) {
-    return (c & kLeafBit) ? boxes[order[c & kFirstMask]] : ibox[c];
-}
-
-// The cheapest split of leaf set S: the partition (P, S \ P) with P holding
-// S's lowest leaf that minimises cost(P) + cost(S \ P), partitions tried in
-// decreasing order of P and the first minimum kept. P = low | Q for Q a
-// proper submask of S \ low (2^m - 1 of them for m bits), and decreasing Q is
-// decreasing P. Four partitions at a time, so that their LDS reads are in
-// flight together; the comparisons stay in order.
-__device__ inline uint32_t best_split(uint32_t S, const float* cost, int stride, float& best) {
-    const uint32_t low = S & (0u - S), R = S ^ low;
-    const uint32_t count = (1u << __builtin_popcount(R)) - 1u;
-    uint32_t Q = (R - 1u) & R;
-    uint32_t bp = 0;
-    best = 0.0f;
-    uint32_t i = 0;
-    for (; i + 4u <= count; i += 4u) {
-        uint32_t P[4];
-        float c[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            P[j] = Q | low;
-            c[j] = cost[P[j] * stride] + cost[(S ^ P[j]) * stride];
-            Q = (Q - 1u) & R;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (bp == 0 || c[j] < best) {
-                best = c[j];
-                bp = P[j];
-            }
-    }
-    for (; i < count; ++i) {
-        const uint32_t P = Q | low;
-        const float c = cost[P * stride] + cost[(S ^ P) * stride];
-        if (bp == 0 || c < best) {
-            best = c;
-            bp = P;
-        }
-        Q = (Q - 1u) & R;
-    }
-    return bp;
-}
-
-// `cost` is this lane's column of a per-workgroup LDS table (entry S at
-// cost[S * stride]); LDS keeps the dynamic programme's 2^7 subset costs
-// close, where a per-lane array would live in scratch memory.
-__device__ void treelet_optimize(uint32_t r, const Box* boxes, const uint32_t* order, uint32_t* left,
-                                 uint32_t* right, uint32_t* rcount, Box* ibox, float* area, float* cost,
-                                 int stride) {
-    uint32_t leaf[kTreeletLeaves], inner[kTreeletLeaves];
-    int nl = 2, ni = 0;
-    leaf[0] = left[r];
-    leaf[1] = right[r];
-    while (nl < kTreeletLeaves) {
-        int best = -1;
-        float best_area = 0.0f;
-        for (int k = 0; k < nl; ++k) {
-            const uint32_t c = leaf[k];
-            if (c & kLeafBit) continue;
-            const float a = area[c];
-            if (best < 0 || a > best_area) {
-                best = k;
-                best_area = a;
-            }
-        }
-        if (best < 0) break;
-        const uint32_t c = leaf[best];
-        inner[ni++] = c;
-        leaf[best] = left[c];
-        leaf[nl++] = right[c];
-    }
-    if (nl < 3) return;
-    // leaf boxes in registers: the loops over them are unrolled to constant
-    // indices (set bits of S beyond nl never occur)
-    Box lb[kTreeletLeaves];
-#pragma unroll
-    for (int k = 0; k < kTreeletLeaves; ++k) lb[k] = k < nl ? bin_box(boxes, order, ibox, leaf[k]) : box_empty();
-    const uint32_t full = (1u << nl) - 1u;
-    for (uint32_t Sl = 1; Sl <= full; ++Sl) {
-        // lanes go through the sets in step (lanes past their `full` have
-        // left the loop), so S is uniform: its table reads are scalar
-        const uint32_t S = (uint32_t)__builtin_amdgcn_readfirstlane((int)Sl);
-        if ((S & (S - 1u)) == 0) {
-            cost[S * stride] = 0.0f;
-            continue;
-        }
-        Box b = box_empty();
-#pragma unroll
-        for (int k = 0; k < kTreeletLeaves; ++k)
-            if (S & (1u << k)) b = box_union(b, lb[k]);
-        float best;
-        best_split(S, cost, stride, best);
-        cost[S * stride] = box_area(b) + best;
-    }
-    uint32_t stk_set[kTreeletLeaves], stk_id[kTreeletLeaves], done[kTreeletLeaves];
-    int sp = 0, no = 0, next = 0;
-    stk_set[sp] = full;
-    stk_id[sp++] = r;
-    while (sp > 0) {
-        --sp;
-        const uint32_t S = stk_set[sp], id = stk_id[sp];
-        done[no++] = id;
-        float unused;
-        const uint32_t P = best_split(S, cost, stride, unused);
-        const uint32_t part[2] = {P, S ^ P};
-        uint32_t ref[2];
-        for (int h = 0; h < 2; ++h)
-            ref[h] = (part[h] & (part[h] - 1u)) ? inner[next++] : leaf[__builtin_ctz(part[h])];
-        left[id] = ref[0];
-        right[id] = ref[1];
-        for (int h = 1; h >= 0; --h)
-            if (part[h] & (part[h] - 1u)) {
-                stk_set[sp] = part[h];
-                stk_id[sp++] = ref[h];
-            }
-    }
-    for (int k = no - 1; k >= 0; --k) {
-        const uint32_t id = done[k], c0 = left[id], c1 = right[id];
-        const Box u = box_union(bin_box(boxes, order, ibox, c0), bin_box(boxes, order, ibox, c1));
-        ibox[id] = u;
-        area[id] = box_area(u);
-        rcount[id] = ((c0 & kLeafBit) ? 1u : rcount[c0]) + ((c1 & kLeafBit) ? 1u : rcount[c1]);
-    }
-}
-
-// One depth level of a pass: every internal node at depth `d` of the tree
-// the pass started from. Launched from the deepest level up, so a node is
-// restructured after its whole subtree; nodes of one level have disjoint
-// subtrees, and a restructured subtree keeps its node set, so the result is
-// the one of any order that visits subtrees first.
-constexpr int kTreeletThreads = 64;
-
-// Restructures the `count` internal nodes of one depth level listed in
-// `nodes` (the level's run of the nodes sorted by depth), so that every
-// workgroup is full of treelets.
-__global__ __launch_bounds__(kTreeletThreads) void k_treelet_level(const uint32_t* nodes, uint32_t count,
-                                                                   const Box* boxes, const uint32_t* order,
-                                                                   uint32_t* left, uint32_t* right, uint32_t* rcount,
-                                                                   Box* ibox, float* area) {
-    __shared__ float s_cost[(1 << kTreeletLeaves) * kTreeletThreads];
-    uint32_t k = blockIdx.x * kTreeletThreads + threadIdx.x;
-    if (k >= count) return;
-    treelet_optimize(nodes[k], boxes, order, left, right, rcount, ibox, area, s_cost + threadIdx.x,
-                     kTreeletThreads);
-}
-
-__global__ __launch_bounds__(256) void k_iota(uint32_t* p, uint32_t n) {
-    uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) p[i] = i;
-}
-
-// First position of each depth in the depth-sorted node list: where the
-// depth differs from its predecessor's. Every depth from 0 to the tree's
-// depth holds a node (the ancestors of a deepest one); the entry past the
-// deepest is the list length, filled beforehand.
-__global__ __launch_bounds__(256) void k_level_starts(const uint32_t* sorted_depth, uint32_t m, uint32_t* start) {
-    uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= m) return;
-    const uint32_t d = sorted_depth[i];
-    if (i == 0 || sorted_depth[i - 1] != d) start[d] = i;
-}
-
-// Parents of the restructured tree (the root keeps none).
-__global__ __launch_bounds__(256) void k_parents(int n, const uint32_t* left, const uint32_t* right,
-                                                 uint32_t* parent) {
-    int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) lbox[i] = boxes[order[i]];
     if (i >= n - 1) return;
-    const uint32_t lc = left[i], rc = right[i];
-    parent[(lc & kLeafBit) ? (n - 1) + (lc & kFirstMask) : lc] = (uint32_t)i;
-    parent[(rc & kLeafBit) ? (n - 1) + (rc & kFirstMask) : rc] = (uint32_t)i;
+    uint32_t child[2], count[2];
+    const uint32_t c = radix_node(keys, n, i, child, count);
+    bin[i] = BinNode{child[0], child[1], 0.0f, 0.0f};
+    rcount[i] = c;
+    tier_roots((uint32_t)i, c, child, count, low, mid, counts);
+}
+
+// ---------------------------------------------------------------------------
+// Up to kSmallBuild primitives: one workgroup makes the records, sorts the
+// codes in LDS and writes the binary tree. A launch of many workgroups per
+// step would be 15 launches of 2 to 5 us each, whatever the count.
+// ---------------------------------------------------------------------------
+constexpr uint32_t kSmallBuild = 8192;
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallWaves = kSmallThreads / 64;
+constexpr int kSmallItems = kSmallBuild / kSmallThreads;
+
+struct SmallSort {
+    uint32_t key[kSmallBuild];
+    uint16_t val[kSmallBuild];
+    uint16_t cnt[kSmallWaves][256];
+    uint32_t part[kSmallWaves];
+    uint32_t bounds[8];
+    uint32_t tiers[2];
+};
+
+struct SmallOut {
+    Box* boxes;
+    Box* lbox;
+    uint32_t* order;
+    BinNode* bin;
+    uint32_t* rcount;
+    uint32_t *low, *mid, *counts, *cb;
+};
+
+// Centre bounds of this thread's primitives, folded over the workgroup.
+struct CentreBounds {
+    uint32_t lo[3], hi[3];
+    __device__ inline CentreBounds() {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            lo[a] = 0xffffffffu;
+            hi[a] = 0u;
+        }
+    }
+    __device__ inline void add(const Box& b) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const float c = centre(b, a);
+            if (!isfinite(c)) continue;
+            lo[a] = min(lo[a], f2ord(c));
+            hi[a] = max(hi[a], f2ord(c));
+        }
+    }
+};
+
+__device__ inline void small_tree(SmallSort& Z, uint32_t n, const CentreBounds& cb, const SmallOut& O) {
+    const uint32_t t = threadIdx.x, lane = t & 63, w = t >> 6;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        uint32_t l = cb.lo[a], h = cb.hi[a];
+        for (int off = 32; off > 0; off >>= 1) {
+            l = min(l, (uint32_t)__shfl_xor((int)l, off));
+            h = max(h, (uint32_t)__shfl_xor((int)h, off));
+        }
+        if (lane == 0) {
+            atomicMin(&Z.bounds[a], l);
+            atomicMax(&Z.bounds[3 + a], h);
+        }
+    }
+    __syncthreads();
+    // wave w holds positions [w * 64 J, (w + 1) * 64 J) of every pass
+    const uint32_t J = (n + kSmallThreads - 1) / kSmallThreads;
+    const uint32_t first = w * 64 * J + lane;
+    uint32_t key[kSmallItems], val[kSmallItems], rank[kSmallItems];
+    {
+        float lo[3], hi[3];
+        bounds_from_words(Z.bounds, lo, hi);
+#pragma unroll
+        for (uint32_t j = 0; j < (uint32_t)kSmallItems; ++j) {
+            const uint32_t p = first + j * 64;
+            key[j] = val[j] = 0;
+            if (j < J && p < n) {
+                key[j] = morton(O.boxes[p], lo, hi);
+                val[j] = p;
+            }
+        }
+    }
+    const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    for (int shift = 0; shift < 32; shift += 8) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) Z.cnt[w][lane + 64 * k] = 0;
+        wave_order();
+#pragma unroll
+        for (uint32_t j = 0; j < (uint32_t)kSmallItems; ++j) {
+            if (j >= J) break;
+            const bool valid = first + j * 64 < n;
+            const uint32_t digit = (key[j] >> shift) & 0xffu;
+            uint64_t peers = __ballot(valid);
+#pragma unroll
+            for (int bit = 0; bit < 8; ++bit) {
+                const uint64_t bal = __ballot((digit >> bit) & 1u);
+                peers &= ((digit >> bit) & 1u) ? bal : ~bal;
+            }
+            const uint32_t before = (uint32_t)__popcll(peers & lt);
+            uint32_t run = 0;
+            if (valid) run = Z.cnt[w][digit];
+            rank[j] = run + before;
+            wave_order();
+            if (valid && before == 0) Z.cnt[w][digit] = (uint16_t)(run + (uint32_t)__popcll(peers));
+            wave_order();
+        }
+        __syncthreads();
+        {
+            // exclusive scan over (digit, wave): four waves' counts per thread
+            const uint32_t d = t >> 2, w0 = (t & 3u) * 4;
+            uint32_t c[4], sum = 0, total;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                c[k] = Z.cnt[w0 + k][d];
+                sum += c[k];
+            }
+            uint32_t run = block_scan<kSmallThreads>(sum, Z.part, total) - sum;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                Z.cnt[w0 + k][d] = (uint16_t)run;
+                run += c[k];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t j = 0; j < (uint32_t)kSmallItems; ++j) {
+            if (j >= J) break;
+            if (first + j * 64 < n) {
+                const uint32_t dst = Z.cnt[w][(key[j] >> shift) & 0xffu] + rank[j];
+                Z.key[dst] = key[j];
+                Z.val[dst] = (uint16_t)val[j];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t j = 0; j < (uint32_t)kSmallItems; ++j) {
+            if (j >= J) break;
+            const uint32_t p = first + j * 64;
+            if (p < n) {
+                key[j] = Z.key[p];
+                val[j] = Z.val[p];
+            }
+        }
+        // the next pass writes Z.key and Z.val only after two barriers
+    }
+    for (uint32_t j = 0; j < J; ++j) {
+        const uint32_t p = first + j * 64;
+        if (p < n) {
+            const uint32_t v = Z.val[p];
+            O.order[p] = v;
+            O.lbox[p] = O.boxes[v];
+        }
+        if (p + 1 < n) {
+            uint32_t child[2], count[2];
+            const uint32_t c = radix_node(Z.key, (int)n, (int)p, child, count);
+            O.bin[p] = BinNode{child[0], child[1], 0.0f, 0.0f};
+            O.rcount[p] = c;
+            tier_roots(p, c, child, count, O.low, O.mid, Z.tiers);
+        }
+    }
+    __syncthreads();
+    if (t < 2) O.counts[t] = Z.tiers[t];
+}
+
+__device__ inline void small_init(SmallSort& Z) {
+    if (threadIdx.x < 8) Z.bounds[threadIdx.x] = threadIdx.x < 3 ? 0xffffffffu : 0u;
+    if (threadIdx.x < 2) Z.tiers[threadIdx.x] = 0;
+    __syncthreads();
+}
+
+__global__ __launch_bounds__(kSmallThreads) void k_small_tris(const GeomDesc* geoms, uint32_t ngeom, uint32_t n,
+                                                              TriRec* tris, SmallOut O, uint32_t* status) {
+    __shared__ SmallSort Z;
+    small_init(Z);
+    CentreBounds cb;
+    for (uint32_t i = threadIdx.x; i < n; i += kSmallThreads) {
+        TriRec r;
+        Box b;
+        make_tri(geoms, ngeom, i, r, b, status);
+        tris[i] = r;
+        O.boxes[i] = b;
+        if (box_has_nan(b)) atomicOr(&O.cb[6], 1u);
+        cb.add(b);
+    }
+    small_tree(Z, n, cb, O);
+}
+
+__global__ __launch_bounds__(kSmallThreads) void k_small_insts(const rtg_instance* inst, uint32_t n,
+                                                               const uint64_t* reg, uint32_t nreg, InstRec* recs,
+                                                               SmallOut O, uint32_t* status) {
+    __shared__ SmallSort Z;
+    small_init(Z);
+    CentreBounds cb;
+    for (uint32_t i = threadIdx.x; i < n; i += kSmallThreads) {
+        InstRec r;
+        Box b;
+        make_inst(inst, i, reg, nreg, r, b, status);
+        recs[i] = r;
+        O.boxes[i] = b;
+        cb.add(b);
+    }
+    small_tree(Z, n, cb, O);
 }
 
 // The single node of a structure with at most leaf_max primitives: one leaf
 // of all of them in input order (or none).
-__global__ void k_wide_single(const Box* boxes, uint32_t n, Node* nodes, uint32_t* order) {
+__global__ void k_wide_single(const Box* boxes, uint32_t n, Node* nodes, uint32_t* order, uint32_t* off,
+                              CollapseState* state) {
     if (threadIdx.x == 0) {
+        off[0] = 0;
+        off[1] = 1;
+        *state = CollapseState{1u, 1u, 1u, 0u};
         Node nd;
         const uint32_t ref = n ? (kLeafBit | ((n - 1) << 27)) : kEmpty;
 #pragma unroll
@@ -689,80 +687,8 @@ __global__ void k_wide_single(const Box* boxes, uint32_t n, Node* nodes, uint32_
     for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) order[k] = k;
 }
 
-// Slots (binary refs) of each wide node of a level: the binary root's two
-// children, then the largest-area openable slot replaced in place by its
-// two children while fewer than four; and the number of slots that become
-// wide nodes of the next level.
-__global__ __launch_bounds__(256) void k_wide_expand(uint32_t lb, uint32_t m, const uint32_t* wroot,
-                                                     const uint32_t* left, const uint32_t* right,
-                                                     const uint32_t* rcount, const float* area, uint32_t leaf_max,
-                                                     uint4* slots, uint32_t* cnt) {
-    uint32_t w = blockIdx.x * 256 + threadIdx.x;
-    if (w >= m) return;
-    uint32_t r = wroot[lb + w];
-    uint32_t s[4] = {left[r], right[r], kEmpty, kEmpty};
-    int nslot = 2;
-    while (nslot < 4) {
-        int best = -1;
-        float best_area = 0.0f;
-        for (int k = 0; k < nslot; ++k) {
-            uint32_t c = s[k];
-            if ((c & kLeafBit) || rcount[c] <= leaf_max) continue;
-            float a = area[c];
-            if (best < 0 || a > best_area) {
-                best = k;
-                best_area = a;
-            }
-        }
-        if (best < 0) break;
-        uint32_t c = s[best];
-        for (int k = nslot; k > best + 1; --k) s[k] = s[k - 1];
-        s[best] = left[c];
-        s[best + 1] = right[c];
-        ++nslot;
-    }
-    uint32_t internal = 0;
-    for (int k = 0; k < nslot; ++k) internal += (!(s[k] & kLeafBit) && rcount[s[k]] > leaf_max) ? 1u : 0u;
-    slots[w] = make_uint4(s[0], s[1], s[2], s[3]);
-    cnt[w] = internal;
-}
-
-// Child refs of each wide node of a level; opened slots get the next
-// level's node numbers from the exclusive prefix sum `base` (node le + base).
-__global__ __launch_bounds__(256) void k_wide_emit(uint32_t lb, uint32_t le, uint32_t m, const uint4* slots,
-                                                   const uint32_t* base, const uint32_t* rfirst,
-                                                   const uint32_t* rcount, uint32_t leaf_max, uint32_t cap,
-                                                   Node* nodes, uint32_t* wroot, uint32_t* next_count) {
-    uint32_t w = blockIdx.x * 256 + threadIdx.x;
-    if (w >= m) return;
-    uint4 sv = slots[w];
-    uint32_t s[4] = {sv.x, sv.y, sv.z, sv.w};
-    uint32_t next = le + base[w];
-    uint32_t internal = 0;
-    Node& nd = nodes[lb + w];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        uint32_t c = s[k], ref = kEmpty;
-        if (c != kEmpty) {
-            if (c & kLeafBit) {
-                ref = c;
-            } else if (rcount[c] <= leaf_max) {
-                ref = kLeafBit | ((rcount[c] - 1u) << 27) | rfirst[c];
-            } else {
-                // a wide tree over n leaves has at most n - 1 nodes (each has
-                // two or more slots); the host checks the count against cap
-                ref = next;
-                if (next < cap) wroot[next] = c;
-                ++next;
-                ++internal;
-            }
-        }
-        nd.child[k] = ref;
-    }
-    if (w == m - 1) *next_count = base[w] + internal;
-}
-
-// Slot boxes of the wide nodes of a level (the levels below are done).
+// Slot boxes of the wide nodes of a level (the levels below are done): the
+// fold by its definition, for structures with a NaN box plane.
 __global__ __launch_bounds__(256) void k_wide_boxes(uint32_t lb, uint32_t m, Node* nodes, const Box* boxes,
                                                     const uint32_t* order) {
     uint32_t w = blockIdx.x * 256 + threadIdx.x;
@@ -775,48 +701,97 @@ __global__ __launch_bounds__(256) void k_wide_boxes(uint32_t lb, uint32_t m, Nod
     }
 }
 
-__global__ void k_header(AsHeader* h, uint32_t kind, uint32_t node_count, uint32_t prim_count, uint32_t geom_count,
-                         uint32_t levels, uint64_t nodes_off, uint64_t prims_off, uint64_t extra_off,
-                         uint64_t level_off, uint64_t leafbox_off, uint64_t total) {
-    if (threadIdx.x != 0) return;
+// Where the parts of a blob lie (bytes from its start).
+struct Layout {
+    uint64_t nodes_off, prims_off, extra_off, level_off, leafbox_off, total;
+    uint32_t node_count;
+};
+
+__device__ inline void write_header(uint8_t* blob, const Layout& L, const Node* nodes, uint32_t kind,
+                                    uint32_t prim_count, uint32_t geom_count, uint32_t levels) {
     AsHeader hd;
     memset(&hd, 0, sizeof(hd));
     hd.magic = kMagic;
     hd.kind = kind;
-    hd.node_count = node_count;
+    hd.node_count = L.node_count;
     hd.prim_count = prim_count;
     hd.geom_count = geom_count;
     hd.max_depth = levels;
     hd.node_width = 4;
     hd.flags = 0;
-    const Node* nodes = reinterpret_cast<const Node*>(reinterpret_cast<const uint8_t*>(h) + nodes_off);
     Box r = node_box(nodes[0]);
     for (int a = 0; a < 3; ++a) {
         hd.lo[a] = r.lo[a];
         hd.hi[a] = r.hi[a];
     }
-    hd.nodes_off = nodes_off;
-    hd.prims_off = prims_off;
-    hd.extra_off = extra_off;
-    hd.level_off = level_off;
-    hd.total_size = total;
-    hd.leafbox_off = leafbox_off;
-    *h = hd;
+    hd.nodes_off = L.nodes_off;
+    hd.prims_off = L.prims_off;
+    hd.extra_off = L.extra_off;
+    hd.level_off = L.level_off;
+    hd.total_size = L.total;
+    hd.leafbox_off = L.leafbox_off;
+    *reinterpret_cast<AsHeader*>(blob) = hd;
 }
 
-__global__ __launch_bounds__(256) void k_gather_tris(const uint32_t* order, const TriRec* in, TriRec* out, uint32_t n) {
-    uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) out[i] = in[order[i]];
+// Copies `bytes` (a multiple of sizeof(T)) over the whole grid, T by T.
+template <class T>
+__device__ inline void grid_copy(void* dst, const void* src, uint64_t bytes) {
+    const uint64_t count = bytes / sizeof(T), step = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < count; i += step)
+        static_cast<T*>(dst)[i] = static_cast<const T*>(src)[i];
 }
-
-__global__ __launch_bounds__(256) void k_gather_insts(const uint32_t* order, const InstRec* in, const Box* boxes,
-                                                      InstRec* out, Box* leafbox, uint32_t n) {
-    uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) {
-        uint32_t s = order[i];
-        out[i] = in[s];
-        leafbox[i] = boxes[s];
+// Records of `words` T each, out[k] = in[order[k]].
+template <class T, uint32_t Words>
+__device__ inline void grid_gather(void* dst, const void* src, const uint32_t* order, uint32_t n) {
+    const uint64_t count = (uint64_t)n * Words, step = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < count; i += step) {
+        const uint32_t k = (uint32_t)(i / Words), w = (uint32_t)(i % Words);
+        static_cast<T*>(dst)[i] = static_cast<const T*>(src)[(uint64_t)order[k] * Words + w];
     }
+}
+// Zeroes the 4-byte words of [from, to) (at most 64 bytes of padding).
+__device__ inline void zero_pad(uint8_t* blob, uint64_t from, uint64_t to) {
+    if (blockIdx.x != 0) return;
+    for (uint64_t o = from + 4ull * threadIdx.x; o < to; o += 4ull * blockDim.x)
+        *reinterpret_cast<uint32_t*>(blob + o) = 0u;
+}
+
+// The blob of a BLAS, and a new version of the registry with its address.
+__global__ __launch_bounds__(256) void k_finish_blas(uint8_t* blob, Layout L, const Node* nodes, const TriRec* tris,
+                                                     const uint32_t* order, const GeomDesc* geoms, uint32_t ngeom,
+                                                     uint32_t n, uint32_t levels, const uint64_t* reg, uint32_t nreg,
+                                                     uint64_t* new_reg) {
+    grid_copy<uint4>(blob + L.nodes_off, nodes, (uint64_t)L.node_count * sizeof(Node));
+    grid_gather<uint4, sizeof(TriRec) / 16>(blob + L.prims_off, tris, order, n);
+    if (blockIdx.x != 0) return;
+    zero_pad(blob, L.prims_off + (uint64_t)n * sizeof(TriRec), L.extra_off);
+    zero_pad(blob, L.extra_off + 4ull * ngeom, L.total);
+    uint32_t* gflags = reinterpret_cast<uint32_t*>(blob + L.extra_off);
+    for (uint32_t g = threadIdx.x; g < ngeom; g += blockDim.x) gflags[g] = geoms[g].flags;
+    if (threadIdx.x == 0) write_header(blob, L, nodes, kKindBlas, n, ngeom, levels);
+    const uint64_t addr = reinterpret_cast<uint64_t>(blob);
+    for (uint32_t k = threadIdx.x; k < nreg; k += blockDim.x) {
+        const uint64_t a = reg[k];
+        new_reg[a < addr ? k : k + 1] = a;
+        if (a < addr && (k + 1 == nreg || reg[k + 1] > addr)) new_reg[k + 1] = addr;
+    }
+    if (threadIdx.x == 0 && (nreg == 0 || reg[0] > addr)) new_reg[0] = addr;
+}
+
+__global__ __launch_bounds__(256) void k_finish_tlas(uint8_t* blob, Layout L, const Node* nodes, const InstRec* recs,
+                                                     const uint32_t* order, const rtg_instance* inst, const Box* lbox,
+                                                     const uint32_t* off, uint32_t n, uint32_t levels) {
+    grid_copy<uint4>(blob + L.nodes_off, nodes, (uint64_t)L.node_count * sizeof(Node));
+    grid_gather<uint4, sizeof(InstRec) / 16>(blob + L.prims_off, recs, order, n);
+    // the caller's records: 8-byte words, their alignment
+    grid_copy<uint64_t>(blob + L.extra_off, inst, (uint64_t)n * sizeof(rtg_instance));
+    grid_copy<uint64_t>(blob + L.leafbox_off, lbox, (uint64_t)n * sizeof(Box));
+    if (blockIdx.x != 0) return;
+    uint32_t* lv = reinterpret_cast<uint32_t*>(blob + L.level_off);
+    for (uint32_t k = threadIdx.x; k < levels + 2; k += blockDim.x) lv[k] = k == 0 ? levels : off[k - 1];
+    zero_pad(blob, L.level_off + 4ull * (levels + 2), L.leafbox_off);
+    zero_pad(blob, L.leafbox_off + (uint64_t)n * sizeof(Box), L.total);
+    if (threadIdx.x == 0) write_header(blob, L, nodes, kKindTlas, n, 0u, levels);
 }
 
 // In-place TLAS UPDATE (src/util_structs.rs:285-357): new instance records,
@@ -869,11 +844,6 @@ __global__ __launch_bounds__(256) void k_tlas_refit(uint8_t* base, const rtg_ins
 static inline uint64_t align64(uint64_t x) { return (x + 63) & ~uint64_t(63); }
 static inline unsigned blocks_for(uint64_t n, unsigned bs) { return (unsigned)((n + bs - 1) / bs); }
 
-struct Layout {
-    uint64_t nodes_off, prims_off, extra_off, level_off, leafbox_off, total;
-    uint32_t node_count;
-};
-
 // Blob layouts for a tree of node_count nodes in `levels` levels.
 static Layout blas_layout(uint32_t n, uint32_t ngeom, uint32_t node_count) {
     Layout L;
@@ -903,208 +873,208 @@ static Layout tlas_layout(uint32_t n, uint32_t node_count, uint32_t levels) {
 // n - 1: every node has two or more slots).
 static inline uint32_t node_cap(uint32_t n) { return n >= 2 ? n - 1 : 1; }
 
-// Scratch needs of the wide-tree build over n primitives.
-static size_t lbvh_scratch_bytes(uint32_t n, size_t rec_bytes) {
-    size_t off = 0;
-    uint32_t ntiles = (n + kRsTile - 1) / kRsTile;
-    uint32_t cap = node_cap(n);
-    carve_size<uint8_t>(off, (size_t)n * rec_bytes);  // unsorted records
-    carve_size<Box>(off, n);                          // primitive boxes
-    carve_size<uint32_t>(off, 8);                     // centre bounds
-    carve_size<uint32_t>(off, n);                     // keys a
-    carve_size<uint32_t>(off, n);                     // keys b
-    carve_size<uint32_t>(off, n);                     // vals a
-    carve_size<uint32_t>(off, n);                     // vals b
-    carve_size<uint32_t>(off, (size_t)256 * std::max(1u, ntiles));
-    carve_size<uint32_t>(off, n);                     // left
-    carve_size<uint32_t>(off, n);                     // right
-    carve_size<uint32_t>(off, 2ull * n);              // parent
-    carve_size<uint32_t>(off, n);                     // arrivals (node depths)
-    carve_size<uint32_t>(off, n);                     // range first
-    carve_size<uint32_t>(off, n);                     // range count
-    carve_size<float>(off, n);                        // binary box areas
-    carve_size<Box>(off, n);                          // binary boxes
-    carve_size<Node>(off, cap);                       // wide nodes
-    carve_size<uint32_t>(off, cap);                   // binary root of each wide node
-    carve_size<uint4>(off, cap);                      // slots of a level
-    carve_size<uint32_t>(off, cap);                   // opened slots per node / prefix sums
-    carve_size<uint32_t>(off, 4 + 257);               // next level size, tree depth, level starts
-    carve_size<GeomDesc>(off, 1);
-    return off + 4096;
-}
-
-struct LbvhBufs {
-    uint8_t* recs;
-    Box* boxes;
-    uint32_t* cb;
-    uint32_t *ka, *kb, *va, *vb, *hist, *left, *right, *parent, *arrivals, *rfirst, *rcount;
-    float* area;
-    Box* ibox;
-    Node* nodes;
-    uint32_t *wroot, *cnt, *next;
-    uint4* slots;
+// Scratch of a build over n primitives (records of rec_bytes each).
+struct BuildBufs {
     GeomDesc* geoms;
+    uint8_t* recs;   // unsorted records
+    Box *boxes, *lbox, *ibox;  // of primitives, of sorted leaves, of binary nodes
+    uint32_t* cb;    // centre bounds and the NaN flag
+    uint32_t *ka, *kb, *va, *vb, *hist, *totals;
+    BinNode* bin;
+    uint32_t *rcount, *low, *mid, *list, *levels, *tiers;
+    Node* nodes;
+    uint32_t *wroot, *off, *sums;
+    uint4* slots;
+    CollapseState* state;
+    size_t bytes;
 };
 
-static LbvhBufs carve_lbvh(void* base, uint32_t n, size_t rec_bytes, uint32_t ngeom = 1) {
+constexpr uint32_t kCollapseSteps = 12;  // levels launched between two looks at the collapse's progress
+
+static BuildBufs carve_build(void* base, uint32_t n, size_t rec_bytes, uint32_t ngeom) {
     Carve c(base);
-    LbvhBufs b;
+    BuildBufs b;
+    const uint32_t ntiles = std::max(1u, (n + kRsTile - 1) / kRsTile), cap = node_cap(n);
     b.geoms = c.take<GeomDesc>(std::max(1u, ngeom));
-    uint32_t ntiles = (n + kRsTile - 1) / kRsTile;
-    uint32_t cap = node_cap(n);
     b.recs = c.take<uint8_t>((size_t)n * rec_bytes);
     b.boxes = c.take<Box>(n);
+    b.lbox = c.take<Box>(n);
+    b.ibox = c.take<Box>(n);
     b.cb = c.take<uint32_t>(8);
     b.ka = c.take<uint32_t>(n);
     b.kb = c.take<uint32_t>(n);
-    b.va = c.take<uint32_t>(n);
+    b.va = c.take<uint32_t>(std::max(1u, n));
     b.vb = c.take<uint32_t>(n);
-    b.hist = c.take<uint32_t>((size_t)256 * std::max(1u, ntiles));
-    b.left = c.take<uint32_t>(n);
-    b.right = c.take<uint32_t>(n);
-    b.parent = c.take<uint32_t>(2ull * n);
-    b.arrivals = c.take<uint32_t>(n);
-    b.rfirst = c.take<uint32_t>(n);
+    b.hist = c.take<uint32_t>((size_t)256 * ntiles);
+    b.totals = c.take<uint32_t>(256);
+    b.bin = c.take<BinNode>(n);
     b.rcount = c.take<uint32_t>(n);
-    b.area = c.take<float>(n);
-    b.ibox = c.take<Box>(n);
+    b.low = c.take<uint32_t>(n);
+    b.mid = c.take<uint32_t>(n / kTierLow + 2);
+    b.list = c.take<uint32_t>(n);
+    b.levels = c.take<uint32_t>(n);
+    b.tiers = c.take<uint32_t>(kTierCounters);
     b.nodes = c.take<Node>(cap);
     b.wroot = c.take<uint32_t>(cap);
     b.slots = c.take<uint4>(cap);
-    b.cnt = c.take<uint32_t>(cap);
-    b.next = c.take<uint32_t>(4 + 257);
+    b.off = c.take<uint32_t>((size_t)cap + kCollapseSteps + 8);
+    b.sums = c.take<uint32_t>(kWideBlocks);
+    b.state = c.take<CollapseState>(1);
+    b.bytes = c.off + 4096;
     return b;
 }
 
-// Sorts the primitives, builds the binary radix tree and collapses it into
-// the wide tree in b.nodes. On return the leaf order is in b.va and
-// level_off holds the level offsets (level_off.back() = node count). Reads
-// each level's size back from the device (synchronises `s`).
-static int wide_hierarchy(LbvhBufs& b, uint32_t n, uint32_t leaf_max, int treelet_rounds, hipStream_t s,
-                          std::vector<uint32_t>& level_off) {
-    level_off.assign(1, 0u);
-    if (n <= leaf_max || n <= 1) {
-        hipLaunchKernelGGL(k_wide_single, dim3(1), dim3(256), 0, s, b.boxes, n, b.nodes, b.va);
-        RTG_HIP(hipGetLastError());
-        level_off.push_back(1u);
-        return RTG_OK;
+static size_t build_scratch_bytes(uint32_t n, size_t rec_bytes, uint32_t ngeom) {
+    return carve_build(nullptr, n, rec_bytes, ngeom).bytes;
+}
+
+// One bottom-up pass (boxes, with treelets when OPT) over the tiers whose
+// roots `tiers` counts.
+template <bool OPT>
+static void launch_pass(const BuildBufs& b, uint32_t n, uint32_t* tiers, int rounds, hipStream_t s) {
+    // a bottom subtree holds 170 of at most 256 primitives on average; the
+    // grid loops, so that the count can stay on the device
+    const unsigned low_grid = std::min(std::max(1u, n / 96), 8192u);
+    hipLaunchKernelGGL((k_tree_bottom<OPT>), dim3(low_grid), dim3(kBottomThreads), 0, s, b.bin, b.ibox, b.rcount,
+                       b.lbox, b.low, tiers, rounds);
+    const GlobalTree T{b.bin, b.ibox, b.rcount, b.lbox};
+    if (n > kTierLow) {
+        const unsigned mid_grid = n > kTierHigh ? std::min(n / kTierLow, 1024u) : 1u;
+        hipLaunchKernelGGL((k_tree_upper<OPT>), dim3(mid_grid), dim3(kUpperThreads), 0, s, T, b.mid, tiers + 1,
+                           kTierLow, n, b.list, b.levels, tiers + 2);
     }
+    if (n > kTierHigh)
+        hipLaunchKernelGGL((k_tree_upper<OPT>), dim3(1), dim3(kUpperThreads), 0, s, T, b.tiers + kTopRoot,
+                           b.tiers + kTopCount, kTierHigh, n, b.list, b.levels, tiers + 3);
+}
+
+// From the binary radix tree (n > 1) to the wide nodes in b.nodes; the level
+// offsets are in b.off.
+static int wide_hierarchy(rtg_ctx* ctx, const BuildBufs& b, uint32_t n, int treelet_rounds, hipStream_t s,
+                          BuildReport& rep) {
+    if (treelet_rounds == 0) {
+        launch_pass<false>(b, n, b.tiers, 1, s);
+    } else if (n <= kTierLow) {
+        launch_pass<true>(b, n, b.tiers, treelet_rounds, s);
+    } else {
+        for (int round = 0; round < treelet_rounds; ++round) {
+            uint32_t* tiers = b.tiers + kTierWords * round;
+            if (round > 0)
+                hipLaunchKernelGGL(k_tier_roots, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, n, b.bin, b.rcount,
+                                   b.low, b.mid, tiers);
+            launch_pass<true>(b, n, tiers, 1, s);
+        }
+    }
+    const WideTree W{b.bin, b.ibox, b.lbox, b.nodes, b.wroot, node_cap(n)};
+    // one workgroup emits 1,024 nodes of a level in about 4 us; beyond a few
+    // thousand the two launches over many workgroups are the faster way
+    const bool one = n <= kSmallBuild;
+    hipLaunchKernelGGL(k_collapse_top, dim3(1), dim3(kCollapseThreads), 0, s, W, one ? n : 2048u, b.off, b.state);
+    do {
+        if (!one) {
+            for (uint32_t k = 0; k < kCollapseSteps; ++k) {
+                hipLaunchKernelGGL(k_wide_expand, dim3(kWideBlocks), dim3(256), 0, s, W, b.off, b.state, k, b.slots,
+                                   b.sums);
+                hipLaunchKernelGGL(k_wide_emit, dim3(kWideBlocks), dim3(256), 0, s, W, b.off, b.state, k, b.slots,
+                                   b.sums);
+            }
+            hipLaunchKernelGGL(k_collapse_advance, dim3(1), dim3(64), 0, s, b.off, b.state, kCollapseSteps);
+        }
+        hipLaunchKernelGGL(k_build_report, dim3(1), dim3(64), 0, s, b.state, ctx->d_status, b.cb + 6,
+                           ctx->build_report);
+        RTG_HIP(hipGetLastError());
+        RTG_HIP(hipStreamSynchronize(s));
+        rep = *ctx->build_report;
+    } while (!one && !rep.done);
+    RTG_REQUIRE(rep.done && rep.nodes <= node_cap(n), RTG_ERROR_DEVICE, "BVH collapse: %u nodes, capacity %u",
+                rep.nodes, node_cap(n));
+    if (rep.nan_boxes) {
+        std::vector<uint32_t> off(rep.levels + 1);
+        RTG_HIP(hipMemcpyAsync(off.data(), b.off, off.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        RTG_HIP(hipStreamSynchronize(s));
+        for (uint32_t L = rep.levels; L-- > 0;) {
+            const uint32_t m = off[L + 1] - off[L];
+            hipLaunchKernelGGL(k_wide_boxes, dim3(blocks_for(m, 256)), dim3(256), 0, s, off[L], m, b.nodes, b.boxes,
+                               b.va);
+        }
+        RTG_HIP(hipGetLastError());
+    }
+    return RTG_OK;
+}
+
+// The radix tree over more than kSmallBuild primitives whose boxes and
+// centre bounds are made; the leaf order ends in b.va.
+static void radix_tree(const BuildBufs& b, uint32_t n, hipStream_t s) {
     hipLaunchKernelGGL(k_morton, dim3(blocks_for(n, 256)), dim3(256), 0, s, b.boxes, n, b.cb, b.ka, b.va);
-    uint32_t ntiles = (n + kRsTile - 1) / kRsTile;
+    const uint32_t ntiles = (n + kRsTile - 1) / kRsTile;
     uint32_t *kin = b.ka, *kout = b.kb, *vin = b.va, *vout = b.vb;
     for (int pass = 0; pass < 4; ++pass) {
         int shift = pass * 8;
         hipLaunchKernelGGL(k_rs_hist, dim3(ntiles), dim3(kRsThreads), 0, s, kin, n, shift, b.hist, ntiles);
-        hipLaunchKernelGGL(k_scan_exclusive, dim3(1), dim3(1024), 0, s, b.hist, 256u * ntiles);
+        hipLaunchKernelGGL(k_rs_scan, dim3(256), dim3(256), 0, s, b.hist, ntiles, b.totals);
         hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles), dim3(kRsThreads), 0, s, kin, vin, kout, vout, n, shift, b.hist,
-                           ntiles);
+                           ntiles, b.totals);
         std::swap(kin, kout);
         std::swap(vin, vout);
     }
     // after 4 passes the sorted data is back in (ka, va)
-    hipLaunchKernelGGL(k_karras, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, b.ka, (int)n, b.left, b.right,
-                       b.parent, b.rfirst, b.rcount);
-    // Bottom-up passes go one depth level per launch, deepest first: the
-    // kernel boundaries order the levels, where arrival counters would need
-    // device-scope atomics and fences, which MI355X serves past its per-XCD
-    // L2s. `b.arrivals` holds the depths; the host reads the tree's depth.
-    uint32_t* depth = b.arrivals;
-    uint32_t* max_depth = b.next + 1;
-    auto tree_depth = [&](uint32_t& out) -> int {
-        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, max_depth, 1ull, 0u);
-        hipLaunchKernelGGL(k_node_depth, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, (int)n, b.parent, depth,
-                           max_depth);
-        RTG_HIP(hipGetLastError());
-        RTG_HIP(hipMemcpyAsync(&out, max_depth, 4, hipMemcpyDeviceToHost, s));
-        RTG_HIP(hipStreamSynchronize(s));
-        RTG_REQUIRE(out < n, RTG_ERROR_DEVICE, "BVH build: tree depth %u over %u primitives", out, n);
-        return RTG_OK;
-    };
-    uint32_t dmax = 0;
-    int st = tree_depth(dmax);
-    if (st != RTG_OK) return st;
-    for (uint32_t d = dmax + 1; d-- > 0;)
-        hipLaunchKernelGGL(k_boxes_level, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, d, depth, b.boxes, b.va,
-                           (int)n, b.left, b.right, b.ibox, b.area);
-    // the treelet passes need single-primitive leaves: a restructured
-    // subtree no longer covers a contiguous range of sorted primitives.
-    // Each pass sorts the internal nodes by depth (one 8-bit radix pass:
-    // depth values in b.arrivals, node numbers from b.ka, which the Morton
-    // codes no longer need, into b.kb / b.vb) and restructures each depth's
-    // run with full workgroups, deepest first.
-    const uint32_t m = n - 1;
-    const uint32_t mtiles = (m + kRsTile - 1) / kRsTile;
-    std::vector<uint32_t> start;
-    for (int round = 0; round < treelet_rounds && leaf_max == 1; ++round) {
-        if (round > 0) {
-            st = tree_depth(dmax);
-            if (st != RTG_OK) return st;
-        }
-        RTG_REQUIRE(dmax < 256u, RTG_ERROR_LIMIT, "BVH build: binary tree depth %u beyond 255", dmax);
-        hipLaunchKernelGGL(k_iota, dim3(blocks_for(m, 256)), dim3(256), 0, s, b.ka, m);
-        hipLaunchKernelGGL(k_rs_hist, dim3(mtiles), dim3(kRsThreads), 0, s, depth, m, 0, b.hist, mtiles);
-        hipLaunchKernelGGL(k_scan_exclusive, dim3(1), dim3(1024), 0, s, b.hist, 256u * mtiles);
-        hipLaunchKernelGGL(k_rs_scatter, dim3(mtiles), dim3(kRsThreads), 0, s, depth, b.ka, b.kb, b.vb, m, 0, b.hist,
-                           mtiles);
-        uint32_t* d_start = b.next + 4;  // 257 words after the collapse's counters
-        hipLaunchKernelGGL(k_fill_u32, dim3(blocks_for(dmax + 2, 256)), dim3(256), 0, s, d_start,
-                           (uint64_t)(dmax + 2), m);
-        hipLaunchKernelGGL(k_level_starts, dim3(blocks_for(m, 256)), dim3(256), 0, s, b.kb, m, d_start);
-        RTG_HIP(hipGetLastError());
-        start.assign(dmax + 2, m);
-        RTG_HIP(hipMemcpyAsync(start.data(), d_start, (dmax + 2) * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-        RTG_HIP(hipStreamSynchronize(s));
-        for (uint32_t d = dmax + 1; d-- > 0;) {
-            const uint32_t count = start[d + 1] - start[d];
-            if (count == 0) continue;
-            hipLaunchKernelGGL(k_treelet_level, dim3(blocks_for(count, kTreeletThreads)), dim3(kTreeletThreads), 0, s,
-                               b.vb + start[d], count, b.boxes, b.va, b.left, b.right, b.rcount, b.ibox, b.area);
-        }
-        hipLaunchKernelGGL(k_parents, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, (int)n, b.left, b.right,
-                           b.parent);
-    }
-    // top-down collapse, one breadth-first level per step
-    const uint32_t cap = node_cap(n);
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, b.wroot, 1ull, 0u);
-    uint32_t lb = 0, le = 1;
-    while (lb < le) {
-        const uint32_t m = le - lb;
-        hipLaunchKernelGGL(k_wide_expand, dim3(blocks_for(m, 256)), dim3(256), 0, s, lb, m, b.wroot, b.left, b.right,
-                           b.rcount, b.area, leaf_max, b.slots, b.cnt);
-        hipLaunchKernelGGL(k_scan_exclusive, dim3(1), dim3(1024), 0, s, b.cnt, m);
-        hipLaunchKernelGGL(k_wide_emit, dim3(blocks_for(m, 256)), dim3(256), 0, s, lb, le, m, b.slots, b.cnt,
-                           b.rfirst, b.rcount, leaf_max, cap, b.nodes, b.wroot, b.next);
-        RTG_HIP(hipGetLastError());
-        uint32_t next = 0;
-        RTG_HIP(hipMemcpyAsync(&next, b.next, 4, hipMemcpyDeviceToHost, s));
-        RTG_HIP(hipStreamSynchronize(s));
-        RTG_REQUIRE(next <= cap - le, RTG_ERROR_DEVICE, "BVH collapse: %u nodes exceed the capacity %u", le + next,
-                    cap);
-        level_off.push_back(le);
-        lb = le;
-        le += next;
-    }
-    const uint32_t levels = (uint32_t)level_off.size() - 1;
-    for (uint32_t L = levels; L-- > 0;) {
-        const uint32_t m = level_off[L + 1] - level_off[L];
-        hipLaunchKernelGGL(k_wide_boxes, dim3(blocks_for(m, 256)), dim3(256), 0, s, level_off[L], m, b.nodes,
-                           b.boxes, b.va);
-    }
+    hipLaunchKernelGGL(k_karras, dim3(blocks_for(n, 256)), dim3(256), 0, s, b.ka, (int)n, b.va, b.boxes, b.lbox, b.bin,
+                       b.rcount, b.low, b.mid, b.tiers);
+}
+
+// At most one primitive: the single node.
+static int single_node(rtg_ctx* ctx, const BuildBufs& b, uint32_t n, hipStream_t s, BuildReport& rep) {
+    hipLaunchKernelGGL(k_wide_single, dim3(1), dim3(256), 0, s, b.boxes, n, b.nodes, b.va, b.off, b.state);
+    hipLaunchKernelGGL(k_build_report, dim3(1), dim3(64), 0, s, b.state, ctx->d_status, b.cb + 6, ctx->build_report);
     RTG_HIP(hipGetLastError());
+    RTG_HIP(hipStreamSynchronize(s));
+    rep = *ctx->build_report;
+    return RTG_OK;
+}
+
+static SmallOut small_out(const BuildBufs& b) {
+    return SmallOut{b.boxes, b.lbox, b.va, b.bin, b.rcount, b.low, b.mid, b.tiers, b.cb};
+}
+
+// Workgroups of a blob's last kernel: 16 bytes a lane and a few rounds.
+static unsigned finish_grid(uint64_t bytes) { return (unsigned)std::min<uint64_t>(bytes / 4096 / 4 + 1, 4096); }
+
+// Room for `count` addresses in the registry arena. Versions are never
+// overwritten: work in flight, and a caller's captured refits, read the one
+// of their launch until the context goes.
+static int registry_room(rtg_ctx* ctx, uint32_t count, uint64_t** out) {
+    if (ctx->registry_used + count > ctx->registry_cap || !ctx->registry_arena) {
+        const size_t cap = std::max<size_t>(8192, 16 * (size_t)count);
+        uint64_t* p = nullptr;
+        RTG_HIP(hipMalloc(&p, cap * sizeof(uint64_t)));
+        if (ctx->registry_arena) ctx->retired.push_back(ctx->registry_arena);
+        ctx->registry_arena = p;
+        ctx->registry_cap = cap;
+        ctx->registry_used = 0;
+    }
+    *out = ctx->registry_arena + ctx->registry_used;
+    return RTG_OK;
+}
+static void registry_commit(rtg_ctx* ctx, uint64_t* version, uint32_t count) {
+    ctx->d_registry = version;
+    ctx->registry_count = count;
+    ctx->registry_used += count;
+}
+
+int build_report_init(rtg_ctx* ctx) {
+    RTG_HIP(hipHostMalloc(reinterpret_cast<void**>(&ctx->build_report), sizeof(BuildReport)));
     return RTG_OK;
 }
 
 int refresh_registry(rtg_ctx* ctx) {
-    std::vector<uint64_t> addrs;
+    std::vector<uint64_t> addrs;  // ascending, as the map holds them
     for (auto& kv : ctx->structures)
         if (kv.second.kind == kKindBlas) addrs.push_back(kv.first);
-    std::sort(addrs.begin(), addrs.end());
     uint64_t* d = nullptr;
-    RTG_HIP(hipMalloc(&d, std::max<size_t>(1, addrs.size()) * sizeof(uint64_t)));
+    int st = registry_room(ctx, (uint32_t)addrs.size(), &d);
+    if (st != RTG_OK) return st;
     if (!addrs.empty()) RTG_HIP(hipMemcpy(d, addrs.data(), addrs.size() * sizeof(uint64_t), hipMemcpyHostToDevice));
-    if (ctx->d_registry) ctx->retired.push_back(ctx->d_registry);
-    ctx->d_registry = d;
-    ctx->registry_count = (uint32_t)addrs.size();
+    registry_commit(ctx, d, (uint32_t)addrs.size());
     return RTG_OK;
 }
 
@@ -1145,7 +1115,7 @@ extern "C" int rtg_blas_query_sizes(rtg_ctx* ctx, const rtg_geometry* geoms, uin
     // an upper bound: the blob of a build holds its actual node count
     Layout L = blas_layout((uint32_t)total, n_geom, node_cap((uint32_t)total));
     out->acceleration_structure_size = L.total;
-    out->build_scratch_size = lbvh_scratch_bytes((uint32_t)total, sizeof(TriRec)) + n_geom * sizeof(GeomDesc);
+    out->build_scratch_size = build_scratch_bytes((uint32_t)total, sizeof(TriRec), n_geom);
     out->update_scratch_size = 0;
     return RTG_OK;
 }
@@ -1156,7 +1126,7 @@ extern "C" int rtg_tlas_query_sizes(rtg_ctx* ctx, uint32_t count, rtg_build_size
     RTG_REQUIRE(count < (1u << 27), RTG_ERROR_LIMIT, "TLAS has %u instances (limit 2^27)", count);
     Layout L = tlas_layout(count, node_cap(count), node_cap(count));
     out->acceleration_structure_size = L.total;
-    out->build_scratch_size = lbvh_scratch_bytes(count, sizeof(InstRec));
+    out->build_scratch_size = build_scratch_bytes(count, sizeof(InstRec), 1);
     out->update_scratch_size = 0;
     return RTG_OK;
 }
@@ -1187,55 +1157,51 @@ extern "C" int rtg_blas_build(rtg_ctx* ctx, const rtg_geometry* geoms, uint32_t 
         RTG_REQUIRE(total < (1ull << 27), RTG_ERROR_LIMIT, "BLAS exceeds 2^27 triangles");
     }
     uint32_t n = (uint32_t)total;
-    size_t need = lbvh_scratch_bytes(n, sizeof(TriRec)) + std::max(1u, n_geom) * sizeof(GeomDesc) + 256;
-    if (ctx->scratch.ensure(need) != RTG_OK) return RTG_ERROR_OUT_OF_MEMORY;
-    LbvhBufs b = carve_lbvh(ctx->scratch.ptr, n, sizeof(TriRec), n_geom);
-    GeomDesc* d_geoms = b.geoms;
+    if (ctx->scratch.ensure(build_scratch_bytes(n, sizeof(TriRec), n_geom)) != RTG_OK) return RTG_ERROR_OUT_OF_MEMORY;
+    const BuildBufs b = carve_build(ctx->scratch.ptr, n, sizeof(TriRec), n_geom);
+    GeomArgs args = {};
+    const uint32_t by_arg = n_geom <= kGeomArgs ? n_geom : 0;
+    std::copy(gd.begin(), gd.begin() + by_arg, args.g);
+    hipLaunchKernelGGL(k_build_init, dim3(1), dim3(64), 0, s, b.cb, b.tiers, args, by_arg, b.geoms);
     // the copy source must outlive the asynchronous copy: the build
     // synchronises its stream before returning
-    RTG_HIP(hipMemcpyAsync(d_geoms, gd.data(), std::max(1u, n_geom) * sizeof(GeomDesc), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_init_bounds, dim3(1), dim3(64), 0, s, b.cb);
-    if (n > 0)
-        hipLaunchKernelGGL(k_tri_setup, dim3(blocks_for(n, 256)), dim3(256), 0, s, d_geoms, n_geom, n,
-                           reinterpret_cast<TriRec*>(b.recs), b.boxes, b.cb, ctx->d_status);
-    std::vector<uint32_t> level_off;
-    int st = wide_hierarchy(b, n, kBlasLeafMax, (flags & RTG_BUILD_PREFER_FAST_TRACE) ? kTreeletRounds : 0, s,
-                            level_off);
+    if (n_geom > kGeomArgs)
+        RTG_HIP(hipMemcpyAsync(b.geoms, gd.data(), n_geom * sizeof(GeomDesc), hipMemcpyHostToDevice, s));
+    TriRec* tris = reinterpret_cast<TriRec*>(b.recs);
+    if (n > 1 && n <= kSmallBuild) {
+        hipLaunchKernelGGL(k_small_tris, dim3(1), dim3(kSmallThreads), 0, s, b.geoms, n_geom, n, tris, small_out(b),
+                           ctx->d_status);
+    } else if (n > 0) {
+        hipLaunchKernelGGL(k_tri_setup, dim3(blocks_for(n, 256)), dim3(256), 0, s, b.geoms, n_geom, n, tris, b.boxes,
+                           b.cb, ctx->d_status);
+        if (n > 1) radix_tree(b, n, s);
+    }
+    BuildReport rep;
+    int st = n > 1 ? wide_hierarchy(ctx, b, n, (flags & RTG_BUILD_PREFER_FAST_TRACE) ? kTreeletRounds : 0, s, rep)
+                   : single_node(ctx, b, n, s, rep);
     if (st != RTG_OK) {
         hipStreamSynchronize(s);  // pending copies read host memory of this frame
         return st;
     }
-    const uint32_t levels = (uint32_t)level_off.size() - 1;
-    Layout L = blas_layout(n, n_geom, level_off.back());
+    if (rep.status & kStatusBadIndex) return check_status(ctx, s, kStatusBadIndex, "rtg_blas_build");
+    const Layout L = blas_layout(n, n_geom, rep.nodes);
+    uint64_t* new_reg = nullptr;
+    st = registry_room(ctx, ctx->registry_count + 1, &new_reg);
+    if (st != RTG_OK) return st;
     uint8_t* blob = nullptr;
     RTG_HIP(hipMalloc(&blob, L.total));
-    hipError_t e = hipMemsetAsync(blob, 0, L.total, s);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(blob + L.nodes_off, b.nodes, (size_t)L.node_count * sizeof(Node), hipMemcpyDeviceToDevice,
-                           s);
+    hipLaunchKernelGGL(k_finish_blas, dim3(finish_grid(L.total)), dim3(256), 0, s, blob, L, b.nodes, tris, b.va,
+                       b.geoms, n_geom, n, rep.levels, ctx->d_registry, ctx->registry_count, new_reg);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) {
         hipFree(blob);
         set_error("rtg_blas_build: %s", hipGetErrorString(e));
         return RTG_ERROR_DEVICE;
     }
-    if (n > 0)
-        hipLaunchKernelGGL(k_gather_tris, dim3(blocks_for(n, 256)), dim3(256), 0, s, b.va,
-                           reinterpret_cast<const TriRec*>(b.recs), reinterpret_cast<TriRec*>(blob + L.prims_off), n);
-    std::vector<uint32_t> gflags(std::max(1u, n_geom));
-    for (uint32_t g = 0; g < n_geom; ++g) gflags[g] = geoms[g].flags;
-    if (n_geom) RTG_HIP(hipMemcpyAsync(blob + L.extra_off, gflags.data(), n_geom * 4, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_header, dim3(1), dim3(64), 0, s, reinterpret_cast<AsHeader*>(blob), kKindBlas, L.node_count,
-                       n, n_geom, levels, L.nodes_off, L.prims_off, L.extra_off, L.level_off, L.leafbox_off, L.total);
-    RTG_HIP(hipGetLastError());
-    st = check_status(ctx, s, kStatusBadIndex, "rtg_blas_build");
-    if (st != RTG_OK) {
-        hipFree(blob);
-        return st;
-    }
     uint64_t addr = reinterpret_cast<uint64_t>(blob);
     ctx->structures[addr] = AsRecord{kKindBlas, n, L.node_count, L.total};
-    st = refresh_registry(ctx);
-    if (st != RTG_OK) return st;
+    registry_commit(ctx, new_reg, ctx->registry_count + 1);
     *out = addr;
     return RTG_OK;
 }
@@ -1248,54 +1214,38 @@ extern "C" int rtg_tlas_build(rtg_ctx* ctx, const rtg_instance* instances, uint3
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     RTG_HIP(hipSetDevice(ctx->device));
     uint32_t n = count;
-    size_t need = lbvh_scratch_bytes(n, sizeof(InstRec));
-    if (ctx->scratch.ensure(need) != RTG_OK) return RTG_ERROR_OUT_OF_MEMORY;
-    LbvhBufs b = carve_lbvh(ctx->scratch.ptr, n, sizeof(InstRec));
-    hipLaunchKernelGGL(k_init_bounds, dim3(1), dim3(64), 0, s, b.cb);
-    if (n > 0)
+    if (ctx->scratch.ensure(build_scratch_bytes(n, sizeof(InstRec), 1)) != RTG_OK) return RTG_ERROR_OUT_OF_MEMORY;
+    const BuildBufs b = carve_build(ctx->scratch.ptr, n, sizeof(InstRec), 1);
+    hipLaunchKernelGGL(k_build_init, dim3(1), dim3(64), 0, s, b.cb, b.tiers, GeomArgs{}, 0u, b.geoms);
+    InstRec* recs = reinterpret_cast<InstRec*>(b.recs);
+    if (n > 1 && n <= kSmallBuild) {
+        hipLaunchKernelGGL(k_small_insts, dim3(1), dim3(kSmallThreads), 0, s, instances, n, ctx->d_registry,
+                           ctx->registry_count, recs, small_out(b), ctx->d_status);
+    } else if (n > 0) {
         hipLaunchKernelGGL(k_inst_setup, dim3(blocks_for(n, 256)), dim3(256), 0, s, instances, n, ctx->d_registry,
-                           ctx->registry_count, reinterpret_cast<InstRec*>(b.recs), b.boxes, b.cb, ctx->d_status);
-    std::vector<uint32_t> level_off;
-    int st = wide_hierarchy(b, n, kTlasLeafMax, (flags & RTG_BUILD_PREFER_FAST_TRACE) ? kTreeletRounds : 0, s,
-                            level_off);
+                           ctx->registry_count, recs, b.boxes, b.cb, ctx->d_status);
+        if (n > 1) radix_tree(b, n, s);
+        else hipMemcpyAsync(b.lbox, b.boxes, sizeof(Box), hipMemcpyDeviceToDevice, s);
+    }
+    BuildReport rep;
+    int st = n > 1 ? wide_hierarchy(ctx, b, n, (flags & RTG_BUILD_PREFER_FAST_TRACE) ? kTreeletRounds : 0, s, rep)
+                   : single_node(ctx, b, n, s, rep);
     if (st != RTG_OK) {
         hipStreamSynchronize(s);
         return st;
     }
-    const uint32_t levels = (uint32_t)level_off.size() - 1;
-    Layout L = tlas_layout(n, level_off.back(), levels);
-    // level data: level_count, level_offsets[level_count + 1]
-    std::vector<uint32_t> level_data(1, levels);
-    level_data.insert(level_data.end(), level_off.begin(), level_off.end());
+    if (rep.status & kStatusBadBlas) return check_status(ctx, s, kStatusBadBlas, "rtg_tlas_build");
+    const Layout L = tlas_layout(n, rep.nodes, rep.levels);
     uint8_t* blob = nullptr;
     RTG_HIP(hipMalloc(&blob, L.total));
-    hipError_t e = hipMemsetAsync(blob, 0, L.total, s);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(blob + L.nodes_off, b.nodes, (size_t)L.node_count * sizeof(Node), hipMemcpyDeviceToDevice,
-                           s);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(blob + L.level_off, level_data.data(), level_data.size() * 4, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess && n > 0)
-        e = hipMemcpyAsync(blob + L.extra_off, instances, (size_t)n * 64, hipMemcpyDeviceToDevice, s);
+    hipLaunchKernelGGL(k_finish_tlas, dim3(finish_grid(L.total)), dim3(256), 0, s, blob, L, b.nodes, recs, b.va,
+                       instances, b.lbox, b.off, n, rep.levels);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) {
-        hipStreamSynchronize(s);
         hipFree(blob);
         set_error("rtg_tlas_build: %s", hipGetErrorString(e));
         return RTG_ERROR_DEVICE;
-    }
-    if (n > 0)
-        hipLaunchKernelGGL(k_gather_insts, dim3(blocks_for(n, 256)), dim3(256), 0, s, b.va,
-                           reinterpret_cast<const InstRec*>(b.recs), b.boxes,
-                           reinterpret_cast<InstRec*>(blob + L.prims_off), reinterpret_cast<Box*>(blob + L.leafbox_off),
-                           n);
-    hipLaunchKernelGGL(k_header, dim3(1), dim3(64), 0, s, reinterpret_cast<AsHeader*>(blob), kKindTlas, L.node_count,
-                       n, 0u, levels, L.nodes_off, L.prims_off, L.extra_off, L.level_off, L.leafbox_off, L.total);
-    RTG_HIP(hipGetLastError());
-    // also keeps level_data alive until its copy has finished
-    st = check_status(ctx, s, kStatusBadBlas, "rtg_tlas_build");
-    if (st != RTG_OK) {
-        hipFree(blob);
-        return st;
     }
     uint64_t addr = reinterpret_cast<uint64_t>(blob);
     ctx->structures[addr] = AsRecord{kKindTlas, n, L.node_count, L.total};

@@ -1,0 +1,960 @@
+// build_tree.hpp -- the binary tree of a build and its collapse: bottom-up
+// boxes, treelet restructuring, and the 4-wide nodes (gfx950).
+//
+// Both bottom-up passes (boxes; boxes with treelets) have to visit a node
+// after its whole subtree. A pass is cut by primitive counts: the subtrees of
+// at most kTierLow primitives are each taken by one workgroup, which holds
+// the subtree in LDS and walks its levels with workgroup barriers; then one
+// workgroup per subtree of at most kTierHigh primitives visits the nodes
+// above those, and one workgroup the rest. A kernel per tier instead of one
+// per depth level, and no host read between them.
+#pragma once
+
+#include "rtg_device.hpp"
+
+namespace rtg {
+
+// ---------------------------------------------------------------------------
+// Boxes
+// ---------------------------------------------------------------------------
+// min/max of box planes as selects: the first operand wins ties, so that
+// +0/-0 resolve the same way on every device.
+__device__ inline float mins(float a, float b) { return b < a ? b : a; }
+__device__ inline float maxs(float a, float b) { return b > a ? b : a; }
+__device__ inline Box box_union(const Box& a, const Box& b) {
+    Box r;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        r.lo[k] = mins(a.lo[k], b.lo[k]);
+        r.hi[k] = maxs(a.hi[k], b.hi[k]);
+    }
+    return r;
+}
+__device__ inline Box box_empty() {
+    Box b;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        b.lo[k] = __builtin_inff();
+        b.hi[k] = -__builtin_inff();
+    }
+    return b;
+}
+
+// Order-preserving map of float to uint (for atomic min/max of centres).
+__device__ inline uint32_t f2ord(float f) {
+    uint32_t u = __float_as_uint(f);
+    return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+__device__ inline float ord2f(uint32_t o) { return __uint_as_float((o & 0x80000000u) ? (o & 0x7fffffffu) : ~o); }
+
+// Surface area of a box (half of it: the build only compares areas).
+__device__ inline float box_area(const Box& b) {
+    float ex = b.hi[0] - b.lo[0], ey = b.hi[1] - b.lo[1], ez = b.hi[2] - b.lo[2];
+    return (ex * ey + ey * ez) + ez * ex;
+}
+
+// A node of the binary tree: its children (internal node number, or kLeafBit
+// and a position in the sorted order) beside the areas of those that are
+// internal, so that opening a child and ranking what it holds takes one load.
+struct alignas(16) BinNode {
+    uint32_t left, right;
+    float area_l, area_r;
+};
+
+constexpr uint32_t kTierLow = 256;     // largest subtree a bottom workgroup holds in LDS
+constexpr uint32_t kTierHigh = 65536;  // largest subtree of the middle tier
+
+// Compiler order of LDS accesses between the lanes of one wave (the hardware
+// serves a wave's LDS accesses in order).
+__device__ __forceinline__ void wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// ---------------------------------------------------------------------------
+// Treelet restructuring (Karras & Aila 2013, HPG, "Fast Parallel
+// Construction of High-Quality Bounding Volume Hierarchies", section 4) of
+// the binary tree, for single-primitive leaves. The treelet of internal node
+// r: r's two children, then, while fewer than kTreeletLeaves, the treelet
+// leaf with the largest area that is an internal node replaced by its left
+// child in place and its right child appended. Its topology becomes the one
+// that minimises the summed surface area of its internal nodes (SAH cost with
+// fixed leaves), by dynamic programming over subsets of treelet leaves:
+// cost(S) = area(S) + min over partitions (P, S\P), P holding S's lowest
+// leaf, of cost(P) + cost(S\P); partitions tried in decreasing order of P,
+// the first minimum kept. New internal nodes reuse the treelet's numbers:
+// r for the whole set, then the expanded nodes in expansion order, handed
+// out as subsets are split from a stack (P's subtree first). A node is
+// processed after its whole subtree, so the result does not depend on timing.
+//
+// One treelet takes a group of G lanes: 16 where a level has treelets for
+// several groups of every wave, 64 where it has no more treelets than waves
+// and the level's time is one treelet's. Lane k holds treelet leaf k while
+// the treelet is formed; the subsets' areas are spread over the lanes by
+// their high bits; the dynamic programme goes by subset size, the sets of a
+// size (or parts of their partitions) side by side in the lanes, its table
+// in LDS. One lane for a whole treelet took 85 us of dependent LDS reads,
+// whatever a level's size; a group of 16 takes about 5 us.
+// ---------------------------------------------------------------------------
+constexpr int kTreeletLeaves = 7;
+constexpr int kTreeletRounds = 5;  // passes with RTG_BUILD_PREFER_FAST_TRACE
+
+struct alignas(16) TreeletScratch {
+    float cost[1 << kTreeletLeaves];
+    float lbox[kTreeletLeaves * 6 + 2];  // boxes of the treelet's leaves
+    float nbox[(kTreeletLeaves - 1) * 6];  // boxes of its new internal nodes
+    float larea[8], narea[8];
+    uint32_t lref[8], lcount[8], inner[8];
+    uint8_t split[1 << kTreeletLeaves];
+    uint32_t pad[12];  // groups of a wave start 16 banks apart
+};
+static_assert(sizeof(TreeletScratch) % 16 == 0, "scratch records stay 16-byte aligned");
+
+// The subsets of 7 treelet leaves by size (2 to 7), ascending within a size,
+// so that those of the first m leaves come first.
+constexpr int kTreeletSets = 120;
+struct TreeletSetTable {
+    uint8_t s[kTreeletSets];
+    constexpr TreeletSetTable() : s() {
+        int n = 0;
+        for (int size = 2; size <= kTreeletLeaves; ++size)
+            for (int v = 1; v < (1 << kTreeletLeaves); ++v) {
+                int bits = 0;
+                for (int b = 0; b < kTreeletLeaves; ++b) bits += (v >> b) & 1;
+                if (bits == size) s[n++] = (uint8_t)v;
+            }
+    }
+};
+__device__ constexpr TreeletSetTable kTreeletSetTable;
+
+constexpr uint32_t binom(uint32_t n, uint32_t k) {
+    uint64_t r = 1;
+    for (uint32_t i = 0; i < k; ++i) r = r * (n - i) / (i + 1);
+    return k > n ? 0u : (uint32_t)r;
+}
+// number of subsets of size m of n <= 7 leaves, for a fixed m
+template <int M>
+__device__ __forceinline__ uint32_t set_count(int n) {
+    constexpr uint64_t packed = ((uint64_t)binom(2, M) << 16) | ((uint64_t)binom(3, M) << 24) |
+                                ((uint64_t)binom(4, M) << 32) | ((uint64_t)binom(5, M) << 40) |
+                                ((uint64_t)binom(6, M) << 48) | ((uint64_t)binom(7, M) << 56);
+    return (uint32_t)(packed >> (8 * n)) & 0xffu;
+}
+constexpr int set_offset(int m) {
+    int o = 0;
+    for (int k = 2; k < m; ++k) o += (int)binom(kTreeletLeaves, k);
+    return o;
+}
+
+template <int Ctrl>
+__device__ __forceinline__ uint32_t dpp_max(uint32_t x) {
+    const uint32_t y = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, Ctrl, 0xf, 0xf, true);
+    return max(x, y);
+}
+// max over the aligned 8 lanes this lane is in
+__device__ __forceinline__ uint32_t max8(uint32_t x) {
+    x = dpp_max<0xB1>(x);   // quad_perm 1,0,3,2
+    x = dpp_max<0x4E>(x);   // quad_perm 2,3,0,1
+    return dpp_max<0x141>(x);  // row_half_mirror
+}
+
+// Costs and splits of the subsets of M treelet leaves. L lanes share a set:
+// lane h of them tries the partitions whose top log2(L) free leaves are the
+// complement of h's bits, so that ascending h is descending P.
+template <int G, int M, int L>
+__device__ __forceinline__ void treelet_size(TreeletScratch* sc, const uint8_t* sets, int nl, int gl) {
+    if (M > nl) return;
+    constexpr int kLog = L == 1 ? 0 : L == 2 ? 1 : L == 4 ? 2 : L == 8 ? 3 : L == 16 ? 4 : 6;
+    constexpr int kSteps = 1 << (M - 1 - kLog);
+    const uint32_t ntask = set_count<M>(nl) * L;
+    for (uint32_t task = gl; task < ntask; task += G) {
+        const uint32_t S = sets[set_offset(M) + task / L], h = task % L;
+        const uint32_t low = S & (0u - S);
+        uint32_t R = S ^ low, P0 = low;
+#pragma unroll
+        for (int b = kLog - 1; b >= 0; --b) {
+            const uint32_t top = 0x80000000u >> __builtin_clz(R);
+            R ^= top;
+            if (!((h >> b) & 1u)) P0 |= top;
+        }
+        // q runs down over the submasks of R; for h = 0 the first one gives
+        // P = S, no partition; the first real one starts the minimum
+        // whatever its value (a NaN cost stays the minimum)
+        float best = __builtin_inff();
+        uint32_t bp = 0, q = R;
+        const uint32_t first_h = kSteps > 1 ? 0u : 1u;
+        constexpr int first_i = kSteps > 1 ? 1 : 0;
+        float c[kSteps];
+        uint32_t P[kSteps];
+#pragma unroll
+        for (int i = 0; i < kSteps; ++i) {
+            P[i] = P0 | q;
+            c[i] = sc->cost[P[i]] + sc->cost[S ^ P[i]];
+            q = (q - 1u) & R;
+        }
+#pragma unroll
+        for (int i = 0; i < kSteps; ++i) {
+            bool take = c[i] < best;
+            if (i == 0) take = take && h != 0u;
+            if (i == first_i) take = take || h == first_h;
+            if (take) {
+                best = c[i];
+                bp = P[i];
+            }
+        }
+#pragma unroll
+        for (int off = 1; off < L; off <<= 1) {
+            const float co = __shfl_xor(best, off);
+            const uint32_t po = (uint32_t)__shfl_xor((int)bp, off);
+            const bool less = co < best || (co == best && (h & off) != 0u);
+            const bool take = po != 0u && (bp == 0u || co != co || (best == best && less));
+            if (take) {
+                best = co;
+                bp = po;
+            }
+        }
+        if (h == 0) {
+            sc->cost[S] = sc->cost[S] + best;
+            sc->split[S] = (uint8_t)bp;
+        }
+    }
+    wave_order();
+}
+
+// Restructures the treelet of node r (three or more primitives below it);
+// the G lanes of a group call it together. Store: rec(id), box(ref),
+// count(ref), put(id, record, box, count).
+template <int G, class Store>
+__device__ void treelet_group(Store& S, uint32_t r, TreeletScratch* sc, const uint8_t* sets) {
+    static_assert(G == 16 || G == 64, "group sizes");
+    constexpr int kLowBits = G == 16 ? 3 : 1;  // subset bits a lane goes through by itself
+    const int gl = threadIdx.x & (G - 1);
+    const int base = (threadIdx.x & 63) & ~(G - 1);
+    // formation: lane k < nl holds leaf k
+    uint32_t ref = kEmpty, inner = 0;
+    float area = 0.0f;
+    {
+        const BinNode nd = S.rec(r);
+        if (gl == 0) ref = nd.left;
+        if (gl == 1) ref = nd.right;
+        if (gl < 2 && !(ref & kLeafBit)) area = box_area(S.box(ref));
+    }
+    int nl = 2;
+    while (nl < kTreeletLeaves) {
+        const bool internal = gl < nl && !(ref & kLeafBit);
+        // largest area, lowest lane; a NaN area wins only in the first
+        // internal leaf and never later, as the comparisons in leaf order do
+        uint32_t key = internal ? f2ord(area + 0.0f) : 0u;
+        const uint64_t cand = (__ballot(internal) >> base) & 0xffu;
+        if (cand == 0) break;
+        if (internal && area != area) key = (int)__builtin_ctzll(cand) == gl ? 0xffffffffu : 1u;
+        const uint32_t top = max8(key);
+        const uint64_t at = (__ballot(internal && key == top) >> base) & 0xffu;
+        const int best = (int)__builtin_ctzll(at);
+        const uint32_t c = (uint32_t)__shfl((int)ref, best, G);
+        const BinNode nd = S.rec(c);
+        if (gl == nl - 2) inner = c;
+        if (gl == best) {
+            ref = nd.left;
+            area = nd.area_l;
+        }
+        if (gl == nl) {
+            ref = nd.right;
+            area = nd.area_r;
+        }
+        ++nl;
+    }
+    if (gl < nl) {
+        const Box b = S.box(ref);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            sc->lbox[gl * 6 + a] = b.lo[a];
+            sc->lbox[gl * 6 + 3 + a] = b.hi[a];
+        }
+        sc->lref[gl] = ref;
+        sc->larea[gl] = area;
+        sc->lcount[gl] = S.count(ref);
+        if (gl == 0) sc->inner[0] = r;
+        if (gl < nl - 2) sc->inner[1 + gl] = inner;
+    }
+    wave_order();
+    // areas of the subsets: the lane's high bits choose leaves kLowBits..6.
+    // fminf/fmaxf fold the same values as the selects of box_union from the
+    // empty box (NaN planes skipped); a zero's sign does not change an area.
+    {
+        float lo[3], hi[3], l[kLowBits][6];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            lo[a] = __builtin_inff();
+            hi[a] = -__builtin_inff();
+        }
+#pragma unroll
+        for (int k = 0; k < kTreeletLeaves; ++k) {
+            float p[6];
+#pragma unroll
+            for (int a = 0; a < 6; ++a) p[a] = sc->lbox[k * 6 + a];
+            if (k < kLowBits) {
+#pragma unroll
+                for (int a = 0; a < 6; ++a) l[k][a] = p[a];
+            } else if ((gl >> (k - kLowBits)) & 1) {
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    lo[a] = fminf(lo[a], p[a]);
+                    hi[a] = fmaxf(hi[a], p[3 + a]);
+                }
+            }
+        }
+#pragma unroll
+        for (int low = 0; low < (1 << kLowBits); ++low) {
+            float bl[3], bh[3];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                bl[a] = lo[a];
+                bh[a] = hi[a];
+#pragma unroll
+                for (int k = 0; k < kLowBits; ++k)
+                    if ((low >> k) & 1) {
+                        bl[a] = fminf(bl[a], l[k][a]);
+                        bh[a] = fmaxf(bh[a], l[k][3 + a]);
+                    }
+            }
+            const float ex = bh[0] - bl[0], ey = bh[1] - bl[1], ez = bh[2] - bl[2];
+            const uint32_t set = ((uint32_t)gl << kLowBits) | (uint32_t)low;
+            if (set < (1u << kTreeletLeaves))
+                sc->cost[set] = (set & (set - 1u)) == 0u ? 0.0f : (ex * ey + ey * ez) + ez * ex;
+        }
+    }
+    wave_order();
+    if (G == 16) {
+        treelet_size<G, 2, 1>(sc, sets, nl, gl);
+        treelet_size<G, 3, 1>(sc, sets, nl, gl);
+        treelet_size<G, 4, 1>(sc, sets, nl, gl);
+        treelet_size<G, 5, 2>(sc, sets, nl, gl);
+        treelet_size<G, 6, 2>(sc, sets, nl, gl);
+        treelet_size<G, 7, 16>(sc, sets, nl, gl);
+    } else {
+        treelet_size<G, 2, 1>(sc, sets, nl, gl);
+        treelet_size<G, 3, 1>(sc, sets, nl, gl);
+        treelet_size<G, 4, 1>(sc, sets, nl, gl);
+        treelet_size<G, 5, 2>(sc, sets, nl, gl);
+        treelet_size<G, 6, 8>(sc, sets, nl, gl);
+        treelet_size<G, 7, 64>(sc, sets, nl, gl);
+    }
+    // The new internal nodes, in the order they come off the stack (every
+    // lane of the group follows it): node j's set, number and children as
+    // codes: 0..6 a treelet leaf, 8 + x internal node number inner[x].
+    uint32_t node[kTreeletLeaves - 1];
+    uint32_t jof = 0;  // 4 bits per internal number: its place in the order
+    {
+        uint64_t st_set = (1u << nl) - 1u, st_id = 0;  // stacks of 8-bit entries
+        uint32_t next = 1;
+#pragma unroll
+        for (int j = 0; j < kTreeletLeaves - 1; ++j) {
+            if (j < nl - 1) {
+                const uint32_t set = (uint32_t)st_set & 0xffu, id = (uint32_t)st_id & 0xffu;
+                st_set >>= 8;
+                st_id >>= 8;
+                jof |= (uint32_t)j << (4 * id);
+                const uint32_t P = sc->split[set], Q = set ^ P;
+                uint32_t c0, c1;
+                const bool m0 = (P & (P - 1u)) != 0u, m1 = (Q & (Q - 1u)) != 0u;
+                c0 = m0 ? 8u + next : (uint32_t)__builtin_ctz(P);
+                next += m0 ? 1u : 0u;
+                c1 = m1 ? 8u + next : (uint32_t)__builtin_ctz(Q);
+                next += m1 ? 1u : 0u;
+                if (m1) {
+                    st_set = (st_set << 8) | Q;
+                    st_id = (st_id << 8) | (c1 - 8u);
+                }
+                if (m0) {
+                    st_set = (st_set << 8) | P;
+                    st_id = (st_id << 8) | (c0 - 8u);
+                }
+                node[j] = set | (id << 8) | (c0 << 12) | (c1 << 16);
+            } else {
+                node[j] = 0;
+            }
+        }
+    }
+    // their boxes, last to first (children come after their parents): lane a
+    // folds plane a
+#pragma unroll
+    for (int j = kTreeletLeaves - 2; j >= 0; --j) {
+        if (j < nl - 1 && gl < 6) {
+            const uint32_t c0 = (node[j] >> 12) & 0xfu, c1 = (node[j] >> 16) & 0xfu;
+            const float x = c0 < 8u ? sc->lbox[c0 * 6 + gl] : sc->nbox[((jof >> (4 * (c0 - 8u))) & 0xfu) * 6 + gl];
+            const float y = c1 < 8u ? sc->lbox[c1 * 6 + gl] : sc->nbox[((jof >> (4 * (c1 - 8u))) & 0xfu) * 6 + gl];
+            sc->nbox[j * 6 + gl] = gl < 3 ? mins(x, y) : maxs(x, y);
+        }
+        wave_order();
+    }
+    uint32_t mine = 0;
+    Box b = box_empty();
+    if (gl < nl - 1) {
+#pragma unroll
+        for (int j = 0; j < kTreeletLeaves - 1; ++j)
+            if (j == gl) mine = node[j];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            b.lo[a] = sc->nbox[gl * 6 + a];
+            b.hi[a] = sc->nbox[gl * 6 + 3 + a];
+        }
+        sc->narea[gl] = box_area(b);
+    }
+    wave_order();
+    if (gl < nl - 1) {
+        BinNode nd;
+        uint32_t count = 0;
+#pragma unroll
+        for (int k = 0; k < kTreeletLeaves; ++k)
+            if ((mine >> k) & 1u) count += sc->lcount[k];
+        const uint32_t c0 = (mine >> 12) & 0xfu, c1 = (mine >> 16) & 0xfu;
+        nd.left = c0 < 8u ? sc->lref[c0] : sc->inner[c0 - 8u];
+        nd.area_l = c0 < 8u ? sc->larea[c0] : sc->narea[(jof >> (4 * (c0 - 8u))) & 0xfu];
+        nd.right = c1 < 8u ? sc->lref[c1] : sc->inner[c1 - 8u];
+        nd.area_r = c1 < 8u ? sc->larea[c1] : sc->narea[(jof >> (4 * (c1 - 8u))) & 0xfu];
+        S.put(sc->inner[(mine >> 8) & 0xfu], nd, b, count);
+    }
+    wave_order();
+}
+
+// ---------------------------------------------------------------------------
+// Bottom tier: one workgroup per subtree of at most kTierLow primitives.
+// The subtree's records live in LDS under local numbers, nodes with three or
+// more primitives from the front in breadth-first order (their levels in
+// `lv`), nodes with two from the back.
+// ---------------------------------------------------------------------------
+struct LdsTree {
+    BinNode rec_[kTierLow];
+    Box box_[kTierLow];
+    Box leaf_[kTierLow];
+    uint32_t gid[kTierLow];       // node number of a local node
+    uint32_t leaf_pos[kTierLow];  // sorted position of a local leaf
+    uint16_t cnt[kTierLow];       // primitives below a local node
+    uint16_t lv[kTierLow + 1];    // first local node of each level
+    uint32_t nfront, nback, nleaf, levels;
+
+    __device__ __forceinline__ BinNode rec(uint32_t i) const { return rec_[i]; }
+    __device__ __forceinline__ Box box(uint32_t ref) const {
+        return (ref & kLeafBit) ? leaf_[ref & 0xffu] : box_[ref];
+    }
+    __device__ __forceinline__ uint32_t count(uint32_t ref) const { return (ref & kLeafBit) ? 1u : cnt[ref]; }
+    __device__ __forceinline__ void put(uint32_t i, const BinNode& nd, const Box& b, uint32_t c) {
+        rec_[i] = nd;
+        box_[i] = b;
+        cnt[i] = (uint16_t)c;
+    }
+};
+
+constexpr int kBottomThreads = 256;
+
+// OPT: treelets, `rounds` passes over the same subtree (more than one only
+// where the subtree is the whole tree: between passes the nodes above a
+// subtree move its nodes); otherwise boxes only.
+template <bool OPT>
+__global__ __launch_bounds__(kBottomThreads) void k_tree_bottom(BinNode* bin, Box* ibox, uint32_t* rcount,
+                                                                const Box* lbox, const uint32_t* roots,
+                                                                const uint32_t* nroots, int rounds) {
+    __shared__ LdsTree T;
+    __shared__ TreeletScratch s_sc[OPT ? kBottomThreads / 16 : 1];
+    __shared__ uint8_t s_sets[OPT ? kTreeletSets : 1];
+    const uint32_t t = threadIdx.x;
+    if (OPT && t < kTreeletSets) s_sets[t] = kTreeletSetTable.s[t];
+    const uint32_t nr = *nroots;
+    for (uint32_t k = blockIdx.x; k < nr; k += gridDim.x) {
+        const uint32_t root = roots[k];
+        for (int round = 0; round < rounds; ++round) {
+            __syncthreads();
+            if (t == 0) {
+                const uint32_t rc = rcount[root];
+                const bool front = rc >= 3;
+                T.gid[front ? 0 : kTierLow - 1] = root;
+                T.nfront = front ? 1 : 0;
+                T.nback = front ? 0 : 1;
+                T.nleaf = 0;
+                T.lv[0] = 0;
+                T.levels = 0;
+            }
+            __syncthreads();
+            // breadth-first: the front nodes of a level hand out local
+            // numbers to their children (order within a level is free: no
+            // result depends on local numbers)
+            uint32_t b = 0, L = 0;
+            while (true) {
+                const uint32_t e = T.nfront;
+                __syncthreads();
+                if (b >= e) break;
+                for (uint32_t q = b + t; q < e; q += kBottomThreads) {
+                    const uint32_t g = T.gid[q];
+                    BinNode nd = bin[g];
+                    T.cnt[q] = (uint16_t)rcount[g];
+                    uint32_t c[2] = {nd.left, nd.right};
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        uint32_t local;
+                        if (c[h] & kLeafBit) {
+                            local = atomicAdd(&T.nleaf, 1u) & 0xffu;
+                            T.leaf_pos[local] = c[h] & kFirstMask;
+                            local |= kLeafBit;
+                        } else if (rcount[c[h]] >= 3) {
+                            local = min(atomicAdd(&T.nfront, 1u), kTierLow - 1);
+                            T.gid[local] = c[h];
+                        } else {
+                            local = (kTierLow - 1 - atomicAdd(&T.nback, 1u)) & 0xffu;
+                            T.gid[local] = c[h];
+                        }
+                        c[h] = local;
+                    }
+                    nd.left = c[0];
+                    nd.right = c[1];
+                    T.rec_[q] = nd;
+                }
+                __syncthreads();
+                b = e;
+                ++L;
+                if (t == 0) T.lv[L] = (uint16_t)e;
+                if (L >= kTierLow) break;
+            }
+            const uint32_t nfront = min(T.nfront, kTierLow), nback = min(T.nback, kTierLow);
+            // the two leaves of each back node
+            for (uint32_t q = t; q < nback; q += kBottomThreads) {
+                const uint32_t i = kTierLow - 1 - q;
+                BinNode nd = bin[T.gid[i]];
+                const uint32_t l = atomicAdd(&T.nleaf, 2u);
+                const uint32_t l0 = l & 0xffu, l1 = (l + 1) & 0xffu;
+                T.leaf_pos[l0] = nd.left & kFirstMask;
+                T.leaf_pos[l1] = nd.right & kFirstMask;
+                const Box b0 = lbox[nd.left & kFirstMask], b1 = lbox[nd.right & kFirstMask];
+                T.box_[i] = box_union(b0, b1);
+                T.leaf_[l0] = b0;
+                T.leaf_[l1] = b1;
+                nd.left = kLeafBit | l0;
+                nd.right = kLeafBit | l1;
+                nd.area_l = nd.area_r = 0.0f;
+                T.rec_[i] = nd;
+                T.cnt[i] = 2;
+            }
+            // the leaves of the front nodes
+            for (uint32_t q = t; q < nfront; q += kBottomThreads) {
+                const BinNode nd = T.rec_[q];
+                if (nd.left & kLeafBit) T.leaf_[nd.left & 0xffu] = lbox[T.leaf_pos[nd.left & 0xffu]];
+                if (nd.right & kLeafBit) T.leaf_[nd.right & 0xffu] = lbox[T.leaf_pos[nd.right & 0xffu]];
+            }
+            __syncthreads();
+            for (uint32_t lev = L; lev-- > 0;) {
+                const uint32_t lb = T.lv[lev], le = T.lv[lev + 1];
+                if (!OPT) {
+                    for (uint32_t q = lb + t; q < le; q += kBottomThreads) {
+                        BinNode nd = T.rec_[q];
+                        const Box x = T.box(nd.left), y = T.box(nd.right);
+                        T.box_[q] = box_union(x, y);
+                        nd.area_l = box_area(x);
+                        nd.area_r = box_area(y);
+                        T.rec_[q] = nd;
+                    }
+                } else if (le - lb <= kBottomThreads / 64) {
+                    const uint32_t w = t >> 6;
+                    if (lb + w < le) treelet_group<64>(T, lb + w, &s_sc[w], s_sets);
+                } else {
+                    for (uint32_t q = lb + (t >> 4); q < le; q += kBottomThreads / 16)
+                        treelet_group<16>(T, q, &s_sc[t >> 4], s_sets);
+                }
+                __syncthreads();
+            }
+            // back to the tree under its own numbers
+            for (uint32_t q = t; q < nfront + nback; q += kBottomThreads) {
+                const uint32_t i = q < nfront ? q : kTierLow - 1 - (q - nfront);
+                BinNode nd = T.rec_[i];
+                nd.left = (nd.left & kLeafBit) ? (kLeafBit | T.leaf_pos[nd.left & 0xffu]) : T.gid[nd.left];
+                nd.right = (nd.right & kLeafBit) ? (kLeafBit | T.leaf_pos[nd.right & 0xffu]) : T.gid[nd.right];
+                const uint32_t g = T.gid[i];
+                bin[g] = nd;
+                ibox[g] = T.box_[i];
+                if (OPT) rcount[g] = T.cnt[i];
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Upper tiers: one workgroup per subtree visits its nodes of more than
+// `lowest` primitives, from the deepest of their levels up, in the tree's own
+// (global) records. `list` and `levels` hold each subtree's nodes breadth
+// first and their level starts; a subtree of c primitives takes c entries of
+// each (it has fewer nodes), from `bump` on.
+// ---------------------------------------------------------------------------
+struct GlobalTree {
+    BinNode* bin;
+    Box* ibox;
+    uint32_t* rcount;
+    const Box* lbox;
+    __device__ __forceinline__ BinNode rec(uint32_t i) const { return bin[i]; }
+    __device__ __forceinline__ Box box(uint32_t ref) const {
+        return (ref & kLeafBit) ? lbox[ref & kFirstMask] : ibox[ref];
+    }
+    __device__ __forceinline__ uint32_t count(uint32_t ref) const { return (ref & kLeafBit) ? 1u : rcount[ref]; }
+    __device__ __forceinline__ void put(uint32_t i, const BinNode& nd, const Box& b, uint32_t c) {
+        bin[i] = nd;
+        ibox[i] = b;
+        rcount[i] = c;
+    }
+};
+
+constexpr int kUpperThreads = 512;
+
+template <bool OPT>
+__global__ __launch_bounds__(kUpperThreads) void k_tree_upper(GlobalTree T, const uint32_t* roots,
+                                                              const uint32_t* nroots, uint32_t lowest, uint32_t n,
+                                                              uint32_t* list_all, uint32_t* levels_all,
+                                                              uint32_t* bump) {
+    __shared__ TreeletScratch s_sc[OPT ? kUpperThreads / 16 : 1];
+    __shared__ uint8_t s_sets[OPT ? kTreeletSets : 1];
+    __shared__ uint32_t s_count, s_base;
+    const uint32_t t = threadIdx.x;
+    if (OPT && t < kTreeletSets) s_sets[t] = kTreeletSetTable.s[t];
+    const uint32_t nr = *nroots;
+    for (uint32_t k = blockIdx.x; k < nr; k += gridDim.x) {
+        const uint32_t root = roots[k];
+        __syncthreads();
+        if (t == 0) {
+            s_base = atomicAdd(bump, T.rcount[root]);
+            s_count = 1;
+        }
+        __syncthreads();
+        const uint32_t base = s_base;
+        if (base >= n) return;  // (never: the subtrees of a tier share no primitive)
+        const uint32_t cap = n - base;
+        uint32_t* list = list_all + base;
+        uint32_t* lv = levels_all + base;
+        if (t == 0) {
+            list[0] = root;
+            lv[0] = 0;
+        }
+        __syncthreads();
+        uint32_t b = 0, L = 0;
+        while (true) {
+            const uint32_t e = min(s_count, cap);
+            __syncthreads();
+            if (b >= e) break;
+            for (uint32_t q = b + t; q < e; q += kUpperThreads) {
+                const BinNode nd = T.bin[list[q]];
+                const uint32_t c[2] = {nd.left, nd.right};
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    if (!(c[h] & kLeafBit) && T.rcount[c[h]] > lowest) {
+                        const uint32_t at = atomicAdd(&s_count, 1u);
+                        if (at < cap) list[at] = c[h];
+                    }
+            }
+            b = e;
+            ++L;
+            if (t == 0 && L < cap) lv[L] = e;
+            __syncthreads();
+        }
+        for (uint32_t lev = L; lev-- > 0;) {
+            const uint32_t lb = lv[lev], le = lev + 1 < L ? lv[lev + 1] : b;
+            if (!OPT) {
+                for (uint32_t q = lb + t; q < le; q += kUpperThreads) {
+                    const uint32_t g = list[q];
+                    BinNode nd = T.bin[g];
+                    const Box x = T.box(nd.left), y = T.box(nd.right);
+                    T.ibox[g] = box_union(x, y);
+                    nd.area_l = box_area(x);
+                    nd.area_r = box_area(y);
+                    T.bin[g] = nd;
+                }
+            } else if (le - lb <= kUpperThreads / 64) {
+                const uint32_t w = t >> 6;
+                if (lb + w < le) treelet_group<64>(T, list[lb + w], &s_sc[w], s_sets);
+            } else {
+                for (uint32_t q = lb + (t >> 4); q < le; q += kUpperThreads / 16)
+                    treelet_group<16>(T, list[q], &s_sc[t >> 4], s_sets);
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// Roots of the bottom and middle tiers: internal children of at most
+// kTierLow (kTierHigh) primitives under a node of more. Their order is free:
+// a tier's subtrees share no node. counts[0], counts[1]: how many.
+__device__ inline void tier_roots(uint32_t i, uint32_t count, const uint32_t* child, const uint32_t* child_count,
+                                  uint32_t* low, uint32_t* mid, uint32_t* counts) {
+    if (i == 0) {
+        if (count <= kTierLow) low[atomicAdd(&counts[0], 1u)] = 0;
+        else if (count <= kTierHigh) mid[atomicAdd(&counts[1], 1u)] = 0;
+    }
+    if (count <= kTierLow) return;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        if (child[h] & kLeafBit) continue;
+        if (child_count[h] <= kTierLow) low[atomicAdd(&counts[0], 1u)] = child[h];
+        else if (count > kTierHigh && child_count[h] <= kTierHigh) mid[atomicAdd(&counts[1], 1u)] = child[h];
+    }
+}
+
+__global__ __launch_bounds__(256) void k_tier_roots(uint32_t n, const BinNode* bin, const uint32_t* rcount,
+                                                    uint32_t* low, uint32_t* mid, uint32_t* counts) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n - 1) return;
+    const uint32_t c = rcount[i];
+    if (c <= kTierLow && i != 0) return;
+    const BinNode nd = bin[i];
+    const uint32_t child[2] = {nd.left, nd.right};
+    uint32_t cc[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) cc[h] = (child[h] & kLeafBit) ? 1u : rcount[child[h]];
+    tier_roots(i, c, child, cc, low, mid, counts);
+}
+
+// ---------------------------------------------------------------------------
+// Collapse into 4-wide nodes, breadth first. A wide node's slots: the binary
+// root's two children, then the largest-area internal slot replaced in place
+// by its two children while fewer than four (first slot on ties). Slot boxes
+// are the binary tree's: a fold of box planes in leaf order gives the same
+// value however it is grouped, as long as no plane is NaN (k_wide_boxes
+// below folds them again where one is).
+// ---------------------------------------------------------------------------
+struct WideTree {
+    const BinNode* bin;
+    const Box* ibox;
+    const Box* lbox;
+    Node* nodes;
+    uint32_t* wroot;  // binary root of each wide node
+    uint32_t cap;     // node capacity (n - 1: every wide node has two or more slots)
+};
+
+// Slots of the wide node rooted at binary node r and how many of them become
+// wide nodes.
+__device__ inline uint32_t wide_slots(const BinNode* bin, uint32_t r, uint32_t s[4]) {
+    BinNode nd = bin[r];
+    float a[4] = {nd.area_l, nd.area_r, 0.0f, 0.0f};
+    s[0] = nd.left;
+    s[1] = nd.right;
+    s[2] = s[3] = kEmpty;
+#pragma unroll
+    for (int nslot = 2; nslot < 4; ++nslot) {
+        int best = -1;
+        float best_area = 0.0f;
+        uint32_t c = 0;
+#pragma unroll
+        for (int k = 0; k < nslot; ++k) {
+            if (s[k] & kLeafBit) continue;
+            if (best < 0 || a[k] > best_area) {
+                best = k;
+                best_area = a[k];
+                c = s[k];
+            }
+        }
+        if (best < 0) break;
+        nd = bin[c];
+#pragma unroll
+        for (int k = 3; k >= 1; --k) {
+            if (k > best + 1) {
+                s[k] = s[k - 1];
+                a[k] = a[k - 1];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (k == best) {
+                s[k] = nd.left;
+                a[k] = nd.area_l;
+            }
+            if (k == best + 1) {
+                s[k] = nd.right;
+                a[k] = nd.area_r;
+            }
+        }
+    }
+    uint32_t internal = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) internal += (s[k] & kLeafBit) ? 0u : 1u;  // kEmpty has the leaf bit
+    return internal;
+}
+
+// Writes wide node w of binary slots s; its internal slots take the node
+// numbers from `next` on.
+__device__ inline void wide_emit(const WideTree& W, uint32_t w, const uint32_t s[4], uint32_t next) {
+    float lo[3][4], hi[3][4];
+    uint32_t ref[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        Box b = box_empty();
+        uint32_t r = s[k];
+        if (r != kEmpty) {
+            if (r & kLeafBit) {
+                b = box_union(b, W.lbox[r & kFirstMask]);
+            } else {
+                b = W.ibox[r];
+                if (next < W.cap) W.wroot[next] = r;
+                r = next++;
+            }
+        }
+        ref[k] = r;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            lo[a][k] = b.lo[a];
+            hi[a][k] = b.hi[a];
+        }
+    }
+    float4* out = reinterpret_cast<float4*>(W.nodes + w);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        out[2 * a] = make_float4(lo[a][0], lo[a][1], lo[a][2], lo[a][3]);
+        out[2 * a + 1] = make_float4(hi[a][0], hi[a][1], hi[a][2], hi[a][3]);
+    }
+    reinterpret_cast<uint4*>(out)[6] = make_uint4(ref[0], ref[1], ref[2], ref[3]);
+    reinterpret_cast<uint4*>(out)[7] = make_uint4(0u, 0u, 0u, 0u);
+}
+
+// Inclusive prefix sum over the workgroup (part: one word per wave).
+template <int BS>
+__device__ inline uint32_t block_scan(uint32_t v, uint32_t* part, uint32_t& total) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t u = (uint32_t)__shfl_up((int)v, off);
+        if (lane >= off) v += u;
+    }
+    if (lane == 63) part[w] = v;
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+#pragma unroll
+    for (int k = 0; k < BS / 64; ++k) {
+        const uint32_t p = part[k];
+        if (k < w) before += p;
+        all += p;
+    }
+    total = all;
+    __syncthreads();
+    return v + before;
+}
+
+// Progress of a collapse: level L holds nodes [off[L], off[L + 1]); `level`
+// is the first level not emitted.
+struct CollapseState {
+    uint32_t level, nodes, done, pad;
+};
+// What the host reads after a build's kernels (host memory, written by the device).
+struct BuildReport {
+    uint32_t levels, nodes, done, status, nan_boxes, pad[3];
+};
+
+// The first levels, by one workgroup, until one holds more than `most`
+// nodes or there is none left.
+constexpr int kCollapseThreads = 1024;
+__global__ __launch_bounds__(kCollapseThreads) void k_collapse_top(WideTree W, uint32_t most, uint32_t* off,
+                                                                   CollapseState* state) {
+    __shared__ uint32_t part[kCollapseThreads / 64];
+    uint32_t lb = 0, le = 1, level = 0;
+    if (threadIdx.x == 0) {
+        W.wroot[0] = 0;
+        off[0] = 0;
+        off[1] = 1;
+    }
+    __syncthreads();
+    while (le - lb <= most && le > lb) {
+        uint32_t next = le;
+        for (uint32_t q = lb; q < le; q += kCollapseThreads) {
+            const uint32_t w = q + threadIdx.x;
+            uint32_t s[4], want = 0, total;
+            if (w < le) want = wide_slots(W.bin, W.wroot[w], s);
+            const uint32_t incl = block_scan<kCollapseThreads>(want, part, total);
+            if (w < le) wide_emit(W, w, s, next + incl - want);
+            next += total;
+        }
+        next = min(next, W.cap);
+        ++level;
+        if (threadIdx.x == 0) off[level + 1] = next;
+        lb = le;
+        le = next;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        state->level = level;
+        state->nodes = le;
+        state->done = le == lb ? 1u : 0u;
+    }
+}
+
+// A later level in two kernels over many workgroups: the slots and the
+// workgroups' counts of new nodes, then the nodes, each workgroup's numbers
+// after those of the workgroups before it. `step`: levels since the one that
+// state->level names.
+constexpr uint32_t kWideBlocks = 1024;
+__device__ inline uint32_t wide_chunk(uint32_t m) { return ((m + kWideBlocks - 1) / kWideBlocks + 255u) & ~255u; }
+
+__global__ __launch_bounds__(256) void k_wide_expand(WideTree W, const uint32_t* off, const CollapseState* state,
+                                                     uint32_t step, uint4* slots, uint32_t* sums) {
+    __shared__ uint32_t part[4];
+    const uint32_t L = state->level + step;
+    const uint32_t lb = off[L], m = off[L + 1] - lb, chunk = wide_chunk(m);
+    const uint32_t b = blockIdx.x * chunk, e = min(m, b + chunk);
+    if (b >= m) return;
+    uint32_t sum = 0;
+    for (uint32_t q = b + threadIdx.x; q < e; q += 256) {
+        uint32_t s[4];
+        sum += wide_slots(W.bin, W.wroot[lb + q], s);
+        slots[q] = make_uint4(s[0], s[1], s[2], s[3]);
+    }
+    uint32_t total;
+    block_scan<256>(sum, part, total);
+    if (threadIdx.x == 0) sums[blockIdx.x] = total;
+}
+
+__global__ __launch_bounds__(256) void k_wide_emit(WideTree W, uint32_t* off, const CollapseState* state,
+                                                   uint32_t step, const uint4* slots, const uint32_t* sums) {
+    __shared__ uint32_t part[4];
+    const uint32_t L = state->level + step;
+    const uint32_t lb = off[L], le = off[L + 1], m = le - lb, chunk = wide_chunk(m);
+    const uint32_t b = blockIdx.x * chunk, e = min(m, b + chunk);
+    if (m == 0) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) off[L + 2] = le;
+        return;
+    }
+    if (b >= m) return;
+    uint32_t before = 0, total;
+    for (uint32_t k = threadIdx.x; k < blockIdx.x; k += 256) before += sums[k];
+    block_scan<256>(before, part, total);
+    uint32_t next = le + total;
+    for (uint32_t q0 = b; q0 < e; q0 += 256) {
+        const uint32_t q = q0 + threadIdx.x;
+        uint32_t s[4] = {kEmpty, kEmpty, kEmpty, kEmpty}, want = 0;
+        if (q < e) {
+            const uint4 v = slots[q];
+            s[0] = v.x;
+            s[1] = v.y;
+            s[2] = v.z;
+            s[3] = v.w;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) want += (s[k] & kLeafBit) ? 0u : 1u;
+        }
+        const uint32_t incl = block_scan<256>(want, part, total);
+        if (q < e) wide_emit(W, lb + q, s, next + incl - want);
+        next += total;
+    }
+    if (e == m && threadIdx.x == 0) off[L + 2] = min(next, W.cap);
+}
+
+// Moves the state past `steps` levels.
+__global__ void k_collapse_advance(const uint32_t* off, CollapseState* state, uint32_t steps) {
+    if (threadIdx.x != 0) return;
+    uint32_t L = state->level;
+    for (uint32_t k = 0; k < steps && off[L + 1] > off[L]; ++k) ++L;
+    state->level = L;
+    state->nodes = off[L + 1];
+    state->done = off[L + 1] == off[L] ? 1u : 0u;
+}
+
+__global__ void k_build_report(const CollapseState* state, const uint32_t* status, const uint32_t* nan_boxes,
+                               BuildReport* out) {
+    if (threadIdx.x != 0) return;
+    out->levels = state->level;
+    out->nodes = state->nodes;
+    out->done = state->done;
+    out->status = *status;
+    out->nan_boxes = *nan_boxes;
+}
+
+}  // namespace rtg

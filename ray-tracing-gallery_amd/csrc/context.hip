@@ -138,6 +138,7 @@ extern "C" int rtg_create(rtg_ctx** out, int device) {
     hipMemset(ctx->d_status, 0, 4);
     hipMemset(ctx->d_counters, 0, sizeof(rtg_trace_counters));
     int st = refresh_registry(ctx);
+    if (st == RTG_OK) st = build_report_init(ctx);
     if (st != RTG_OK) {
         rtg_destroy(ctx);
         return st;
@@ -154,7 +155,8 @@ extern "C" void rtg_destroy(rtg_ctx* ctx) {
     for (auto& kv : ctx->structures) hipFree(reinterpret_cast<void*>(kv.first));
     ctx->structures.clear();
     for (void* p : ctx->retired) hipFree(p);
-    if (ctx->d_registry) hipFree(ctx->d_registry);
+    if (ctx->registry_arena) hipFree(ctx->registry_arena);
+    if (ctx->build_report) hipHostFree(ctx->build_report);
     ctx->scratch.release();
     free_frame_arena(ctx);
     if (ctx->d_srgb_lut) hipFree(ctx->d_srgb_lut);

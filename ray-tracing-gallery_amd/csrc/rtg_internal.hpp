@@ -81,6 +81,7 @@ struct TimedLaunch {
 };
 
 struct FrameArena;  // trace.hip
+struct BuildReport;  // build_tree.hpp
 
 // Launch parameters of the traversal kernels (defaults, overridable through
 // the environment: RTG_REFILL_CLOSEST, RTG_REFILL_OCCLUSION (0 selects the
@@ -129,7 +130,12 @@ struct rtg_ctx {
     // sorted addresses of live BLASes, on the device (TLAS build/refit validate against it)
     uint64_t* d_registry = nullptr;
     uint32_t registry_count = 0;
-    std::vector<void*> retired;  // old registry buffers (freed at destroy)
+    // the registry's versions are cut from an arena, none overwritten while
+    // the context lives; arenas that filled up are in `retired`
+    uint64_t* registry_arena = nullptr;
+    size_t registry_cap = 0, registry_used = 0;
+    std::vector<void*> retired;
+    rtg::BuildReport* build_report = nullptr;  // host memory that a build's kernels write
     rtg::DeviceBuffer scratch;   // build scratch arena
     float* d_srgb_lut = nullptr;
     uint32_t* d_status = nullptr;  // sticky kernel status bits
@@ -146,6 +152,8 @@ struct rtg_ctx {
 
 namespace rtg {
 int refresh_registry(rtg_ctx* ctx);
+// Host memory for a build's report (rtg_create).
+int build_report_init(rtg_ctx* ctx);
 // Event pair around a launch when timing is enabled.
 struct LaunchTimer {
     rtg_ctx* ctx;

@@ -220,7 +220,9 @@ int rtg_tlas_query_sizes(rtg_ctx* ctx, uint32_t count, rtg_build_sizes* out);
 int rtg_tlas_build(rtg_ctx* ctx, const rtg_instance* instances, uint32_t count,
                    uint32_t build_flags, rtg_tlas* out, void* stream);
 /* In-place UPDATE (src == dst, util_structs.rs:318-319): new transforms and
- * BLAS references with the same instance count; topology is kept. One kernel. */
+ * BLAS references with the same instance count; topology is kept. One kernel
+ * for up to 256 instances, else one for the instances and one or more for
+ * the levels. */
 int rtg_tlas_refit(rtg_ctx* ctx, rtg_tlas tlas, const rtg_instance* instances, uint32_t count,
                    void* stream);
 /* CLONE mode copy into a new TLAS (src/main.rs:622). */

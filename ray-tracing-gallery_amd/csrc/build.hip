@@ -795,47 +795,107 @@ __global__ __launch_bounds__(256) void k_finish_tlas(uint8_t* blob, Layout L, co
 }
 
 // In-place TLAS UPDATE (src/util_structs.rs:285-357): new instance records,
-// same topology. One workgroup walks the level lists from the deepest level
-// to the root with a barrier between levels. 256 lanes, one wave per SIMD:
-// while another frame's traversal waves fill the GPU, such a workgroup finds
-// room on a CU long before a 1024-lane one (four waves per SIMD) would.
+// same topology, slot boxes again from the deepest level up. Instance k's
+// record waits on a chain of dependent loads (its index, the caller's
+// record, the registry, the BLAS header), so it pays to have all chains in
+// flight: one workgroup going through 20,000 instances took 350 us, a lane
+// each in as many workgroups as they need 6 us. The registry goes to LDS
+// first (a binary search per instance).
+constexpr uint32_t kRegistryLds = 1024;
+
+struct TlasParts {
+    AsHeader* h;
+    Node* nodes;
+    InstRec* recs;
+    rtg_instance* src;
+    Box* leafbox;
+};
+__device__ inline TlasParts tlas_parts(uint8_t* base) {
+    AsHeader* h = reinterpret_cast<AsHeader*>(base);
+    return TlasParts{h, reinterpret_cast<Node*>(base + h->nodes_off), reinterpret_cast<InstRec*>(base + h->prims_off),
+                     reinterpret_cast<rtg_instance*>(base + h->extra_off),
+                     reinterpret_cast<Box*>(base + h->leafbox_off)};
+}
+__device__ inline const uint64_t* registry_to_lds(const uint64_t* reg, uint32_t nreg, uint64_t* lds) {
+    if (nreg > kRegistryLds) return reg;
+    for (uint32_t k = threadIdx.x; k < nreg; k += blockDim.x) lds[k] = reg[k];
+    return lds;
+}
+__device__ inline void refit_inst(const TlasParts& P, uint32_t k, const rtg_instance* inst, const uint64_t* reg,
+                                  uint32_t nreg, uint32_t* status) {
+    uint32_t s = P.recs[k].index;
+    rtg_instance in = inst[s];
+    const AsHeader* bh = checked_blas(in, reg, nreg, status);
+    InstRec r;
+    fill_inst_rec(r, in, s, bh ? in.acceleration_structure_reference : 0);
+    P.recs[k] = r;
+    P.leafbox[k] = instance_world_box(in, bh);
+    P.src[s] = in;
+}
+// Slot i & 3 of node i >> 2 (the levels below are done).
+__device__ inline void refit_slot(const TlasParts& P, uint32_t i) {
+    Node& nd = P.nodes[i >> 2];
+    const uint32_t s = i & 3u;
+    set_slot(nd, s, ref_box(P.nodes, nd.child[s], P.leafbox, nullptr));
+}
+__device__ inline void refit_bounds(const TlasParts& P) {
+    if (threadIdx.x != 0) return;
+    Box r = node_box(P.nodes[0]);
+    for (int a = 0; a < 3; ++a) {
+        P.h->lo[a] = r.lo[a];
+        P.h->hi[a] = r.hi[a];
+    }
+}
+
+// The whole update in one workgroup of 256 lanes, one wave per SIMD: while
+// another frame's traversal waves fill the GPU, such a workgroup finds room
+// on a CU long before a 1024-lane one (four waves per SIMD) would.
 __global__ __launch_bounds__(256) void k_tlas_refit(uint8_t* base, const rtg_instance* inst, uint32_t n,
                                                     const uint64_t* reg, uint32_t nreg, uint32_t* status) {
-    AsHeader* h = reinterpret_cast<AsHeader*>(base);
-    Node* nodes = reinterpret_cast<Node*>(base + h->nodes_off);
-    InstRec* recs = reinterpret_cast<InstRec*>(base + h->prims_off);
-    rtg_instance* src = reinterpret_cast<rtg_instance*>(base + h->extra_off);
-    Box* leafbox = reinterpret_cast<Box*>(base + h->leafbox_off);
-    for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) {
-        uint32_t s = recs[k].index;
-        rtg_instance in = inst[s];
-        const AsHeader* bh = checked_blas(in, reg, nreg, status);
-        InstRec r;
-        fill_inst_rec(r, in, s, bh ? in.acceleration_structure_reference : 0);
-        recs[k] = r;
-        leafbox[k] = instance_world_box(in, bh);
-        src[s] = in;
-    }
+    __shared__ uint64_t s_reg[kRegistryLds];
+    const TlasParts P = tlas_parts(base);
+    reg = registry_to_lds(reg, nreg, s_reg);
     __syncthreads();
-    // same topology: slot boxes again, deepest level first
-    const uint32_t* lv = reinterpret_cast<const uint32_t*>(base + h->level_off);
+    for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) refit_inst(P, k, inst, reg, nreg, status);
+    __syncthreads();
+    const uint32_t* lv = reinterpret_cast<const uint32_t*>(base + P.h->level_off);
     const uint32_t levels = lv[0];
     const uint32_t* offs = lv + 1;
     for (uint32_t L = levels; L-- > 0;) {
-        for (uint32_t q = offs[L] + threadIdx.x; q < offs[L + 1]; q += blockDim.x) {
-            Node& nd = nodes[q];
-#pragma unroll
-            for (int s = 0; s < 4; ++s) set_slot(nd, s, ref_box(nodes, nd.child[s], leafbox, nullptr));
-        }
+        for (uint32_t i = 4 * offs[L] + threadIdx.x; i < 4 * offs[L + 1]; i += blockDim.x) refit_slot(P, i);
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        Box r = node_box(nodes[0]);
-        for (int a = 0; a < 3; ++a) {
-            h->lo[a] = r.lo[a];
-            h->hi[a] = r.hi[a];
-        }
+    refit_bounds(P);
+}
+
+__global__ __launch_bounds__(256) void k_refit_insts(uint8_t* base, const rtg_instance* inst, uint32_t n,
+                                                     const uint64_t* reg, uint32_t nreg, uint32_t* status) {
+    __shared__ uint64_t s_reg[kRegistryLds];
+    const TlasParts P = tlas_parts(base);
+    reg = registry_to_lds(reg, nreg, s_reg);
+    __syncthreads();
+    const uint32_t k = blockIdx.x * 256 + threadIdx.x;
+    if (k < n) refit_inst(P, k, inst, reg, nreg, status);
+}
+
+// Consecutive levels [from, to) in one workgroup, deepest first.
+struct LevelArgs {
+    uint32_t off[kReportLevels + 1];
+};
+__global__ __launch_bounds__(1024) void k_refit_levels(uint8_t* base, LevelArgs A, uint32_t from, uint32_t to) {
+    const TlasParts P = tlas_parts(base);
+    for (uint32_t L = to; L-- > from;) {
+        for (uint32_t i = 4 * A.off[L] + threadIdx.x; i < 4 * A.off[L + 1]; i += blockDim.x) refit_slot(P, i);
+        __syncthreads();
     }
+    if (from == 0) refit_bounds(P);
+}
+
+// One level of nodes [first, end).
+__global__ __launch_bounds__(256) void k_refit_level(uint8_t* base, uint32_t first, uint32_t end) {
+    const TlasParts P = tlas_parts(base);
+    const uint32_t i = 4 * first + blockIdx.x * 256 + threadIdx.x;
+    if (i < 4 * end) refit_slot(P, i);
 }
 
 // ---------------------------------------------------------------------------
@@ -980,7 +1040,7 @@ static int wide_hierarchy(rtg_ctx* ctx, const BuildBufs& b, uint32_t n, int tree
             }
             hipLaunchKernelGGL(k_collapse_advance, dim3(1), dim3(64), 0, s, b.off, b.state, kCollapseSteps);
         }
-        hipLaunchKernelGGL(k_build_report, dim3(1), dim3(64), 0, s, b.state, ctx->d_status, b.cb + 6,
+        hipLaunchKernelGGL(k_build_report, dim3(1), dim3(64), 0, s, b.state, b.off, ctx->d_status, b.cb + 6,
                            ctx->build_report);
         RTG_HIP(hipGetLastError());
         RTG_HIP(hipStreamSynchronize(s));
@@ -1025,7 +1085,8 @@ static void radix_tree(const BuildBufs& b, uint32_t n, hipStream_t s) {
 // At most one primitive: the single node.
 static int single_node(rtg_ctx* ctx, const BuildBufs& b, uint32_t n, hipStream_t s, BuildReport& rep) {
     hipLaunchKernelGGL(k_wide_single, dim3(1), dim3(256), 0, s, b.boxes, n, b.nodes, b.va, b.off, b.state);
-    hipLaunchKernelGGL(k_build_report, dim3(1), dim3(64), 0, s, b.state, ctx->d_status, b.cb + 6, ctx->build_report);
+    hipLaunchKernelGGL(k_build_report, dim3(1), dim3(64), 0, s, b.state, b.off, ctx->d_status, b.cb + 6,
+                       ctx->build_report);
     RTG_HIP(hipGetLastError());
     RTG_HIP(hipStreamSynchronize(s));
     rep = *ctx->build_report;
@@ -1035,6 +1096,10 @@ static int single_node(rtg_ctx* ctx, const BuildBufs& b, uint32_t n, hipStream_t
 static SmallOut small_out(const BuildBufs& b) {
     return SmallOut{b.boxes, b.lbox, b.va, b.bin, b.rcount, b.low, b.mid, b.tiers, b.cb};
 }
+
+// Largest level that a refit walks in one workgroup with its neighbours
+// (1,024 lanes, a lane per slot: about 1.2 us per 256 nodes, a launch 3 us).
+constexpr uint32_t kRefitGroupNodes = 768;
 
 // Workgroups of a blob's last kernel: 16 bytes a lane and a few rounds.
 static unsigned finish_grid(uint64_t bytes) { return (unsigned)std::min<uint64_t>(bytes / 4096 / 4 + 1, 4096); }
@@ -1078,10 +1143,35 @@ int refresh_registry(rtg_ctx* ctx) {
     return RTG_OK;
 }
 
-int launch_refit(rtg_ctx* ctx, uint8_t* tlas, const rtg_instance* instances, uint32_t count, hipStream_t s) {
+int launch_refit(rtg_ctx* ctx, uint8_t* tlas, const std::vector<uint32_t>& level_off, const rtg_instance* instances,
+                 uint32_t count, hipStream_t s) {
     LaunchTimer timer(ctx, RTG_KERNEL_REFIT, s);
-    hipLaunchKernelGGL(k_tlas_refit, dim3(1), dim3(256), 0, s, tlas, instances, count, ctx->d_registry,
-                       ctx->registry_count, ctx->d_status);
+    const uint32_t levels = level_off.empty() ? 0 : (uint32_t)level_off.size() - 1;
+    // one workgroup takes about 4 us per 256 instances, a second launch 3 us
+    if (count <= 256 || levels == 0) {
+        hipLaunchKernelGGL(k_tlas_refit, dim3(1), dim3(256), 0, s, tlas, instances, count, ctx->d_registry,
+                           ctx->registry_count, ctx->d_status);
+        RTG_HIP(hipGetLastError());
+        return RTG_OK;
+    }
+    hipLaunchKernelGGL(k_refit_insts, dim3(blocks_for(count, 256)), dim3(256), 0, s, tlas, instances, count,
+                       ctx->d_registry, ctx->registry_count, ctx->d_status);
+    LevelArgs A = {};
+    std::copy(level_off.begin(), level_off.end(), A.off);
+    auto nodes = [&](uint32_t L) { return level_off[L + 1] - level_off[L]; };
+    for (uint32_t to = levels; to > 0;) {
+        // runs of levels that one workgroup walks faster than a launch each
+        uint32_t from = to, most = 0;
+        while (from > 0 && nodes(from - 1) <= kRefitGroupNodes) most = std::max(most, nodes(--from));
+        if (from < to) {
+            hipLaunchKernelGGL(k_refit_levels, dim3(1), dim3(most <= 256 ? 256 : 1024), 0, s, tlas, A, from, to);
+        } else {
+            --from;
+            hipLaunchKernelGGL(k_refit_level, dim3(blocks_for(4ull * nodes(from), 256)), dim3(256), 0, s, tlas,
+                               level_off[from], level_off[from + 1]);
+        }
+        to = from;
+    }
     RTG_HIP(hipGetLastError());
     return RTG_OK;
 }
@@ -1200,7 +1290,7 @@ extern "C" int rtg_blas_build(rtg_ctx* ctx, const rtg_geometry* geoms, uint32_t 
         return RTG_ERROR_DEVICE;
     }
     uint64_t addr = reinterpret_cast<uint64_t>(blob);
-    ctx->structures[addr] = AsRecord{kKindBlas, n, L.node_count, L.total};
+    ctx->structures[addr] = AsRecord{kKindBlas, n, L.node_count, L.total, {}};
     registry_commit(ctx, new_reg, ctx->registry_count + 1);
     *out = addr;
     return RTG_OK;
@@ -1248,7 +1338,9 @@ extern "C" int rtg_tlas_build(rtg_ctx* ctx, const rtg_instance* instances, uint3
         return RTG_ERROR_DEVICE;
     }
     uint64_t addr = reinterpret_cast<uint64_t>(blob);
-    ctx->structures[addr] = AsRecord{kKindTlas, n, L.node_count, L.total};
+    std::vector<uint32_t> level_off;
+    if (rep.levels <= kReportLevels) level_off.assign(rep.off, rep.off + rep.levels + 1);
+    ctx->structures[addr] = AsRecord{kKindTlas, n, L.node_count, L.total, level_off};
     *out = addr;
     return RTG_OK;
 }
@@ -1262,7 +1354,8 @@ extern "C" int rtg_tlas_refit(rtg_ctx* ctx, rtg_tlas tlas, const rtg_instance* i
                 "rtg_tlas_refit: 0x%llx is not a TLAS of this context", (unsigned long long)tlas);
     RTG_REQUIRE(it->second.prim_count == count, RTG_ERROR_INVALID_ARGUMENT,
                 "rtg_tlas_refit: %u instances, the TLAS was built with %u", count, it->second.prim_count);
-    return launch_refit(ctx, reinterpret_cast<uint8_t*>(tlas), instances, count, reinterpret_cast<hipStream_t>(stream));
+    return launch_refit(ctx, reinterpret_cast<uint8_t*>(tlas), it->second.level_off, instances, count,
+                        reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" int rtg_tlas_clone(rtg_ctx* ctx, rtg_tlas src, rtg_tlas* out, void* stream) {

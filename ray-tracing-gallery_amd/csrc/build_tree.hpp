@@ -837,8 +837,10 @@ struct CollapseState {
     uint32_t level, nodes, done, pad;
 };
 // What the host reads after a build's kernels (host memory, written by the device).
+constexpr uint32_t kReportLevels = 60;
 struct BuildReport {
     uint32_t levels, nodes, done, status, nan_boxes, pad[3];
+    uint32_t off[kReportLevels + 1];  // the first level offsets
 };
 
 // The first levels, by one workgroup, until one holds more than `most`
@@ -947,8 +949,10 @@ __global__ void k_collapse_advance(const uint32_t* off, CollapseState* state, ui
     state->done = off[L + 1] == off[L] ? 1u : 0u;
 }
 
-__global__ void k_build_report(const CollapseState* state, const uint32_t* status, const uint32_t* nan_boxes,
-                               BuildReport* out) {
+__global__ __launch_bounds__(64) void k_build_report(const CollapseState* state, const uint32_t* off,
+                                                     const uint32_t* status, const uint32_t* nan_boxes,
+                                                     BuildReport* out) {
+    if (threadIdx.x <= min(state->level, kReportLevels)) out->off[threadIdx.x] = off[threadIdx.x];
     if (threadIdx.x != 0) return;
     out->levels = state->level;
     out->nodes = state->nodes;

@@ -34,6 +34,7 @@ using namespace rtg;
 struct rtg_frames {
     rtg_ctx* ctx = nullptr;
     uint32_t count = 0;  // instances of the TLAS
+    std::vector<uint32_t> level_off;  // and its levels
     std::vector<FrameSlot> slots;
 };
 
@@ -70,6 +71,7 @@ extern "C" int rtg_frames_create(rtg_ctx* ctx, rtg_tlas tlas, uint32_t frames_in
     rtg_frames* f = new rtg_frames();
     f->ctx = ctx;
     f->count = it->second.prim_count;
+    f->level_off = it->second.level_off;
     f->slots.resize(frames_in_flight);
     const size_t bytes = std::max<size_t>(1, f->count) * sizeof(rtg_instance);
     // the template's source instances seed every slot's mapping
@@ -120,7 +122,7 @@ extern "C" int rtg_frames_submit(rtg_frames* f, uint64_t frame, const rtg_image_
     RTG_HIP(hipSetDevice(f->ctx->device));
     if (f->count)
         RTG_HIP(hipMemcpyAsync(s.dev, s.host, (size_t)f->count * sizeof(rtg_instance), hipMemcpyHostToDevice, st));
-    int r = launch_refit(f->ctx, reinterpret_cast<uint8_t*>(s.tlas), s.dev, f->count, st);
+    int r = launch_refit(f->ctx, reinterpret_cast<uint8_t*>(s.tlas), f->level_off, s.dev, f->count, st);
     if (r != RTG_OK) return r;
     rtg_image_job j = *job;
     j.tlas = s.tlas;

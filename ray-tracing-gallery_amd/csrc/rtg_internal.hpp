@@ -38,6 +38,9 @@ struct AsRecord {
     uint32_t prim_count;
     uint32_t node_count;
     uint64_t size;
+    // TLAS: first node of each level and the node count (empty for more
+    // levels than a build reports)
+    std::vector<uint32_t> level_off;
 };
 
 // Grow-only device buffer.
@@ -217,6 +220,8 @@ void suppress_timing_on_this_thread();
 // Takes the device address of rtg_trace_rays_static's scratch array on
 // `device` (which must be current); once per device, at rtg_create.
 int static_scratch_init(int device);
-// One-kernel refit of the TLAS blob at `tlas` (no registry lookup).
-int launch_refit(rtg_ctx* ctx, uint8_t* tlas, const rtg_instance* instances, uint32_t count, hipStream_t stream);
+// Refit of the TLAS blob at `tlas`, a structure with the levels `level_off`
+// (AsRecord) or a copy of one.
+int launch_refit(rtg_ctx* ctx, uint8_t* tlas, const std::vector<uint32_t>& level_off, const rtg_instance* instances,
+                 uint32_t count, hipStream_t stream);
 }  // namespace rtg

@@ -32,6 +32,7 @@ struct ServerScene {
     uint64_t tlas_bytes;
     uint32_t instance_count;
     rtg_scene_bindings bindings;
+    std::vector<uint32_t> level_off;  // levels of its TLAS (AsRecord)
 };
 
 struct PendingRequest {
@@ -155,7 +156,7 @@ bool rtg_server::launch(Slot& s) {
             if (hipMemcpyAsync(copy, reinterpret_cast<const void*>(sc.tlas), sc.tlas_bytes, hipMemcpyDeviceToDevice,
                                s.stream) != hipSuccess)
                 return false;
-            if (launch_refit(ctx, copy, r.instances, sc.instance_count, s.stream) != RTG_OK) return false;
+            if (launch_refit(ctx, copy, sc.level_off, r.instances, sc.instance_count, s.stream) != RTG_OK) return false;
             tlas = reinterpret_cast<uint64_t>(copy);
         }
         rtg_image_job& j = jobs[k];
@@ -349,6 +350,7 @@ extern "C" int rtg_server_add_scene(rtg_server* srv, rtg_tlas tlas, const rtg_sc
     ServerScene sc;
     sc.tlas = tlas;
     sc.tlas_bytes = it->second.size;
+    sc.level_off = it->second.level_off;
     sc.instance_count = it->second.prim_count;
     sc.bindings = *scene;
     srv->scenes.push_back(sc);

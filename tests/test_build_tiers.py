@@ -11,7 +11,8 @@ import torch
 
 import oracle_host as oh
 from rtg import abi, scenes
-from rtg.device import device_to_host
+from rtg.device import DeviceScene, device_to_host
+from rtg.frames import FrameDriver
 from rtg.lib import check, load
 
 pytestmark = pytest.mark.gpu
@@ -99,3 +100,52 @@ def test_nine_geometries(ctx):
         o = np.frombuffer(C.string_at(p.value, size.value), dtype=np.uint8).copy()
         oh.lib().orc_free(p)
         assert np.array_equal(g, o)
+
+
+def _masked(blob, n):
+    """TLAS blob bytes without the BLAS addresses (device or host pointers)."""
+    b = np.frombuffer(blob, dtype=np.uint8).copy()
+    hdr = b[:128].view(np.uint64)
+    for off, at in ((int(hdr[9]), 48), (int(hdr[10]), 56)):
+        b[off:off + 64 * n].reshape(n, 64)[:, at:at + 8] = 0
+    return b
+
+
+@pytest.mark.parametrize("n", [1, 2, 256, 257, 1500, 5003, 8192, 8193, 20011])
+def test_tlas_bytes_and_refit_equal_the_oracle(ctx, n):
+    """The build, and the update whose launches go by the levels' sizes: of a
+    clone, of the structure itself, and of a frame slot's copy."""
+    rng = scenes.Rng(7 + n)
+    s = scenes.Scene("crowd")
+    s.add_mesh(scenes.icosphere(1))
+    s.add_mesh(scenes.quad(2.0, 1.0))
+    s.models.append(scenes.Model(0, [(0, 0, -1)]))
+    scenes._base_textures(s, 7)
+    side = np.sqrt(n)
+    p = rng.uniform(3 * n, -side, side).reshape(n, 3)
+    for k in range(n):
+        s.instances.append(scenes.InstanceData(scenes.affine(p[k], None, 0.7), 0, k % 2))
+    ds, hs = DeviceScene(ctx, s), oh.HostScene(s)
+    assert np.array_equal(_masked(ds.as_bytes(ds.tlas), n), _masked(hs.tlas.bytes(), n))
+    turn = rng.uniform(3 * n).reshape(n, 3)
+    step = rng.uniform(3 * n, -1.0, 1.0).reshape(n, 3)
+    xf = [scenes.affine(p[k] + step[k], scenes.rotation_from_uniform(*turn[k]), 0.9) for k in range(n)]
+    clone, buf = ds.clone_tlas(), ds.instance_buffer(xf)
+    torch.cuda.synchronize()
+    hs.refit(xf)
+    want = _masked(hs.tlas.bytes(), n)
+    for tlas in (clone, ds.tlas):
+        ds.refit(buf, tlas=tlas)
+        torch.cuda.synchronize()
+        assert np.array_equal(_masked(ds.as_bytes(tlas), n), want)
+    driver = FrameDriver(ds, 1)
+    inst, slot = driver.begin(0)
+    inst["transform"] = np.asarray(xf, np.float32)
+    s.width = s.height = 8
+    out = ds.make_outputs()
+    driver.submit(0, ds.job(out))
+    torch.cuda.synchronize()
+    assert np.array_equal(_masked(ds.as_bytes(slot), n), want)
+    driver.close()
+    check(load().rtg_tlas_destroy(ctx.ptr, clone), "rtg_tlas_destroy")
+    ds.destroy()

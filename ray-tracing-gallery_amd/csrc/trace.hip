@@ -23,10 +23,10 @@ namespace rtg {
 
 constexpr int kTraceThreads = 256;
 constexpr int kCountSlots = 16;
-constexpr int kFeedLevel = 8;    // counts[kFeedLevel + level]: feed counter of a trace level
-constexpr int kFeedShadow = 12;  // counts[kFeedShadow]: feed counter of the shadow queue
+// queues of the feed counters (Frame::feeds): the trace levels, then
+constexpr int kFeedShadow = 4;      // the shadow queue
+constexpr int kFeedShadowRest = 5;  // the shadow rays after those of trace level 0
 constexpr int kShadowFirst = 5;      // counts[5]: shadow rays of trace level 0
-constexpr int kFeedShadowRest = 13;  // counts[13]: feed counter of the shadow rays after them
 constexpr int kStatusSlot = 14;      // counts[14]: status bits of the trace (merged into the context's)
 constexpr int kPartAll = 0, kPartFirst = 1, kPartRest = 2;  // parts of the shadow queue
 // path of a shadow-queue padding slot (after an odd count of a path's rays)
@@ -107,8 +107,8 @@ struct Frame {
     float2* hit_b;       // u, v
     Queue sq;            // shadow rays
     uint32_t* counts;    // [0..3] queue sizes per trace level, [4] shadow rays, [5] shadow
-                         // rays of level 0, [8..11] feed counters per trace level,
-                         // [12], [13] shadow feed counters
+                         // rays of level 0, [14] status bits
+    uint32_t* feeds;     // feed counters of queue q: feeds[q + k * kFeedStride]
     uint64_t* counters;  // rtg_trace_counters
     uint2* spill;
     uint32_t order;           // pixel order along paths (0 row-major, 1 8x8 bands)
@@ -202,7 +202,7 @@ template <bool OCC, bool COUNT>
 __global__ __launch_bounds__(kTraceThreads) void k_trace_rays(const uint8_t* tlas, SceneView S, const rtg_ray* rays,
                                                               uint32_t n, uint32_t ray_flags, uint32_t cull_mask,
                                                               uint32_t sbt_offset, rtg_hit* hits, uint32_t* occ,
-                                                              uint2* spill, uint32_t* feed_counter,
+                                                              uint2* spill, uint32_t* feeds, uint32_t feed_stride,
                                                               uint64_t* counters, uint32_t* status, int refill_min,
                                                               uint32_t feed_chunk, int stack_lds) {
     extern __shared__ uint2 s_stack[];
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_rays(const uint8_t* tla
     TravCounters cnt = {0, 0, 0, 0, 0};
     Traverser<OCC, COUNT> tr;
     WaveFeeder feeder;
-    feeder.init(feed_chunk);
+    feeder.init(n, feed_chunk, 64, gtid >> 6, gridDim.x * (kTraceThreads / 64), feed_stride);
     bool active = false;
     uint32_t ray = 0;
     uint32_t it = 0;  // iteration parity: leaf visits on even, instance entries on odd iterations
@@ -221,7 +221,7 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_rays(const uint8_t* tla
         ++it;
         uint64_t idle = __ballot(!active);
         if (want_refill(idle, feeder, refill_min)) {
-            uint32_t id = feeder.feed(idle, !active, feed_counter, n);
+            uint32_t id = feeder.feed(idle, !active, feeds, n);
             if (id != ~0u) {
                 const float4* rp = reinterpret_cast<const float4*>(rays + id);
                 float4 a = rp[0], b = rp[1];
@@ -258,8 +258,9 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_rays(const uint8_t* tla
 // ---------------------------------------------------------------------------
 // Wavefront pipeline
 // ---------------------------------------------------------------------------
-__global__ void k_frame_begin(uint32_t* counts, uint64_t* counters, bool reset_counters) {
+__global__ void k_frame_begin(uint32_t* counts, uint32_t* feeds, uint64_t* counters, bool reset_counters) {
     if (threadIdx.x < kCountSlots) counts[threadIdx.x] = 0;
+    feeds[threadIdx.x] = 0;
     if (reset_counters && threadIdx.x < kCounterSlots) counters[threadIdx.x] = 0;
 }
 
@@ -272,8 +273,8 @@ __global__ void k_shadow_snapshot(uint32_t* counts) {
     if (threadIdx.x == 0) counts[kShadowFirst] = counts[4];
 }
 
-__global__ void k_zero_u32(uint32_t* p, uint32_t n) {
-    if (threadIdx.x < n) p[threadIdx.x] = 0;
+__global__ void k_zero_feed(uint32_t* feed, uint32_t stride) {
+    if (threadIdx.x < kFeedGroups) feed[threadIdx.x * stride] = 0;
 }
 
 __global__ void k_reset_counters(uint64_t* counters, uint64_t primary) {
@@ -351,7 +352,7 @@ __device__ __forceinline__ void trace_closest(Frame F, int level, const uint32_t
     TravCounters cnt = {0, 0, 0, 0, 0};
     Traverser<false, COUNT> tr;
     WaveFeeder feeder;
-    feeder.init(F.feed_chunk);
+    feeder.init(n, F.feed_chunk, 64, gtid >> 6, gridDim.x * (kTraceThreads / 64));
     bool active = false;
     uint32_t slot = 0;
     const JobDev* J = SINGLE ? &F.jobs[0] : nullptr;
@@ -363,7 +364,7 @@ __device__ __forceinline__ void trace_closest(Frame F, int level, const uint32_t
         ++it;
         uint64_t idle = __ballot(!active);
         if (want_refill(idle, feeder, F.refill_closest)) {
-            uint32_t id = feeder.feed(idle, !active, &F.counts[kFeedLevel + level], n);
+            uint32_t id = feeder.feed(idle, !active, F.feeds + level, n);
             if (id != ~0u) {
                 slot = id;
                 uint32_t path = Q.path[id];
@@ -764,7 +765,7 @@ __global__ __launch_bounds__(256) void k_shade(Frame F, int level, const uint32_
 __device__ inline void shadow_part(const Frame& F, int part, uint32_t& lo, uint32_t& hi, uint32_t*& feed) {
     hi = min(part == kPartFirst ? F.counts[kShadowFirst] : F.counts[4], F.shadow_cap);
     lo = min(part == kPartRest ? F.counts[kShadowFirst] : 0u, hi);
-    feed = &F.counts[part == kPartRest ? kFeedShadowRest : kFeedShadow];
+    feed = F.feeds + (part == kPartRest ? kFeedShadowRest : kFeedShadow);
 }
 
 // The pair of shadow-queue entries 2q, 2q + 1 of [lo, hi): a path's shadow
@@ -816,7 +817,7 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_occlusion(Frame F, uint
     TravCounters cnt = {0, 0, 0, 0, 0};
     PairTraverser<COUNT> tr;
     WaveFeeder feeder;
-    feeder.init(F.feed_chunk);
+    feeder.init(npairs, F.feed_chunk, 64, gtid >> 6, gridDim.x * (kTraceThreads / 64));
     bool active = false;
     uint32_t e0 = 0, started = 0, path = 0;
     const JobDev* J = nullptr;
@@ -990,7 +991,7 @@ __global__ __launch_bounds__(256) void k_resolve(Frame F, uint64_t total_pixels)
 struct FrameArena {
     DeviceBuffer buf;
     DeviceBuffer spill;
-    DeviceBuffer feed;  // feed counter of rtg_trace_rays
+    DeviceBuffer feed;  // feed counters of rtg_trace_rays
     uint64_t paths_cap = 0, shadow_cap = 0;
     uint32_t jobs_cap = 0;
     JobDev* h_jobs = nullptr;  // pinned staging
@@ -1002,6 +1003,7 @@ struct FrameArena {
     Frame F;
     JobDev* d_jobs = nullptr;
     uint32_t* d_counts = nullptr;
+    uint32_t* d_feeds = nullptr;
     // grow to exactly the size asked (no headroom): a server slot's arena,
     // whose device bytes count against an HBM budget
     bool exact = false;
@@ -1064,8 +1066,9 @@ size_t frame_bytes(uint64_t paths, uint64_t shadow, uint32_t njobs) {
     carve_size<float4>(off, shadow);
     carve_size<uint32_t>(off, shadow);
     carve_size<uint32_t>(off, kCountSlots);
+    carve_size<uint32_t>(off, kFeedWords);
     carve_size<JobDev>(off, njobs);
-    return off + 4096;
+    return off + 2048;
 }
 
 static int trace_grid(rtg_ctx* ctx, const Tuning& tune) {
@@ -1080,8 +1083,7 @@ size_t spill_bytes(rtg_ctx* ctx, const Tuning& tune) {
 }
 
 static int ensure_spill(rtg_ctx* ctx, FrameArena* a, const Tuning& tune) {
-    if (a->spill.ensure(spill_bytes(ctx, tune), !a->exact) != RTG_OK) return RTG_ERROR_OUT_OF_MEMORY;
-    return a->feed.ensure(256, !a->exact);
+    return a->spill.ensure(spill_bytes(ctx, tune), !a->exact);
 }
 
 size_t arena_bytes_after(const FrameArena* a, uint64_t paths, uint64_t shadow, uint32_t njobs) {
@@ -1136,6 +1138,7 @@ static int ensure_frame(rtg_ctx* ctx, FrameArena* a, uint64_t paths, uint64_t sh
         F.sq.d = c.take<float4>(S);
         F.sq.path = c.take<uint32_t>(S);
         a->d_counts = c.take<uint32_t>(kCountSlots);
+        a->d_feeds = c.take<uint32_t>(kFeedWords);
         a->d_jobs = c.take<JobDev>(NJ);
         a->paths_cap = P;
         a->shadow_cap = S;
@@ -1258,6 +1261,7 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
     F.njobs = P.njobs;
     F.paths = P.paths;
     F.counts = a->d_counts;
+    F.feeds = a->d_feeds;
     F.counters = ctx->d_counters;
     F.spill = reinterpret_cast<uint2*>(a->spill.ptr);
     F.order = (uint32_t)tune.path_order;
@@ -1272,7 +1276,7 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
     const unsigned G = (unsigned)trace_grid(ctx, tune);
     const size_t lds = stack_lds_bytes(tune.stack_lds);  // a traversal workgroup's stacks
     const unsigned Gsmall = (unsigned)std::min<uint64_t>((P.paths + 255) / 256, (uint64_t)ctx->cu_count * 16);
-    hipLaunchKernelGGL(k_frame_begin, dim3(1), dim3(64), 0, s, a->d_counts, ctx->d_counters, cnt);
+    hipLaunchKernelGGL(k_frame_begin, dim3(1), dim3(kFeedWords), 0, s, a->d_counts, a->d_feeds, ctx->d_counters, cnt);
     {
         LaunchTimer t(ctx, RTG_KERNEL_RAYGEN, s, timed);
         hipLaunchKernelGGL(k_raygen, dim3(Gsmall), dim3(256), 0, s, F, cnt);
@@ -1441,12 +1445,12 @@ static int check_ray_query(rtg_ctx* ctx, rtg_tlas tlas, const rtg_ray* rays, uin
     return RTG_OK;
 }
 
-// Clears the feed counter and launches the query kernel on `G` persistent
+// Clears the feed counters (`feed_stride` words apart) and launches the query kernel on `G` persistent
 // blocks whose spill stacks start at `spill` (G * kTraceThreads lanes).
 static void launch_ray_query(rtg_ctx* ctx, rtg_tlas tlas, const rtg_scene_bindings* scene, const rtg_ray* rays,
                              uint32_t count, uint32_t mode, uint32_t ray_flags, uint32_t cull_mask,
                              uint32_t sbt_offset, rtg_hit* hits, uint32_t* occluded, uint2* spill, uint32_t* feed,
-                             unsigned G, bool timed, hipStream_t s) {
+                             uint32_t feed_stride, unsigned G, bool timed, hipStream_t s) {
     SceneView S;
     S.models = scene ? reinterpret_cast<const rtg_model_info*>(scene->model_info) : nullptr;
     S.textures = scene ? reinterpret_cast<const rtg_texture*>(scene->textures) : nullptr;
@@ -1455,14 +1459,15 @@ static void launch_ray_query(rtg_ctx* ctx, rtg_tlas tlas, const rtg_scene_bindin
     S.texture_count = scene ? scene->texture_count : 0;
     const bool cnt = ctx->counters_enabled;
     uint8_t* tl = reinterpret_cast<uint8_t*>(tlas);
-    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, feed, 1u);
+    if (count > G * kTraceThreads)  // else the waves' first chunks are all there is
+        hipLaunchKernelGGL(k_zero_feed, dim3(1), dim3(64), 0, s, feed, feed_stride);
     // the primary ray count of a ray query is the query size
     if (cnt) hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, ctx->d_counters, (uint64_t)count);
     LaunchTimer t(ctx, mode == RTG_QUERY_CLOSEST ? RTG_KERNEL_TRACE_CLOSEST : RTG_KERNEL_TRACE_OCCLUSION, s, timed);
     cull_mask &= 0xffu;
 #define RTG_LAUNCH_RAYS(OCC, CNT)                                                                                \
     hipLaunchKernelGGL((k_trace_rays<OCC, CNT>), dim3(G), dim3(kTraceThreads), stack_lds_bytes(ctx->tune.stack_lds), \
-                       s, tl, S, rays, count, ray_flags, cull_mask, sbt_offset, hits, occluded, spill, feed,         \
+                       s, tl, S, rays, count, ray_flags, cull_mask, sbt_offset, hits, occluded, spill, feed, feed_stride, \
                        ctx->d_counters, ctx->d_status, ctx->tune.refill_rays, (uint32_t)ctx->tune.feed_chunk,       \
                        ctx->tune.stack_lds)
     if (mode == RTG_QUERY_CLOSEST) {
@@ -1490,16 +1495,17 @@ extern "C" int rtg_trace_rays(rtg_ctx* ctx, rtg_tlas tlas, const rtg_scene_bindi
                 "rtg_trace_rays: the frame state of stream %p is in use by another call (a context is used by one "
                 "thread at a time)",
                 (void*)s);
-    if (ensure_spill(ctx, a, ctx->tune) != RTG_OK) return RTG_ERROR_OUT_OF_MEMORY;
+    if (ensure_spill(ctx, a, ctx->tune) != RTG_OK || a->feed.ensure(kFeedWords * sizeof(uint32_t)) != RTG_OK)
+        return RTG_ERROR_OUT_OF_MEMORY;
     const unsigned G = (unsigned)std::min<uint64_t>((count + kTraceThreads - 1) / kTraceThreads, trace_grid(ctx));
     launch_ray_query(ctx, tlas, scene, rays, count, mode, ray_flags, cull_mask, sbt_offset, hits, occluded,
-                     reinterpret_cast<uint2*>(a->spill.ptr), reinterpret_cast<uint32_t*>(a->feed.ptr), G, true, s);
+                     reinterpret_cast<uint2*>(a->spill.ptr), reinterpret_cast<uint32_t*>(a->feed.ptr), kFeedStride, G, true, s);
     RTG_HIP(hipGetLastError());
     return RTG_OK;
 }
 
 // ---------------------------------------------------------------------------
-// rtg_trace_rays_static: the ray query with its scratch (the feed counter and
+// rtg_trace_rays_static: the ray query with its scratch (the feed counters and
 // the spill stacks of kStaticBlocks persistent workgroups) in a file-scope
 // device array instead of the context's arenas, for callers that cannot
 // allocate. Every GPU holds its own copy of `scratch` while the process
@@ -1558,7 +1564,8 @@ extern "C" int rtg_trace_rays_static(rtg_ctx* ctx, rtg_tlas tlas, const rtg_scen
     const unsigned G = (unsigned)std::min<uint64_t>(
         std::min<uint64_t>((count + kTraceThreads - 1) / kTraceThreads, trace_grid(ctx)), kStaticBlocks);
     launch_ray_query(ctx, tlas, scene, rays, count, mode, ray_flags, cull_mask, sbt_offset, hits, occluded,
-                     reinterpret_cast<uint2*>(base + kStaticFeedBytes), reinterpret_cast<uint32_t*>(base), G, false,
+                     reinterpret_cast<uint2*>(base + kStaticFeedBytes), reinterpret_cast<uint32_t*>(base),
+                     (uint32_t)(kStaticFeedBytes / kFeedGroups / sizeof(uint32_t)), G, false,
                      reinterpret_cast<hipStream_t>(stream));
     RTG_HIP(hipGetLastError());
     return RTG_OK;

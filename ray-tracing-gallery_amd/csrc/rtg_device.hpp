@@ -1074,6 +1074,457 @@ struct PairTraverser {
     __device__ inline uint32_t occluded(uint32_t started) const { return started & ~alive; }
 };
 
+// ---------------------------------------------------------------------------
+// Four lanes per ray. A launch with fewer rays than the GPU has lanes is as
+// long as its longest rays, and a ray's time is the chain of its visits: a
+// node's loads, four slab tests, the ordering and the stack, some 150
+// instructions in one lane. A quad of lanes makes the visit together: lane s
+// tests slot s (seven 4-byte loads instead of seven 16-byte ones), the slots
+// are ranked with quad permutes, the overlapped ones push their entries with
+// one store; an instance's rays are transformed, and their components
+// inverted, a row per lane; a triangle's vertices are sheared and its edge
+// functions formed a vertex per lane. The visits, their order and every
+// operation's operands and rounding are those of Traverser.
+// ---------------------------------------------------------------------------
+template <int Ctrl>
+__device__ __forceinline__ float quad_perm(float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), Ctrl, 0xf, 0xf, true));
+}
+template <int Ctrl>
+__device__ __forceinline__ uint32_t quad_perm(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, Ctrl, 0xf, 0xf, true);
+}
+// lane K's value in all four lanes
+template <int K, class T>
+__device__ __forceinline__ T quad_bcast(T x) {
+    return quad_perm<K * 0x55>(x);
+}
+// lane (i + K) & 3's value in lane i
+template <int K>
+__device__ __forceinline__ float quad_rot(float x) {
+    return quad_perm<K == 1 ? 0x39 : K == 2 ? 0x4E : 0x93>(x);
+}
+__device__ __forceinline__ uint32_t quad_or(uint32_t x) {
+    x |= quad_perm<0xB1>(x);
+    return x | quad_perm<0x4E>(x);
+}
+__device__ __forceinline__ uint32_t quad_mask(bool b, uint32_t sub) { return quad_or(b ? 1u << sub : 0u); }
+
+// The watertight test of tri_test with vertex s in lane s (0..2) of a quad:
+// lane 0 forms V, lane 1 W, lane 2 U, each from its vertex and the one before.
+// axes: kx | ky << 2 | kz << 4.
+__device__ inline bool quad_tri_test(const float4& vtx, uint32_t sub, V3 o, float sx, float sy, float sz,
+                                     uint32_t axes, float tmin, float tmax, float& t_out, float& u_out,
+                                     float& v_out) {
+    const V3 P = v3(vtx.x, vtx.y, vtx.z) - o;
+    const int kx = (int)(axes & 3u), ky = (int)((axes >> 2) & 3u), kz = (int)(axes >> 4);
+    const float Pz = sel3(P, kz);
+    const float X = sel3(P, kx) - sx * Pz, Y = sel3(P, ky) - sy * Pz;
+    constexpr int kPrev = 2 | (0 << 2) | (1 << 4) | (3 << 6);
+    const float Xp = quad_perm<kPrev>(X), Yp = quad_perm<kPrev>(Y);
+    float E = X * Yp - Y * Xp;
+    const bool tri = sub < 3u;
+    if (quad_or((tri && E == 0.0f) ? 1u : 0u)) E = (float)((double)X * (double)Yp - (double)Y * (double)Xp);
+    const uint32_t signs = quad_or((tri && E < 0.0f ? 1u : 0u) | (tri && E > 0.0f ? 2u : 0u));
+    if (signs == 3u) return false;
+    const float V = quad_bcast<0>(E), W = quad_bcast<1>(E), U = quad_bcast<2>(E);
+    const float det = (U + V) + W;
+    if (det == 0.0f) return false;
+    const float Z = sz * Pz;
+    const float Ts = (U * quad_bcast<0>(Z) + V * quad_bcast<1>(Z)) + W * quad_bcast<2>(Z);
+    // the three quotients a lane each
+    const float q = (sub == 0u ? Ts : sub == 1u ? V : W) / det;
+    const float t = quad_bcast<0>(q);
+    if (!(t >= tmin && t <= tmax)) return false;
+    t_out = t;
+    u_out = quad_bcast<1>(q);
+    v_out = quad_bcast<2>(q);
+    return true;
+}
+
+// Shear setup of the watertight test (as ray_setup).
+__device__ inline void shear_setup(V3 d, V3 inv, float& sx, float& sy, float& sz, uint32_t& axes) {
+    const float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
+    const int kz = ax > ay ? (ax > az ? 0 : 2) : (ay > az ? 1 : 2);
+    int kx = kz + 1 == 3 ? 0 : kz + 1;
+    int ky = kx + 1 == 3 ? 0 : kx + 1;
+    if (sel3(d, kz) < 0.0f) {
+        const int t = kx;
+        kx = ky;
+        ky = t;
+    }
+    sz = sel3(inv, kz);
+    sx = sel3(d, kx) * sz;
+    sy = sel3(d, ky) * sz;
+    axes = (uint32_t)kx | ((uint32_t)ky << 2) | ((uint32_t)kz << 4);
+}
+
+// The ray's stack, shared by its four lanes: consecutive entries of a ray lie
+// side by side in LDS (a visit's pushes are one conflict-free store), rays an
+// odd number of entries apart; deeper entries in the spill areas of the
+// quad's lanes.
+struct QuadStack {
+    uint2* lds;
+    uint2* spill;
+    int lds_n;
+    int sp;
+    // `entries`: 8-byte entries per lane the launch's LDS holds
+    __device__ inline void init(uint2* lds_words, int entries, uint8_t* spill_area, uint32_t gtid, int lane) {
+        lds_n = 4 * entries - 1;
+        lds = lds_words + (lane >> 2) * lds_n;
+        spill = reinterpret_cast<uint2*>(spill_area + (size_t)(gtid & ~3u) * kSpillLaneBytes);
+        sp = 0;
+    }
+    __device__ inline void put(int at, uint32_t ref, uint32_t word) {
+        if (at < lds_n) {
+            lds[at] = make_uint2(ref, word);
+        } else {
+            rtg_u2v v = {ref, word};
+            *(RTG_GLOBAL rtg_u2v*)(spill + (at - lds_n)) = v;
+        }
+    }
+    __device__ inline uint2 pop() {
+        --sp;
+        return sp < lds_n ? lds[sp] : gld_u2(spill + (sp - lds_n));
+    }
+};
+
+template <bool OCCLUSION>
+struct QuadTraverser {
+    V3 wo, wd, winv;     // world ray
+    V3 ao, ainv;         // the ray of the structure being walked
+    float sx, sy, sz;    // shear of the object-space ray
+    uint32_t axes;       // kx | ky << 2 | kz << 4
+    const Node* nodes;
+    const TriRec* tris;
+    float tmin, tcur;
+    uint32_t ray_flags, cull_mask, sbt_offset;
+    uint32_t inst_index, inst_flags;
+    uint32_t cur;
+    bool in_blas;
+    HitRec best;
+
+    __device__ inline void start(const TlasView& T, V3 o, V3 d, float tmin_, float tmax_, uint32_t flags,
+                                 uint32_t mask, uint32_t sbt, QuadStack& st) {
+        wo = o;
+        wd = d;
+        winv = v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+        ao = wo;
+        ainv = winv;
+        in_blas = false;
+        nodes = T.nodes;
+        tris = nullptr;
+        tmin = tmin_;
+        tcur = tmax_;
+        ray_flags = flags;
+        cull_mask = mask;
+        sbt_offset = sbt;
+        inst_index = inst_flags = 0;
+        best.t = tmax_;
+        best.u = best.v = 0.0f;
+        best.inst = best.prim = best.geom = RTG_NO_HIT;
+        st.sp = 0;
+        cur = 0;
+    }
+
+    __device__ inline int done() const { return best.inst != RTG_NO_HIT ? kRayHit : kRayMiss; }
+
+    __device__ inline bool pop(const TlasView& T, QuadStack& st) {
+        while (st.sp > 0) {
+            const uint2 e = st.pop();
+            if (e.x == kSentinel) {
+                in_blas = false;
+                nodes = T.nodes;
+                ao = wo;
+                ainv = winv;
+                continue;
+            }
+            if (!OCCLUSION && u2f(e.y) > tcur) continue;
+            cur = e.x;
+            return true;
+        }
+        return false;
+    }
+
+    __device__ inline int node_step(const TlasView& T, QuadStack& st, uint32_t sub) {
+        const float* np = reinterpret_cast<const float*>(nodes + cur) + sub;
+        const uint32_t ix = (f2u(ainv.x) >> 31) * 4u, iy = (f2u(ainv.y) >> 31) * 4u, iz = (f2u(ainv.z) >> 31) * 4u;
+        const float nx = gld_f32(np + ix), fx = gld_f32(np + (ix ^ 4u));
+        const float ny = gld_f32(np + 8 + iy), fy = gld_f32(np + 8 + (iy ^ 4u));
+        const float nz = gld_f32(np + 16 + iz), fz = gld_f32(np + 16 + (iz ^ 4u));
+        const uint32_t c = gld_u32(np + 24);
+        RayCtx r;
+        r.o = ao;
+        r.inv = ainv;
+        float t;
+        const bool h = slab(nx, fx, ny, fy, nz, fz, r, tmin, tcur, t) && c != kEmpty;
+        const uint32_t hits = quad_mask(h, sub);
+        if (hits == 0u) {
+            if (!pop(T, st)) return done();
+            return kRayActive;
+        }
+        const int nh = __builtin_popcount(hits);
+        if (st.sp + nh - 1 > kStackMax) return kRayOverflow;
+        // rank of this lane's slot among the overlapped ones: in slot order
+        // for occlusion, in ascending (entry distance, slot) order otherwise
+        int rank;
+        if (OCCLUSION) {
+            rank = __builtin_popcount(hits & ((1u << sub) - 1u));
+        } else {
+            const float tt = h ? t : __builtin_nanf("");
+            const float t1 = quad_rot<1>(tt), t2 = quad_rot<2>(tt), t3 = quad_rot<3>(tt);
+            rank = (int)(sub == 3u ? t1 <= tt : t1 < tt) + (int)(sub >= 2u ? t2 <= tt : t2 < tt) +
+                   (int)(sub >= 1u ? t3 <= tt : t3 < tt);
+        }
+        if (h && rank > 0) st.put(st.sp + nh - 1 - rank, c, f2u(t));
+        cur = quad_or(h && rank == 0 ? c : 0u);
+        st.sp += nh - 1;
+        return kRayActive;
+    }
+
+    __device__ inline int instance_step(const TlasView& T, QuadStack& st, uint32_t sub) {
+        // lane s has row s of the world-to-object matrix; lane 3 the BLAS
+        // address, the instance's index and its mask and flags
+        const float4* rp = reinterpret_cast<const float4*>(T.recs + (cur & kFirstMask)) + sub;
+        const float4 m = gld_f4(rp);
+        const uint32_t blo = quad_bcast<3>(f2u(m.x)), bhi = quad_bcast<3>(f2u(m.y));
+        const uint32_t mf = quad_bcast<3>(f2u(m.w));
+        const uint8_t* bb = reinterpret_cast<const uint8_t*>((uint64_t)blo | ((uint64_t)bhi << 32));
+        if (((mf & 0xffu) & cull_mask) == 0 || bb == nullptr) {
+            if (!pop(T, st)) return done();
+            return kRayActive;
+        }
+        if (st.sp >= kStackMax) return kRayOverflow;
+        if (sub == 0u) st.put(st.sp, kSentinel, 0xff800000u);
+        ++st.sp;
+        inst_index = quad_bcast<3>(f2u(m.z));
+        inst_flags = (mf >> 8) & 0xffu;
+        const AsHeader* bh = reinterpret_cast<const AsHeader*>(bb);
+        nodes = reinterpret_cast<const Node*>(bb + gld_u64(&bh->nodes_off));
+        tris = reinterpret_cast<const TriRec*>(bb + gld_u64(&bh->prims_off));
+        const float po = ((m.x * wo.x + m.y * wo.y) + m.z * wo.z) + m.w;
+        const float pd = (m.x * wd.x + m.y * wd.y) + m.z * wd.z;
+        const float pi = 1.0f / pd;
+        ao = v3(quad_bcast<0>(po), quad_bcast<1>(po), quad_bcast<2>(po));
+        const V3 d = v3(quad_bcast<0>(pd), quad_bcast<1>(pd), quad_bcast<2>(pd));
+        ainv = v3(quad_bcast<0>(pi), quad_bcast<1>(pi), quad_bcast<2>(pi));
+        shear_setup(d, ainv, sx, sy, sz, axes);
+        in_blas = true;
+        cur = 0;
+        return kRayActive;
+    }
+
+    __device__ inline int leaf_step(const TlasView& T, const SceneView& S, QuadStack& st, uint32_t sub) {
+        const uint32_t first = cur & kFirstMask;
+        const uint32_t count = ((cur >> 27) & 0xfu) + 1u;
+        for (uint32_t k = first; k < first + count; ++k) {
+            const float4 vtx = gld_f4(reinterpret_cast<const float4*>(tris + k) + (sub < 3u ? sub : 2u));
+            float t, u, v;
+            if (!quad_tri_test(vtx, sub, ao, sx, sy, sz, axes, tmin, tcur, t, u, v)) continue;
+            const uint32_t prim = quad_bcast<0>(f2u(vtx.w)), gword = quad_bcast<1>(f2u(vtx.w));
+            const uint32_t geom = gword & ~kNonOpaqueBit;
+            if (!OCCLUSION &&
+                !(t < best.t || (t == best.t && key_less(inst_index, geom, prim, best.inst, best.geom, best.prim))))
+                continue;
+            if (!is_opaque(gword, inst_flags, ray_flags)) {
+                const uint32_t group = (gld_u32(&T.src[inst_index].sbt_offset_and_flags) & 0xffffffu) + sbt_offset;
+                if (group < RTG_HIT_GROUP_COUNT) {
+                    if (!alpha_clip_keep(S, T.src, inst_index, geom, prim, u, v)) continue;
+                }
+            }
+            best.t = t;
+            best.u = u;
+            best.v = v;
+            best.inst = inst_index;
+            best.geom = geom;
+            best.prim = prim;
+            if (OCCLUSION || (ray_flags & RTG_RAY_FLAG_TERMINATE_ON_FIRST_HIT)) return kRayHit;
+            tcur = t;
+        }
+        if (!pop(T, st)) return done();
+        return kRayActive;
+    }
+
+    // One iteration, as Traverser::step.
+    __device__ inline int step(const TlasView& T, const SceneView& S, QuadStack& st, uint32_t sub) {
+        if ((cur & kLeafBit) && in_blas) {
+            const int r = leaf_step(T, S, st, sub);
+            if (r != kRayActive) return r;
+        }
+        if ((cur & kLeafBit) && !in_blas) {
+            const int r = instance_step(T, st, sub);
+            if (r != kRayActive) return r;
+        }
+        if (!(cur & kLeafBit)) return node_step(T, st, sub);
+        return kRayActive;
+    }
+};
+
+// Two shadow rays of one path walked by a quad of lanes: PairTraverser's
+// visits and tests, a slot, a matrix row or a vertex per lane.
+struct QuadPairTraverser {
+    V3 wo, wd0, wd1, winv0, winv1;  // world rays (shared origin)
+    V3 ao, ainv0, ainv1;            // the rays of the structure being walked
+    float sx0, sy0, sz0, sx1, sy1, sz1;
+    uint32_t axes0, axes1;
+    const Node* nodes;
+    const TriRec* tris;
+    float tmin, tcur;
+    uint32_t inst_index, inst_flags;
+    uint32_t cur, mask, alive;
+    bool in_blas;
+
+    __device__ inline void start(const TlasView& T, V3 o, V3 d0, V3 d1, uint32_t m, float tmin_, float tmax_,
+                                 QuadStack& st) {
+        wo = o;
+        wd0 = d0;
+        wd1 = d1;
+        winv0 = v3(1.0f / d0.x, 1.0f / d0.y, 1.0f / d0.z);
+        winv1 = v3(1.0f / d1.x, 1.0f / d1.y, 1.0f / d1.z);
+        in_blas = false;
+        ao = wo;
+        ainv0 = winv0;
+        ainv1 = winv1;
+        nodes = T.nodes;
+        tris = nullptr;
+        tmin = tmin_;
+        tcur = tmax_;
+        inst_index = inst_flags = 0;
+        st.sp = 0;
+        cur = 0;
+        mask = m;
+        alive = m;
+    }
+    __device__ inline bool pop(const TlasView& T, QuadStack& st) {
+        while (st.sp > 0) {
+            const uint2 e = st.pop();
+            if (e.x == kSentinel) {
+                in_blas = false;
+                nodes = T.nodes;
+                ao = wo;
+                ainv0 = winv0;
+                ainv1 = winv1;
+                continue;
+            }
+            if ((e.y & alive) == 0) continue;
+            cur = e.x;
+            mask = e.y & alive;
+            return true;
+        }
+        return false;
+    }
+    __device__ inline int node_step(const TlasView& T, QuadStack& st, uint32_t sub) {
+        const float* np = reinterpret_cast<const float*>(nodes + cur) + sub;
+        const uint32_t ix = (f2u(ainv0.x) >> 31) * 4u, iy = (f2u(ainv0.y) >> 31) * 4u, iz = (f2u(ainv0.z) >> 31) * 4u;
+        const float nx = gld_f32(np + ix), fx = gld_f32(np + (ix ^ 4u));
+        const float ny = gld_f32(np + 8 + iy), fy = gld_f32(np + 8 + (iy ^ 4u));
+        const float nz = gld_f32(np + 16 + iz), fz = gld_f32(np + 16 + (iz ^ 4u));
+        const uint32_t child = gld_u32(np + 24);
+        RayCtx r0, r1;
+        r0.o = r1.o = ao;
+        r0.inv = ainv0;
+        r1.inv = ainv1;
+        float t;
+        uint32_t c = ((mask & 1u) && slab(nx, fx, ny, fy, nz, fz, r0, tmin, tcur, t)) ? 1u : 0u;
+        // ray 1's near planes where its direction's signs differ
+        const bool sx = ((f2u(ainv0.x) ^ f2u(ainv1.x)) >> 31) != 0u;
+        const bool sy = ((f2u(ainv0.y) ^ f2u(ainv1.y)) >> 31) != 0u;
+        const bool sz = ((f2u(ainv0.z) ^ f2u(ainv1.z)) >> 31) != 0u;
+        c |= ((mask & 2u) && slab(sx ? fx : nx, sx ? nx : fx, sy ? fy : ny, sy ? ny : fy, sz ? fz : nz, sz ? nz : fz,
+                                  r1, tmin, tcur, t))
+                 ? 2u
+                 : 0u;
+        if (child == kEmpty) c = 0u;
+        const uint32_t hits = quad_mask(c != 0u, sub);
+        if (hits == 0u) {
+            if (!pop(T, st)) return kRayMiss;
+            return kRayActive;
+        }
+        const int nh = __builtin_popcount(hits);
+        if (st.sp + nh - 1 > kStackMax) return kRayOverflow;
+        const int rank = __builtin_popcount(hits & ((1u << sub) - 1u));
+        if (c != 0u && rank > 0) st.put(st.sp + nh - 1 - rank, child, c);
+        const bool first = c != 0u && rank == 0;
+        cur = quad_or(first ? child : 0u);
+        mask = quad_or(first ? c : 0u);
+        st.sp += nh - 1;
+        return kRayActive;
+    }
+    __device__ inline int instance_step(const TlasView& T, QuadStack& st, uint32_t sub) {
+        const float4* rp = reinterpret_cast<const float4*>(T.recs + (cur & kFirstMask)) + sub;
+        const float4 m = gld_f4(rp);
+        const uint32_t blo = quad_bcast<3>(f2u(m.x)), bhi = quad_bcast<3>(f2u(m.y));
+        const uint32_t mf = quad_bcast<3>(f2u(m.w));
+        const uint8_t* bb = reinterpret_cast<const uint8_t*>((uint64_t)blo | ((uint64_t)bhi << 32));
+        if ((mf & 0xffu) == 0 || bb == nullptr) {  // shadow rays' cull mask is 0xff
+            if (!pop(T, st)) return kRayMiss;
+            return kRayActive;
+        }
+        if (st.sp >= kStackMax) return kRayOverflow;
+        if (sub == 0u) st.put(st.sp, kSentinel, 0u);
+        ++st.sp;
+        inst_index = quad_bcast<3>(f2u(m.z));
+        inst_flags = (mf >> 8) & 0xffu;
+        const AsHeader* bh = reinterpret_cast<const AsHeader*>(bb);
+        nodes = reinterpret_cast<const Node*>(bb + gld_u64(&bh->nodes_off));
+        tris = reinterpret_cast<const TriRec*>(bb + gld_u64(&bh->prims_off));
+        const float po = ((m.x * wo.x + m.y * wo.y) + m.z * wo.z) + m.w;
+        const float p0 = (m.x * wd0.x + m.y * wd0.y) + m.z * wd0.z;
+        const float p1 = (m.x * wd1.x + m.y * wd1.y) + m.z * wd1.z;
+        const float i0 = 1.0f / p0, i1 = 1.0f / p1;
+        ao = v3(quad_bcast<0>(po), quad_bcast<1>(po), quad_bcast<2>(po));
+        ainv0 = v3(quad_bcast<0>(i0), quad_bcast<1>(i0), quad_bcast<2>(i0));
+        ainv1 = v3(quad_bcast<0>(i1), quad_bcast<1>(i1), quad_bcast<2>(i1));
+        shear_setup(v3(quad_bcast<0>(p0), quad_bcast<1>(p0), quad_bcast<2>(p0)), ainv0, sx0, sy0, sz0, axes0);
+        shear_setup(v3(quad_bcast<0>(p1), quad_bcast<1>(p1), quad_bcast<2>(p1)), ainv1, sx1, sy1, sz1, axes1);
+        in_blas = true;
+        cur = 0;
+        return kRayActive;
+    }
+    __device__ inline int leaf_step(const TlasView& T, const SceneView& S, QuadStack& st, uint32_t sub) {
+        const uint32_t first = cur & kFirstMask;
+        const uint32_t count = ((cur >> 27) & 0xfu) + 1u;
+        for (uint32_t k = first; k < first + count; ++k) {
+            const float4 vtx = gld_f4(reinterpret_cast<const float4*>(tris + k) + (sub < 3u ? sub : 2u));
+            for (uint32_t r = 0; r < 2; ++r) {
+                const uint32_t bit = 1u << r;
+                if (!(mask & alive & bit)) continue;
+                float t, u, v;
+                if (!quad_tri_test(vtx, sub, ao, r ? sx1 : sx0, r ? sy1 : sy0, r ? sz1 : sz0, r ? axes1 : axes0, tmin,
+                                   tcur, t, u, v))
+                    continue;
+                const uint32_t prim = quad_bcast<0>(f2u(vtx.w)), gword = quad_bcast<1>(f2u(vtx.w));
+                const uint32_t geom = gword & ~kNonOpaqueBit;
+                if (!is_opaque(gword, inst_flags,
+                               RTG_RAY_FLAG_TERMINATE_ON_FIRST_HIT | RTG_RAY_FLAG_SKIP_CLOSEST_HIT_SHADER)) {
+                    // hit group offset 1 (closest_hit_textured.glsl:159-172)
+                    const uint32_t group = (gld_u32(&T.src[inst_index].sbt_offset_and_flags) & 0xffffffu) + 1u;
+                    if (group < RTG_HIT_GROUP_COUNT) {
+                        if (!alpha_clip_keep(S, T.src, inst_index, geom, prim, u, v)) continue;
+                    }
+                }
+                alive &= ~bit;
+            }
+            if (alive == 0u) return kRayHit;
+        }
+        if (!pop(T, st)) return kRayMiss;
+        return kRayActive;
+    }
+    __device__ inline int step(const TlasView& T, const SceneView& S, QuadStack& st, uint32_t sub) {
+        if ((cur & kLeafBit) && in_blas) {
+            const int r = leaf_step(T, S, st, sub);
+            if (r != kRayActive) return r;
+        }
+        if ((cur & kLeafBit) && !in_blas) {
+            const int r = instance_step(T, st, sub);
+            if (r != kRayActive) return r;
+        }
+        if (!(cur & kLeafBit)) return node_step(T, st, sub);
+        return kRayActive;
+    }
+    __device__ inline uint32_t occluded(uint32_t started) const { return started & ~alive; }
+};
+
 // Runs one ray to completion. Returns 1 for an accepted hit, 0 for none, -1
 // if the stack overflowed.
 template <bool OCCLUSION, bool COUNT>
@@ -1124,6 +1575,7 @@ struct WaveFeeder {
     // wave holds at once; `wave` of the launch's `waves`
     __device__ inline void init(uint32_t n, uint32_t most, uint32_t slots, uint32_t wave, uint32_t waves,
                                 uint32_t stride_ = kFeedStride) {
+        wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave);
         const bool fixed = n <= (uint64_t)waves * slots;
         chunk = fixed ? max(1u, (n + waves - 1) / waves) : most;
         handed = fixed ? waves * chunk : 0u;
@@ -1137,8 +1589,16 @@ struct WaveFeeder {
     // `idle` is the wave's ballot of lanes asking for work (wave-uniform);
     // returns this lane's entry or ~0u. counters: the queue's feed counters.
     __device__ inline uint32_t feed(uint64_t idle, bool want, uint32_t* counters, uint32_t n) {
+        return feed_ranked(idle, threadIdx.x & 63, want, counters, n);
+    }
+    // The same for idle quads of lanes (each asks with all four lanes).
+    __device__ inline uint32_t feed_quads(uint64_t idle, bool want, uint32_t* counters, uint32_t n) {
+        return feed_ranked(idle & 0x1111111111111111ull, (threadIdx.x & 63) & ~3, want, counters, n);
+    }
+    // one entry per set bit of `idle`; `at`: this lane's bit or that of its group
+    __device__ inline uint32_t feed_ranked(uint64_t idle, int at, bool want, uint32_t* counters, uint32_t n) {
         const int lane = threadIdx.x & 63;
-        const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+        const uint64_t lt = at == 0 ? 0ull : (~0ull >> (64 - at));
         uint32_t rank = (uint32_t)__popcll(idle & lt);
         uint32_t k = (uint32_t)__popcll(idle);
         uint32_t mine = ~0u;
@@ -1148,7 +1608,7 @@ struct WaveFeeder {
                 while (handed < n && tries > 0u) {
                     uint32_t c = 0;
                     if (lane == 0) c = atomicAdd(counters + group * stride, 1u);
-                    c = (uint32_t)__shfl((int)c, 0);
+                    c = (uint32_t)__builtin_amdgcn_readfirstlane((int)c);  // wave-uniform: scalar registers
                     base = handed + (c * kFeedGroups + group) * chunk;
                     if (base < n) break;
                     group = (group + 1u) & (kFeedGroups - 1);

@@ -112,7 +112,7 @@ struct Tuning {
     // persistent blocks given to the bounce stream beside the first level's
     // shadow rays (0: all levels in sequence on the caller's stream): its
     // shadow-ray launch takes them all, its bounce-level launches at most
-    // 128, and the first level's shadow rays the rest of the grid. 192 of
+    // 192, and the first level's shadow rays the rest of the grid. 192 of
     // 1,024 measured best on the 1080p scene with two frames in flight
     // (3,668-3,738 Mrays/s in seven runs on two boxes); 224, 256 and 320
     // often settled into a slower overlap of the two frames, 384 once in

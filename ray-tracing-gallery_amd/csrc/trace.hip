@@ -117,6 +117,7 @@ struct Frame {
     uint32_t feed_chunk;      // queue entries a wave takes per atomic
     int stack_lds;            // closest-hit stack entries per lane in LDS (the launches' LDS holds them)
     uint32_t side;            // 1 on the bounce stream (counts its shadow rays apart)
+    uint32_t quad_max;        // most rays (pairs) a bounce level traces with four lanes each
     // capacities of the path and shadow queues: sizes read from the device
     // are clamped to them and entries checked, so that a frame state driven
     // by two traces at once drops rays (kStatusQueueRange) instead of
@@ -188,6 +189,10 @@ __device__ inline void flush_counters(uint64_t* counters, const TravCounters& c,
     wave_add_counter(&counters[spill_slot(base)], c.spills);
 }
 
+// Idle quads of a wave (of 16) before they take new rays (8: the same time
+// on a 320x180 frame, 2 % more on two 1080p frames).
+constexpr int kQuadRefill = 16;
+
 // Lanes of a persistent traversal kernel keep tracing rays until the queue is
 // empty: a lane that finishes asks the wave's feeder for the next entry once
 // at least `refill_min` lanes are idle (or all are).
@@ -253,6 +258,46 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_rays(const uint8_t* tla
         }
     }
     if (COUNT) flush_counters(counters, cnt, OCC ? kCountersOcclusion : kCountersClosest);
+}
+
+// The same queries with four lanes per ray (QuadTraverser).
+template <bool OCC>
+__global__ __launch_bounds__(kTraceThreads) void k_trace_rays_quad(const uint8_t* tlas, SceneView S,
+                                                                   const rtg_ray* rays, uint32_t n,
+                                                                   uint32_t ray_flags, uint32_t cull_mask,
+                                                                   uint32_t sbt_offset, rtg_hit* hits, uint32_t* occ,
+                                                                   uint2* spill, uint32_t* status, int stack_lds) {
+    extern __shared__ uint2 s_stack[];
+    const uint32_t gtid = blockIdx.x * kTraceThreads + threadIdx.x;
+    const uint32_t waves = gridDim.x * (kTraceThreads / 64), per_wave = (n + waves - 1) / waves;  // 1..16
+    const uint32_t quad = (threadIdx.x & 63u) >> 2, sub = threadIdx.x & 3u;
+    const uint32_t ray = (gtid >> 6) * per_wave + quad;
+    if (quad >= per_wave || ray >= n) return;
+    const TlasView T = tlas_view(tlas);
+    QuadStack st;
+    st.init(s_stack, stack_lds, reinterpret_cast<uint8_t*>(spill), gtid, threadIdx.x);
+    QuadTraverser<OCC> tr;
+    const float4* rp = reinterpret_cast<const float4*>(rays + ray);
+    const float4 a = rp[0], b = rp[1];
+    tr.start(T, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, ray_flags, cull_mask, sbt_offset, st);
+    int res;
+    while ((res = tr.step(T, S, st, sub)) == kRayActive) {
+    }
+    if (res == kRayOverflow) atomicOr(status, (uint32_t)kStatusStackOverflow);
+    if (sub != 0u) return;
+    if (OCC) {
+        occ[ray] = res == kRayHit ? 1u : 0u;
+    } else {
+        const HitRec& h = tr.best;
+        rtg_hit o;
+        o.t = h.t;
+        o.instance = h.inst;
+        o.primitive = h.prim;
+        o.geometry = h.geom;
+        o.u = h.u;
+        o.v = h.v;
+        hits[ray] = o;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -400,6 +445,86 @@ __device__ __forceinline__ void trace_closest(Frame F, int level, const uint32_t
         }
     }
     if (COUNT) flush_counters(F.counters, cnt, SIDE ? kCountersClosestSide : kCountersClosest);
+}
+
+// Closest-hit traversal with four lanes per ray (QuadTraverser), for levels
+// of few rays; no traversal counters.
+template <bool SIDE, bool SINGLE>
+__device__ __forceinline__ void quad_closest(const Frame& F, int level, uint32_t n, uint32_t* status,
+                                             uint2* s_stack) {
+    if (SIDE) bounce_stream_priority();
+    else frame_chain_priority();
+    const Queue Q = F.q[level & 1];
+    const uint32_t gtid = blockIdx.x * kTraceThreads + threadIdx.x, sub = threadIdx.x & 3u;
+    QuadStack st;
+    st.init(s_stack, F.stack_lds, reinterpret_cast<uint8_t*>(F.spill), gtid, threadIdx.x);
+    QuadTraverser<false> tr;
+    WaveFeeder feeder;
+    feeder.init(n, 16, 16, gtid >> 6, gridDim.x * (kTraceThreads / 64));
+    bool active = false;
+    uint32_t slot = 0;
+    const JobDev* J = SINGLE ? &F.jobs[0] : nullptr;
+    TlasView T;
+    if (SINGLE) T = tlas_view(J->tlas);
+    uint32_t c0 = 0;
+    while (true) {
+        const uint64_t idle = __ballot(!active) & 0x1111111111111111ull;
+        if (idle != 0 && !feeder.exhausted && __popcll(idle) >= kQuadRefill) {
+            const uint32_t id = feeder.feed_quads(idle, !active, F.feeds + level, n);
+            if (id != ~0u) {
+                slot = id;
+                uint32_t path = Q.path[id];
+                if (path >= F.paths) {
+                    queue_range_error(F);
+                    path = 0;  // traced as path 0's ray; the shade stage drops it
+                }
+                if (!SINGLE) {
+                    J = &F.jobs[find_job(F.jobs, F.njobs, path, false)];
+                    T = tlas_view(J->tlas);
+                }
+                const float4 a = Q.o[id], b = Q.d[id];
+                tr.start(T, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, RTG_RAY_FLAG_NONE, 0xffu, 0u, st);
+                if (J->flags & RTG_TRACE_HEATMAP) c0 = (uint32_t)__builtin_readcyclecounter();
+                active = true;
+            }
+        }
+        if (__ballot(active) == 0) break;
+        if (active) {
+            const int res = tr.step(T, J->scene, st, sub);
+            if (res != kRayActive) {
+                active = false;
+                if (res == kRayOverflow) atomicOr(status, (uint32_t)kStatusStackOverflow);
+                if (sub == 0u) {
+                    if (J->flags & RTG_TRACE_HEATMAP) {
+                        const uint32_t path = Q.path[slot];
+                        atomicAdd(&F.cycles[path < F.paths ? path : 0u], (uint32_t)__builtin_readcyclecounter() - c0);
+                    }
+                    const HitRec& h = tr.best;
+                    F.hit_a[slot] = make_uint4(f2u(h.t), h.inst, h.prim, h.geom);
+                    F.hit_b[slot] = make_float2(h.u, h.v);
+                }
+            }
+        }
+    }
+}
+
+template <bool SINGLE>
+__global__ __launch_bounds__(kTraceThreads) void k_trace_closest_quad(Frame F, int level, const uint32_t* count_ptr,
+                                                                      uint32_t fixed_count, uint32_t* status) {
+    extern __shared__ uint2 s_stack[];
+    const uint32_t n = min(count_ptr ? *count_ptr : fixed_count, F.path_cap);
+    quad_closest<false, SINGLE>(F, level, n, status, s_stack);
+}
+
+// A bounce level, whose ray count only the device knows: four lanes per ray
+// up to F.quad_max rays.
+template <bool SIDE, bool SINGLE>
+__global__ __launch_bounds__(kTraceThreads) void k_trace_closest_any(Frame F, int level, const uint32_t* count_ptr,
+                                                                     uint32_t fixed_count, uint32_t* status) {
+    extern __shared__ uint2 s_stack[];
+    const uint32_t n = min(count_ptr ? *count_ptr : fixed_count, F.path_cap);
+    if (n <= F.quad_max) quad_closest<SIDE, SINGLE>(F, level, n, status, s_stack);
+    else trace_closest<false, SIDE, SINGLE>(F, level, count_ptr, fixed_count, status, s_stack);
 }
 
 // Launches of one job (held to 96 VGPRs, five waves per SIMD).
@@ -804,8 +929,7 @@ __device__ inline uint32_t shadow_pair(const Frame& F, uint32_t e0, uint32_t hi,
 // shadow ray, plain stores (no atomics). A pair lane holds 121 VGPRs (four
 // waves per SIMD).
 template <bool COUNT, bool SIDE>
-__global__ __launch_bounds__(kTraceThreads) void k_trace_occlusion(Frame F, uint32_t* status, int part) {
-    extern __shared__ uint2 s_stack[];
+__device__ __forceinline__ void trace_occlusion(const Frame& F, uint32_t* status, int part, uint2* s_stack) {
     if (SIDE) bounce_stream_priority();
     uint32_t lo, hi;
     uint32_t* feed;
@@ -856,6 +980,83 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_occlusion(Frame F, uint
         }
     }
     if (COUNT) flush_counters(F.counters, cnt, SIDE ? kCountersOcclusionSide : kCountersOcclusion);
+}
+
+template <bool COUNT, bool SIDE>
+__global__ __launch_bounds__(kTraceThreads) void k_trace_occlusion(Frame F, uint32_t* status, int part) {
+    extern __shared__ uint2 s_stack[];
+    trace_occlusion<COUNT, SIDE>(F, status, part, s_stack);
+}
+
+// The same pairs with four lanes each (QuadPairTraverser), for few of them; no
+// traversal counters.
+template <bool SIDE>
+__device__ __forceinline__ void quad_occlusion(const Frame& F, uint32_t* status, uint32_t lo, uint32_t hi,
+                                               uint32_t* feed, uint2* s_stack) {
+    if (SIDE) bounce_stream_priority();
+    const uint32_t npairs = (hi - lo + 1) / 2;
+    const uint32_t gtid = blockIdx.x * kTraceThreads + threadIdx.x, sub = threadIdx.x & 3u;
+    QuadStack st;
+    st.init(s_stack, F.stack_lds, reinterpret_cast<uint8_t*>(F.spill), gtid, threadIdx.x);
+    QuadPairTraverser tr;
+    WaveFeeder feeder;
+    feeder.init(npairs, 16, 16, gtid >> 6, gridDim.x * (kTraceThreads / 64));
+    bool active = false;
+    uint32_t e0 = 0, started = 0, path = 0;
+    const JobDev* J = nullptr;
+    TlasView T;
+    uint32_t c0 = 0;
+    while (true) {
+        const uint64_t idle = __ballot(!active) & 0x1111111111111111ull;
+        if (idle != 0 && !feeder.exhausted && __popcll(idle) >= kQuadRefill) {
+            const uint32_t q = feeder.feed_quads(idle, !active, feed, npairs);
+            if (q != ~0u) {
+                e0 = lo + 2 * q;
+                float4 o, d0, d1;
+                started = shadow_pair(F, e0, hi, path, o, d0, d1);
+                J = &F.jobs[find_job(F.jobs, F.njobs, path, false)];
+                T = tlas_view(J->tlas);
+                tr.start(T, v3(o.x, o.y, o.z), v3(d0.x, d0.y, d0.z), v3(d1.x, d1.y, d1.z), started, o.w, d0.w, st);
+                if (J->flags & RTG_TRACE_HEATMAP) c0 = (uint32_t)__builtin_readcyclecounter();
+                active = true;
+            }
+        }
+        if (__ballot(active) == 0) break;
+        if (active) {
+            const int res = tr.step(T, J->scene, st, sub);
+            if (res != kRayActive) {
+                active = false;
+                // a stack overflow leaves both rays unresolved: not visible
+                const uint32_t occ = res == kRayOverflow ? started : tr.occluded(started);
+                if (res == kRayOverflow) atomicOr(status, (uint32_t)kStatusStackOverflow);
+                if (sub == 0u) {
+                    if (J->flags & RTG_TRACE_HEATMAP)
+                        atomicAdd(&F.cycles[path], (uint32_t)__builtin_readcyclecounter() - c0);
+                    F.sflag[e0] = (occ & 1u) ? 0 : 1;
+                    if (started & 2u) F.sflag[e0 + 1] = (occ & 2u) ? 0 : 1;
+                }
+            }
+        }
+    }
+}
+
+__global__ __launch_bounds__(kTraceThreads) void k_trace_occlusion_quad(Frame F, uint32_t* status, int part) {
+    extern __shared__ uint2 s_stack[];
+    uint32_t lo, hi;
+    uint32_t* feed;
+    shadow_part(F, part, lo, hi, feed);
+    quad_occlusion<false>(F, status, lo, hi, feed, s_stack);
+}
+
+// The shadow rays that the bounce levels add: four lanes per pair up to
+// F.quad_max pairs.
+__global__ __launch_bounds__(kTraceThreads) void k_trace_occlusion_any(Frame F, uint32_t* status, int part) {
+    extern __shared__ uint2 s_stack[];
+    uint32_t lo, hi;
+    uint32_t* feed;
+    shadow_part(F, part, lo, hi, feed);
+    if ((hi - lo + 1) / 2 <= F.quad_max) quad_occlusion<true>(F, status, lo, hi, feed, s_stack);
+    else trace_occlusion<false, true>(F, status, part, s_stack);
 }
 
 // The same pairs, one per lane and grid-stride round (refill_occlusion 0).
@@ -1078,6 +1279,19 @@ static int trace_grid(rtg_ctx* ctx, const Tuning& tune) {
 }
 static int trace_grid(rtg_ctx* ctx) { return trace_grid(ctx, ctx->tune); }
 
+// Rays that a grid of `blocks` workgroups holds at once with four lanes a ray,
+// and the workgroups for `rays` of them, as thin as one ray to a wave. Up to
+// that many rays (65,536 on the default grid) the longest rays set a launch's
+// time and four lanes a ray are the faster way: closest hits of 4,096 and
+// 65,536 rays among 20,011 instances take 54 and 109 us (one lane a ray 139
+// and 196), in a 1 M-triangle soup 95 and 211 (259 and 292). Beyond, rays
+// wait for lanes and the quads' four times as many cost: 131,072 rays took
+// 375 us in the soup (one lane a ray 308).
+static uint64_t quad_capacity(unsigned blocks) { return (uint64_t)blocks * (kTraceThreads / 4); }
+static unsigned quad_grid(uint64_t rays, unsigned blocks) {
+    return (unsigned)std::min<uint64_t>((rays + kTraceThreads / 64 - 1) / (kTraceThreads / 64), blocks);
+}
+
 size_t spill_bytes(rtg_ctx* ctx, const Tuning& tune) {
     return (size_t)trace_grid(ctx, tune) * kTraceThreads * kSpillLaneBytes;
 }
@@ -1274,6 +1488,7 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
     F.shadow_cap = (uint32_t)std::min<uint64_t>(a->shadow_cap, 0xffffffffu);
     F.status = a->d_counts + kStatusSlot;
     const unsigned G = (unsigned)trace_grid(ctx, tune);
+    F.quad_max = (uint32_t)quad_capacity(G);
     const size_t lds = stack_lds_bytes(tune.stack_lds);  // a traversal workgroup's stacks
     const unsigned Gsmall = (unsigned)std::min<uint64_t>((P.paths + 255) / 256, (uint64_t)ctx->cu_count * 16);
     hipLaunchKernelGGL(k_frame_begin, dim3(1), dim3(kFeedWords), 0, s, a->d_counts, a->d_feeds, ctx->d_counters, cnt);
@@ -1298,7 +1513,13 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
                     hipLaunchKernelGGL((cnt ? k_trace_closest_rounds<true, false> : k_trace_closest_rounds<false, false>),
                                        dim3(g), dim3(kTraceThreads), lds, st, Fl, (int)level, cp, fixed, Fl.status);
             } else {
-                auto kernel = side ? (cnt ? (single ? k_trace_closest_one<true, true> : k_trace_closest<true, true>)
+                const bool quad = !cnt && level == 0 && P.paths <= quad_capacity(G);
+                if (quad) g = quad_grid(P.paths, G);
+                auto kernel = quad ? (single ? k_trace_closest_quad<true> : k_trace_closest_quad<false>)
+                              : !cnt && level > 0
+                                  ? (side ? (single ? k_trace_closest_any<true, true> : k_trace_closest_any<true, false>)
+                                          : (single ? k_trace_closest_any<false, true> : k_trace_closest_any<false, false>))
+                              : side ? (cnt ? (single ? k_trace_closest_one<true, true> : k_trace_closest<true, true>)
                                           : (single ? k_trace_closest_one<false, true> : k_trace_closest<false, true>))
                                    : (cnt ? (single ? k_trace_closest_one<true, false> : k_trace_closest<true, false>)
                                           : (single ? k_trace_closest_one<false, false> : k_trace_closest<false, false>));
@@ -1325,8 +1546,11 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
             else
                 hipLaunchKernelGGL((cnt ? k_trace_occlusion_rounds<true, false> : k_trace_occlusion_rounds<false, false>),
                                    dim3(g), dim3(kTraceThreads), lds, st, Fo, Fo.status, part);
+        } else if (!cnt && !side && P.shadow / 2 <= quad_capacity(G)) {
+            hipLaunchKernelGGL(k_trace_occlusion_quad, dim3(quad_grid(P.shadow / 2, g)), dim3(kTraceThreads), lds, st,
+                               Fo, Fo.status, part);
         } else if (side) {
-            hipLaunchKernelGGL((cnt ? k_trace_occlusion<true, true> : k_trace_occlusion<false, true>), dim3(g),
+            hipLaunchKernelGGL((cnt ? k_trace_occlusion<true, true> : k_trace_occlusion_any), dim3(g),
                                dim3(kTraceThreads), lds, st, Fo, Fo.status, part);
         } else {
             hipLaunchKernelGGL((cnt ? k_trace_occlusion<true, false> : k_trace_occlusion<false, false>), dim3(g),
@@ -1354,12 +1578,12 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
             // timed as one span: its kernels share the GPU with the shadow rays
             LaunchTimer t(ctx, RTG_KERNEL_BOUNCE_SIDE, a->side, timed);
             // The bounce levels' traversal and shading launches take at most
-            // 128 workgroups (32 k lanes; a 1080p frame has about 46 k and
-            // 3 k bounce rays): a launch ends only once each of its
-            // workgroups has been dispatched, which waits for free slots while
-            // the other frame's persistent kernels hold the CUs (the bounce
-            // part of the frame: 1.70-1.78 instead of 1.82 ms).
-            const unsigned Gbounce = std::min(Gside, 128u);
+            // 192 workgroups (12 k rays at once with four lanes each; a 1080p
+            // frame has about 46 k and 3 k bounce rays): a launch ends only
+            // once each of its workgroups has been dispatched, which waits
+            // for free slots while the other frame's persistent kernels hold
+            // the CUs (two 1080p frames: 4.58 ms, with 128 workgroups 4.73).
+            const unsigned Gbounce = std::min(Gside, 192u);
             for (uint32_t level = 1; level < P.max_traces; ++level)
                 level_step(Fs, level, Gbounce, std::min(Gsmall, Gbounce), a->side, false);
             occlusion(Fs, kPartRest, Gside, a->side, false);
@@ -1445,12 +1669,13 @@ static int check_ray_query(rtg_ctx* ctx, rtg_tlas tlas, const rtg_ray* rays, uin
     return RTG_OK;
 }
 
-// Clears the feed counters (`feed_stride` words apart) and launches the query kernel on `G` persistent
-// blocks whose spill stacks start at `spill` (G * kTraceThreads lanes).
+// Clears the feed counters (`feed_stride` words apart) and launches the query
+// kernel on at most `max_blocks` persistent blocks, whose spill stacks start
+// at `spill` (max_blocks * kTraceThreads lanes).
 static void launch_ray_query(rtg_ctx* ctx, rtg_tlas tlas, const rtg_scene_bindings* scene, const rtg_ray* rays,
                              uint32_t count, uint32_t mode, uint32_t ray_flags, uint32_t cull_mask,
                              uint32_t sbt_offset, rtg_hit* hits, uint32_t* occluded, uint2* spill, uint32_t* feed,
-                             uint32_t feed_stride, unsigned G, bool timed, hipStream_t s) {
+                             uint32_t feed_stride, unsigned max_blocks, bool timed, hipStream_t s) {
     SceneView S;
     S.models = scene ? reinterpret_cast<const rtg_model_info*>(scene->model_info) : nullptr;
     S.textures = scene ? reinterpret_cast<const rtg_texture*>(scene->textures) : nullptr;
@@ -1459,12 +1684,21 @@ static void launch_ray_query(rtg_ctx* ctx, rtg_tlas tlas, const rtg_scene_bindin
     S.texture_count = scene ? scene->texture_count : 0;
     const bool cnt = ctx->counters_enabled;
     uint8_t* tl = reinterpret_cast<uint8_t*>(tlas);
+    cull_mask &= 0xffu;
+    if (!cnt && count <= quad_capacity(max_blocks)) {
+        LaunchTimer t(ctx, mode == RTG_QUERY_CLOSEST ? RTG_KERNEL_TRACE_CLOSEST : RTG_KERNEL_TRACE_OCCLUSION, s, timed);
+        hipLaunchKernelGGL((mode == RTG_QUERY_CLOSEST ? k_trace_rays_quad<false> : k_trace_rays_quad<true>),
+                           dim3(quad_grid(count, max_blocks)), dim3(kTraceThreads),
+                           stack_lds_bytes(ctx->tune.stack_lds), s, tl, S, rays, count, ray_flags, cull_mask,
+                           sbt_offset, hits, occluded, spill, ctx->d_status, ctx->tune.stack_lds);
+        return;
+    }
+    const unsigned G = (unsigned)std::min<uint64_t>((count + kTraceThreads - 1) / kTraceThreads, max_blocks);
     if (count > G * kTraceThreads)  // else the waves' first chunks are all there is
         hipLaunchKernelGGL(k_zero_feed, dim3(1), dim3(64), 0, s, feed, feed_stride);
     // the primary ray count of a ray query is the query size
     if (cnt) hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, ctx->d_counters, (uint64_t)count);
     LaunchTimer t(ctx, mode == RTG_QUERY_CLOSEST ? RTG_KERNEL_TRACE_CLOSEST : RTG_KERNEL_TRACE_OCCLUSION, s, timed);
-    cull_mask &= 0xffu;
 #define RTG_LAUNCH_RAYS(OCC, CNT)                                                                                \
     hipLaunchKernelGGL((k_trace_rays<OCC, CNT>), dim3(G), dim3(kTraceThreads), stack_lds_bytes(ctx->tune.stack_lds), \
                        s, tl, S, rays, count, ray_flags, cull_mask, sbt_offset, hits, occluded, spill, feed, feed_stride, \
@@ -1497,9 +1731,9 @@ extern "C" int rtg_trace_rays(rtg_ctx* ctx, rtg_tlas tlas, const rtg_scene_bindi
                 (void*)s);
     if (ensure_spill(ctx, a, ctx->tune) != RTG_OK || a->feed.ensure(kFeedWords * sizeof(uint32_t)) != RTG_OK)
         return RTG_ERROR_OUT_OF_MEMORY;
-    const unsigned G = (unsigned)std::min<uint64_t>((count + kTraceThreads - 1) / kTraceThreads, trace_grid(ctx));
     launch_ray_query(ctx, tlas, scene, rays, count, mode, ray_flags, cull_mask, sbt_offset, hits, occluded,
-                     reinterpret_cast<uint2*>(a->spill.ptr), reinterpret_cast<uint32_t*>(a->feed.ptr), kFeedStride, G, true, s);
+                     reinterpret_cast<uint2*>(a->spill.ptr), reinterpret_cast<uint32_t*>(a->feed.ptr), kFeedStride,
+                     (unsigned)trace_grid(ctx), true, s);
     RTG_HIP(hipGetLastError());
     return RTG_OK;
 }
@@ -1561,11 +1795,10 @@ extern "C" int rtg_trace_rays_static(rtg_ctx* ctx, rtg_tlas tlas, const rtg_scen
                 ctx->device);
     // the grid is capped by the spill stacks the array holds; the launch
     // shape never changes results
-    const unsigned G = (unsigned)std::min<uint64_t>(
-        std::min<uint64_t>((count + kTraceThreads - 1) / kTraceThreads, trace_grid(ctx)), kStaticBlocks);
     launch_ray_query(ctx, tlas, scene, rays, count, mode, ray_flags, cull_mask, sbt_offset, hits, occluded,
                      reinterpret_cast<uint2*>(base + kStaticFeedBytes), reinterpret_cast<uint32_t*>(base),
-                     (uint32_t)(kStaticFeedBytes / kFeedGroups / sizeof(uint32_t)), G, false,
+                     (uint32_t)(kStaticFeedBytes / kFeedGroups / sizeof(uint32_t)),
+                     std::min((unsigned)trace_grid(ctx), kStaticBlocks), false,
                      reinterpret_cast<hipStream_t>(stream));
     RTG_HIP(hipGetLastError());
     return RTG_OK;

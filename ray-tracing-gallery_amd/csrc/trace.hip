@@ -29,8 +29,9 @@ constexpr int kFeedShadowRest = 5;  // the shadow rays after those of trace leve
 constexpr int kShadowFirst = 5;      // counts[5]: shadow rays of trace level 0
 constexpr int kStatusSlot = 14;      // counts[14]: status bits of the trace (merged into the context's)
 constexpr int kPartAll = 0, kPartFirst = 1, kPartRest = 2;  // parts of the shadow queue
-// path of a shadow-queue padding slot (after an odd count of a path's rays)
-constexpr uint32_t kNoPath = 0xFFFFFFFFu;
+// intervals of the camera, continuation and shadow rays (lib.rs:146-149,
+// closest_hit_textured.glsl:159-172)
+constexpr float kPathTmin = 0.01f, kShadowTmin = 0.001f, kRayTmax = 10000.0f;
 
 // Order of an image's pixels along its paths: bands of 8 rows, each band
 // walked column by column, so that the 64 lanes of a wavefront cover an 8x8
@@ -75,6 +76,7 @@ struct JobDev {
     SceneView scene;
     float view_inverse[16];
     float proj_inverse[16];
+    float origin[3];  // of every camera ray
     float sun[3];
     float sun_radius;
     uint32_t bn_index;
@@ -97,15 +99,16 @@ struct Frame {
     const JobDev* jobs;
     uint32_t njobs;
     uint64_t paths;
-    float4* path_rgb;    // final colour of paths that did not end on a textured hit
     float4* shade_a;     // NoL, combined.xyz of a textured hit
-    float4* shade_b;     // ambient.xyz; w: bits of 1 + the path's first shadow ray if textured, else 0
+    float4* shade_b;     // a textured hit's ambient.xyz and (bits of w) 1 + the path's first
+                         // shadow ray; else the path's colour and 0
     uint8_t* sflag;      // per shadow-queue entry: 1 if the shadow ray saw the sun
-    uint32_t* cycles;    // heatmap cycle counts
-    Queue q[2];
+    uint32_t* cycles;    // heatmap cycle counts (jobs with RTG_TRACE_HEATMAP)
+    Queue q[2];          // rays of a trace level; of level 0, ray i is path i's: only q[0].d is kept
     uint4* hit_a;        // t bits, instance, primitive, geometry
     float2* hit_b;       // u, v
-    Queue sq;            // shadow rays
+    float4* pair_o;      // shadow rays in pairs (slots 2j, 2j + 1) of one path: origin.xyz, path
+    float4* pair_d;      // per slot: direction.xyz; of the first, 3 in w's bits, or 1 without a second
     uint32_t* counts;    // [0..3] queue sizes per trace level, [4] shadow rays, [5] shadow
                          // rays of level 0, [14] status bits
     uint32_t* feeds;     // feed counters of queue q: feeds[q + k * kFeedStride]
@@ -365,6 +368,10 @@ __global__ void k_reset_counters(uint64_t* counters, uint64_t primary) {
 // ray_generation (shaders/ray-tracing/src/lib.rs:94-142): one path per
 // (pixel, sample). Sample s > 0 of a multi-sample pixel moves the pixel
 // centre by the R2 sequence; sample 0 of one sample is the reference's +0.5.
+// Writes the direction alone (16 bytes a path): the origin is the job's, the
+// path the ray's number, and the shading of level 0 writes every path's
+// state. With the whole ray and cleared state, 72 bytes, the launch took
+// 100 us on average over a set of served requests, now 56.
 __global__ __launch_bounds__(256) void k_raygen(Frame F, bool count) {
     uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t p = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; p < F.paths; p += stride) {
@@ -381,20 +388,14 @@ __global__ __launch_bounds__(256) void k_raygen(Frame F, bool count) {
         float pcx = (float)px + jx, pcy = (float)py + jy;
         float tcx = pcx / (float)J.width, tcy = pcy / (float)J.height;
         float rcx = tcx * 2.0f - 1.0f, rcy = tcy * 2.0f - 1.0f;
-        float zo[4] = {0.0f, 0.0f, 0.0f, 1.0f}, tmp[4];
-        mat4_mul(J.view_inverse, zo, tmp);
-        V3 origin = v3(tmp[0], tmp[1], tmp[2]);
+        float tmp[4];
         float tv[4] = {rcx, rcy, 1.0f, 1.0f};
         mat4_mul(J.proj_inverse, tv, tmp);
         V3 ld = normalize(v3(tmp[0], tmp[1], tmp[2]));
         float dv[4] = {ld.x, ld.y, ld.z, 0.0f};
         mat4_mul(J.view_inverse, dv, tmp);
-        F.q[0].o[p] = make_float4(origin.x, origin.y, origin.z, 0.01f);
-        F.q[0].d[p] = make_float4(tmp[0], tmp[1], tmp[2], 10000.0f);
-        F.q[0].path[p] = (uint32_t)p;
-        F.path_rgb[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        F.shade_b[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        F.cycles[p] = 0;
+        F.q[0].d[p] = make_float4(tmp[0], tmp[1], tmp[2], kRayTmax);
+        if (J.flags & RTG_TRACE_HEATMAP) F.cycles[p] = 0;
     }
     if (count && blockIdx.x == 0 && threadIdx.x == 0) atomicAdd((unsigned long long*)&F.counters[0], F.paths);
 }
@@ -413,6 +414,19 @@ __global__ __launch_bounds__(256) void k_raygen(Frame F, bool count) {
 // (1 of 16 runs on three boxes, against 3 of 12; the others 0.7 % faster).
 __device__ __forceinline__ void bounce_stream_priority() { __builtin_amdgcn_s_setprio(2); }
 __device__ __forceinline__ void frame_chain_priority() { __builtin_amdgcn_s_setprio(1); }
+
+// Path and origin (with tmin) of entry i of a trace level's queue.
+__device__ inline uint32_t level_path(const Frame& F, const Queue& Q, int level, uint32_t i) {
+    if (level == 0) return i;
+    const uint32_t path = Q.path[i];
+    if (path < F.paths) return path;
+    queue_range_error(F);
+    return 0;  // traced as path 0's ray; the shade stage drops it
+}
+__device__ inline float4 level_origin(const Queue& Q, int level, uint32_t i, const JobDev& J) {
+    if (level == 0) return make_float4(J.origin[0], J.origin[1], J.origin[2], kPathTmin);
+    return Q.o[i];
+}
 
 // Closest-hit traversal of trace level b (count from the device unless fixed).
 // SIDE instances run the bounce levels on the bounce stream. SINGLE instances
@@ -448,16 +462,12 @@ __device__ __forceinline__ void trace_closest(Frame F, int level, const uint32_t
             uint32_t id = feeder.feed(idle, !active, F.feeds + level, n);
             if (id != ~0u) {
                 slot = id;
-                uint32_t path = Q.path[id];
-                if (path >= F.paths) {
-                    queue_range_error(F);
-                    path = 0;  // traced as path 0's ray; the shade stage drops it
-                }
+                const uint32_t path = level_path(F, Q, level, id);
                 if (!SINGLE) {
                     J = &F.jobs[find_job(F.jobs, F.njobs, path, false)];
                     T = tlas_view(J->tlas);
                 }
-                float4 a = Q.o[id], b = Q.d[id];
+                const float4 a = level_origin(Q, level, id, *J), b = Q.d[id];
                 tr.start(T, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, RTG_RAY_FLAG_NONE, 0xffu, 0u, st);
                 if (J->flags & RTG_TRACE_HEATMAP) c0 = (uint32_t)__builtin_readcyclecounter();
                 active = true;
@@ -470,8 +480,7 @@ __device__ __forceinline__ void trace_closest(Frame F, int level, const uint32_t
                 if (res == kRayOverflow) atomicOr(status, (uint32_t)kStatusStackOverflow);
                 if (J->flags & RTG_TRACE_HEATMAP) {
                     // the path is read again rather than kept live through the traversal
-                    const uint32_t path = Q.path[slot];
-                    atomicAdd(&F.cycles[path < F.paths ? path : 0u], (uint32_t)__builtin_readcyclecounter() - c0);
+                    atomicAdd(&F.cycles[level_path(F, Q, level, slot)], (uint32_t)__builtin_readcyclecounter() - c0);
                 }
                 const HitRec& h = tr.best;
                 F.hit_a[slot] = make_uint4(f2u(h.t), h.inst, h.prim, h.geom);
@@ -509,16 +518,12 @@ __device__ __forceinline__ void quad_closest(const Frame& F, int level, uint32_t
             const uint32_t id = feeder.feed_quads(idle, !active, F.feeds + level, n);
             if (id != ~0u) {
                 slot = id;
-                uint32_t path = Q.path[id];
-                if (path >= F.paths) {
-                    queue_range_error(F);
-                    path = 0;  // traced as path 0's ray; the shade stage drops it
-                }
+                const uint32_t path = level_path(F, Q, level, id);
                 if (!SINGLE) {
                     J = &F.jobs[find_job(F.jobs, F.njobs, path, false)];
                     T = tlas_view(J->tlas);
                 }
-                const float4 a = Q.o[id], b = Q.d[id];
+                const float4 a = level_origin(Q, level, id, *J), b = Q.d[id];
                 tr.start(T, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w, RTG_RAY_FLAG_NONE, 0xffu, 0u, st);
                 if (J->flags & RTG_TRACE_HEATMAP) c0 = (uint32_t)__builtin_readcyclecounter();
                 active = true;
@@ -532,8 +537,8 @@ __device__ __forceinline__ void quad_closest(const Frame& F, int level, uint32_t
                 if (res == kRayOverflow) atomicOr(status, (uint32_t)kStatusStackOverflow);
                 if (sub == 0u) {
                     if (J->flags & RTG_TRACE_HEATMAP) {
-                        const uint32_t path = Q.path[slot];
-                        atomicAdd(&F.cycles[path < F.paths ? path : 0u], (uint32_t)__builtin_readcyclecounter() - c0);
+                        atomicAdd(&F.cycles[level_path(F, Q, level, slot)],
+                                  (uint32_t)__builtin_readcyclecounter() - c0);
                     }
                     const HitRec& h = tr.best;
                     F.hit_a[slot] = make_uint4(f2u(h.t), h.inst, h.prim, h.geom);
@@ -599,14 +604,10 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_closest_rounds(Frame F,
     for (uint32_t r = 0; r < rounds; ++r) {
         uint32_t i = r * stride + gtid;
         if (i < n) {
-            uint32_t p = Q.path[i];
-            if (p >= F.paths) {
-                queue_range_error(F);
-                p = 0;  // traced as path 0's ray; the shade stage drops it
-            }
+            const uint32_t p = level_path(F, Q, level, i);
             const JobDev& J = F.jobs[find_job(F.jobs, F.njobs, p, false)];
             const TlasView T = tlas_view(J.tlas);
-            float4 a = Q.o[i], b = Q.d[i];
+            const float4 a = level_origin(Q, level, i, J), b = Q.d[i];
             HitRec h;
             int res = traverse<false, COUNT>(T, J.scene, v3(a.x, a.y, a.z), v3(b.x, b.y, b.z), a.w, b.w,
                                              RTG_RAY_FLAG_NONE, 0xffu, 0u, h, st, cnt);
@@ -722,11 +723,14 @@ __global__ __launch_bounds__(256) void k_shade(Frame F, int level, const uint32_
         bool want_next = false;
         V3 sh_origin = v3(0, 0, 0), next_o = v3(0, 0, 0), next_d = v3(0, 0, 0), amb = v3(0, 0, 0);
         V3 sun = v3(0, 0, 0);
+        // the path's colour, if its trace ends here without shadow rays
+        float4 result = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        bool ends = level == 0;
         float sun_radius = 0.0f;
         uint32_t p = 0, px = 0, py = 0, frame = 0, bn_index = 0;
         const JobDev* J = nullptr;
         if (active) {
-            p = Q.path[i];
+            p = level == 0 ? i : Q.path[i];
             if (p >= F.paths) {
                 queue_range_error(F);
                 active = false;
@@ -746,7 +750,7 @@ __global__ __launch_bounds__(256) void k_shade(Frame F, int level, const uint32_
             float2 hb = F.hit_b[i];
             float t = u2f(ha.x);
             uint32_t inst = ha.y, prim = ha.z, geom = ha.w;
-            float4 ro = Q.o[i], rd = Q.d[i];
+            const float4 ro = level_origin(Q, level, i, *J), rd = Q.d[i];
             V3 o = v3(ro.x, ro.y, ro.z), d = v3(rd.x, rd.y, rd.z);
             if (level == 0 && J->out_hits) {
                 rtg_hit oh;
@@ -763,7 +767,8 @@ __global__ __launch_bounds__(256) void k_shade(Frame F, int level, const uint32_
                 // primary_ray_miss (lib.rs:40-51)
                 float cs = cos_own(sun_radius);
                 V3 c = dot(d, sun) > cs ? v3(1.0f, 1.0f, 1.0f) : v3(0.0f, 0.0f, 0.05f);
-                F.path_rgb[p] = make_float4(c.x, c.y, c.z, 0.0f);
+                result = make_float4(c.x, c.y, c.z, 0.0f);
+                ends = true;
             } else {
                 const TlasView T = tlas_view(J->tlas);
                 const float4* sp = reinterpret_cast<const float4*>(T.src + inst);
@@ -848,7 +853,7 @@ __global__ __launch_bounds__(256) void k_shade(Frame F, int level, const uint32_
             }
         }
         // compaction: one atomic per workgroup for each queue; a path's shadow
-        // rays take an even number of slots (a padding slot after an odd
+        // rays take an even number of slots (an unused one after an odd
         // count) so that the occlusion kernel's pairs never span two paths
         const uint32_t shadow_slots = want_shadow + (want_shadow & 1u);
         uint32_t sbase, nbase;
@@ -861,11 +866,13 @@ __global__ __launch_bounds__(256) void k_shade(Frame F, int level, const uint32_
             queue_range_error(F);
             want_shadow = 0;
         }
-        // a textured hit's ambient term and where its shadow rays' flags lie
-        if (want_shadow) F.shade_b[p] = make_float4(amb.x, amb.y, amb.z, u2f(sbase + 1u));
+        // a textured hit's ambient term and where its shadow rays' flags lie;
+        // level 0 writes every path's record, a continued path's colour as 0
+        if (want_shadow) result = make_float4(amb.x, amb.y, amb.z, u2f(sbase + 1u));
+        if (active && (ends || want_shadow)) F.shade_b[p] = result;
         if (want_next) {
-            NQ.o[nbase] = make_float4(next_o.x, next_o.y, next_o.z, 0.01f);
-            NQ.d[nbase] = make_float4(next_d.x, next_d.y, next_d.z, 10000.0f);
+            NQ.o[nbase] = make_float4(next_o.x, next_o.y, next_o.z, kPathTmin);
+            NQ.d[nbase] = make_float4(next_d.x, next_d.y, next_d.z, kRayTmax);
             NQ.path[nbase] = p;
             n_bounce++;
         }
@@ -897,14 +904,12 @@ __global__ __launch_bounds__(256) void k_shade(Frame F, int level, const uint32_
                     if (k < want_shadow) {
                         float rx = fractf(n1[j] + anim), ry = fractf(n2[j] + anim);
                         V3 sd = sample_dir_light(rx, ry, sun, lt, lb, sun_radius);
-                        uint32_t slot = sbase + k;
-                        F.sq.o[slot] = make_float4(sh_origin.x, sh_origin.y, sh_origin.z, 0.001f);
-                        F.sq.d[slot] = make_float4(sd.x, sd.y, sd.z, 10000.0f);
-                        F.sq.path[slot] = p;
+                        const uint32_t slot = sbase + k;
+                        if (!(k & 1u)) F.pair_o[slot / 2] = make_float4(sh_origin.x, sh_origin.y, sh_origin.z, u2f(p));
+                        F.pair_d[slot] = make_float4(sd.x, sd.y, sd.z, u2f(k + 1 < want_shadow ? 3u : 1u));
                     }
                 }
             }
-            if (want_shadow & 1u) F.sq.path[sbase + want_shadow] = kNoPath;
             n_shadow += want_shadow;
             n_textured++;
         }
@@ -930,32 +935,23 @@ __device__ inline void shadow_part(const Frame& F, int part, uint32_t& lo, uint3
     feed = F.feeds + (part == kPartRest ? kFeedShadowRest : kFeedShadow);
 }
 
-// The pair of shadow-queue entries 2q, 2q + 1 of [lo, hi): a path's shadow
-// rays are allocated from an even slot, so a pair holds the rays 2j, 2j + 1
-// of one path, or ray 2j alone when the path has an odd count (its last slot
-// is padding, path kNoPath). Returns the pair's mask (3, or 1 for ray 2j
-// alone) and its rays.
-__device__ inline uint32_t shadow_pair(const Frame& F, uint32_t e0, uint32_t hi, uint32_t& path, float4& o,
-                                       float4& d0, float4& d1) {
-    path = F.sq.path[e0];
+// The pair of shadow rays in slots e0, e0 + 1: the rays 2j, 2j + 1 of one
+// path, or ray 2j alone when the path has an odd count. Returns the pair's
+// mask (3, or 1 for ray 2j alone) and its rays. A pair shares one origin
+// record, so it takes 48 bytes where two whole rays took 72 (with the camera
+// rays' records: served requests 12.9 -> 10.8 ms a set).
+__device__ inline uint32_t shadow_pair(const Frame& F, uint32_t e0, uint32_t& path, float4& o, float4& d0,
+                                       float4& d1) {
+    o = F.pair_o[e0 / 2];
+    d0 = F.pair_d[e0];
+    path = f2u(o.w);
     if (path >= F.paths) {
         queue_range_error(F);
         path = 0;
     }
-    o = F.sq.o[e0];
-    d0 = F.sq.d[e0];
     d1 = d0;
-    if (e0 + 1 >= hi) return 1u;
-    const uint32_t p1 = F.sq.path[e0 + 1];
-    if (p1 == kNoPath) return 1u;
-    if (p1 != path) {
-        // entries of different paths in one pair: a frame state driven by
-        // two traces at once; its second ray is dropped (reported visible)
-        queue_range_error(F);
-        F.sflag[e0 + 1] = 1;
-        return 1u;
-    }
-    d1 = F.sq.d[e0 + 1];
+    if (f2u(d0.w) != 3u) return 1u;
+    d1 = F.pair_d[e0 + 1];
     return 3u;
 }
 
@@ -993,10 +989,11 @@ __device__ __forceinline__ void trace_occlusion(const Frame& F, uint32_t* status
             if (q != ~0u) {
                 e0 = lo + 2 * q;
                 float4 o, d0, d1;
-                started = shadow_pair(F, e0, hi, path, o, d0, d1);
+                started = shadow_pair(F, e0, path, o, d0, d1);
                 J = &F.jobs[find_job(F.jobs, F.njobs, path, false)];
                 T = tlas_view(J->tlas);
-                tr.start(T, v3(o.x, o.y, o.z), v3(d0.x, d0.y, d0.z), v3(d1.x, d1.y, d1.z), started, o.w, d0.w, st);
+                tr.start(T, v3(o.x, o.y, o.z), v3(d0.x, d0.y, d0.z), v3(d1.x, d1.y, d1.z), started, kShadowTmin,
+                         kRayTmax, st);
                 if (J->flags & RTG_TRACE_HEATMAP) c0 = (uint32_t)__builtin_readcyclecounter();
                 active = true;
             }
@@ -1050,10 +1047,11 @@ __device__ __forceinline__ void quad_occlusion(const Frame& F, uint32_t* status,
             if (q != ~0u) {
                 e0 = lo + 2 * q;
                 float4 o, d0, d1;
-                started = shadow_pair(F, e0, hi, path, o, d0, d1);
+                started = shadow_pair(F, e0, path, o, d0, d1);
                 J = &F.jobs[find_job(F.jobs, F.njobs, path, false)];
                 T = tlas_view(J->tlas);
-                tr.start(T, v3(o.x, o.y, o.z), v3(d0.x, d0.y, d0.z), v3(d1.x, d1.y, d1.z), started, o.w, d0.w, st);
+                tr.start(T, v3(o.x, o.y, o.z), v3(d0.x, d0.y, d0.z), v3(d1.x, d1.y, d1.z), started, kShadowTmin,
+                         kRayTmax, st);
                 if (J->flags & RTG_TRACE_HEATMAP) c0 = (uint32_t)__builtin_readcyclecounter();
                 active = true;
             }
@@ -1117,11 +1115,12 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_occlusion_rounds(Frame 
             const uint32_t e0 = lo + 2 * q;
             uint32_t path;
             float4 o, d0, d1;
-            const uint32_t started = shadow_pair(F, e0, hi, path, o, d0, d1);
+            const uint32_t started = shadow_pair(F, e0, path, o, d0, d1);
             const JobDev& J = F.jobs[find_job(F.jobs, F.njobs, path, false)];
             const TlasView T = tlas_view(J.tlas);
             PairTraverser<COUNT> tr;
-            tr.start(T, v3(o.x, o.y, o.z), v3(d0.x, d0.y, d0.z), v3(d1.x, d1.y, d1.z), started, o.w, d0.w, st);
+            tr.start(T, v3(o.x, o.y, o.z), v3(d0.x, d0.y, d0.z), v3(d1.x, d1.y, d1.z), started, kShadowTmin,
+                         kRayTmax, st);
             int res;
             while ((res = tr.step(T, J.scene, st, cnt)) == kRayActive) {
             }
@@ -1192,11 +1191,10 @@ __global__ __launch_bounds__(256) void k_resolve(Frame F, uint64_t total_pixels)
                 float in_nol = sf * a.x;
                 c = v3(a.y * in_nol + b.x, a.z * in_nol + b.y, a.w * in_nol + b.z);
             } else {
-                float4 r = F.path_rgb[p];
-                c = v3(r.x, r.y, r.z);
+                c = v3(b.x, b.y, b.z);
             }
             acc = acc + c;
-            cycles += F.cycles[p];
+            if (J.flags & RTG_TRACE_HEATMAP) cycles += F.cycles[p];
         }
         V3 col = J.spp == 1 ? acc : acc * (1.0f / (float)J.spp);
         if (J.flags & RTG_TRACE_HEATMAP) {
@@ -1288,7 +1286,6 @@ void free_frame_arena(rtg_ctx* ctx) {
 // shadow rays and `njobs` jobs: the buffer ensure_frame carves.
 size_t frame_bytes(uint64_t paths, uint64_t shadow, uint32_t njobs) {
     size_t off = 0;
-    carve_size<float4>(off, paths);    // path_rgb
     carve_size<float4>(off, paths);    // shade_a
     carve_size<float4>(off, paths);    // shade_b
     carve_size<uint8_t>(off, shadow);  // sflag
@@ -1300,9 +1297,8 @@ size_t frame_bytes(uint64_t paths, uint64_t shadow, uint32_t njobs) {
     }
     carve_size<uint4>(off, paths);
     carve_size<float2>(off, paths);
+    carve_size<float4>(off, (shadow + 1) / 2);
     carve_size<float4>(off, shadow);
-    carve_size<float4>(off, shadow);
-    carve_size<uint32_t>(off, shadow);
     carve_size<uint32_t>(off, kCountSlots);
     carve_size<uint32_t>(off, kFeedWords);
     carve_size<JobDev>(off, njobs);
@@ -1373,7 +1369,6 @@ static int ensure_frame(rtg_ctx* ctx, FrameArena* a, uint64_t paths, uint64_t sh
         if (a->buf.ensure(frame_bytes(P, S, NJ), !a->exact) != RTG_OK) return RTG_ERROR_OUT_OF_MEMORY;
         Carve c(a->buf.ptr);
         Frame& F = a->F;
-        F.path_rgb = c.take<float4>(P);
         F.shade_a = c.take<float4>(P);
         F.shade_b = c.take<float4>(P);
         F.sflag = c.take<uint8_t>(S);
@@ -1385,9 +1380,8 @@ static int ensure_frame(rtg_ctx* ctx, FrameArena* a, uint64_t paths, uint64_t sh
         }
         F.hit_a = c.take<uint4>(P);
         F.hit_b = c.take<float2>(P);
-        F.sq.o = c.take<float4>(S);
-        F.sq.d = c.take<float4>(S);
-        F.sq.path = c.take<uint32_t>(S);
+        F.pair_o = c.take<float4>((S + 1) / 2);
+        F.pair_d = c.take<float4>(S);
         a->d_counts = c.take<uint32_t>(kCountSlots);
         a->d_feeds = c.take<uint32_t>(kFeedWords);
         a->d_jobs = c.take<JobDev>(NJ);
@@ -1477,6 +1471,11 @@ int plan_jobs(rtg_ctx* ctx, const rtg_image_job* jobs, uint32_t njobs, FrameAren
         d.scene.texture_count = j.scene.texture_count;
         memcpy(d.view_inverse, j.uniforms.view_inverse, sizeof(d.view_inverse));
         memcpy(d.proj_inverse, j.uniforms.proj_inverse, sizeof(d.proj_inverse));
+        // view_inverse * (0, 0, 0, 1), in mat4_mul's order
+        for (int r = 0; r < 3; ++r) {
+            const float* m = j.uniforms.view_inverse + r;
+            d.origin[r] = ((m[0] * 0.0f + m[4] * 0.0f) + m[8] * 0.0f) + m[12] * 1.0f;
+        }
         memcpy(d.sun, j.uniforms.sun_dir, sizeof(d.sun));
         d.sun_radius = j.uniforms.sun_radius;
         d.bn_index = j.uniforms.blue_noise_texture_index;

@@ -641,6 +641,7 @@ struct Traverser {
     uint32_t inst_index, inst_flags;
     uint32_t cur;
     bool in_blas;
+    bool pending;  // the next entry has to come off the stack
     HitRec best;  // best.inst stays RTG_NO_HIT until a hit is accepted
 
     using StackT = Stack<OCCLUSION>;
@@ -649,6 +650,7 @@ struct Traverser {
                                  uint32_t mask, uint32_t sbt, StackT& st) {
         ray_setup_box(world, o, d);
         in_blas = false;
+        pending = false;
         nodes = T.nodes;
         tris = nullptr;
         tmin = tmin_;
@@ -682,6 +684,23 @@ struct Traverser {
         return false;
     }
 
+    // After a visit with nothing to go on to: an occlusion query pops its next
+    // entry here, a closest-hit query in step()'s one place.  The pop loop
+    // (stack words, the culled-by-distance test, leaving an instance) inlined
+    // behind each kind of visit is run by every subset of the wave in turn;
+    // one copy after the leaves serves them together.  16 M closest rays on a
+    // triangle soup 9785 -> 9363 us, the 1080p frame loop 4325 -> 4282.  An
+    // occlusion pop tests no distance and its lanes end at the first hit:
+    // there the shared pop only adds a pass (3 M rays 1122 -> 1196 us), so
+    // occlusion keeps the inlined one.
+    __device__ inline int next(const TlasView& T, StackT& st) {
+        if (!OCCLUSION) {
+            pending = true;
+            return kRayActive;
+        }
+        return pop(T, st) ? kRayActive : done();
+    }
+
     // pushes from stack position sp0 on that went past the LDS part
     __device__ static inline uint32_t spilled(int sp0, int sp1, int lds) {
         const int from = sp0 > lds ? sp0 : lds;
@@ -710,8 +729,7 @@ struct Traverser {
         bool h3 = slab(NX.w, FX.w, NY.w, FY.w, NZ.w, FZ.w, cr, tmin, tcur, t3) && C.w != kEmpty;
         const int nh = (int)h0 + (int)h1 + (int)h2 + (int)h3;
         if (nh == 0) {
-            if (!pop(T, st)) return done();
-            return kRayActive;
+            return next(T, st);
         }
         if (st.sp + nh - 1 > kStackMax) return kRayOverflow;
         if (COUNT) cnt.spills += spilled(st.sp, st.sp + nh - 1, st.lds_n);
@@ -751,8 +769,7 @@ struct Traverser {
         uint32_t mf = tail.w;
         const uint8_t* bb = reinterpret_cast<const uint8_t*>((uint64_t)tail.x | ((uint64_t)tail.y << 32));
         if (((mf & 0xffu) & cull_mask) == 0 || bb == nullptr) {
-            if (!pop(T, st)) return done();
-            return kRayActive;
+            return next(T, st);
         }
         if (COUNT) cnt.insts++;
         if (st.sp >= kStackMax) return kRayOverflow;
@@ -806,8 +823,7 @@ struct Traverser {
             if (OCCLUSION || (ray_flags & RTG_RAY_FLAG_TERMINATE_ON_FIRST_HIT)) return kRayHit;
             tcur = t;
         }
-        if (!pop(T, st)) return done();
-        return kRayActive;
+        return next(T, st);
     }
 
     // One iteration: a BLAS leaf, then a TLAS leaf, then an internal node,
@@ -826,6 +842,10 @@ struct Traverser {
             if (!leaf_turn) return kRayActive;
             const int r = leaf_step(T, S, st, cnt);
             if (r != kRayActive) return r;
+        }
+        if (!OCCLUSION && pending) {
+            if (!pop(T, st)) return done();
+            pending = false;
         }
         if ((cur & kLeafBit) && !in_blas) {
             if (!inst_turn) return kRayActive;

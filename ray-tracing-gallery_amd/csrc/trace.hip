@@ -1705,13 +1705,28 @@ static int check_ray_query(rtg_ctx* ctx, rtg_tlas tlas, const rtg_ray* rays, uin
     return RTG_OK;
 }
 
+// A closest-hit query on lanes takes a fifth workgroup per CU where the spill
+// area holds it, as a stream's area does (it is allocated with a quarter to
+// spare): the registers are few enough, and 15 stack entries a lane fit the
+// 160 KB of LDS five times. Incoherent rays fetch nodes and triangles past L2,
+// and a fifth wave per SIMD hides more of that than the entries spilled beyond
+// the 15th cost: 16 M rays in a 1 M-triangle soup 9,460 -> 8,530 us (15
+// entries on four workgroups 9,480, 12 on six 8,650). Occlusion queries lose
+// (3 M rays 1,104 -> 1,188 us), and so do frames (the 1080p loop 4,312 ->
+// 4,452): coherent rays hit the caches. A tuning other than four workgroups
+// is taken as it is.
+constexpr unsigned kQueryBlocksPerCu = 5;
+constexpr int kQueryStackLds = 15;
+
 // Clears the feed counters (`feed_stride` words apart) and launches the query
-// kernel on at most `max_blocks` persistent blocks, whose spill stacks start
-// at `spill` (max_blocks * kTraceThreads lanes).
+// kernel on at most `max_blocks` persistent blocks, closest hits on up to
+// `spill_blocks` where more pay: the workgroups whose spill stacks `spill`
+// holds (kTraceThreads lanes each).
 static void launch_ray_query(rtg_ctx* ctx, rtg_tlas tlas, const rtg_scene_bindings* scene, const rtg_ray* rays,
                              uint32_t count, uint32_t mode, uint32_t ray_flags, uint32_t cull_mask,
                              uint32_t sbt_offset, rtg_hit* hits, uint32_t* occluded, uint2* spill, uint32_t* feed,
-                             uint32_t feed_stride, unsigned max_blocks, bool timed, hipStream_t s) {
+                             uint32_t feed_stride, unsigned max_blocks, unsigned spill_blocks, bool timed,
+                             hipStream_t s) {
     SceneView S;
     S.models = scene ? reinterpret_cast<const rtg_model_info*>(scene->model_info) : nullptr;
     S.textures = scene ? reinterpret_cast<const rtg_texture*>(scene->textures) : nullptr;
@@ -1729,6 +1744,13 @@ static void launch_ray_query(rtg_ctx* ctx, rtg_tlas tlas, const rtg_scene_bindin
                            sbt_offset, hits, occluded, spill, ctx->d_status, ctx->tune.stack_lds);
         return;
     }
+    int entries = ctx->tune.stack_lds;
+    const unsigned wide = (unsigned)ctx->cu_count * kQueryBlocksPerCu;
+    if (!cnt && mode == RTG_QUERY_CLOSEST && max_blocks == (unsigned)ctx->cu_count * (kQueryBlocksPerCu - 1) &&
+        spill_blocks >= wide) {
+        max_blocks = wide;
+        entries = std::min(entries, kQueryStackLds);
+    }
     const unsigned G = (unsigned)std::min<uint64_t>((count + kTraceThreads - 1) / kTraceThreads, max_blocks);
     if (count > G * kTraceThreads)  // else the waves' first chunks are all there is
         hipLaunchKernelGGL(k_zero_feed, dim3(1), dim3(64), 0, s, feed, feed_stride);
@@ -1736,10 +1758,10 @@ static void launch_ray_query(rtg_ctx* ctx, rtg_tlas tlas, const rtg_scene_bindin
     if (cnt) hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, ctx->d_counters, (uint64_t)count);
     LaunchTimer t(ctx, mode == RTG_QUERY_CLOSEST ? RTG_KERNEL_TRACE_CLOSEST : RTG_KERNEL_TRACE_OCCLUSION, s, timed);
 #define RTG_LAUNCH_RAYS(OCC, CNT)                                                                                \
-    hipLaunchKernelGGL((k_trace_rays<OCC, CNT>), dim3(G), dim3(kTraceThreads), stack_lds_bytes(ctx->tune.stack_lds), \
+    hipLaunchKernelGGL((k_trace_rays<OCC, CNT>), dim3(G), dim3(kTraceThreads), stack_lds_bytes(entries),            \
                        s, tl, S, rays, count, ray_flags, cull_mask, sbt_offset, hits, occluded, spill, feed, feed_stride, \
                        ctx->d_counters, ctx->d_status, ctx->tune.refill_rays, (uint32_t)ctx->tune.feed_chunk,       \
-                       ctx->tune.stack_lds)
+                       entries)
     if (mode == RTG_QUERY_CLOSEST) {
         if (cnt) RTG_LAUNCH_RAYS(false, true);
         else RTG_LAUNCH_RAYS(false, false);
@@ -1769,7 +1791,7 @@ extern "C" int rtg_trace_rays(rtg_ctx* ctx, rtg_tlas tlas, const rtg_scene_bindi
         return RTG_ERROR_OUT_OF_MEMORY;
     launch_ray_query(ctx, tlas, scene, rays, count, mode, ray_flags, cull_mask, sbt_offset, hits, occluded,
                      reinterpret_cast<uint2*>(a->spill.ptr), reinterpret_cast<uint32_t*>(a->feed.ptr), kFeedStride,
-                     (unsigned)trace_grid(ctx), true, s);
+                     (unsigned)trace_grid(ctx), (unsigned)(a->spill.size / (kTraceThreads * kSpillLaneBytes)), true, s);
     RTG_HIP(hipGetLastError());
     return RTG_OK;
 }
@@ -1834,7 +1856,7 @@ extern "C" int rtg_trace_rays_static(rtg_ctx* ctx, rtg_tlas tlas, const rtg_scen
     launch_ray_query(ctx, tlas, scene, rays, count, mode, ray_flags, cull_mask, sbt_offset, hits, occluded,
                      reinterpret_cast<uint2*>(base + kStaticFeedBytes), reinterpret_cast<uint32_t*>(base),
                      (uint32_t)(kStaticFeedBytes / kFeedGroups / sizeof(uint32_t)),
-                     std::min((unsigned)trace_grid(ctx), kStaticBlocks), false,
+                     std::min((unsigned)trace_grid(ctx), kStaticBlocks), kStaticBlocks, false,
                      reinterpret_cast<hipStream_t>(stream));
     RTG_HIP(hipGetLastError());
     return RTG_OK;

@@ -477,7 +477,9 @@ typedef struct rtg_tuning {
                                   bounce levels (on at most 192 of them) and the shadow rays they add
                                   (on all) beside the first level's shadow rays (taken from the
                                   blocks_per_cu grid, at most half of it); 192 by default;
-                                  0 = every level in sequence on the caller's stream */
+                                  0 = every level in sequence on the caller's stream, as is an
+                                  uncounted trace enqueued while another of the context is in
+                                  flight (on another stream, frame slot or server slot) */
     uint32_t stack_lds_entries; /* traversal stack entries per lane kept in LDS (8..32, multiple of 4;
                                   0 = 16): a workgroup takes entries * 2 KB of LDS, deeper entries
                                   spill to global memory; the occlusion queries of rtg_trace_rays

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <atomic>
 #include <map>
 #include <string>
 #include <vector>
@@ -84,6 +85,7 @@ struct TimedLaunch {
 };
 
 struct FrameArena;  // trace.hip
+constexpr int kFlightSlots = 64;
 struct BuildReport;  // build_tree.hpp
 
 // Launch parameters of the traversal kernels (defaults, overridable through
@@ -112,11 +114,10 @@ struct Tuning {
     // persistent blocks given to the bounce stream beside the first level's
     // shadow rays (0: all levels in sequence on the caller's stream): its
     // shadow-ray launch takes them all, its bounce-level launches at most
-    // 192, and the first level's shadow rays the rest of the grid. 192 of
-    // 1,024 measured best on the 1080p scene with two frames in flight
-    // (3,668-3,738 Mrays/s in seven runs on two boxes); 224, 256 and 320
-    // often settled into a slower overlap of the two frames, 384 once in
-    // seven runs, and 448 or more slowed the first level's shadow rays
+    // 192, and the first level's shadow rays the rest of the grid. Frames
+    // alone on the GPU (traces beside others in flight run in sequence) take
+    // 410 us at 480x270 and 681 at 1280x720 with 192 of 1,024, 423 and 762
+    // with 128, 451 and 977 with 64
     int bounce_blocks = 192;
     // stack entries per lane kept in LDS by every traversal launch (8-B
     // entries; the single-ray occlusion queries of the ray API keep twice as
@@ -150,6 +151,12 @@ struct rtg_ctx {
     uint64_t kernel_launches[RTG_KERNEL_COUNT] = {};
     // frame state of the context's own calls, one per stream they are made on
     std::map<void*, rtg::FrameArena*> frames;
+    // Traces in flight, by arena: how many each has started, and (in host
+    // memory, written by a trace's last kernel) the last that ended. More
+    // arenas than words share them: that can only make a trace look in flight.
+    std::atomic<uint32_t> flight_started[rtg::kFlightSlots] = {};
+    std::atomic<uint32_t> flight_next{0};
+    uint32_t* flight_done = nullptr;
     rtg::Tuning tune;
 };
 
@@ -210,9 +217,11 @@ void arena_pointers(const FrameArena* a, const void* out[3]);
 int upload_jobs(FrameArena* a, const TracePlan& P, hipStream_t stream);
 // Device half: the kernels of the step and nothing else (no copy, memset or
 // allocation), so that it can be captured into a graph. Launch parameters
-// come from `tune`; `timed` records kernel events when timing is on.
+// come from `tune`; `timed` records kernel events when timing is on; `flight`
+// enters the trace in the context's flight table (not for kernels that are
+// captured to run later).
 void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning& tune, bool counters, bool timed,
-                   hipStream_t stream);
+                   hipStream_t stream, bool flight = false);
 // Device bytes of the spill area of the persistent traversal grid.
 size_t spill_bytes(rtg_ctx* ctx, const Tuning& tune);
 // Launches made by the calling thread are not timed (a server's worker).

@@ -348,9 +348,11 @@ __global__ void k_frame_begin(uint32_t* counts, uint32_t* feeds, uint64_t* count
     if (reset_counters && threadIdx.x < kCounterSlots) counters[threadIdx.x] = 0;
 }
 
-// ORs a trace's status bits into the context's sticky ones.
-__global__ void k_status_merge(const uint32_t* trace_status, uint32_t* ctx_status) {
+// ORs a trace's status bits into the context's sticky ones; `done`, if not
+// null, is the host word that says which trace of its arena has ended.
+__global__ void k_status_merge(const uint32_t* trace_status, uint32_t* ctx_status, uint32_t* done, uint32_t seq) {
     if (threadIdx.x == 0 && *trace_status) atomicOr(ctx_status, *trace_status);
+    if (threadIdx.x == 0 && done) __hip_atomic_store(done, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __global__ void k_shadow_snapshot(uint32_t* counts) {
@@ -1243,6 +1245,7 @@ struct FrameArena {
     // grow to exactly the size asked (no headroom): a server slot's arena,
     // whose device bytes count against an HBM budget
     bool exact = false;
+    int flight = -1;  // its word in the context's flight table, from its first trace on
     // host calls using the arena now: a second one at the same time (two
     // threads tracing on one stream of one context) is refused
     std::atomic<int> users{0};
@@ -1504,8 +1507,19 @@ int upload_jobs(FrameArena* a, const TracePlan& P, hipStream_t s) {
     return RTG_OK;
 }
 
+// Whether a trace of another arena than `a` is on the GPU, as far as the host
+// words tell (a moment's view, which changes launch shapes only).
+static bool others_in_flight(rtg_ctx* ctx, const FrameArena* a) {
+    for (int k = 0; k < kFlightSlots; ++k)
+        if (k != a->flight &&
+            ctx->flight_started[k].load(std::memory_order_relaxed) !=
+                __atomic_load_n(&ctx->flight_done[k], __ATOMIC_RELAXED))
+            return true;
+    return false;
+}
+
 void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning& tune, bool cnt, bool timed,
-                   hipStream_t s) {
+                   hipStream_t s, bool flight) {
     Frame F = a->F;
     F.jobs = a->d_jobs;
     F.njobs = P.njobs;
@@ -1594,7 +1608,15 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
         }
     };
     level_step(F, 0, G, Gsmall, s, timed);
-    const unsigned Gside = std::min<unsigned>((unsigned)tune.bounce_blocks, G / 2);
+    // With another trace in flight the bounce levels leave no gap to fill,
+    // and a second stream costs: streams share the process's four hardware
+    // queues, where its waits hold up the other traces' kernels. Two frames
+    // in flight, levels in sequence against side by side: 4,157 us to 4,226
+    // at 1920x1080, 1,680 to 2,170 at 960x540, 1,004 to 1,500 at 480x270. A
+    // frame alone is the faster side by side: 410 us to 505 at 480x270, 681
+    // to 775 at 1280x720. Counted traces keep the setting's split.
+    const bool crowded = flight && !cnt && others_in_flight(ctx, a);
+    const unsigned Gside = crowded ? 0 : std::min<unsigned>((unsigned)tune.bounce_blocks, G / 2);
     if (P.max_traces > 1 && Gside > 0) {
         // The bounce levels hold few rays, so their launches are short of
         // work and bound by the latency of their longest rays. They run on
@@ -1636,7 +1658,14 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
         unsigned Gr = (unsigned)std::min<uint64_t>((P.pixels + 255) / 256, (uint64_t)ctx->cu_count * 16);
         hipLaunchKernelGGL(k_resolve, dim3(Gr), dim3(256), 0, s, F, P.pixels);
     }
-    hipLaunchKernelGGL(k_status_merge, dim3(1), dim3(64), 0, s, F.status, ctx->d_status);
+    uint32_t* done = nullptr;
+    uint32_t seq = 0;
+    if (flight) {
+        if (a->flight < 0) a->flight = (int)(ctx->flight_next.fetch_add(1) % kFlightSlots);
+        done = ctx->flight_done + a->flight;
+        seq = ctx->flight_started[a->flight].fetch_add(1) + 1;
+    }
+    hipLaunchKernelGGL(k_status_merge, dim3(1), dim3(64), 0, s, F.status, ctx->d_status, done, seq);
 }
 
 // Marks an arena as used by this host call for its duration.
@@ -1661,7 +1690,7 @@ int trace_jobs(rtg_ctx* ctx, const rtg_image_job* jobs, uint32_t njobs, hipStrea
     if (st != RTG_OK) return st;
     st = upload_jobs(a, P, s);
     if (st != RTG_OK) return st;
-    enqueue_trace(ctx, a, P, t, ctx->counters_enabled, true, s);
+    enqueue_trace(ctx, a, P, t, ctx->counters_enabled, true, s, true);
     RTG_HIP(hipGetLastError());
     return RTG_OK;
 }

@@ -94,21 +94,25 @@ __device__ __forceinline__ void wave_order() {
 // their high bits; the dynamic programme goes by subset size, the sets of a
 // size (or parts of their partitions) side by side in the lanes, its table
 // in LDS. One lane for a whole treelet took 85 us of dependent LDS reads,
-// whatever a level's size; a group of 16 takes about 5 us.
+// whatever a level's size; a group of 16 takes about 5 us, a chain of some
+// 750 VALU operations and 30 LDS round trips of one wave: records read ahead
+// of the choice between them, minima over lanes by DPP, a lane's sets in
+// registers, the new boxes straight from the leaves (1 M triangles 5,880 ->
+// 5,720 us).
 // ---------------------------------------------------------------------------
 constexpr int kTreeletLeaves = 7;
 constexpr int kTreeletRounds = 5;  // passes with RTG_BUILD_PREFER_FAST_TRACE
 
 struct alignas(16) TreeletScratch {
     float cost[1 << kTreeletLeaves];
-    float lbox[kTreeletLeaves * 6 + 2];  // boxes of the treelet's leaves
-    float nbox[(kTreeletLeaves - 1) * 6];  // boxes of its new internal nodes
-    float larea[8], narea[8];
-    uint32_t lref[8], lcount[8], inner[8];
+    float4 leaf[kTreeletLeaves][2];  // lo.xyz, hi.x; hi.yz, area, reference
+    uint32_t lcount[8], inner[8];
     uint8_t split[1 << kTreeletLeaves];
-    uint32_t pad[12];  // groups of a wave start 16 banks apart
+    float nbox[kTreeletLeaves - 1][6];  // boxes of the new nodes, where their order matters
+    uint32_t pad[4];  // groups of a wave start 16 banks apart
 };
 static_assert(sizeof(TreeletScratch) % 16 == 0, "scratch records stay 16-byte aligned");
+static_assert(sizeof(TreeletScratch) / 4 % 32 == 16, "groups of a wave start 16 banks apart");
 
 // The subsets of 7 treelet leaves by size (2 to 7), ascending within a size,
 // so that those of the first m leaves come first.
@@ -158,17 +162,99 @@ __device__ __forceinline__ uint32_t max8(uint32_t x) {
     return dpp_max<0x141>(x);  // row_half_mirror
 }
 
+// The sets a lane works on, a byte each, in the order of treelet_sizes: fixed
+// by its place in the group, so read once per kernel.
+template <int G>
+struct TreeletLane {
+    static constexpr int kWords = G == 16 ? 3 : 2;
+    uint32_t w[kWords];
+    __device__ __forceinline__ uint32_t set(int k) const { return (w[k / 4] >> (8 * (k % 4))) & 0xffu; }
+    template <int M, int L, int K>
+    __device__ __forceinline__ void fill(int gl) {
+        constexpr int kTasks = (int)binom(kTreeletLeaves, M) * L, kIters = (kTasks + G - 1) / G;
+#pragma unroll
+        for (int it = 0; it < kIters; ++it) {
+            const int task = it * G + gl;
+            const uint32_t s = kTreeletSetTable.s[set_offset(M) + (task < kTasks ? task : 0) / L];
+            w[(K + it) / 4] |= s << (8 * ((K + it) % 4));
+        }
+    }
+    __device__ __forceinline__ void init() {
+        const int gl = threadIdx.x & (G - 1);
+#pragma unroll
+        for (int k = 0; k < kWords; ++k) w[k] = 0;
+        if constexpr (G == 16) {
+            fill<2, 1, 0>(gl);
+            fill<3, 1, 2>(gl);
+            fill<4, 1, 5>(gl);
+            fill<5, 2, 8>(gl);
+            fill<6, 2, 11>(gl);
+        } else {
+            fill<2, 1, 0>(gl);
+            fill<3, 1, 1>(gl);
+            fill<4, 1, 2>(gl);
+            fill<5, 2, 3>(gl);
+            fill<6, 8, 4>(gl);
+        }
+    }
+};
+
+// One step of split_min: the other lane's (cost, split), taken if it is the
+// better or, at the same cost, the larger split. Split 0 holds none; a NaN
+// (only the first partition's cost can be one here) is taken as it stands.
+__device__ __forceinline__ void split_take(float& best, uint32_t& bp, float co, uint32_t po) {
+    const bool less = co < best || (co == best && po > bp);
+    const bool take = po != 0u && (bp == 0u || co != co || (best == best && less));
+    if (take) {
+        best = co;
+        bp = po;
+    }
+}
+template <int Ctrl>
+__device__ __forceinline__ void split_take_dpp(float& best, uint32_t& bp) {
+    const float co =
+        __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(best), Ctrl, 0xf, 0xf, true));
+    const uint32_t po = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)bp, Ctrl, 0xf, 0xf, true);
+    split_take(best, bp, co, po);
+}
+// The least cost and its split over the aligned L lanes this lane is in (L =
+// 64: in every lane the wave's).
+template <int L>
+__device__ __forceinline__ void split_min(float& best, uint32_t& bp) {
+    if (L >= 2) split_take_dpp<0xB1>(best, bp);    // quad_perm 1,0,3,2
+    if (L >= 4) split_take_dpp<0x4E>(best, bp);    // quad_perm 2,3,0,1
+    if (L >= 8) split_take_dpp<0x141>(best, bp);   // row_half_mirror
+    if (L >= 16) split_take_dpp<0x140>(best, bp);  // row_mirror
+    if (L == 64) {
+        float c[4];
+        uint32_t p[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            c[r] = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(best), 16 * r));
+            p[r] = (uint32_t)__builtin_amdgcn_readlane((int)bp, 16 * r);
+        }
+        best = c[0];
+        bp = p[0];
+#pragma unroll
+        for (int r = 1; r < 4; ++r) split_take(best, bp, c[r], p[r]);
+    }
+}
+
 // Costs and splits of the subsets of M treelet leaves. L lanes share a set:
 // lane h of them tries the partitions whose top log2(L) free leaves are the
-// complement of h's bits, so that ascending h is descending P.
-template <int G, int M, int L>
-__device__ __forceinline__ void treelet_size(TreeletScratch* sc, const uint8_t* sets, int nl, int gl) {
+// complement of h's bits, so that ascending h is descending P. K: the lane's
+// first set of this size. The sets of a lane are independent, so their table
+// reads go out together; lanes without a set read another's and write none.
+template <int G, int M, int L, int K>
+__device__ __forceinline__ void treelet_size(TreeletScratch* sc, const TreeletLane<G>& lane, int nl, int gl) {
     if (M > nl) return;
     constexpr int kLog = L == 1 ? 0 : L == 2 ? 1 : L == 4 ? 2 : L == 8 ? 3 : L == 16 ? 4 : 6;
     constexpr int kSteps = 1 << (M - 1 - kLog);
-    const uint32_t ntask = set_count<M>(nl) * L;
-    for (uint32_t task = gl; task < ntask; task += G) {
-        const uint32_t S = sets[set_offset(M) + task / L], h = task % L;
+    constexpr int kIters = ((int)binom(kTreeletLeaves, M) * L + G - 1) / G;
+    const uint32_t ntask = set_count<M>(nl) * L, h = (uint32_t)gl % L;
+#pragma unroll
+    for (int it = 0; it < kIters; ++it) {
+        const uint32_t S = M == kTreeletLeaves ? (1u << kTreeletLeaves) - 1u : lane.set(K + it);
         const uint32_t low = S & (0u - S);
         uint32_t R = S ^ low, P0 = low;
 #pragma unroll
@@ -180,12 +266,11 @@ __device__ __forceinline__ void treelet_size(TreeletScratch* sc, const uint8_t* 
         // q runs down over the submasks of R; for h = 0 the first one gives
         // P = S, no partition; the first real one starts the minimum
         // whatever its value (a NaN cost stays the minimum)
-        float best = __builtin_inff();
-        uint32_t bp = 0, q = R;
         const uint32_t first_h = kSteps > 1 ? 0u : 1u;
         constexpr int first_i = kSteps > 1 ? 1 : 0;
-        float c[kSteps];
-        uint32_t P[kSteps];
+        const float area = sc->cost[S];
+        float c[kSteps], best = __builtin_inff();
+        uint32_t P[kSteps], bp = 0, q = R;
 #pragma unroll
         for (int i = 0; i < kSteps; ++i) {
             P[i] = P0 | q;
@@ -202,105 +287,118 @@ __device__ __forceinline__ void treelet_size(TreeletScratch* sc, const uint8_t* 
                 bp = P[i];
             }
         }
-#pragma unroll
-        for (int off = 1; off < L; off <<= 1) {
-            const float co = __shfl_xor(best, off);
-            const uint32_t po = (uint32_t)__shfl_xor((int)bp, off);
-            const bool less = co < best || (co == best && (h & off) != 0u);
-            const bool take = po != 0u && (bp == 0u || co != co || (best == best && less));
-            if (take) {
-                best = co;
-                bp = po;
-            }
-        }
-        if (h == 0) {
-            sc->cost[S] = sc->cost[S] + best;
+        split_min<L>(best, bp);
+        if (h == 0 && (uint32_t)(it * G + gl) < ntask) {
+            sc->cost[S] = area + best;
             sc->split[S] = (uint8_t)bp;
         }
+        if (kSteps >= 8) __builtin_amdgcn_sched_barrier(0);
     }
     wave_order();
+}
+
+__device__ __forceinline__ void treelet_planes(const TreeletScratch* sc, float pl[kTreeletLeaves][6]) {
+#pragma unroll
+    for (int k = 0; k < kTreeletLeaves; ++k) {
+        const float4 x = sc->leaf[k][0], y = sc->leaf[k][1];
+        pl[k][0] = x.x; pl[k][1] = x.y; pl[k][2] = x.z;
+        pl[k][3] = x.w; pl[k][4] = y.x; pl[k][5] = y.y;
+    }
 }
 
 // Restructures the treelet of node r (three or more primitives below it);
 // the G lanes of a group call it together. Store: rec(id), box(ref),
 // count(ref), put(id, record, box, count).
 template <int G, class Store>
-__device__ void treelet_group(Store& S, uint32_t r, TreeletScratch* sc, const uint8_t* sets) {
+__device__ __forceinline__ void treelet_group(Store& S, uint32_t r, TreeletScratch* sc, TreeletLane<G> lane) {
     static_assert(G == 16 || G == 64, "group sizes");
+    // opaque here, or everything that follows from the sets alone is kept in
+    // registers across treelets (256 of them, and spills)
+#pragma unroll
+    for (int k = 0; k < TreeletLane<G>::kWords; ++k) asm volatile("" : "+v"(lane.w[k]));
     constexpr int kLowBits = G == 16 ? 3 : 1;  // subset bits a lane goes through by itself
     const int gl = threadIdx.x & (G - 1);
     const int base = (threadIdx.x & 63) & ~(G - 1);
-    // formation: lane k < nl holds leaf k
-    uint32_t ref = kEmpty, inner = 0;
+    // formation: lane k < nl holds leaf k and, if it is an internal node, its
+    // record, read ahead of the choice that may open it
+    uint32_t ref = kEmpty;
     float area = 0.0f;
-    {
-        const BinNode nd = S.rec(r);
-        if (gl == 0) ref = nd.left;
-        if (gl == 1) ref = nd.right;
-        if (gl < 2 && !(ref & kLeafBit)) area = box_area(S.box(ref));
+    BinNode nd = S.rec(r);
+    if (gl == 0) ref = nd.left;
+    if (gl == 1) ref = nd.right;
+    if (gl < 2 && !(ref & kLeafBit)) {
+        nd = S.rec(ref);
+        area = box_area(S.box(ref));
     }
+    if (gl == 0) sc->inner[0] = r;
     int nl = 2;
     while (nl < kTreeletLeaves) {
         const bool internal = gl < nl && !(ref & kLeafBit);
         // largest area, lowest lane; a NaN area wins only in the first
         // internal leaf and never later, as the comparisons in leaf order do
-        uint32_t key = internal ? f2ord(area + 0.0f) : 0u;
-        const uint64_t cand = (__ballot(internal) >> base) & 0xffu;
+        const uint32_t cand = (uint32_t)(__ballot(internal) >> base) & 0xffu;
         if (cand == 0) break;
-        if (internal && area != area) key = (int)__builtin_ctzll(cand) == gl ? 0xffffffffu : 1u;
+        uint32_t key = internal ? f2ord(area + 0.0f) : 0u;
+        if (__ballot(area != area) != 0) {
+            if (internal && area != area) key = __builtin_ctz(cand) == gl ? 0xffffffffu : 1u;
+        }
         const uint32_t top = max8(key);
-        const uint64_t at = (__ballot(internal && key == top) >> base) & 0xffu;
-        const int best = (int)__builtin_ctzll(at);
-        const uint32_t c = (uint32_t)__shfl((int)ref, best, G);
-        const BinNode nd = S.rec(c);
-        if (gl == nl - 2) inner = c;
+        const int best = __builtin_ctz((uint32_t)(__ballot(internal && key == top) >> base) & 0xffu);
+        uint32_t right;
+        float area_r;
+        if (G == 64) {
+            right = (uint32_t)__builtin_amdgcn_readlane((int)nd.right, best);
+            area_r = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(nd.area_r), best));
+        } else {
+            right = (uint32_t)__shfl((int)nd.right, best, G);
+            area_r = __shfl(nd.area_r, best, G);
+        }
         if (gl == best) {
+            sc->inner[nl - 1] = ref;
             ref = nd.left;
             area = nd.area_l;
         }
         if (gl == nl) {
-            ref = nd.right;
-            area = nd.area_r;
+            ref = right;
+            area = area_r;
         }
+        if ((gl == best || gl == nl) && !(ref & kLeafBit)) nd = S.rec(ref);
         ++nl;
     }
+    // A box plane that is NaN or -0 makes a box depend on the order its
+    // leaves are folded in; without one any order gives the same bits.
+    bool ordered = false;
     if (gl < nl) {
         const Box b = S.box(ref);
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            sc->lbox[gl * 6 + a] = b.lo[a];
-            sc->lbox[gl * 6 + 3 + a] = b.hi[a];
+            ordered = ordered || b.lo[a] != b.lo[a] || __float_as_uint(b.lo[a]) == 0x80000000u;
+            ordered = ordered || b.hi[a] != b.hi[a] || __float_as_uint(b.hi[a]) == 0x80000000u;
         }
-        sc->lref[gl] = ref;
-        sc->larea[gl] = area;
+        sc->leaf[gl][0] = make_float4(b.lo[0], b.lo[1], b.lo[2], b.hi[0]);
+        sc->leaf[gl][1] = make_float4(b.hi[1], b.hi[2], area, __uint_as_float(ref));
         sc->lcount[gl] = S.count(ref);
-        if (gl == 0) sc->inner[0] = r;
-        if (gl < nl - 2) sc->inner[1 + gl] = inner;
     }
+    ordered = ((__ballot(ordered) >> base) & 0xffu) != 0;
     wave_order();
     // areas of the subsets: the lane's high bits choose leaves kLowBits..6.
     // fminf/fmaxf fold the same values as the selects of box_union from the
     // empty box (NaN planes skipped); a zero's sign does not change an area.
     {
-        float lo[3], hi[3], l[kLowBits][6];
+        float lo[3], hi[3], pl[kTreeletLeaves][6];
+        treelet_planes(sc, pl);
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
             lo[a] = __builtin_inff();
             hi[a] = -__builtin_inff();
         }
 #pragma unroll
-        for (int k = 0; k < kTreeletLeaves; ++k) {
-            float p[6];
-#pragma unroll
-            for (int a = 0; a < 6; ++a) p[a] = sc->lbox[k * 6 + a];
-            if (k < kLowBits) {
-#pragma unroll
-                for (int a = 0; a < 6; ++a) l[k][a] = p[a];
-            } else if ((gl >> (k - kLowBits)) & 1) {
+        for (int k = kLowBits; k < kTreeletLeaves; ++k) {
+            if ((gl >> (k - kLowBits)) & 1) {
 #pragma unroll
                 for (int a = 0; a < 3; ++a) {
-                    lo[a] = fminf(lo[a], p[a]);
-                    hi[a] = fmaxf(hi[a], p[3 + a]);
+                    lo[a] = fminf(lo[a], pl[k][a]);
+                    hi[a] = fmaxf(hi[a], pl[k][3 + a]);
                 }
             }
         }
@@ -314,8 +412,8 @@ __device__ void treelet_group(Store& S, uint32_t r, TreeletScratch* sc, const ui
 #pragma unroll
                 for (int k = 0; k < kLowBits; ++k)
                     if ((low >> k) & 1) {
-                        bl[a] = fminf(bl[a], l[k][a]);
-                        bh[a] = fmaxf(bh[a], l[k][3 + a]);
+                        bl[a] = fminf(bl[a], pl[k][a]);
+                        bh[a] = fmaxf(bh[a], pl[k][3 + a]);
                     }
             }
             const float ex = bh[0] - bl[0], ey = bh[1] - bl[1], ez = bh[2] - bl[2];
@@ -325,95 +423,100 @@ __device__ void treelet_group(Store& S, uint32_t r, TreeletScratch* sc, const ui
         }
     }
     wave_order();
-    if (G == 16) {
-        treelet_size<G, 2, 1>(sc, sets, nl, gl);
-        treelet_size<G, 3, 1>(sc, sets, nl, gl);
-        treelet_size<G, 4, 1>(sc, sets, nl, gl);
-        treelet_size<G, 5, 2>(sc, sets, nl, gl);
-        treelet_size<G, 6, 2>(sc, sets, nl, gl);
-        treelet_size<G, 7, 16>(sc, sets, nl, gl);
+    if constexpr (G == 16) {
+        treelet_size<G, 2, 1, 0>(sc, lane, nl, gl);
+        treelet_size<G, 3, 1, 2>(sc, lane, nl, gl);
+        treelet_size<G, 4, 1, 5>(sc, lane, nl, gl);
+        treelet_size<G, 5, 2, 8>(sc, lane, nl, gl);
+        treelet_size<G, 6, 2, 11>(sc, lane, nl, gl);
+        treelet_size<G, 7, 16, 0>(sc, lane, nl, gl);
     } else {
-        treelet_size<G, 2, 1>(sc, sets, nl, gl);
-        treelet_size<G, 3, 1>(sc, sets, nl, gl);
-        treelet_size<G, 4, 1>(sc, sets, nl, gl);
-        treelet_size<G, 5, 2>(sc, sets, nl, gl);
-        treelet_size<G, 6, 8>(sc, sets, nl, gl);
-        treelet_size<G, 7, 64>(sc, sets, nl, gl);
+        treelet_size<G, 2, 1, 0>(sc, lane, nl, gl);
+        treelet_size<G, 3, 1, 1>(sc, lane, nl, gl);
+        treelet_size<G, 4, 1, 2>(sc, lane, nl, gl);
+        treelet_size<G, 5, 2, 3>(sc, lane, nl, gl);
+        treelet_size<G, 6, 8, 4>(sc, lane, nl, gl);
+        treelet_size<G, 7, 64, 0>(sc, lane, nl, gl);
     }
-    // The new internal nodes, in the order they come off the stack (every
-    // lane of the group follows it): node j's set, number and children as
-    // codes: 0..6 a treelet leaf, 8 + x internal node number inner[x].
-    uint32_t node[kTreeletLeaves - 1];
-    uint32_t jof = 0;  // 4 bits per internal number: its place in the order
+    // The new internal nodes in the order they come off the stack: lane j
+    // walks down the splits to node j. A node j0 over P and Q is followed by
+    // P's internal nodes, |P| - 1 of them, then Q's; splitting it hands out
+    // the numbers of those of P and Q that are internal, `next` on. Children
+    // as codes: 0..6 a treelet leaf, 8 + x internal node number inner[x].
+    const bool mine = gl < nl - 1;
+    uint32_t set = (1u << nl) - 1u, id = 0, next = 1, c0 = 0, c1 = 0, np = 0;
     {
-        uint64_t st_set = (1u << nl) - 1u, st_id = 0;  // stacks of 8-bit entries
-        uint32_t next = 1;
-#pragma unroll
-        for (int j = 0; j < kTreeletLeaves - 1; ++j) {
-            if (j < nl - 1) {
-                const uint32_t set = (uint32_t)st_set & 0xffu, id = (uint32_t)st_id & 0xffu;
-                st_set >>= 8;
-                st_id >>= 8;
-                jof |= (uint32_t)j << (4 * id);
+        int j0 = 0;
+        bool walking = mine;
+        while (__ballot(walking) != 0) {
+            if (walking) {
                 const uint32_t P = sc->split[set], Q = set ^ P;
-                uint32_t c0, c1;
-                const bool m0 = (P & (P - 1u)) != 0u, m1 = (Q & (Q - 1u)) != 0u;
-                c0 = m0 ? 8u + next : (uint32_t)__builtin_ctz(P);
-                next += m0 ? 1u : 0u;
-                c1 = m1 ? 8u + next : (uint32_t)__builtin_ctz(Q);
-                next += m1 ? 1u : 0u;
-                if (m1) {
-                    st_set = (st_set << 8) | Q;
-                    st_id = (st_id << 8) | (c1 - 8u);
+                np = (uint32_t)__popc(P);
+                const uint32_t m0 = np > 1u ? 1u : 0u, m1 = (Q & (Q - 1u)) != 0u ? 1u : 0u;
+                if (j0 == gl) {
+                    c0 = m0 ? 8u + next : (uint32_t)__builtin_ctz(P);
+                    c1 = m1 ? 8u + next + m0 : (uint32_t)__builtin_ctz(Q);
+                    walking = false;
+                } else {
+                    const bool in_p = gl < j0 + (int)np;
+                    set = in_p ? P : Q;
+                    id = in_p ? next : next + m0;
+                    next += m0 + m1 + (in_p || np < 2u ? 0u : np - 2u);
+                    j0 += in_p ? 1 : (int)np;
                 }
-                if (m0) {
-                    st_set = (st_set << 8) | P;
-                    st_id = (st_id << 8) | (c0 - 8u);
-                }
-                node[j] = set | (id << 8) | (c0 << 12) | (c1 << 16);
-            } else {
-                node[j] = 0;
             }
         }
     }
-    // their boxes, last to first (children come after their parents): lane a
-    // folds plane a
-#pragma unroll
-    for (int j = kTreeletLeaves - 2; j >= 0; --j) {
-        if (j < nl - 1 && gl < 6) {
-            const uint32_t c0 = (node[j] >> 12) & 0xfu, c1 = (node[j] >> 16) & 0xfu;
-            const float x = c0 < 8u ? sc->lbox[c0 * 6 + gl] : sc->nbox[((jof >> (4 * (c0 - 8u))) & 0xfu) * 6 + gl];
-            const float y = c1 < 8u ? sc->lbox[c1 * 6 + gl] : sc->nbox[((jof >> (4 * (c1 - 8u))) & 0xfu) * 6 + gl];
-            sc->nbox[j * 6 + gl] = gl < 3 ? mins(x, y) : maxs(x, y);
-        }
-        wave_order();
-    }
-    uint32_t mine = 0;
     Box b = box_empty();
-    if (gl < nl - 1) {
+    if (__ballot(ordered && mine) == 0) {
+        float pl[kTreeletLeaves][6];
+        treelet_planes(sc, pl);
 #pragma unroll
-        for (int j = 0; j < kTreeletLeaves - 1; ++j)
-            if (j == gl) mine = node[j];
+        for (int k = 0; k < kTreeletLeaves; ++k) {
+            const bool in = ((set >> k) & 1u) != 0u;
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            b.lo[a] = sc->nbox[gl * 6 + a];
-            b.hi[a] = sc->nbox[gl * 6 + 3 + a];
+            for (int a = 0; a < 3; ++a) {
+                b.lo[a] = fminf(b.lo[a], in ? pl[k][a] : __builtin_inff());
+                b.hi[a] = fmaxf(b.hi[a], in ? pl[k][3 + a] : -__builtin_inff());
+            }
         }
-        sc->narea[gl] = box_area(b);
+    } else {
+        // last to first (children come after their parents)
+        for (int j = kTreeletLeaves - 2; j >= 0; --j) {
+            if (mine && gl == j) {
+                Box x, y;
+#pragma unroll
+                for (int a = 0; a < 6; ++a) {
+                    const float u = c0 < 8u ? reinterpret_cast<const float*>(sc->leaf[c0])[a] : sc->nbox[j + 1][a];
+                    const float v = c1 < 8u ? reinterpret_cast<const float*>(sc->leaf[c1])[a]
+                                            : sc->nbox[j + (int)np][a];
+                    (a < 3 ? x.lo[a % 3] : x.hi[a % 3]) = u;
+                    (a < 3 ? y.lo[a % 3] : y.hi[a % 3]) = v;
+                }
+                b = box_union(x, y);
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    sc->nbox[j][a] = b.lo[a];
+                    sc->nbox[j][3 + a] = b.hi[a];
+                }
+            }
+            wave_order();
+        }
     }
-    wave_order();
-    if (gl < nl - 1) {
-        BinNode nd;
+    const float my_area = box_area(b);
+    const float area_p = __shfl(my_area, (gl + 1) & (G - 1), G), area_q = __shfl(my_area, (gl + (int)np) & (G - 1), G);
+    if (mine) {
         uint32_t count = 0;
 #pragma unroll
         for (int k = 0; k < kTreeletLeaves; ++k)
-            if ((mine >> k) & 1u) count += sc->lcount[k];
-        const uint32_t c0 = (mine >> 12) & 0xfu, c1 = (mine >> 16) & 0xfu;
-        nd.left = c0 < 8u ? sc->lref[c0] : sc->inner[c0 - 8u];
-        nd.area_l = c0 < 8u ? sc->larea[c0] : sc->narea[(jof >> (4 * (c0 - 8u))) & 0xfu];
-        nd.right = c1 < 8u ? sc->lref[c1] : sc->inner[c1 - 8u];
-        nd.area_r = c1 < 8u ? sc->larea[c1] : sc->narea[(jof >> (4 * (c1 - 8u))) & 0xfu];
-        S.put(sc->inner[(mine >> 8) & 0xfu], nd, b, count);
+            if ((set >> k) & 1u) count += sc->lcount[k];
+        const float4 l0 = sc->leaf[c0 & 7u][1], l1 = sc->leaf[c1 & 7u][1];
+        BinNode out;
+        out.left = c0 < 8u ? __float_as_uint(l0.w) : sc->inner[c0 - 8u];
+        out.area_l = c0 < 8u ? l0.z : area_p;
+        out.right = c1 < 8u ? __float_as_uint(l1.w) : sc->inner[c1 - 8u];
+        out.area_r = c1 < 8u ? l1.z : area_q;
+        S.put(sc->inner[id], out, b, count);
     }
     wave_order();
 }
@@ -446,20 +549,24 @@ struct LdsTree {
     }
 };
 
-constexpr int kBottomThreads = 256;
 
 // OPT: treelets, `rounds` passes over the same subtree (more than one only
 // where the subtree is the whole tree: between passes the nodes above a
 // subtree move its nodes); otherwise boxes only.
-template <bool OPT>
-__global__ __launch_bounds__(kBottomThreads) void k_tree_bottom(BinNode* bin, Box* ibox, uint32_t* rcount,
+// THREADS: see launch_pass.
+template <bool OPT, int THREADS>
+__global__ __launch_bounds__(THREADS, 4) void k_tree_bottom(BinNode* bin, Box* ibox, uint32_t* rcount,
                                                                 const Box* lbox, const uint32_t* roots,
                                                                 const uint32_t* nroots, int rounds) {
     __shared__ LdsTree T;
-    __shared__ TreeletScratch s_sc[OPT ? kBottomThreads / 16 : 1];
-    __shared__ uint8_t s_sets[OPT ? kTreeletSets : 1];
+    __shared__ TreeletScratch s_sc[OPT ? THREADS / 16 : 1];
     const uint32_t t = threadIdx.x;
-    if (OPT && t < kTreeletSets) s_sets[t] = kTreeletSetTable.s[t];
+    TreeletLane<64> lane64;
+    TreeletLane<16> lane16;
+    if (OPT) {
+        lane64.init();
+        lane16.init();
+    }
     const uint32_t nr = *nroots;
     for (uint32_t k = blockIdx.x; k < nr; k += gridDim.x) {
         const uint32_t root = roots[k];
@@ -484,7 +591,7 @@ __global__ __launch_bounds__(kBottomThreads) void k_tree_bottom(BinNode* bin, Bo
                 const uint32_t e = T.nfront;
                 __syncthreads();
                 if (b >= e) break;
-                for (uint32_t q = b + t; q < e; q += kBottomThreads) {
+                for (uint32_t q = b + t; q < e; q += THREADS) {
                     const uint32_t g = T.gid[q];
                     BinNode nd = bin[g];
                     T.cnt[q] = (uint16_t)rcount[g];
@@ -517,7 +624,7 @@ __global__ __launch_bounds__(kBottomThreads) void k_tree_bottom(BinNode* bin, Bo
             }
             const uint32_t nfront = min(T.nfront, kTierLow), nback = min(T.nback, kTierLow);
             // the two leaves of each back node
-            for (uint32_t q = t; q < nback; q += kBottomThreads) {
+            for (uint32_t q = t; q < nback; q += THREADS) {
                 const uint32_t i = kTierLow - 1 - q;
                 BinNode nd = bin[T.gid[i]];
                 const uint32_t l = atomicAdd(&T.nleaf, 2u);
@@ -535,7 +642,7 @@ __global__ __launch_bounds__(kBottomThreads) void k_tree_bottom(BinNode* bin, Bo
                 T.cnt[i] = 2;
             }
             // the leaves of the front nodes
-            for (uint32_t q = t; q < nfront; q += kBottomThreads) {
+            for (uint32_t q = t; q < nfront; q += THREADS) {
                 const BinNode nd = T.rec_[q];
                 if (nd.left & kLeafBit) T.leaf_[nd.left & 0xffu] = lbox[T.leaf_pos[nd.left & 0xffu]];
                 if (nd.right & kLeafBit) T.leaf_[nd.right & 0xffu] = lbox[T.leaf_pos[nd.right & 0xffu]];
@@ -544,7 +651,7 @@ __global__ __launch_bounds__(kBottomThreads) void k_tree_bottom(BinNode* bin, Bo
             for (uint32_t lev = L; lev-- > 0;) {
                 const uint32_t lb = T.lv[lev], le = T.lv[lev + 1];
                 if (!OPT) {
-                    for (uint32_t q = lb + t; q < le; q += kBottomThreads) {
+                    for (uint32_t q = lb + t; q < le; q += THREADS) {
                         BinNode nd = T.rec_[q];
                         const Box x = T.box(nd.left), y = T.box(nd.right);
                         T.box_[q] = box_union(x, y);
@@ -552,17 +659,17 @@ __global__ __launch_bounds__(kBottomThreads) void k_tree_bottom(BinNode* bin, Bo
                         nd.area_r = box_area(y);
                         T.rec_[q] = nd;
                     }
-                } else if (le - lb <= kBottomThreads / 64) {
+                } else if (le - lb <= THREADS / 64) {
                     const uint32_t w = t >> 6;
-                    if (lb + w < le) treelet_group<64>(T, lb + w, &s_sc[w], s_sets);
+                    if (lb + w < le) treelet_group<64>(T, lb + w, &s_sc[w], lane64);
                 } else {
-                    for (uint32_t q = lb + (t >> 4); q < le; q += kBottomThreads / 16)
-                        treelet_group<16>(T, q, &s_sc[t >> 4], s_sets);
+                    for (uint32_t q = lb + (t >> 4); q < le; q += THREADS / 16)
+                        treelet_group<16>(T, q, &s_sc[t >> 4], lane16);
                 }
                 __syncthreads();
             }
             // back to the tree under its own numbers
-            for (uint32_t q = t; q < nfront + nback; q += kBottomThreads) {
+            for (uint32_t q = t; q < nfront + nback; q += THREADS) {
                 const uint32_t i = q < nfront ? q : kTierLow - 1 - (q - nfront);
                 BinNode nd = T.rec_[i];
                 nd.left = (nd.left & kLeafBit) ? (kLeafBit | T.leaf_pos[nd.left & 0xffu]) : T.gid[nd.left];
@@ -608,10 +715,14 @@ __global__ __launch_bounds__(kUpperThreads) void k_tree_upper(GlobalTree T, cons
                                                               uint32_t* list_all, uint32_t* levels_all,
                                                               uint32_t* bump) {
     __shared__ TreeletScratch s_sc[OPT ? kUpperThreads / 16 : 1];
-    __shared__ uint8_t s_sets[OPT ? kTreeletSets : 1];
     __shared__ uint32_t s_count, s_base;
     const uint32_t t = threadIdx.x;
-    if (OPT && t < kTreeletSets) s_sets[t] = kTreeletSetTable.s[t];
+    TreeletLane<64> lane64;
+    TreeletLane<16> lane16;
+    if (OPT) {
+        lane64.init();
+        lane16.init();
+    }
     const uint32_t nr = *nroots;
     for (uint32_t k = blockIdx.x; k < nr; k += gridDim.x) {
         const uint32_t root = roots[k];
@@ -665,10 +776,10 @@ __global__ __launch_bounds__(kUpperThreads) void k_tree_upper(GlobalTree T, cons
                 }
             } else if (le - lb <= kUpperThreads / 64) {
                 const uint32_t w = t >> 6;
-                if (lb + w < le) treelet_group<64>(T, list[lb + w], &s_sc[w], s_sets);
+                if (lb + w < le) treelet_group<64>(T, list[lb + w], &s_sc[w], lane64);
             } else {
                 for (uint32_t q = lb + (t >> 4); q < le; q += kUpperThreads / 16)
-                    treelet_group<16>(T, list[q], &s_sc[t >> 4], s_sets);
+                    treelet_group<16>(T, list[q], &s_sc[t >> 4], lane16);
             }
             __syncthreads();
         }

@@ -314,24 +314,33 @@ __global__ __launch_bounds__(256) void k_morton(const Box* boxes, uint32_t n, co
 }
 
 // ---------------------------------------------------------------------------
-// Stable LSD radix sort, 8-bit digits, tiles of 256 threads x 16 keys.
+// Stable LSD radix sort, 8-bit digits, tiles of 256 threads x 8 keys.
 // ---------------------------------------------------------------------------
 constexpr int kRsThreads = 256;
-constexpr int kRsItems = 16;
+constexpr int kRsItems = 8;
 constexpr int kRsTile = kRsThreads * kRsItems;
+// Up to this many tiles (262,144 keys) a scatter workgroup sums the tiles'
+// counts itself; beyond, a kernel between the two scans them. A build of
+// 130,000 triangles without treelets takes 503 us summing itself and 506 with
+// the scan, of 500,000 triangles 674 and 625.
+constexpr uint32_t kRsSelfTiles = 128;
 
+// SELF: the counts tile by tile, else digit by digit.
+template <bool SELF>
 __global__ __launch_bounds__(kRsThreads) void k_rs_hist(const uint32_t* keys, uint32_t n, int shift, uint32_t* hist,
-                                                        uint32_t ntiles) {
+                                                         uint32_t ntiles) {
     __shared__ uint32_t h[256];
     h[threadIdx.x] = 0;
     __syncthreads();
-    uint32_t base = blockIdx.x * kRsTile;
-    for (int r = 0; r < kRsItems; ++r) {
-        uint32_t i = base + r * kRsThreads + threadIdx.x;
-        if (i < n) atomicAdd(&h[(keys[i] >> shift) & 0xffu], 1u);
-    }
+    const uint32_t base = blockIdx.x * kRsTile + threadIdx.x;
+    uint32_t key[kRsItems];
+#pragma unroll
+    for (int r = 0; r < kRsItems; ++r) key[r] = base + r * kRsThreads < n ? keys[base + r * kRsThreads] : 0u;
+#pragma unroll
+    for (int r = 0; r < kRsItems; ++r)
+        if (base + r * kRsThreads < n) atomicAdd(&h[(key[r] >> shift) & 0xffu], 1u);
     __syncthreads();
-    hist[(size_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
+    hist[SELF ? (size_t)blockIdx.x * 256 + threadIdx.x : (size_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
 }
 
 // Exclusive scan of each digit's counts over the tiles (one workgroup per
@@ -351,64 +360,80 @@ __global__ __launch_bounds__(256) void k_rs_scan(uint32_t* hist, uint32_t ntiles
     if (threadIdx.x == 0) totals[blockIdx.x] = run;
 }
 
+// A tile's keys to their places. Each wave ranks a run of kRsItems * 64
+// consecutive keys against its own counts, 64 at a time, with no barrier in
+// between and all of its keys loaded ahead; then the waves' counts become
+// first places: 8.3 us a pass over 81,920 keys, bound by the chain of the
+// eight ranks, where three barriers and a load per 256 keys and tiles of 4,096
+// took 16.8 (a build of 82,000 triangles without treelets 538 -> 467 us).
+template <bool SELF>
 __global__ __launch_bounds__(kRsThreads) void k_rs_scatter(const uint32_t* kin, const uint32_t* vin, uint32_t* kout,
-                                                           uint32_t* vout, uint32_t n, int shift,
-                                                           const uint32_t* offsets, uint32_t ntiles,
-                                                           const uint32_t* totals) {
+                                                            uint32_t* vout, uint32_t n, int shift,
+                                                            const uint32_t* hist, uint32_t ntiles,
+                                                            const uint32_t* totals) {
     constexpr int kWaves = kRsThreads / 64;
     static_assert(kRsThreads == 256, "a thread per digit");
     __shared__ uint32_t part[kWaves];
-    __shared__ uint32_t base_off[256];
-    __shared__ uint32_t running[256];
     __shared__ uint32_t wave_cnt[kWaves][256];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    {
-        // first position of each digit: the totals of the digits below it
-        const uint32_t mine = totals[threadIdx.x];
-        uint32_t all;
-        base_off[threadIdx.x] =
-            block_scan<256>(mine, part, all) - mine + offsets[(size_t)threadIdx.x * ntiles + blockIdx.x];
+    const uint32_t first = blockIdx.x * kRsTile + w * (64 * kRsItems) + lane;
+    uint32_t key[kRsItems], val[kRsItems], rank[kRsItems];
+#pragma unroll
+    for (int r = 0; r < kRsItems; ++r) {
+        const bool valid = first + r * 64 < n;
+        key[r] = valid ? kin[first + r * 64] : 0u;
+        val[r] = valid ? vin[first + r * 64] : 0u;
     }
-    running[threadIdx.x] = 0;
+    // first position of each digit in the tile: the totals of the digits
+    // below it and its counts in the tiles before
+    uint32_t place = 0, mine = 0;
+    if (SELF) {
+#pragma unroll 8
+        for (uint32_t t = 0; t < ntiles; ++t) {
+            const uint32_t c = hist[(size_t)t * 256 + threadIdx.x];
+            mine += c;
+            place += t < blockIdx.x ? c : 0u;
+        }
+    } else {
+        mine = totals[threadIdx.x];
+        place = hist[(size_t)threadIdx.x * ntiles + blockIdx.x];
+    }
+    uint32_t all;
+    place += block_scan<256>(mine, part, all) - mine;
     for (int k = 0; k < kWaves; ++k) wave_cnt[k][threadIdx.x] = 0;
     __syncthreads();
     const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    uint32_t tile = blockIdx.x * kRsTile;
+#pragma unroll
     for (int r = 0; r < kRsItems; ++r) {
-        uint32_t i = tile + r * kRsThreads + threadIdx.x;
-        bool valid = i < n;
-        uint32_t key = valid ? kin[i] : 0u;
-        uint32_t val = valid ? vin[i] : 0u;
-        uint32_t digit = (key >> shift) & 0xffu;
+        const bool valid = first + r * 64 < n;
+        const uint32_t digit = (key[r] >> shift) & 0xffu;
         // lanes of this wave holding the same digit
         uint64_t peers = __ballot(valid);
 #pragma unroll
         for (int bit = 0; bit < 8; ++bit) {
-            uint64_t bal = __ballot((digit >> bit) & 1u);
+            const uint64_t bal = __ballot((digit >> bit) & 1u);
             peers &= ((digit >> bit) & 1u) ? bal : ~bal;
         }
-        uint32_t rank_in_wave = (uint32_t)__popcll(peers & lt_mask);
-        bool leader = valid && (peers & lt_mask) == 0;
-        if (leader) wave_cnt[w][digit] = (uint32_t)__popcll(peers);
-        __syncthreads();
-        if (valid) {
-            uint32_t off = running[digit] + rank_in_wave;
-            for (int k = 0; k < w; ++k) off += wave_cnt[k][digit];
-            uint32_t dst = base_off[digit] + off;
-            kout[dst] = key;
-            vout[dst] = val;
+        const uint32_t before = wave_cnt[w][digit];
+        rank[r] = before + (uint32_t)__popcll(peers & lt_mask);
+        wave_order();
+        if (valid && (peers & lt_mask) == 0) wave_cnt[w][digit] = before + (uint32_t)__popcll(peers);
+        wave_order();
+    }
+    __syncthreads();
+    for (int k = 0; k < kWaves; ++k) {
+        const uint32_t c = wave_cnt[k][threadIdx.x];
+        wave_cnt[k][threadIdx.x] = place;
+        place += c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kRsItems; ++r) {
+        if (first + r * 64 < n) {
+            const uint32_t dst = wave_cnt[w][(key[r] >> shift) & 0xffu] + rank[r];
+            kout[dst] = key[r];
+            vout[dst] = val[r];
         }
-        __syncthreads();
-        {
-            uint32_t d = threadIdx.x;
-            uint32_t s = 0;
-            for (int k = 0; k < kWaves; ++k) {
-                s += wave_cnt[k][d];
-                wave_cnt[k][d] = 0;
-            }
-            running[d] += s;
-        }
-        __syncthreads();
     }
 }
 
@@ -1078,10 +1103,12 @@ static void radix_tree(const BuildBufs& b, uint32_t n, hipStream_t s) {
     uint32_t *kin = b.ka, *kout = b.kb, *vin = b.va, *vout = b.vb;
     for (int pass = 0; pass < 4; ++pass) {
         int shift = pass * 8;
-        hipLaunchKernelGGL(k_rs_hist, dim3(ntiles), dim3(kRsThreads), 0, s, kin, n, shift, b.hist, ntiles);
-        hipLaunchKernelGGL(k_rs_scan, dim3(256), dim3(256), 0, s, b.hist, ntiles, b.totals);
-        hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles), dim3(kRsThreads), 0, s, kin, vin, kout, vout, n, shift, b.hist,
-                           ntiles, b.totals);
+        const bool self = ntiles <= kRsSelfTiles;
+        hipLaunchKernelGGL((self ? k_rs_hist<true> : k_rs_hist<false>), dim3(ntiles), dim3(kRsThreads), 0, s, kin, n,
+                           shift, b.hist, ntiles);
+        if (!self) hipLaunchKernelGGL(k_rs_scan, dim3(256), dim3(256), 0, s, b.hist, ntiles, b.totals);
+        hipLaunchKernelGGL((self ? k_rs_scatter<true> : k_rs_scatter<false>), dim3(ntiles), dim3(kRsThreads), 0, s, kin,
+                           vin, kout, vout, n, shift, b.hist, ntiles, b.totals);
         std::swap(kin, kout);
         std::swap(vin, vout);
     }

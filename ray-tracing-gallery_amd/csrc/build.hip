@@ -974,6 +974,8 @@ struct BuildBufs {
     size_t bytes;
 };
 
+// Words of a row of a collapse's turn counts (k_wide_level).
+static uint32_t sums_stride(uint32_t cap) { return cap / kWideTurn + 8; }
 constexpr uint32_t kCollapseSteps = 12;  // levels launched between two looks at the collapse's progress
 
 static BuildBufs carve_build(void* base, uint32_t n, size_t rec_bytes, uint32_t ngeom) {
@@ -1003,7 +1005,7 @@ static BuildBufs carve_build(void* base, uint32_t n, size_t rec_bytes, uint32_t 
     b.wroot = c.take<uint32_t>(cap);
     b.slots = c.take<uint4>(cap);
     b.off = c.take<uint32_t>((size_t)cap + kCollapseSteps + 8);
-    b.sums = c.take<uint32_t>(kWideBlocks);
+    b.sums = c.take<uint32_t>((size_t)3 * sums_stride(cap));
     b.state = c.take<CollapseState>(1);
     b.bytes = c.off + 4096;
     return b;
@@ -1062,15 +1064,15 @@ static int wide_hierarchy(rtg_ctx* ctx, const BuildBufs& b, uint32_t n, int tree
     // one workgroup emits 1,024 nodes of a level in about 4 us; beyond a few
     // thousand the two launches over many workgroups are the faster way
     const bool one = n <= kSmallBuild;
+    const unsigned wide_grid = std::min(n / 1024 + 1, kWideBlocks);
     hipLaunchKernelGGL(k_collapse_top, dim3(1), dim3(kCollapseThreads), 0, s, W, one ? n : 2048u, b.off, b.state);
     do {
         if (!one) {
-            for (uint32_t k = 0; k < kCollapseSteps; ++k) {
-                hipLaunchKernelGGL(k_wide_expand, dim3(kWideBlocks), dim3(256), 0, s, W, b.off, b.state, k, b.slots,
-                                   b.sums);
-                hipLaunchKernelGGL(k_wide_emit, dim3(kWideBlocks), dim3(256), 0, s, W, b.off, b.state, k, b.slots,
-                                   b.sums);
-            }
+            hipLaunchKernelGGL(k_wide_expand, dim3(wide_grid), dim3(kWideTurn), 0, s, W, b.off, b.state, b.slots,
+                               b.sums, sums_stride(W.cap));
+            for (uint32_t k = 0; k < kCollapseSteps; ++k)
+                hipLaunchKernelGGL(k_wide_level, dim3(wide_grid), dim3(kWideTurn), 0, s, W, b.off, b.state, k, b.slots,
+                                   b.sums, sums_stride(W.cap));
             hipLaunchKernelGGL(k_collapse_advance, dim3(1), dim3(64), 0, s, b.off, b.state, kCollapseSteps);
         }
         hipLaunchKernelGGL(k_build_report, dim3(1), dim3(64), 0, s, b.state, b.off, ctx->d_status, b.cb + 6,

@@ -26,7 +26,8 @@ constexpr int kCountSlots = 16;
 // queues of the feed counters (Frame::feeds): the trace levels, then
 constexpr int kFeedShadow = 4;      // the shadow queue
 constexpr int kFeedShadowRest = 5;  // the shadow rays after those of trace level 0
-constexpr int kShadowFirst = 5;      // counts[5]: shadow rays of trace level 0
+constexpr int kShadowFirst = 4;      // counts[4]: shadow-queue slots of trace level 0, the queue's first
+constexpr int kShadowRest = 5;       // counts[5]: those of the bounce levels, which follow them
 constexpr int kStatusSlot = 14;      // counts[14]: status bits of the trace (merged into the context's)
 constexpr int kPartAll = 0, kPartFirst = 1, kPartRest = 2;  // parts of the shadow queue
 // intervals of the camera, continuation and shadow rays (lib.rs:146-149,
@@ -343,23 +344,6 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_rays_quad(const uint8_t
 // ---------------------------------------------------------------------------
 // Wavefront pipeline
 // ---------------------------------------------------------------------------
-__global__ void k_frame_begin(uint32_t* counts, uint32_t* feeds, uint64_t* counters, bool reset_counters) {
-    if (threadIdx.x < kCountSlots) counts[threadIdx.x] = 0;
-    feeds[threadIdx.x] = 0;
-    if (reset_counters && threadIdx.x < kCounterSlots) counters[threadIdx.x] = 0;
-}
-
-// ORs a trace's status bits into the context's sticky ones; `done`, if not
-// null, is the host word that says which trace of its arena has ended.
-__global__ void k_status_merge(const uint32_t* trace_status, uint32_t* ctx_status, uint32_t* done, uint32_t seq) {
-    if (threadIdx.x == 0 && *trace_status) atomicOr(ctx_status, *trace_status);
-    if (threadIdx.x == 0 && done) __hip_atomic_store(done, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-__global__ void k_shadow_snapshot(uint32_t* counts) {
-    if (threadIdx.x == 0) counts[kShadowFirst] = counts[4];
-}
-
 __global__ void k_zero_feed(uint32_t* feed, uint32_t stride) {
     if (threadIdx.x < kFeedGroups) feed[threadIdx.x * stride] = 0;
 }
@@ -374,8 +358,15 @@ __global__ void k_reset_counters(uint64_t* counters, uint64_t primary) {
 // Writes the direction alone (16 bytes a path): the origin is the job's, the
 // path the ray's number, and the shading of level 0 writes every path's
 // state. With the whole ray and cleared state, 72 bytes, the launch took
-// 100 us on average over a set of served requests, now 56.
+// 100 us on average over a set of served requests, now 56. Its first
+// workgroup also clears the queue counts, the status word and the feed
+// counters, which the frame's later kernels use.
+static_assert(kFeedWords == 256 && kCountSlots <= 256, "a thread per word");
 __global__ __launch_bounds__(256) void k_raygen(Frame F, bool count) {
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < kCountSlots) F.counts[threadIdx.x] = 0;
+        F.feeds[threadIdx.x] = 0;
+    }
     uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t p = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; p < F.paths; p += stride) {
         uint32_t j = find_job(F.jobs, F.njobs, p, false);
@@ -860,7 +851,9 @@ __global__ __launch_bounds__(256) void k_shade(Frame F, int level, const uint32_
         // count) so that the occlusion kernel's pairs never span two paths
         const uint32_t shadow_slots = want_shadow + (want_shadow & 1u);
         uint32_t sbase, nbase;
-        block_alloc<ONE>(s_alloc, shadow_slots, &F.counts[4], want_next, next_count, sbase, nbase);
+        block_alloc<ONE>(s_alloc, shadow_slots, &F.counts[level == 0 ? kShadowFirst : kShadowRest], want_next,
+                         next_count, sbase, nbase);
+        if (level > 0) sbase += F.counts[kShadowFirst];
         if (want_next && nbase >= F.path_cap) {
             queue_range_error(F);
             want_next = false;
@@ -930,11 +923,12 @@ __global__ __launch_bounds__(256) void k_shade(Frame F, int level, const uint32_
 }
 
 // Parts of the shadow queue an occlusion launch traces: all of it, or the
-// rays of the first trace level (counts[kShadowFirst] of them, the queue's
-// size when the first shade finished) and the rays appended after them.
+// rays of the first trace level (counts[kShadowFirst] slots, final once the
+// first shade has finished) and those of the bounce levels after them.
 __device__ inline void shadow_part(const Frame& F, int part, uint32_t& lo, uint32_t& hi, uint32_t*& feed) {
-    hi = min(part == kPartFirst ? F.counts[kShadowFirst] : F.counts[4], F.shadow_cap);
-    lo = min(part == kPartRest ? F.counts[kShadowFirst] : 0u, hi);
+    const uint32_t first = min(F.counts[kShadowFirst], F.shadow_cap);
+    hi = part == kPartFirst ? first : min(first + F.counts[kShadowRest], F.shadow_cap);
+    lo = part == kPartRest ? first : 0u;
     feed = F.feeds + (part == kPartRest ? kFeedShadowRest : kFeedShadow);
 }
 
@@ -1182,7 +1176,11 @@ __device__ inline V3 heatmap_temperature(float heat) {
     return v3(o[0], o[1], o[2]);
 }
 
-__global__ __launch_bounds__(256) void k_resolve(Frame F, uint64_t total_pixels) {
+// The trace's last kernel: it also ORs the trace's status bits into the
+// context's sticky ones; `done`, if not null, is the host word that says which
+// trace of its arena has ended.
+__global__ __launch_bounds__(256) void k_resolve(Frame F, uint64_t total_pixels, uint32_t* ctx_status, uint32_t* done,
+                                                 uint32_t seq) {
     uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t q = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; q < total_pixels; q += stride) {
         // lanes take pixels in path order, so that they read consecutive
@@ -1234,6 +1232,10 @@ __global__ __launch_bounds__(256) void k_resolve(Frame F, uint64_t total_pixels)
             }
             J.out_rgba8[pix] = r | (g << 8) | (b << 16) | (255u << 24);
         }
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (*F.status) atomicOr(ctx_status, *F.status);
+        if (done) __hip_atomic_store(done, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -1556,7 +1558,7 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
     F.quad_max = (uint32_t)quad_capacity(G);
     const size_t lds = stack_lds_bytes(tune.stack_lds);  // a traversal workgroup's stacks
     const unsigned Gsmall = (unsigned)std::min<uint64_t>((P.paths + 255) / 256, (uint64_t)ctx->cu_count * 16);
-    hipLaunchKernelGGL(k_frame_begin, dim3(1), dim3(kFeedWords), 0, s, a->d_counts, a->d_feeds, ctx->d_counters, cnt);
+    if (cnt) hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, ctx->d_counters, (uint64_t)0);
     {
         LaunchTimer t(ctx, RTG_KERNEL_RAYGEN, s, timed);
         hipLaunchKernelGGL(k_raygen, dim3(Gsmall), dim3(256), 0, s, F, cnt);
@@ -1645,7 +1647,6 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
                                             (size_t)Gmain * kTraceThreads * kSpillLaneBytes);
         Fs.side = 1;
         Fs.main_lanes = Gmain * kTraceThreads;
-        hipLaunchKernelGGL(k_shadow_snapshot, dim3(1), dim3(64), 0, s, a->d_counts);
         hipEventRecord(a->fork, s);
         hipStreamWaitEvent(a->side, a->fork, 0);
         {
@@ -1669,11 +1670,6 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
         for (uint32_t level = 1; level < P.max_traces; ++level) level_step(F, level, G, Gsmall, s, timed);
         occlusion(F, kPartAll, G, s, timed);
     }
-    {
-        LaunchTimer t(ctx, RTG_KERNEL_RESOLVE, s, timed);
-        unsigned Gr = (unsigned)std::min<uint64_t>((P.pixels + 255) / 256, (uint64_t)ctx->cu_count * 16);
-        hipLaunchKernelGGL(k_resolve, dim3(Gr), dim3(256), 0, s, F, P.pixels);
-    }
     uint32_t* done = nullptr;
     uint32_t seq = 0;
     if (flight) {
@@ -1681,7 +1677,11 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
         done = ctx->flight_done + a->flight;
         seq = ctx->flight_started[a->flight].fetch_add(1) + 1;
     }
-    hipLaunchKernelGGL(k_status_merge, dim3(1), dim3(64), 0, s, F.status, ctx->d_status, done, seq);
+    {
+        LaunchTimer t(ctx, RTG_KERNEL_RESOLVE, s, timed);
+        unsigned Gr = (unsigned)std::min<uint64_t>((P.pixels + 255) / 256, (uint64_t)ctx->cu_count * 16);
+        hipLaunchKernelGGL(k_resolve, dim3(Gr), dim3(256), 0, s, F, P.pixels, ctx->d_status, done, seq);
+    }
 }
 
 // Marks an arena as used by this host call for its duration.

@@ -473,7 +473,7 @@ typedef struct rtg_tuning {
                                   0 = non-persistent kernel (grid-stride rounds) */
     uint32_t refill_occlusion; /* the same for occlusion rays */
     uint32_t path_order;       /* 0 = row-major paths, 1 = 8x8 pixel blocks per wavefront */
-    uint32_t bounce_blocks;    /* persistent workgroups (0..4096) of a second stream that traces the
+    uint32_t bounce_blocks;    /* persistent workgroups (0..4096) of a stream (the bounce stream) that traces the
                                   bounce levels (on at most 192 of them) and the shadow rays they add
                                   (on all) beside the first level's shadow rays (taken from the
                                   blocks_per_cu grid, at most half of it); 192 by default;

@@ -1637,21 +1637,28 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
     if (P.max_traces > 1 && Gside > 0) {
         // The bounce levels hold few rays, so their launches are short of
         // work and bound by the latency of their longest rays. They run on
-        // the side stream, on Gside persistent blocks, while the first
-        // level's shadow rays take the other blocks; the shadow rays the
-        // bounce levels add are traced on the side stream after them. The
-        // two grids use disjoint spill areas.
+        // Gside persistent blocks, while on another stream the first level's
+        // shadow rays take the other blocks; the shadow rays the bounce
+        // levels add are traced after them. The two grids use disjoint spill
+        // areas.
         const unsigned Gmain = G - Gside;
         Frame Fs = F;
         Fs.spill = reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(F.spill) +
                                             (size_t)Gmain * kTraceThreads * kSpillLaneBytes);
         Fs.side = 1;
         Fs.main_lanes = Gmain * kTraceThreads;
+        // A wait for another stream's event holds a chain up for about 16 us.
+        // The bounce levels' chain is the longer one in small frames, so it
+        // stays on the caller's stream and the first level's shadow rays go
+        // to the side stream (a 320x180 frame 333 -> 321 us, 1280x720 679 ->
+        // 671). In a captured graph the other way round is the faster one (a
+        // batch of one scene 3,160 us, 3,236 swapped).
+        hipStream_t bounces = flight ? s : a->side, firsts = flight ? a->side : s;
         hipEventRecord(a->fork, s);
         hipStreamWaitEvent(a->side, a->fork, 0);
         {
             // timed as one span: its kernels share the GPU with the shadow rays
-            LaunchTimer t(ctx, RTG_KERNEL_BOUNCE_SIDE, a->side, timed);
+            LaunchTimer t(ctx, RTG_KERNEL_BOUNCE_SIDE, bounces, timed);
             // The bounce levels' traversal and shading launches take at most
             // 192 workgroups (12 k rays at once with four lanes each; a 1080p
             // frame has about 46 k and 3 k bounce rays): a launch ends only
@@ -1660,11 +1667,11 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
             // the CUs (two 1080p frames: 4.58 ms, with 128 workgroups 4.73).
             const unsigned Gbounce = std::min(Gside, 192u);
             for (uint32_t level = 1; level < P.max_traces; ++level)
-                level_step(Fs, level, Gbounce, std::min(Gsmall, Gbounce), a->side, false);
-            occlusion(Fs, kPartRest, Gside, a->side, false);
+                level_step(Fs, level, Gbounce, std::min(Gsmall, Gbounce), bounces, false);
+            occlusion(Fs, kPartRest, Gside, bounces, false);
         }
+        occlusion(F, kPartFirst, Gmain, firsts, timed);
         hipEventRecord(a->join, a->side);
-        occlusion(F, kPartFirst, Gmain, s, timed);
         hipStreamWaitEvent(s, a->join, 0);
     } else {
         for (uint32_t level = 1; level < P.max_traces; ++level) level_step(F, level, G, Gsmall, s, timed);

@@ -478,8 +478,10 @@ typedef struct rtg_tuning {
                                   (on all) beside the first level's shadow rays (taken from the
                                   blocks_per_cu grid, at most half of it); 192 by default;
                                   0 = every level in sequence on the caller's stream, as is an
-                                  uncounted trace enqueued while another of the context is in
-                                  flight (on another stream, frame slot or server slot) */
+                                  uncounted trace enqueued while others of the context are in
+                                  flight (on other streams, frame slots or server slots) and
+                                  GPU_MAX_HW_QUEUES, as rtg_create found it (4 if unset), is too
+                                  small for two queues each and one more */
     uint32_t stack_lds_entries; /* traversal stack entries per lane kept in LDS (8..32, multiple of 4;
                                   0 = 16): a workgroup takes entries * 2 KB of LDS, deeper entries
                                   spill to global memory; the occlusion queries of rtg_trace_rays

@@ -157,6 +157,7 @@ struct rtg_ctx {
     std::atomic<uint32_t> flight_started[rtg::kFlightSlots] = {};
     std::atomic<uint32_t> flight_next{0};
     uint32_t* flight_done = nullptr;
+    int hw_queues = 4;  // GPU_MAX_HW_QUEUES, HIP's hardware queues per process
     rtg::Tuning tune;
 };
 

@@ -1523,15 +1523,15 @@ int upload_jobs(FrameArena* a, const TracePlan& P, hipStream_t s) {
     return RTG_OK;
 }
 
-// Whether a trace of another arena than `a` is on the GPU, as far as the host
+// How many other arenas than `a` have a trace on the GPU, as far as the host
 // words tell (a moment's view, which changes launch shapes only).
-static bool others_in_flight(rtg_ctx* ctx, const FrameArena* a) {
+static int others_in_flight(rtg_ctx* ctx, const FrameArena* a) {
+    int n = 0;
     for (int k = 0; k < kFlightSlots; ++k)
-        if (k != a->flight &&
-            ctx->flight_started[k].load(std::memory_order_relaxed) !=
-                __atomic_load_n(&ctx->flight_done[k], __ATOMIC_RELAXED))
-            return true;
-    return false;
+        if (k != a->flight && ctx->flight_started[k].load(std::memory_order_relaxed) !=
+                                  __atomic_load_n(&ctx->flight_done[k], __ATOMIC_RELAXED))
+            ++n;
+    return n;
 }
 
 void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning& tune, bool cnt, bool timed,
@@ -1586,8 +1586,7 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
                               : !cnt && level > 0
                                   ? (side ? (single ? k_trace_closest_any<true, true> : k_trace_closest_any<true, false>)
                                           : (single ? k_trace_closest_any<false, true> : k_trace_closest_any<false, false>))
-                              : side ? (cnt ? (single ? k_trace_closest_one<true, true> : k_trace_closest<true, true>)
-                                          : (single ? k_trace_closest_one<false, true> : k_trace_closest<false, true>))
+                              : side ? (single ? k_trace_closest_one<true, true> : k_trace_closest<true, true>)
                                    : (cnt ? (single ? k_trace_closest_one<true, false> : k_trace_closest<true, false>)
                                           : (single ? k_trace_closest_one<false, false> : k_trace_closest<false, false>));
                 hipLaunchKernelGGL(kernel, dim3(g), dim3(kTraceThreads), lds, st, Fl, (int)level, cp, fixed, Fl.status);
@@ -1625,14 +1624,19 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
         }
     };
     level_step(F, 0, G, Gsmall, s, timed);
-    // With another trace in flight the bounce levels leave no gap to fill,
-    // and a second stream costs: streams share the process's four hardware
-    // queues, where its waits hold up the other traces' kernels. Two frames
-    // in flight, levels in sequence against side by side: 4,157 us to 4,226
-    // at 1920x1080, 1,680 to 2,170 at 960x540, 1,004 to 1,500 at 480x270. A
-    // frame alone is the faster side by side: 410 us to 505 at 480x270, 681
-    // to 775 at 1280x720. Counted traces keep the setting's split.
-    const bool crowded = flight && !cnt && others_in_flight(ctx, a);
+    // A trace takes two streams to run its bounce levels beside the first
+    // level's shadow rays. HIP maps a process's streams onto few hardware
+    // queues, and where traces in flight share one, its waits hold up another
+    // trace's kernels: levels go in sequence unless every trace in flight can
+    // have two queues beside one for the caller's copies. Two frames in
+    // flight, side by side against in sequence: on four queues (HIP's
+    // default) 1,094 us to 1,015 at 480x270, 2,445 to 1,681 at 960x540 and
+    // 6,908 to 4,164 at 1920x1080, on five to sixteen 803 to 1,011, 1,485 to
+    // 1,650 and 4,067..4,130 to 4,155; six served requests on eight queues
+    // 7,276 to 5,681. A frame alone is the faster side by side (404 us to 505
+    // at 480x270). Counted traces keep the setting's split.
+    const int others = flight && !cnt ? others_in_flight(ctx, a) : 0;
+    const bool crowded = others > 0 && 2 * (others + 1) + 1 > ctx->hw_queues;
     const unsigned Gside = crowded ? 0 : std::min<unsigned>((unsigned)tune.bounce_blocks, G / 2);
     if (P.max_traces > 1 && Gside > 0) {
         // The bounce levels hold few rays, so their launches are short of

@@ -475,17 +475,21 @@ __device__ inline uint32_t radix_node(const uint32_t* keys, int n, int i, uint32
 }
 
 // The radix tree, the leaf boxes in sorted order and the first pass's tiers.
-__global__ __launch_bounds__(256) void k_karras(const uint32_t* keys, int n, const uint32_t* order, const Box* boxes,
-                                                Box* lbox, BinNode* bin, uint32_t* rcount, uint32_t* low,
-                                                uint32_t* mid, uint32_t* counts) {
-    int i = blockIdx.x * 256 + threadIdx.x;
+__global__ __launch_bounds__(kRootThreads) void k_karras(const uint32_t* keys, int n, const uint32_t* order,
+                                                         const Box* boxes, Box* lbox, BinNode* bin, uint32_t* rcount,
+                                                         uint32_t* low, uint32_t* mid, uint32_t* counts) {
+    __shared__ RootList R;
+    R.clear();
+    const int i = blockIdx.x * kRootThreads + threadIdx.x;
     if (i < n) lbox[i] = boxes[order[i]];
-    if (i >= n - 1) return;
-    uint32_t child[2], count[2];
-    const uint32_t c = radix_node(keys, n, i, child, count);
-    bin[i] = BinNode{child[0], child[1], 0.0f, 0.0f};
-    rcount[i] = c;
-    tier_roots((uint32_t)i, c, child, count, low, mid, counts);
+    if (i < n - 1) {
+        uint32_t child[2], count[2];
+        const uint32_t c = radix_node(keys, n, i, child, count);
+        bin[i] = BinNode{child[0], child[1], 0.0f, 0.0f};
+        rcount[i] = c;
+        tier_roots((uint32_t)i, c, child, count, [&](int tier, uint32_t k) { R.add(tier, k); });
+    }
+    R.write(low, mid, counts);
 }
 
 // ---------------------------------------------------------------------------
@@ -644,7 +648,9 @@ __device__ inline void small_tree(SmallSort& Z, uint32_t n, const CentreBounds& 
             const uint32_t c = radix_node(Z.key, (int)n, (int)p, child, count);
             O.bin[p] = BinNode{child[0], child[1], 0.0f, 0.0f};
             O.rcount[p] = c;
-            tier_roots(p, c, child, count, O.low, O.mid, Z.tiers);
+            tier_roots(p, c, child, count, [&](int tier, uint32_t k) {
+                (tier == 0 ? O.low : O.mid)[atomicAdd(&Z.tiers[tier], 1u)] = k;
+            });
         }
     }
     __syncthreads();
@@ -1055,8 +1061,8 @@ static int wide_hierarchy(rtg_ctx* ctx, const BuildBufs& b, uint32_t n, int tree
         for (int round = 0; round < treelet_rounds; ++round) {
             uint32_t* tiers = b.tiers + kTierWords * round;
             if (round > 0)
-                hipLaunchKernelGGL(k_tier_roots, dim3(blocks_for(n - 1, 256)), dim3(256), 0, s, n, b.bin, b.rcount,
-                                   b.low, b.mid, tiers);
+                hipLaunchKernelGGL(k_tier_roots, dim3(blocks_for(n - 1, kRootThreads)), dim3(kRootThreads), 0, s, n, b.bin,
+                                   b.rcount, b.low, b.mid, tiers);
             launch_pass<true>(b, n, tiers, 1, s);
         }
     }
@@ -1115,8 +1121,8 @@ static void radix_tree(const BuildBufs& b, uint32_t n, hipStream_t s) {
         std::swap(vin, vout);
     }
     // after 4 passes the sorted data is back in (ka, va)
-    hipLaunchKernelGGL(k_karras, dim3(blocks_for(n, 256)), dim3(256), 0, s, b.ka, (int)n, b.va, b.boxes, b.lbox, b.bin,
-                       b.rcount, b.low, b.mid, b.tiers);
+    hipLaunchKernelGGL(k_karras, dim3(blocks_for(n, kRootThreads)), dim3(kRootThreads), 0, s, b.ka, (int)n, b.va, b.boxes,
+                       b.lbox, b.bin, b.rcount, b.low, b.mid, b.tiers);
 }
 
 // At most one primitive: the single node.

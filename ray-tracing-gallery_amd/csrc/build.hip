@@ -65,15 +65,35 @@ __device__ inline Box ref_box(const Node* nodes, uint32_t c, const Box* leaf_box
     return node_box(nodes[c]);
 }
 
-// Block-wide reduction of centre bounds, then one atomic per block and axis.
+// Centre bounds of this thread's primitives, folded over the workgroup after.
+struct CentreBounds {
+    uint32_t lo[3], hi[3];
+    __device__ inline CentreBounds() {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            lo[a] = 0xffffffffu;
+            hi[a] = 0u;
+        }
+    }
+    __device__ inline void add(const Box& b) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const float c = centre(b, a);
+            if (!isfinite(c)) continue;
+            lo[a] = min(lo[a], f2ord(c));
+            hi[a] = max(hi[a], f2ord(c));
+        }
+    }
+};
+
+// Block-wide reduction of centre bounds, then one atomic per block and bound.
 template <int BS>
-__device__ inline void reduce_centre_bounds(float c[3], bool valid[3], uint32_t* cb) {
+__device__ inline void reduce_centre_bounds(const CentreBounds& c, uint32_t* cb) {
     __shared__ uint32_t s_lo[3][BS / 64], s_hi[3][BS / 64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        uint32_t lo = valid[a] ? f2ord(c[a]) : 0xffffffffu;
-        uint32_t hi = valid[a] ? f2ord(c[a]) : 0u;
+        uint32_t lo = c.lo[a], hi = c.hi[a];
         for (int off = 32; off > 0; off >>= 1) {
             lo = min(lo, (uint32_t)__shfl_xor((int)lo, off));
             hi = max(hi, (uint32_t)__shfl_xor((int)hi, off));
@@ -95,6 +115,11 @@ __device__ inline void reduce_centre_bounds(float c[3], bool valid[3], uint32_t*
         if (hi != 0u) atomicMax(&cb[3 + a], hi);
     }
 }
+// k_tri_setup's workgroups, and the most of them: their atomics on the six
+// bounds pass one after another (1 M triangles: 99 us with 3,906 workgroups
+// of 256 lanes, 33 with these).
+constexpr int kSetupThreads = 1024;
+constexpr unsigned kSetupBlocks = 512;
 
 struct GeomDesc {
     const uint8_t* vertices;
@@ -173,25 +198,20 @@ __device__ inline bool box_has_nan(const Box& b) {
 }
 
 // Triangle records, primitive boxes, centre bounds.
-__global__ __launch_bounds__(256) void k_tri_setup(const GeomDesc* geoms, uint32_t ngeom, uint32_t ntri, TriRec* tris,
-                                                   Box* boxes, uint32_t* cb, uint32_t* status) {
-    uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    float c[3] = {0, 0, 0};
-    bool valid[3] = {false, false, false};
-    if (i < ntri) {
+__global__ __launch_bounds__(kSetupThreads) void k_tri_setup(const GeomDesc* geoms, uint32_t ngeom, uint32_t ntri,
+                                                             TriRec* tris, Box* boxes, uint32_t* cb,
+                                                             uint32_t* status) {
+    CentreBounds c;
+    for (uint32_t i = blockIdx.x * kSetupThreads + threadIdx.x; i < ntri; i += gridDim.x * kSetupThreads) {
         TriRec r;
         Box b;
         make_tri(geoms, ngeom, i, r, b, status);
         tris[i] = r;
         boxes[i] = b;
         if (box_has_nan(b)) atomicOr(&cb[6], 1u);
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            c[k] = centre(b, k);
-            valid[k] = isfinite(c[k]);
-        }
+        c.add(b);
     }
-    reduce_centre_bounds<256>(c, valid, cb);
+    reduce_centre_bounds<kSetupThreads>(c, cb);
 }
 
 __device__ inline bool registry_has(const uint64_t* reg, uint32_t n, uint64_t a) {
@@ -258,22 +278,17 @@ __device__ inline void make_inst(const rtg_instance* inst, uint32_t i, const uin
 __global__ __launch_bounds__(256) void k_inst_setup(const rtg_instance* inst, uint32_t n, const uint64_t* reg,
                                                     uint32_t nreg, InstRec* recs, Box* boxes, uint32_t* cb,
                                                     uint32_t* status) {
-    uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    float c[3] = {0, 0, 0};
-    bool valid[3] = {false, false, false};
+    CentreBounds c;
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
     if (i < n) {
         InstRec r;
         Box b;
         make_inst(inst, i, reg, nreg, r, b, status);
         recs[i] = r;
         boxes[i] = b;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            c[k] = centre(b, k);
-            valid[k] = isfinite(c[k]);
-        }
+        c.add(b);
     }
-    reduce_centre_bounds<256>(c, valid, cb);
+    reduce_centre_bounds<256>(c, cb);
 }
 
 __device__ inline uint32_t spread3(uint32_t v) {
@@ -518,27 +533,6 @@ struct SmallOut {
     BinNode* bin;
     uint32_t* rcount;
     uint32_t *low, *mid, *counts, *cb;
-};
-
-// Centre bounds of this thread's primitives, folded over the workgroup.
-struct CentreBounds {
-    uint32_t lo[3], hi[3];
-    __device__ inline CentreBounds() {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            lo[a] = 0xffffffffu;
-            hi[a] = 0u;
-        }
-    }
-    __device__ inline void add(const Box& b) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            const float c = centre(b, a);
-            if (!isfinite(c)) continue;
-            lo[a] = min(lo[a], f2ord(c));
-            hi[a] = max(hi[a], f2ord(c));
-        }
-    }
 };
 
 __device__ inline void small_tree(SmallSort& Z, uint32_t n, const CentreBounds& cb, const SmallOut& O) {
@@ -1305,7 +1299,7 @@ extern "C" int rtg_blas_build(rtg_ctx* ctx, const rtg_geometry* geoms, uint32_t 
         hipLaunchKernelGGL(k_small_tris, dim3(1), dim3(kSmallThreads), 0, s, b.geoms, n_geom, n, tris, small_out(b),
                            ctx->d_status);
     } else if (n > 0) {
-        hipLaunchKernelGGL(k_tri_setup, dim3(blocks_for(n, 256)), dim3(256), 0, s, b.geoms, n_geom, n, tris, b.boxes,
+        hipLaunchKernelGGL(k_tri_setup, dim3(std::min(blocks_for(n, kSetupThreads), kSetupBlocks)), dim3(kSetupThreads), 0, s, b.geoms, n_geom, n, tris, b.boxes,
                            b.cb, ctx->d_status);
         if (n > 1) radix_tree(b, n, s);
     }

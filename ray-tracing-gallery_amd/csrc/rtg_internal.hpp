@@ -92,21 +92,21 @@ struct BuildReport;  // build_tree.hpp
 // the environment: RTG_REFILL_CLOSEST, RTG_REFILL_OCCLUSION (0 selects the
 // non-persistent kernels), RTG_REFILL_RAYS, RTG_PATH_ORDER,
 // RTG_TRACE_BLOCKS_PER_CU, RTG_FEED_CHUNK, RTG_BOUNCE_BLOCKS).
-// Measured on MI355X (1080p large scene, 4-wide BVH): refilling lanes before
-// the whole wave is idle loses 13-16 % on the occlusion kernel, so the
-// default refills only an idle wave, one 64-ray batch per atomic; four
-// persistent workgroups per CU match the traversal kernels' occupancy
-// (4 waves per SIMD at their register count) and beat 5 and 8 slightly.
+// Measured on MI355X (two 1080p frames in flight): refilling lanes before the
+// whole wave is idle takes 4,694 to 4,859 us with 32 to 56 idle occlusion
+// lanes and 4,636 to 4,655 with as many closest-hit lanes, against 4,439, so
+// the default refills only an idle wave, one 64-ray batch per atomic; four
+// persistent workgroups per CU match the traversal kernels' occupancy (4
+// waves per SIMD at their register count; five take 4,452 us against 4,312).
 struct Tuning {
     int refill_closest = 64;
     int refill_occlusion = 64;
     // idle lanes before a wavefront of rtg_trace_rays takes new rays (both
     // modes). Not part of rtg_tuning: a frame's rays start together and end
-    // alike, but incoherent queries leave waves with a few long rays, and
-    // refilling at 16 idle lanes measured 1,384/2,479 Mrays/s (closest /
-    // occlusion; 16M rays, origins uniform in the unit cube, directions
-    // uniform on the sphere, into 1M random triangles) against 1,006/1,604
-    // at 64; 8 and 24 were within 4 %
+    // alike, but incoherent queries leave waves with a few long rays. 16 M
+    // random rays into 1 M triangles (closest / 3 M occlusion): 9,355 / 1,104
+    // us at 16 idle lanes, 9,273 / 1,126 at 8, 9,747 / 1,115 at 24; at 64 the
+    // queries took half as long again
     int refill_rays = 16;
     int path_order = 1;
     int blocks_per_cu = 4;
@@ -115,7 +115,7 @@ struct Tuning {
     // shadow rays (0: all levels in sequence on the caller's stream): its
     // shadow-ray launch takes them all, its bounce-level launches at most
     // 192, and the first level's shadow rays the rest of the grid. Frames
-    // alone on the GPU (traces beside others in flight run in sequence) take
+    // alone on the GPU (beside others see enqueue_trace) take
     // 410 us at 480x270 and 681 at 1280x720 with 192 of 1,024, 423 and 762
     // with 128, 451 and 977 with 64
     int bounce_blocks = 192;

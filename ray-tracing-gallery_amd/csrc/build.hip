@@ -1284,7 +1284,7 @@ extern "C" int rtg_blas_build(rtg_ctx* ctx, const rtg_geometry* geoms, uint32_t 
         RTG_REQUIRE(total < (1ull << 27), RTG_ERROR_LIMIT, "BLAS exceeds 2^27 triangles");
     }
     uint32_t n = (uint32_t)total;
-    if (ctx->scratch.ensure(build_scratch_bytes(n, sizeof(TriRec), n_geom)) != RTG_OK) return RTG_ERROR_OUT_OF_MEMORY;
+    if (ensure_room(ctx, ctx->scratch, build_scratch_bytes(n, sizeof(TriRec), n_geom)) != RTG_OK) return RTG_ERROR_OUT_OF_MEMORY;
     const BuildBufs b = carve_build(ctx->scratch.ptr, n, sizeof(TriRec), n_geom);
     GeomArgs args = {};
     const uint32_t by_arg = n_geom <= kGeomArgs ? n_geom : 0;
@@ -1315,8 +1315,11 @@ extern "C" int rtg_blas_build(rtg_ctx* ctx, const rtg_geometry* geoms, uint32_t 
     uint64_t* new_reg = nullptr;
     st = registry_room(ctx, ctx->registry_count + 1, &new_reg);
     if (st != RTG_OK) return st;
-    uint8_t* blob = nullptr;
-    RTG_HIP(hipMalloc(&blob, L.total));
+    void* block = nullptr;
+    uint64_t alloc = 0;
+    st = ctx->blobs.take(L.total, &block, &alloc);
+    if (st != RTG_OK) return st;
+    uint8_t* blob = static_cast<uint8_t*>(block);
     hipLaunchKernelGGL(k_finish_blas, dim3(finish_grid(L.total)), dim3(256), 0, s, blob, L, b.nodes, tris, b.va,
                        b.geoms, n_geom, n, rep.levels, ctx->d_registry, ctx->registry_count, new_reg);
     hipError_t e = hipGetLastError();
@@ -1327,7 +1330,7 @@ extern "C" int rtg_blas_build(rtg_ctx* ctx, const rtg_geometry* geoms, uint32_t 
         return RTG_ERROR_DEVICE;
     }
     uint64_t addr = reinterpret_cast<uint64_t>(blob);
-    ctx->structures[addr] = AsRecord{kKindBlas, n, L.node_count, L.total, {}};
+    ctx->structures[addr] = AsRecord{kKindBlas, n, L.node_count, L.total, alloc, {}};
     registry_commit(ctx, new_reg, ctx->registry_count + 1);
     *out = addr;
     return RTG_OK;
@@ -1341,7 +1344,7 @@ extern "C" int rtg_tlas_build(rtg_ctx* ctx, const rtg_instance* instances, uint3
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     RTG_HIP(hipSetDevice(ctx->device));
     uint32_t n = count;
-    if (ctx->scratch.ensure(build_scratch_bytes(n, sizeof(InstRec), 1)) != RTG_OK) return RTG_ERROR_OUT_OF_MEMORY;
+    if (ensure_room(ctx, ctx->scratch, build_scratch_bytes(n, sizeof(InstRec), 1)) != RTG_OK) return RTG_ERROR_OUT_OF_MEMORY;
     const BuildBufs b = carve_build(ctx->scratch.ptr, n, sizeof(InstRec), 1);
     hipLaunchKernelGGL(k_build_init, dim3(1), dim3(64), 0, s, b.cb, b.tiers, GeomArgs{}, 0u, b.geoms);
     InstRec* recs = reinterpret_cast<InstRec*>(b.recs);
@@ -1363,8 +1366,11 @@ extern "C" int rtg_tlas_build(rtg_ctx* ctx, const rtg_instance* instances, uint3
     }
     if (rep.status & kStatusBadBlas) return check_status(ctx, s, kStatusBadBlas, "rtg_tlas_build");
     const Layout L = tlas_layout(n, rep.nodes, rep.levels);
-    uint8_t* blob = nullptr;
-    RTG_HIP(hipMalloc(&blob, L.total));
+    void* block = nullptr;
+    uint64_t alloc = 0;
+    st = ctx->blobs.take(L.total, &block, &alloc);
+    if (st != RTG_OK) return st;
+    uint8_t* blob = static_cast<uint8_t*>(block);
     hipLaunchKernelGGL(k_finish_tlas, dim3(finish_grid(L.total)), dim3(256), 0, s, blob, L, b.nodes, recs, b.va,
                        instances, b.lbox, b.off, n, rep.levels);
     hipError_t e = hipGetLastError();
@@ -1377,7 +1383,7 @@ extern "C" int rtg_tlas_build(rtg_ctx* ctx, const rtg_instance* instances, uint3
     uint64_t addr = reinterpret_cast<uint64_t>(blob);
     std::vector<uint32_t> level_off;
     if (rep.levels <= kReportLevels) level_off.assign(rep.off, rep.off + rep.levels + 1);
-    ctx->structures[addr] = AsRecord{kKindTlas, n, L.node_count, L.total, level_off};
+    ctx->structures[addr] = AsRecord{kKindTlas, n, L.node_count, L.total, alloc, level_off};
     *out = addr;
     return RTG_OK;
 }
@@ -1403,11 +1409,15 @@ extern "C" int rtg_tlas_clone(rtg_ctx* ctx, rtg_tlas src, rtg_tlas* out, void* s
                 "rtg_tlas_clone: 0x%llx is not a TLAS of this context", (unsigned long long)src);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     RTG_HIP(hipSetDevice(ctx->device));
-    uint8_t* blob = nullptr;
-    RTG_HIP(hipMalloc(&blob, it->second.size));
+    void* blob = nullptr;
+    uint64_t alloc = 0;
+    const int st = ctx->blobs.take(it->second.size, &blob, &alloc);
+    if (st != RTG_OK) return st;
     RTG_HIP(hipMemcpyAsync(blob, reinterpret_cast<const void*>(src), it->second.size, hipMemcpyDeviceToDevice, s));
     uint64_t addr = reinterpret_cast<uint64_t>(blob);
-    ctx->structures[addr] = it->second;
+    AsRecord rec = it->second;
+    rec.alloc = alloc;
+    ctx->structures[addr] = rec;
     *out = addr;
     return RTG_OK;
 }
@@ -1419,7 +1429,7 @@ static int destroy_as(rtg_ctx* ctx, uint64_t addr, uint32_t kind, const char* wh
     RTG_REQUIRE(it != ctx->structures.end() && it->second.kind == kind, RTG_ERROR_NOT_FOUND,
                 "%s: 0x%llx is not a live structure of this kind", what, (unsigned long long)addr);
     RTG_HIP(hipDeviceSynchronize());
-    RTG_HIP(hipFree(reinterpret_cast<void*>(addr)));
+    ctx->blobs.put(reinterpret_cast<void*>(addr), it->second.alloc);
     ctx->structures.erase(it);
     if (kind == kKindBlas) return refresh_registry(ctx);
     return RTG_OK;

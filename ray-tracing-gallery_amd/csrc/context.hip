@@ -43,6 +43,63 @@ int DeviceBuffer::ensure(size_t bytes, bool slack) {
     return RTG_OK;
 }
 
+int ensure_room(rtg_ctx* ctx, DeviceBuffer& b, size_t bytes, bool slack) {
+    const int st = b.ensure(bytes, slack);
+    if (st != RTG_ERROR_OUT_OF_MEMORY || !ctx->blobs.release()) return st;
+    hipGetLastError();  // the allocation's error is answered here
+    clear_error();
+    return b.ensure(bytes, slack);
+}
+
+int BlobPool::take(size_t want, void** ptr, uint64_t* size) {
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        size_t best = blocks.size();
+        for (size_t k = 0; k < blocks.size(); ++k)
+            if (blocks[k].size >= want && blocks[k].size <= want + want / 4 &&
+                (best == blocks.size() || blocks[k].size < blocks[best].size))
+                best = k;
+        if (best < blocks.size()) {
+            *ptr = blocks[best].ptr;
+            *size = blocks[best].size;
+            bytes -= blocks[best].size;
+            blocks.erase(blocks.begin() + best);
+            return RTG_OK;
+        }
+    }
+    hipError_t e = hipMalloc(ptr, want);
+    if (e == hipErrorOutOfMemory && release()) {
+        hipGetLastError();  // the first attempt's error is answered here
+        e = hipMalloc(ptr, want);
+    }
+    if (e != hipSuccess) {
+        set_error("hipMalloc(%zu) failed: %s", want, hipGetErrorString(e));
+        return RTG_ERROR_DEVICE;
+    }
+    *size = want;
+    return RTG_OK;
+}
+
+void BlobPool::put(void* ptr, size_t size) {
+    std::lock_guard<std::mutex> lk(mu);
+    blocks.push_back(Block{ptr, size});
+    bytes += size;
+    while (bytes > kBlobPoolBytes || blocks.size() > kBlobPoolBlocks) {
+        hipFree(blocks.front().ptr);
+        bytes -= blocks.front().size;
+        blocks.erase(blocks.begin());
+    }
+}
+
+bool BlobPool::release() {
+    std::lock_guard<std::mutex> lk(mu);
+    const bool any = !blocks.empty();
+    for (const Block& b : blocks) hipFree(b.ptr);
+    blocks.clear();
+    bytes = 0;
+    return any;
+}
+
 void DeviceBuffer::release() {
     if (ptr) hipFree(ptr);
     ptr = nullptr;
@@ -161,6 +218,7 @@ extern "C" void rtg_destroy(rtg_ctx* ctx) {
     drain_timers(ctx);
     for (auto& kv : ctx->structures) hipFree(reinterpret_cast<void*>(kv.first));
     ctx->structures.clear();
+    ctx->blobs.release();
     for (void* p : ctx->retired) hipFree(p);
     if (ctx->registry_arena) hipFree(ctx->registry_arena);
     if (ctx->build_report) hipHostFree(ctx->build_report);

@@ -143,7 +143,7 @@ bool rtg_server::launch(Slot& s) {
         arena_reset(s.arena);
         s.tlas_copies.release();
     }
-    if (copy_bytes && s.tlas_copies.ensure(copy_bytes, false) != RTG_OK) return false;
+    if (copy_bytes && ensure_room(ctx, s.tlas_copies, copy_bytes, false) != RTG_OK) return false;
     std::vector<rtg_image_job> jobs(s.batch.size());
     size_t off = 0;
     for (size_t k = 0; k < s.batch.size(); ++k) {

@@ -1349,7 +1349,7 @@ size_t spill_bytes(rtg_ctx* ctx, const Tuning& tune) {
 }
 
 static int ensure_spill(rtg_ctx* ctx, FrameArena* a, const Tuning& tune) {
-    return a->spill.ensure(spill_bytes(ctx, tune), !a->exact);
+    return ensure_room(ctx, a->spill, spill_bytes(ctx, tune), !a->exact);
 }
 
 size_t arena_bytes_after(const FrameArena* a, uint64_t paths, uint64_t shadow, uint32_t njobs) {
@@ -1385,7 +1385,7 @@ static int ensure_frame(rtg_ctx* ctx, FrameArena* a, uint64_t paths, uint64_t sh
         uint64_t P = std::max<uint64_t>(paths, a->paths_cap);
         uint64_t S = std::max<uint64_t>(shadow, a->shadow_cap);
         uint32_t NJ = std::max<uint32_t>(njobs, a->jobs_cap);
-        if (a->buf.ensure(frame_bytes(P, S, NJ), !a->exact) != RTG_OK) return RTG_ERROR_OUT_OF_MEMORY;
+        if (ensure_room(ctx, a->buf, frame_bytes(P, S, NJ), !a->exact) != RTG_OK) return RTG_ERROR_OUT_OF_MEMORY;
         Carve c(a->buf.ptr);
         Frame& F = a->F;
         F.shade_a = c.take<float4>(P);

@@ -1055,8 +1055,8 @@ static int wide_hierarchy(rtg_ctx* ctx, const BuildBufs& b, uint32_t n, int tree
         for (int round = 0; round < treelet_rounds; ++round) {
             uint32_t* tiers = b.tiers + kTierWords * round;
             if (round > 0)
-                hipLaunchKernelGGL(k_tier_roots, dim3(blocks_for(n - 1, kRootThreads)), dim3(kRootThreads), 0, s, n, b.bin,
-                                   b.rcount, b.low, b.mid, tiers);
+                hipLaunchKernelGGL(k_tier_roots, dim3(blocks_for(n - 1, kRootThreads)), dim3(kRootThreads), 0, s, n,
+                                   b.bin, b.rcount, b.low, b.mid, tiers);
             launch_pass<true>(b, n, tiers, 1, s);
         }
     }
@@ -1115,8 +1115,8 @@ static void radix_tree(const BuildBufs& b, uint32_t n, hipStream_t s) {
         std::swap(vin, vout);
     }
     // after 4 passes the sorted data is back in (ka, va)
-    hipLaunchKernelGGL(k_karras, dim3(blocks_for(n, kRootThreads)), dim3(kRootThreads), 0, s, b.ka, (int)n, b.va, b.boxes,
-                       b.lbox, b.bin, b.rcount, b.low, b.mid, b.tiers);
+    hipLaunchKernelGGL(k_karras, dim3(blocks_for(n, kRootThreads)), dim3(kRootThreads), 0, s, b.ka, (int)n, b.va,
+                       b.boxes, b.lbox, b.bin, b.rcount, b.low, b.mid, b.tiers);
 }
 
 // At most one primitive: the single node.
@@ -1148,7 +1148,7 @@ static int registry_room(rtg_ctx* ctx, uint32_t count, uint64_t** out) {
     if (ctx->registry_used + count > ctx->registry_cap || !ctx->registry_arena) {
         const size_t cap = std::max<size_t>(8192, 16 * (size_t)count);
         uint64_t* p = nullptr;
-        RTG_HIP(hipMalloc(&p, cap * sizeof(uint64_t)));
+        RTG_HIP(ctx->blobs.allocate(reinterpret_cast<void**>(&p), cap * sizeof(uint64_t)));
         if (ctx->registry_arena) ctx->retired.push_back(ctx->registry_arena);
         ctx->registry_arena = p;
         ctx->registry_cap = cap;
@@ -1284,7 +1284,8 @@ extern "C" int rtg_blas_build(rtg_ctx* ctx, const rtg_geometry* geoms, uint32_t 
         RTG_REQUIRE(total < (1ull << 27), RTG_ERROR_LIMIT, "BLAS exceeds 2^27 triangles");
     }
     uint32_t n = (uint32_t)total;
-    if (ensure_room(ctx, ctx->scratch, build_scratch_bytes(n, sizeof(TriRec), n_geom)) != RTG_OK) return RTG_ERROR_OUT_OF_MEMORY;
+    if (ensure_room(ctx, ctx->scratch, build_scratch_bytes(n, sizeof(TriRec), n_geom)) != RTG_OK)
+        return RTG_ERROR_OUT_OF_MEMORY;
     const BuildBufs b = carve_build(ctx->scratch.ptr, n, sizeof(TriRec), n_geom);
     GeomArgs args = {};
     const uint32_t by_arg = n_geom <= kGeomArgs ? n_geom : 0;
@@ -1299,8 +1300,8 @@ extern "C" int rtg_blas_build(rtg_ctx* ctx, const rtg_geometry* geoms, uint32_t 
         hipLaunchKernelGGL(k_small_tris, dim3(1), dim3(kSmallThreads), 0, s, b.geoms, n_geom, n, tris, small_out(b),
                            ctx->d_status);
     } else if (n > 0) {
-        hipLaunchKernelGGL(k_tri_setup, dim3(std::min(blocks_for(n, kSetupThreads), kSetupBlocks)), dim3(kSetupThreads), 0, s, b.geoms, n_geom, n, tris, b.boxes,
-                           b.cb, ctx->d_status);
+        hipLaunchKernelGGL(k_tri_setup, dim3(std::min(blocks_for(n, kSetupThreads), kSetupBlocks)),
+                           dim3(kSetupThreads), 0, s, b.geoms, n_geom, n, tris, b.boxes, b.cb, ctx->d_status);
         if (n > 1) radix_tree(b, n, s);
     }
     BuildReport rep;
@@ -1344,7 +1345,8 @@ extern "C" int rtg_tlas_build(rtg_ctx* ctx, const rtg_instance* instances, uint3
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     RTG_HIP(hipSetDevice(ctx->device));
     uint32_t n = count;
-    if (ensure_room(ctx, ctx->scratch, build_scratch_bytes(n, sizeof(InstRec), 1)) != RTG_OK) return RTG_ERROR_OUT_OF_MEMORY;
+    if (ensure_room(ctx, ctx->scratch, build_scratch_bytes(n, sizeof(InstRec), 1)) != RTG_OK)
+        return RTG_ERROR_OUT_OF_MEMORY;
     const BuildBufs b = carve_build(ctx->scratch.ptr, n, sizeof(InstRec), 1);
     hipLaunchKernelGGL(k_build_init, dim3(1), dim3(64), 0, s, b.cb, b.tiers, GeomArgs{}, 0u, b.geoms);
     InstRec* recs = reinterpret_cast<InstRec*>(b.recs);

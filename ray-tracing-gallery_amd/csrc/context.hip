@@ -67,17 +67,22 @@ int BlobPool::take(size_t want, void** ptr, uint64_t* size) {
             return RTG_OK;
         }
     }
-    hipError_t e = hipMalloc(ptr, want);
-    if (e == hipErrorOutOfMemory && release()) {
-        hipGetLastError();  // the first attempt's error is answered here
-        e = hipMalloc(ptr, want);
-    }
+    const hipError_t e = allocate(ptr, want);
     if (e != hipSuccess) {
         set_error("hipMalloc(%zu) failed: %s", want, hipGetErrorString(e));
         return RTG_ERROR_DEVICE;
     }
     *size = want;
     return RTG_OK;
+}
+
+hipError_t BlobPool::allocate(void** ptr, size_t size) {
+    hipError_t e = hipMalloc(ptr, size);
+    if (e == hipErrorOutOfMemory && release()) {
+        hipGetLastError();  // the first attempt's error is answered here
+        e = hipMalloc(ptr, size);
+    }
+    return e;
 }
 
 void BlobPool::put(void* ptr, size_t size) {

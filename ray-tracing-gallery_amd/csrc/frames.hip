@@ -82,7 +82,7 @@ extern "C" int rtg_frames_create(rtg_ctx* ctx, rtg_tlas tlas, uint32_t frames_in
     for (FrameSlot& s : f->slots) {
         int st = e == hipSuccess ? rtg_tlas_clone(ctx, tlas, &s.tlas, nullptr) : RTG_ERROR_DEVICE;
         if (st == RTG_OK && (hipHostMalloc(reinterpret_cast<void**>(&s.host), bytes) != hipSuccess ||
-                             hipMalloc(&s.dev, bytes) != hipSuccess ||
+                             ctx->blobs.allocate(reinterpret_cast<void**>(&s.dev), bytes) != hipSuccess ||
                              hipEventCreateWithFlags(&s.done, hipEventDisableTiming) != hipSuccess))
             st = RTG_ERROR_OUT_OF_MEMORY;
         if (st == RTG_OK && f->count &&

@@ -66,6 +66,8 @@ struct BlobPool {
     // `size`: the block's
     int take(size_t want, void** ptr, uint64_t* size);
     void put(void* ptr, size_t size);
+    // hipMalloc, once more with the pool given back if it fails
+    hipError_t allocate(void** ptr, size_t size);
     bool release();  // true if there was something to give back
 };
 

@@ -1843,7 +1843,7 @@ extern "C" int rtg_trace_rays(rtg_ctx* ctx, rtg_tlas tlas, const rtg_scene_bindi
                 "rtg_trace_rays: the frame state of stream %p is in use by another call (a context is used by one "
                 "thread at a time)",
                 (void*)s);
-    if (ensure_spill(ctx, a, ctx->tune) != RTG_OK || a->feed.ensure(kFeedWords * sizeof(uint32_t)) != RTG_OK)
+    if (ensure_spill(ctx, a, ctx->tune) != RTG_OK || ensure_room(ctx, a->feed, kFeedWords * sizeof(uint32_t)) != RTG_OK)
         return RTG_ERROR_OUT_OF_MEMORY;
     launch_ray_query(ctx, tlas, scene, rays, count, mode, ray_flags, cull_mask, sbt_offset, hits, occluded,
                      reinterpret_cast<uint2*>(a->spill.ptr), reinterpret_cast<uint32_t*>(a->feed.ptr), kFeedStride,

@@ -18,6 +18,7 @@
 
 #include "rtg_device.hpp"
 #include "rtg_internal.hpp"
+#include "queue_alloc.hpp"
 
 namespace rtg {
 
@@ -142,58 +143,6 @@ __device__ inline uint32_t find_job(const JobDev* jobs, uint32_t njobs, uint64_t
         else hi = mid;
     }
     return lo;
-}
-
-// Allocation from two queues by a whole workgroup (every lane calls it; lanes
-// that need nothing pass 0): one atomic per queue and 256 lanes. Atomics to
-// one address pass one at a time, about 13 ns each, which bound the shading of
-// large images when every wave made its own (7.4 M paths: 115 k of them,
-// 1.5 ms). EVEN: every lane wants the same number of entries of the first
-// queue or none, so ranks come from a ballot.
-struct QueueAlloc {
-    uint32_t total[2][4], base[2];
-};
-__device__ inline uint32_t wave_rank(uint32_t want, bool even, uint32_t& total) {
-    const int lane = threadIdx.x & 63;
-    if (even) {
-        const uint64_t m = __ballot(want != 0u);
-        const uint32_t each = m ? (uint32_t)__shfl((int)want, (int)__builtin_ctzll(m)) : 0u;
-        total = each * (uint32_t)__popcll(m);
-        return each * (uint32_t)__popcll(m & (lane == 0 ? 0ull : (~0ull >> (64 - lane))));
-    }
-    uint32_t incl = want;
-    for (int off = 1; off < 64; off <<= 1) {
-        uint32_t v = (uint32_t)__shfl_up((int)incl, off);
-        if (lane >= off) incl += v;
-    }
-    total = (uint32_t)__shfl((int)incl, 63);
-    return incl - want;
-}
-template <bool EVEN>
-__device__ inline void block_alloc(QueueAlloc& A, uint32_t want0, uint32_t* counter0, bool want1, uint32_t* counter1,
-                                   uint32_t& slot0, uint32_t& slot1) {
-    const int w = threadIdx.x >> 6;
-    uint32_t t0, t1;
-    const uint32_t r0 = wave_rank(want0, EVEN, t0), r1 = wave_rank(want1 ? 1u : 0u, true, t1);
-    if ((threadIdx.x & 63) == 0) {
-        A.total[0][w] = t0;
-        A.total[1][w] = t1;
-    }
-    __syncthreads();
-    if (threadIdx.x < 2) {
-        const uint32_t* tt = A.total[threadIdx.x];
-        const uint32_t sum = (tt[0] + tt[1]) + (tt[2] + tt[3]);
-        A.base[threadIdx.x] = sum ? atomicAdd(threadIdx.x ? counter1 : counter0, sum) : 0u;
-    }
-    __syncthreads();
-    uint32_t b0 = A.base[0], b1 = A.base[1];
-    for (int k = 0; k < 3; ++k)
-        if (k < w) {
-            b0 += A.total[0][k];
-            b1 += A.total[1][k];
-        }
-    slot0 = b0 + r0;
-    slot1 = b1 + r1;
 }
 
 __device__ inline void wave_add_counter(uint64_t* c, uint32_t v) {
@@ -851,7 +800,7 @@ __global__ __launch_bounds__(256) void k_shade(Frame F, int level, const uint32_
         // count) so that the occlusion kernel's pairs never span two paths
         const uint32_t shadow_slots = want_shadow + (want_shadow & 1u);
         uint32_t sbase, nbase;
-        block_alloc<ONE>(s_alloc, shadow_slots, &F.counts[level == 0 ? kShadowFirst : kShadowRest], want_next,
+        block_alloc<ONE>(s_alloc, r, shadow_slots, &F.counts[level == 0 ? kShadowFirst : kShadowRest], want_next,
                          next_count, sbase, nbase);
         if (level > 0) sbase += F.counts[kShadowFirst];
         if (want_next && nbase >= F.path_cap) {

@@ -64,13 +64,6 @@ struct alignas(16) BinNode {
 constexpr uint32_t kTierLow = 256;     // largest subtree a bottom workgroup holds in LDS
 constexpr uint32_t kTierHigh = 65536;  // largest subtree of the middle tier
 
-// Compiler order of LDS accesses between the lanes of one wave (the hardware
-// serves a wave's LDS accesses in order).
-__device__ __forceinline__ void wave_order() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // ---------------------------------------------------------------------------
 // Treelet restructuring (Karras & Aila 2013, HPG, "Fast Parallel
 // Construction of High-Quality Bounding Volume Hierarchies", section 4) of

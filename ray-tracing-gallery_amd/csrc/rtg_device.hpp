@@ -1179,6 +1179,13 @@ __device__ inline void shear_setup(V3 d, V3 inv, float& sx, float& sy, float& sz
     axes = (uint32_t)kx | ((uint32_t)ky << 2) | ((uint32_t)kz << 4);
 }
 
+// Compiler order of memory accesses between the lanes of one wave (the
+// hardware serves a wave's LDS accesses in order, and its global ones).
+__device__ __forceinline__ void wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // The ray's stack, shared by its four lanes: consecutive entries of a ray lie
 // side by side in LDS (a visit's pushes are one conflict-free store), rays an
 // odd number of entries apart; deeper entries in the spill areas of the
@@ -1203,7 +1210,10 @@ struct QuadStack {
             *(RTG_GLOBAL rtg_u2v*)(spill + (at - lds_n)) = v;
         }
     }
+    // an entry may be another lane's, pushed just before: its store has to
+    // stay ahead of this load
     __device__ inline uint2 pop() {
+        wave_order();
         --sp;
         return sp < lds_n ? lds[sp] : gld_u2(spill + (sp - lds_n));
     }

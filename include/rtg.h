@@ -207,9 +207,9 @@ int rtg_blas_query_sizes(rtg_ctx* ctx, const rtg_geometry* geometries, uint32_t 
 int rtg_blas_build(rtg_ctx* ctx, const rtg_geometry* geometries, uint32_t geometry_count,
                    uint32_t build_flags, rtg_blas* out, void* stream);
 /* Waits for the device. The context keeps up to 128 MiB of destroyed
- * structures' memory for its next builds and clones; it gives it back when a
- * device allocation of its own fails, and in rtg_destroy. The same holds for
- * rtg_tlas_destroy. */
+ * structures' memory for its next builds and clones (a larger structure's is
+ * freed at once); it gives it back when a device allocation of its own fails,
+ * and in rtg_destroy. The same holds for rtg_tlas_destroy. */
 int rtg_blas_destroy(rtg_ctx* ctx, rtg_blas blas);
 
 /* ------------------------------------------------------------------------ */

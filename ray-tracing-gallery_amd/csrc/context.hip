@@ -86,6 +86,10 @@ hipError_t BlobPool::allocate(void** ptr, size_t size) {
 }
 
 void BlobPool::put(void* ptr, size_t size) {
+    if (size > kBlobPoolBytes) {  // it would push every kept block out and then go itself
+        hipFree(ptr);
+        return;
+    }
     std::lock_guard<std::mutex> lk(mu);
     blocks.push_back(Block{ptr, size});
     bytes += size;

@@ -49,9 +49,10 @@ struct AsRecord {
 // Device memory of destroyed structures, kept for the context's next builds
 // (hipMalloc and hipFree: rebuilding an 81,920-triangle mesh 489 -> 445 us
 // without them, one of 1 M triangles 5,478 -> 5,064). At most kBlobPoolBytes
-// in kBlobPoolBlocks blocks, the oldest given up first; all of it is given
-// back when a device allocation of the context fails, and with the context. A
-// block comes in after a device synchronisation, so any stream may use it.
+// in kBlobPoolBlocks blocks, the oldest given up first; a larger block (a mesh
+// of some 1.3 M triangles) is freed at once. All of it is given back when a
+// device allocation of the context fails, and with the context. A block comes
+// in after a device synchronisation, so any stream may use it.
 constexpr size_t kBlobPoolBytes = size_t(128) << 20;
 constexpr size_t kBlobPoolBlocks = 64;
 struct BlobPool {

@@ -32,3 +32,19 @@ def test_destroyed_structures_are_bounded_and_given_back():
         assert before - torch.cuda.mem_get_info()[0] <= (128 << 20) + (8 << 20)
     c.close()
     assert torch.cuda.mem_get_info()[0] >= before
+
+
+def test_a_block_beyond_the_bound_leaves_the_kept_ones():
+    """A structure of more than 128 MiB is never kept; destroying it leaves
+    what the context keeps of smaller ones."""
+    c = Context(0)
+    rng = np.random.default_rng(3)
+    large, small = (rng.random((n, 3, 3), dtype=np.float32) for n in (2_000_000, 1_000_000))
+    assert len(gpu_blob(c, large, 0)) > 128 << 20  # and the build's scratch at its largest
+    torch.cuda.empty_cache()
+    before = torch.cuda.mem_get_info()[0]
+    kept = len(gpu_blob(c, small, 0))
+    gpu_blob(c, large, 0)
+    torch.cuda.empty_cache()
+    assert before - torch.cuda.mem_get_info()[0] >= kept
+    c.close()

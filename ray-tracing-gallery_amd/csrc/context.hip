@@ -206,12 +206,12 @@ extern "C" int rtg_create(rtg_ctx** out, int device) {
     hipMemset(ctx->d_counters, 0, sizeof(rtg_trace_counters));
     int st = refresh_registry(ctx);
     if (st == RTG_OK) st = build_report_init(ctx);
-    if (st == RTG_OK && hipHostMalloc(reinterpret_cast<void**>(&ctx->flight_done),
-                                      kFlightSlots * sizeof(uint32_t), hipHostMallocMapped) != hipSuccess) {
+    if (st == RTG_OK && hipHostMalloc(reinterpret_cast<void**>(&ctx->flight.ended),
+                                      kFlightWords * sizeof(uint32_t), hipHostMallocMapped) != hipSuccess) {
         set_error("rtg_create: host allocation failed");
         st = RTG_ERROR_OUT_OF_MEMORY;
     }
-    if (st == RTG_OK) memset(ctx->flight_done, 0, kFlightSlots * sizeof(uint32_t));
+    if (st == RTG_OK) memset(ctx->flight.ended, 0, kFlightWords * sizeof(uint32_t));
     if (st != RTG_OK) {
         rtg_destroy(ctx);
         return st;
@@ -231,9 +231,9 @@ extern "C" void rtg_destroy(rtg_ctx* ctx) {
     for (void* p : ctx->retired) hipFree(p);
     if (ctx->registry_arena) hipFree(ctx->registry_arena);
     if (ctx->build_report) hipHostFree(ctx->build_report);
-    if (ctx->flight_done) hipHostFree(ctx->flight_done);
     ctx->scratch.release();
     free_frame_arena(ctx);
+    if (ctx->flight.ended) hipHostFree(ctx->flight.ended);
     if (ctx->d_srgb_lut) hipFree(ctx->d_srgb_lut);
     if (ctx->d_status) hipFree(ctx->d_status);
     if (ctx->d_counters) hipFree(ctx->d_counters);

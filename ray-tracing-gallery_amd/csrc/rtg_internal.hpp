@@ -4,11 +4,12 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
-#include <atomic>
 #include <map>
 #include <mutex>
 #include <string>
 #include <vector>
+
+#include "flight.hpp"
 
 #include "../../include/rtg.h"
 
@@ -113,7 +114,6 @@ struct TimedLaunch {
 };
 
 struct FrameArena;  // trace.hip
-constexpr int kFlightSlots = 64;
 struct BuildReport;  // build_tree.hpp
 
 // Launch parameters of the traversal kernels (defaults, overridable through
@@ -180,12 +180,7 @@ struct rtg_ctx {
     uint64_t kernel_launches[RTG_KERNEL_COUNT] = {};
     // frame state of the context's own calls, one per stream they are made on
     std::map<void*, rtg::FrameArena*> frames;
-    // Traces in flight, by arena: how many each has started, and (in host
-    // memory, written by a trace's last kernel) the last that ended. More
-    // arenas than words share them: that can only make a trace look in flight.
-    std::atomic<uint32_t> flight_started[rtg::kFlightSlots] = {};
-    std::atomic<uint32_t> flight_next{0};
-    uint32_t* flight_done = nullptr;
+    rtg::FlightTable flight;
     int hw_queues = 4;  // GPU_MAX_HW_QUEUES, HIP's hardware queues per process
     rtg::Tuning tune;
 };

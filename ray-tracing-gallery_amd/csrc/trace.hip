@@ -1210,7 +1210,9 @@ struct FrameArena {
     // grow to exactly the size asked (no headroom): a server slot's arena,
     // whose device bytes count against an HBM budget
     bool exact = false;
-    int flight = -1;  // its word in the context's flight table, from its first trace on
+    // its word in the context's flight table, from its first trace on
+    FlightTable* flights = nullptr;
+    int flight = -1;
     // host calls using the arena now: a second one at the same time (two
     // threads tracing on one stream of one context) is refused
     std::atomic<int> users{0};
@@ -1236,6 +1238,7 @@ void delete_frame_arena(FrameArena* a) {
     }
     if (a->fork) hipEventDestroy(a->fork);
     if (a->join) hipEventDestroy(a->join);
+    if (a->flights) a->flights->give(a->flight);
     delete a;
 }
 
@@ -1472,17 +1475,6 @@ int upload_jobs(FrameArena* a, const TracePlan& P, hipStream_t s) {
     return RTG_OK;
 }
 
-// How many other arenas than `a` have a trace on the GPU, as far as the host
-// words tell (a moment's view, which changes launch shapes only).
-static int others_in_flight(rtg_ctx* ctx, const FrameArena* a) {
-    int n = 0;
-    for (int k = 0; k < kFlightSlots; ++k)
-        if (k != a->flight && ctx->flight_started[k].load(std::memory_order_relaxed) !=
-                                  __atomic_load_n(&ctx->flight_done[k], __ATOMIC_RELAXED))
-            ++n;
-    return n;
-}
-
 void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning& tune, bool cnt, bool timed,
                    hipStream_t s, bool flight) {
     Frame F = a->F;
@@ -1584,7 +1576,7 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
     // 1,650 and 4,067..4,130 to 4,155; six served requests on eight queues
     // 7,276 to 5,681. A frame alone is the faster side by side (404 us to 505
     // at 480x270). Counted traces keep the setting's split.
-    const int others = flight && !cnt ? others_in_flight(ctx, a) : 0;
+    const int others = flight && !cnt ? ctx->flight.others(a->flight) : 0;
     const bool crowded = others > 0 && 2 * (others + 1) + 1 > ctx->hw_queues;
     const unsigned Gside = crowded ? 0 : std::min<unsigned>((unsigned)tune.bounce_blocks, G / 2);
     if (P.max_traces > 1 && Gside > 0) {
@@ -1633,9 +1625,14 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
     uint32_t* done = nullptr;
     uint32_t seq = 0;
     if (flight) {
-        if (a->flight < 0) a->flight = (int)(ctx->flight_next.fetch_add(1) % kFlightSlots);
-        done = ctx->flight_done + a->flight;
-        seq = ctx->flight_started[a->flight].fetch_add(1) + 1;
+        if (a->flight < 0) {
+            a->flights = &ctx->flight;
+            a->flight = ctx->flight.take();
+        }
+        if (a->flight >= 0) {
+            done = ctx->flight.ended + a->flight;
+            seq = ctx->flight.start(a->flight);
+        }
     }
     {
         LaunchTimer t(ctx, RTG_KERNEL_RESOLVE, s, timed);

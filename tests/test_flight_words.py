@@ -1,0 +1,75 @@
+"""Which traces count as in flight: the table of csrc/flight.hpp on the CPU,
+and on the GPU the choice made by it, seen in whether a frame launches the
+bounce levels beside the first level's shadow rays or in sequence."""
+import os
+import subprocess
+
+import pytest
+import torch
+
+from conftest import PKG, REPO
+from rtg import abi, scenes
+from rtg.device import DeviceScene
+from rtg.frames import FrameDriver
+from rtg.lib import Context
+
+
+def test_the_table(tmp_path):
+    exe = str(tmp_path / "flight_words")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-I", os.path.join(PKG, "csrc"), "-o", exe,
+                    os.path.join(REPO, "tests", "flight_words.cpp")], check=True, timeout=120)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
+    assert "flight words: ok" in r.stdout
+
+
+def launched_side_by_side(c, enqueue):
+    """Whether a frame that `enqueue` traces runs its bounce levels beside the
+    first level's shadow rays."""
+    c.set_timing(True)
+    enqueue()
+    n = c.kernel_time(abi.RTG_KERNEL_BOUNCE_SIDE)[1]
+    c.set_timing(False)
+    return n > 0
+
+
+class LongTrace:
+    """A frame of several milliseconds (16.6 M paths), enqueued again and again."""
+
+    def __init__(self, ds):
+        self.opts = ds.scene.trace_opts()
+        self.opts.spp = 8
+        self.out = ds.make_outputs(width=1920, height=1080, hits=False)
+        self.job = ds.job(self.out, opts=self.opts, width=1920, height=1080)
+
+
+@pytest.mark.gpu
+def test_more_arenas_than_a_small_table_has_words(monkeypatch):
+    """136 frame slots: a frame sees the trace of any other slot, and sees none
+    once all have ended."""
+    monkeypatch.setenv("GPU_MAX_HW_QUEUES", "4")
+    c = Context(0)
+    ds = DeviceScene(c, scenes.default_scene(n_tori=12, width=96, height=54))
+    out = ds.make_outputs(hits=False)
+    drivers = [FrameDriver(ds, 8) for _ in range(17)]
+    s0, s1 = torch.cuda.Stream(), torch.cuda.Stream()
+
+    def frame(slot, job, stream):
+        drivers[slot // 8].begin(slot % 8)
+        drivers[slot // 8].submit(slot % 8, job, stream)
+
+    short, long = ds.job(out), LongTrace(ds)
+    for slot in range(136):
+        frame(slot, short, s1)
+    frame(0, long.job, s0)
+    torch.cuda.synchronize()
+    for slot in (1, 64, 128, 135):
+        assert launched_side_by_side(c, lambda: frame(slot, short, s1)), slot
+        torch.cuda.synchronize()
+        frame(0, long.job, s0)
+        assert not launched_side_by_side(c, lambda: frame(slot, short, s1)), slot
+        torch.cuda.synchronize()
+    for d in drivers:
+        d.close()
+    ds.destroy()
+    c.close()

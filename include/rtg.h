@@ -482,8 +482,9 @@ typedef struct rtg_tuning {
                                   (on all) beside the first level's shadow rays (taken from the
                                   blocks_per_cu grid, at most half of it); 192 by default;
                                   0 = every level in sequence on the caller's stream, as is an
-                                  uncounted trace enqueued while others of the context are in
-                                  flight (on other streams, frame slots or server slots) and
+                                  uncounted trace enqueued while others of the process are in
+                                  flight on the device (of any context, on other streams, frame
+                                  slots or server slots; replays of an rtg_batch don't count) and
                                   GPU_MAX_HW_QUEUES, as rtg_create found it (4 if unset), is too
                                   small for two queues each and one more */
     uint32_t stack_lds_entries; /* traversal stack entries per lane kept in LDS (8..32, multiple of 4;

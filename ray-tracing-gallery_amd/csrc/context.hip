@@ -133,6 +133,26 @@ LaunchTimer::~LaunchTimer() {
     ctx->pending.push_back(TimedLaunch{kind, a, b});
 }
 
+// The flight table of a device (which must be current): one for all contexts,
+// made with the first and freed with the last of them and their arenas.
+static std::shared_ptr<FlightTable> flight_table(int device) {
+    static std::mutex mu;
+    static std::map<int, std::weak_ptr<FlightTable>> tables;
+    std::lock_guard<std::mutex> lk(mu);
+    std::shared_ptr<FlightTable> t = tables[device].lock();
+    if (t) return t;
+    void* words = nullptr;
+    if (hipHostMalloc(&words, kFlightWords * sizeof(uint32_t), hipHostMallocMapped) != hipSuccess) return nullptr;
+    memset(words, 0, kFlightWords * sizeof(uint32_t));
+    t = std::shared_ptr<FlightTable>(new FlightTable(), [](FlightTable* p) {
+        hipHostFree(p->ended);
+        delete p;
+    });
+    t->ended = static_cast<uint32_t*>(words);
+    tables[device] = t;
+    return t;
+}
+
 static int drain_timers(rtg_ctx* ctx) {
     for (auto& t : ctx->pending) {
         hipEventSynchronize(t.stop);
@@ -206,12 +226,13 @@ extern "C" int rtg_create(rtg_ctx** out, int device) {
     hipMemset(ctx->d_counters, 0, sizeof(rtg_trace_counters));
     int st = refresh_registry(ctx);
     if (st == RTG_OK) st = build_report_init(ctx);
-    if (st == RTG_OK && hipHostMalloc(reinterpret_cast<void**>(&ctx->flight.ended),
-                                      kFlightWords * sizeof(uint32_t), hipHostMallocMapped) != hipSuccess) {
-        set_error("rtg_create: host allocation failed");
-        st = RTG_ERROR_OUT_OF_MEMORY;
+    if (st == RTG_OK) {
+        ctx->flight = flight_table(device);
+        if (!ctx->flight) {
+            set_error("rtg_create: host allocation failed");
+            st = RTG_ERROR_OUT_OF_MEMORY;
+        }
     }
-    if (st == RTG_OK) memset(ctx->flight.ended, 0, kFlightWords * sizeof(uint32_t));
     if (st != RTG_OK) {
         rtg_destroy(ctx);
         return st;
@@ -233,7 +254,6 @@ extern "C" void rtg_destroy(rtg_ctx* ctx) {
     if (ctx->build_report) hipHostFree(ctx->build_report);
     ctx->scratch.release();
     free_frame_arena(ctx);
-    if (ctx->flight.ended) hipHostFree(ctx->flight.ended);
     if (ctx->d_srgb_lut) hipFree(ctx->d_srgb_lut);
     if (ctx->d_status) hipFree(ctx->d_status);
     if (ctx->d_counters) hipFree(ctx->d_counters);

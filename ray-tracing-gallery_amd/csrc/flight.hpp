@@ -1,4 +1,4 @@
-// flight.hpp -- which traces are on the GPU. Host code without HIP, so that a
+// flight.hpp -- which of a process's traces are on a GPU. Host code without HIP, so that a
 // CPU build can run it.
 #pragma once
 

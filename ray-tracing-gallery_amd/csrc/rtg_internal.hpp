@@ -5,6 +5,7 @@
 
 #include <cstdint>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -180,7 +181,9 @@ struct rtg_ctx {
     uint64_t kernel_launches[RTG_KERNEL_COUNT] = {};
     // frame state of the context's own calls, one per stream they are made on
     std::map<void*, rtg::FrameArena*> frames;
-    rtg::FlightTable flight;
+    // traces in flight on the device, of all its contexts: they share the
+    // process's hardware queues
+    std::shared_ptr<rtg::FlightTable> flight;
     int hw_queues = 4;  // GPU_MAX_HW_QUEUES, HIP's hardware queues per process
     rtg::Tuning tune;
 };
@@ -245,7 +248,7 @@ int upload_jobs(FrameArena* a, const TracePlan& P, hipStream_t stream);
 // Device half: the kernels of the step and nothing else (no copy, memset or
 // allocation), so that it can be captured into a graph. Launch parameters
 // come from `tune`; `timed` records kernel events when timing is on; `flight`
-// enters the trace in the context's flight table (not for kernels that are
+// enters the trace in the device's flight table (not for kernels that are
 // captured to run later).
 void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning& tune, bool counters, bool timed,
                    hipStream_t stream, bool flight = false);

@@ -1210,8 +1210,8 @@ struct FrameArena {
     // grow to exactly the size asked (no headroom): a server slot's arena,
     // whose device bytes count against an HBM budget
     bool exact = false;
-    // its word in the context's flight table, from its first trace on
-    FlightTable* flights = nullptr;
+    // its word in the device's flight table, from its first trace on
+    std::shared_ptr<FlightTable> flights;
     int flight = -1;
     // host calls using the arena now: a second one at the same time (two
     // threads tracing on one stream of one context) is refused
@@ -1575,8 +1575,15 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
     // 6,908 to 4,164 at 1920x1080, on five to sixteen 803 to 1,011, 1,485 to
     // 1,650 and 4,067..4,130 to 4,155; six served requests on eight queues
     // 7,276 to 5,681. A frame alone is the faster side by side (404 us to 505
-    // at 480x270). Counted traces keep the setting's split.
-    const int others = flight && !cnt ? ctx->flight.others(a->flight) : 0;
+    // at 480x270). The queues are the process's, so traces of other contexts
+    // count: two contexts with a 1080p frame each on four queues take 4,110
+    // to 4,160 us (5,090 where both streams have one queue), side by side
+    // 4,160 to 6,580 with which streams share one. Replays of a captured
+    // batch are not counted: four scenes replayed beside six 480x270 frames
+    // take 9,565 us with the frames side by side and 10,632 in sequence,
+    // beside one of 1920x1080 7,391 and 7,265. Counted traces keep the
+    // setting's split.
+    const int others = flight && !cnt ? ctx->flight->others(a->flight) : 0;
     const bool crowded = others > 0 && 2 * (others + 1) + 1 > ctx->hw_queues;
     const unsigned Gside = crowded ? 0 : std::min<unsigned>((unsigned)tune.bounce_blocks, G / 2);
     if (P.max_traces > 1 && Gside > 0) {
@@ -1626,12 +1633,12 @@ void enqueue_trace(rtg_ctx* ctx, FrameArena* a, const TracePlan& P, const Tuning
     uint32_t seq = 0;
     if (flight) {
         if (a->flight < 0) {
-            a->flights = &ctx->flight;
-            a->flight = ctx->flight.take();
+            a->flights = ctx->flight;
+            a->flight = ctx->flight->take();
         }
         if (a->flight >= 0) {
-            done = ctx->flight.ended + a->flight;
-            seq = ctx->flight.start(a->flight);
+            done = ctx->flight->ended + a->flight;
+            seq = ctx->flight->start(a->flight);
         }
     }
     {

@@ -4,11 +4,14 @@ bounce levels beside the first level's shadow rays or in sequence."""
 import os
 import subprocess
 
+import numpy as np
 import pytest
 import torch
 
+import oracle_host as oh
 from conftest import PKG, REPO
 from rtg import abi, scenes
+from rtg.batch import trace_batch
 from rtg.device import DeviceScene
 from rtg.frames import FrameDriver
 from rtg.lib import Context
@@ -34,11 +37,11 @@ def launched_side_by_side(c, enqueue):
 
 
 class LongTrace:
-    """A frame of several milliseconds (16.6 M paths), enqueued again and again."""
+    """A frame of some 25 ms (33 M paths), enqueued again and again."""
 
     def __init__(self, ds):
         self.opts = ds.scene.trace_opts()
-        self.opts.spp = 8
+        self.opts.spp = 16
         self.out = ds.make_outputs(width=1920, height=1080, hits=False)
         self.job = ds.job(self.out, opts=self.opts, width=1920, height=1080)
 
@@ -73,3 +76,37 @@ def test_more_arenas_than_a_small_table_has_words(monkeypatch):
         d.close()
     ds.destroy()
     c.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("queues", [4, 8])
+def test_two_contexts(monkeypatch, queues):
+    """The hardware queues are the process's: a frame sees the traces of other
+    contexts, and side by side or in sequence its image is the oracle's."""
+    monkeypatch.setenv("GPU_MAX_HW_QUEUES", str(queues))
+    a, b = Context(0), Context(0)
+    s = scenes.default_scene(n_tori=12, width=133, height=77)
+    want = oh.HostScene(s).trace_image(frame_index=0, want_hits=False)[0]
+    da, db = DeviceScene(a, s), DeviceScene(b, s)
+    s0, s1 = torch.cuda.Stream(), torch.cuda.Stream()
+    long = LongTrace(da)
+    outs = [db.make_outputs(hits=False) for _ in range(4)]
+    trace_batch(a, [long.job], s0)
+    torch.cuda.synchronize()
+    beside = []
+    for k, o in enumerate(outs):
+        if k % 2:
+            trace_batch(a, [long.job], s0)
+        beside.append(launched_side_by_side(b, lambda: trace_batch(b, [db.job(o, frame_index=0)], s1)))
+        torch.cuda.synchronize()
+    assert beside == [True, queues > 4, True, queues > 4]
+    for o in outs:
+        assert np.array_equal(o[0].cpu().numpy().view(np.uint32), want)
+    # a context that goes takes its words along and leaves the others'
+    trace_batch(b, [db.job(outs[0], frame_index=0)], s1)
+    torch.cuda.synchronize()
+    da.destroy()
+    a.close()
+    assert launched_side_by_side(b, lambda: trace_batch(b, [db.job(outs[0], frame_index=0)], s1))
+    db.destroy()
+    b.close()

@@ -1,8 +1,10 @@
 """Which traces count as in flight: the table of csrc/flight.hpp on the CPU,
 and on the GPU the choice made by it, seen in whether a frame launches the
 bounce levels beside the first level's shadow rays or in sequence."""
+import ctypes
 import os
 import subprocess
+import time
 
 import numpy as np
 import pytest
@@ -110,3 +112,47 @@ def test_two_contexts(monkeypatch, queues):
     assert launched_side_by_side(b, lambda: trace_batch(b, [db.job(outs[0], frame_index=0)], s1))
     db.destroy()
     b.close()
+
+
+@pytest.mark.gpu
+def test_streams_that_share_a_queue():
+    """A frame's two streams on one hardware queue run one after the other. The
+    bounce levels' last launch helps with the first level's shadow rays, so it
+    has to come after their own launch: in front of it, it traced all of them
+    on its 192 workgroups, and a 1920x1080 frame took 2.2 times as long as with
+    two queues (2,410 us and 1,111). In this order it takes 1.4 times as long."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    x = torch.zeros(16, device="cuda:0")
+    raw = []
+
+    def stream():
+        p = ctypes.c_void_p()
+        assert hip.hipStreamCreateWithFlags(ctypes.byref(p), 1) == 0  # non-blocking
+        raw.append(p)
+        s = torch.cuda.ExternalStream(p.value)
+        with torch.cuda.stream(s):
+            x.add_(1)
+        return s
+
+    s = scenes.default_scene(width=1920, height=1080)
+    times = []
+    for between in range(5):  # streams in use between the frame's two
+        c = Context(0)
+        ds = DeviceScene(c, s)
+        out = ds.make_outputs(hits=False)
+        st = stream()
+        for _ in range(between):
+            stream()
+        v = []
+        for k in range(12):
+            t0 = time.perf_counter()
+            trace_batch(c, [ds.job(out, frame_index=0)], st)
+            torch.cuda.synchronize()
+            v.append(time.perf_counter() - t0)
+        times.append(sorted(v[2:])[5])
+        ds.destroy()
+        c.close()
+    torch.cuda.synchronize()
+    for p in raw:
+        assert hip.hipStreamDestroy(p) == 0
+    assert max(times) < 1.8 * min(times), times

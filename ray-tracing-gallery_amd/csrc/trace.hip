@@ -1300,7 +1300,26 @@ size_t spill_bytes(rtg_ctx* ctx, const Tuning& tune) {
     return (size_t)trace_grid(ctx, tune) * kTraceThreads * kSpillLaneBytes;
 }
 
+// A closest-hit query on lanes takes a fifth workgroup per CU where the spill
+// area holds it, as a stream's area does (ensure_spill): the registers are few
+// enough, and 15 stack entries a lane fit the 160 KB of LDS five times.
+// Incoherent rays fetch nodes and triangles past L2, and a fifth wave per SIMD
+// hides more of that than the entries spilled beyond the 15th cost: 16 M rays
+// in a 1 M-triangle soup 9,460 -> 8,530 us (15 entries on four workgroups
+// 9,480, 12 on six 8,650). Occlusion queries lose (3 M rays 1,104 -> 1,188
+// us), and so do frames (the 1080p loop 4,312 -> 4,452): coherent rays hit the
+// caches. A tuning other than four workgroups is taken as it is.
+constexpr unsigned kQueryBlocksPerCu = 5;
+constexpr int kQueryStackLds = 15;
+
+// Spill stacks of the grid; for four workgroups per CU also those of the fifth
+// (a server slot's area, which counts against a budget and serves no queries,
+// has the grid's alone).
 static int ensure_spill(rtg_ctx* ctx, FrameArena* a, const Tuning& tune) {
+    if (!a->exact && tune.blocks_per_cu == (int)kQueryBlocksPerCu - 1) {
+        const size_t wide = (size_t)ctx->cu_count * kQueryBlocksPerCu * kTraceThreads * kSpillLaneBytes;
+        return ensure_room(ctx, a->spill, wide, false);
+    }
     return ensure_room(ctx, a->spill, spill_bytes(ctx, tune), !a->exact);
 }
 
@@ -1718,19 +1737,6 @@ static int check_ray_query(rtg_ctx* ctx, rtg_tlas tlas, const rtg_ray* rays, uin
                 ray_flags & ~allowed);
     return RTG_OK;
 }
-
-// A closest-hit query on lanes takes a fifth workgroup per CU where the spill
-// area holds it, as a stream's area does (it is allocated with a quarter to
-// spare): the registers are few enough, and 15 stack entries a lane fit the
-// 160 KB of LDS five times. Incoherent rays fetch nodes and triangles past L2,
-// and a fifth wave per SIMD hides more of that than the entries spilled beyond
-// the 15th cost: 16 M rays in a 1 M-triangle soup 9,460 -> 8,530 us (15
-// entries on four workgroups 9,480, 12 on six 8,650). Occlusion queries lose
-// (3 M rays 1,104 -> 1,188 us), and so do frames (the 1080p loop 4,312 ->
-// 4,452): coherent rays hit the caches. A tuning other than four workgroups
-// is taken as it is.
-constexpr unsigned kQueryBlocksPerCu = 5;
-constexpr int kQueryStackLds = 15;
 
 // Clears the feed counters (`feed_stride` words apart) and launches the query
 // kernel on at most `max_blocks` persistent blocks, closest hits on up to

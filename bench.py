@@ -637,17 +637,42 @@ def main():
     elapsed = t1 - t0
     value = rays / elapsed / 1e6
 
+    # In the timed frames the bounce stream's last launch takes over part of
+    # the first level's shadow rays, more or fewer as the two frames overlap,
+    # so the counters don't tell what the occlusion launch traced. Its roofline
+    # is of the same frames one at a time with their levels in sequence, where
+    # one launch traces a frame's whole shadow queue.
+    def one_by_one(each):
+        for f in range(W, W + K):
+            frame(f)
+            torch.cuda.synchronize()
+            each()
+
+    saved = ctx.tuning()
+    ctx.set_tuning(abi.Tuning.make(**{**saved.as_dict(), "bounce_blocks": 0}))
+    ctx.set_timing(True)
+    one_by_one(lambda: None)
+    seq_time = ctx.kernel_time(abi.RTG_KERNEL_TRACE_OCCLUSION)
+    ctx.set_timing(False)
+    ctx.set_counters(True)
+    seq_counts = []
+    one_by_one(lambda: seq_counts.append(ctx.counters().as_dict()))
+    ctx.set_counters(False)
+    ctx.set_tuning(saved)
+    seq_tot = {k: sum(c[k] for c in seq_counts) for k in tot}
+    assert seq_tot["side_shadow_rays"] == 0 and seq_tot["shadow_rays"] == tot["shadow_rays"]
+
     # rooflines of the frame stream's traversal and shading launches: the
     # algorithmic bytes of their launches (the counters of the same frames)
     # over their HIP-event time on that stream, beside what the committed
     # rocprofv3 passes measured for the same launches. The dominant kernel,
     # whose figures are the line's `roofline`, is the one that moves the most
-    # algorithmic bytes: the level-0 shadow rays.
+    # algorithmic bytes: the shadow rays.
     per_kernel = {}
-    for kind, name, nbytes in (("trace_closest", "k_trace_closest", algorithmic_bytes(tot, "closest")),
-                               ("trace_occlusion", "k_trace_occlusion", algorithmic_bytes(tot, "occlusion")),
-                               ("shade", "k_shade", shade_bytes(tot))):
-        ms, launches = ktime[kind]
+    for name, (ms, launches), nbytes in (
+            ("k_trace_closest", ktime["trace_closest"], algorithmic_bytes(tot, "closest")),
+            ("k_trace_occlusion", seq_time, algorithmic_bytes(seq_tot, "occlusion")),
+            ("k_shade", ktime["shade"], shade_bytes(tot))):
         per_kernel[name] = kernel_roofline(name, nbytes / max(1, launches), ms / max(1, launches), launches)
     dom = max(("k_trace_closest", "k_trace_occlusion"), key=lambda k: per_kernel[k]["algorithmic_bytes_per_launch"])
     roofline = {"bound": "hbm", "peak": HBM_PEAK_GBS, "unit": "GB/s", **per_kernel[dom],

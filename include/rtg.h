@@ -434,12 +434,14 @@ int rtg_get_status(rtg_ctx* ctx, uint32_t* bits, int clear);
 #define RTG_KERNEL_RAYGEN 0u
 #define RTG_KERNEL_TRACE_CLOSEST 1u
 #define RTG_KERNEL_SHADE 2u
-#define RTG_KERNEL_TRACE_OCCLUSION 3u
+#define RTG_KERNEL_TRACE_OCCLUSION 3u /* beside a bounce stream: the first level's shadow rays, less
+                                         those that the bounce stream's last launch takes over */
 #define RTG_KERNEL_RESOLVE 4u
 #define RTG_KERNEL_REFIT 5u
 #define RTG_KERNEL_BATCH_GRAPH 6u /* one replay of an rtg_batch graph (all its kernels) */
-#define RTG_KERNEL_BOUNCE_SIDE 7u /* the bounce levels and their shadow rays on the bounce stream,
-                                     beside the first level's shadow rays (one span per frame) */
+#define RTG_KERNEL_BOUNCE_SIDE 7u /* the bounce levels, their shadow rays and what their last launch
+                                     takes over of the first level's, on the bounce stream beside the
+                                     first level's shadow rays (one span per frame) */
 #define RTG_KERNEL_COUNT 8u
 int rtg_set_timing(rtg_ctx* ctx, int enable);
 int rtg_get_kernel_time(rtg_ctx* ctx, uint32_t kind, double* total_ms, uint64_t* launches);

@@ -13,7 +13,7 @@ import torch
 import oracle_host as oh
 from conftest import PKG, REPO
 from rtg import abi, scenes
-from rtg.batch import trace_batch
+from rtg.batch import Batch, trace_batch
 from rtg.device import DeviceScene
 from rtg.frames import FrameDriver
 from rtg.lib import Context
@@ -156,3 +156,45 @@ def test_streams_that_share_a_queue():
     for p in raw:
         assert hip.hipStreamDestroy(p) == 0
     assert max(times) < 1.8 * min(times), times
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("queues", [4, 8])
+def test_frames_beside_a_replayed_batch(monkeypatch, queues):
+    """Replays of a captured batch and frames on two other streams at once, all
+    of one context: every image equals the one traced alone."""
+    monkeypatch.setenv("GPU_MAX_HW_QUEUES", str(queues))
+    c = Context(0)
+    ds = [DeviceScene(c, scenes.default_scene(n_tori=n, width=w, height=h))
+          for n, w, h in ((5, 201, 113), (30, 320, 180), (12, 400, 300))]
+
+    def traced(d, f):
+        out = d.make_outputs(hits=False)
+        return out, d.job(out, frame_index=f)
+
+    alone = []
+    for d in ds:
+        out, job = traced(d, 1)
+        trace_batch(c, [job])
+        torch.cuda.synchronize()
+        alone.append(out[0].clone())
+    in_batch = [traced(d, 1) for d in ds[:2]]
+    batch = Batch(c, [job for _, job in in_batch])
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    for replay in range(6):
+        for out, _ in in_batch:
+            out[0].fill_(-1)
+        frames = [traced(ds[2], 1) for _ in range(4)]
+        torch.cuda.synchronize()
+        batch.launch(streams[0])
+        for k, (_, job) in enumerate(frames):
+            trace_batch(c, [job], streams[1 + k % 2])
+        torch.cuda.synchronize()
+        for want, (out, _) in zip(alone, in_batch):
+            assert torch.equal(out[0], want), replay
+        for out, _ in frames:
+            assert torch.equal(out[0], alone[2]), replay
+    batch.close()
+    for d in ds:
+        d.destroy()
+    c.close()

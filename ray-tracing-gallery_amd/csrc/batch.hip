@@ -86,6 +86,7 @@ struct TuneRig {
     FrameArena* arena = nullptr;
     ~TuneRig() {
         if (s) hipStreamSynchronize(s);
+        if (arena) arena_forget_stream(arena);
         if (e0) hipEventDestroy(e0);
         if (e1) hipEventDestroy(e1);
         if (s) hipStreamDestroy(s);
@@ -240,6 +241,7 @@ static int batch_capture(rtg_batch* b, const rtg_image_job* jobs, uint32_t n) {
     RTG_HIP(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
     st = upload_jobs(b->arena, b->plan, cs);
     hipError_t e = hipStreamSynchronize(cs);
+    arena_forget_stream(b->arena);
     if (st == RTG_OK && e != hipSuccess) {
         set_error("rtg_batch_create: job upload: %s", hipGetErrorString(e));
         st = RTG_ERROR_DEVICE;

@@ -218,6 +218,7 @@ void arena_reset(FrameArena* a);
 // The device word with the status bits of the arena's last trace.
 const uint32_t* arena_status_word(const FrameArena* a);
 void delete_frame_arena(FrameArena* a);
+void arena_forget_stream(FrameArena* a);
 size_t frame_bytes(uint64_t paths, uint64_t shadow, uint32_t njobs);
 // Shadow-queue slots a path with `shadow_rays` rays takes: an even number
 // (the occlusion kernel traces the slots in pairs of one path).

@@ -1224,12 +1224,20 @@ FrameArena* new_frame_arena(bool exact) {
     return a;
 }
 
+// HIP asks an event's stream whether it is under capture, so an event must not
+// outlive its stream: called before a stream that the arena's last upload went
+// through is destroyed, when that upload is done.
+void arena_forget_stream(FrameArena* a) {
+    if (a->staging_free) hipEventDestroy(a->staging_free);
+    a->staging_free = nullptr;
+}
+
+// Of an arena whose work is done (the callers synchronise its streams).
 void delete_frame_arena(FrameArena* a) {
     if (!a) return;
     a->buf.release();
     a->spill.release();
     a->feed.release();
-    if (a->staging_free) hipEventSynchronize(a->staging_free);
     if (a->h_jobs) hipHostFree(a->h_jobs);
     if (a->staging_free) hipEventDestroy(a->staging_free);
     if (a->side) {

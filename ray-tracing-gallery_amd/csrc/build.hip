@@ -335,9 +335,11 @@ constexpr int kRsThreads = 256;
 constexpr int kRsItems = 8;
 constexpr int kRsTile = kRsThreads * kRsItems;
 // Up to this many tiles (262,144 keys) a scatter workgroup sums the tiles'
-// counts itself; beyond, a kernel between the two scans them. A build of
-// 130,000 triangles without treelets takes 503 us summing itself and 506 with
-// the scan, of 500,000 triangles 674 and 625.
+// counts itself; beyond, a kernel between the two scans them. Builds without
+// treelets, summing themselves / with the scan: 60,000 triangles 238 / 244 us,
+// 100,000 253 / 256, 130,000 267 / 267, 160,000 278 / 271, 200,000 288 / 284,
+// 262,144 303 / 293, 300,000 321 / 307, 500,000 395 / 365. The two cross near
+// 130,000, so between there and this line the scan would save 1 to 3 %.
 constexpr uint32_t kRsSelfTiles = 128;
 
 // SELF: the counts tile by tile, else digit by digit.
@@ -1025,9 +1027,12 @@ static void launch_pass(const BuildBufs& b, uint32_t n, uint32_t* tiers, int rou
     // Where the CUs hold every subtree at two workgroups each, a subtree's
     // levels are the launch's time, and 512 lanes take them in fewer turns
     // than 256: builds with treelets of 1,000 triangles 1,205 -> 1,044 us,
-    // 20,000 1,560 -> 1,431, 80,000 1,969 -> 1,909. Beyond, the CUs hold more
-    // of the smaller workgroups: 120,000 take 2,240 us with 256 lanes and
-    // 2,434 with 512, 1 M 6,150 and 7,730.
+    // 20,000 1,043 -> 964 (256 / 512 lanes; all from here on with kept
+    // blocks), 80,000 1,382 / 1,325, 100,000 1,470 / 1,390, 110,000 1,499 /
+    // 1,412. Beyond, the CUs hold more of the smaller workgroups: 120,000
+    // take 1,613 us with 256 lanes and 1,773 with 512, 1 M (before kept
+    // blocks) 6,150 and 7,730. The subtrees of a count vary with the mesh, so
+    // the line lies a quarter below where uniform meshes cross (256 CUs).
     const bool wide = OPT && n <= 80000;
     auto bottom = wide ? k_tree_bottom<OPT, OPT ? 512 : 256> : k_tree_bottom<OPT, 256>;
     hipLaunchKernelGGL(bottom, dim3(low_grid), dim3(wide ? 512 : 256), 0, s, b.bin, b.ibox, b.rcount, b.lbox, b.low,
@@ -1062,7 +1067,7 @@ static int wide_hierarchy(rtg_ctx* ctx, const BuildBufs& b, uint32_t n, int tree
     }
     const WideTree W{b.bin, b.ibox, b.lbox, b.nodes, b.wroot, node_cap(n)};
     // one workgroup emits 1,024 nodes of a level in about 4 us; beyond a few
-    // thousand the two launches over many workgroups are the faster way
+    // thousand a launch over many workgroups is the faster way
     const bool one = n <= kSmallBuild;
     const unsigned wide_grid = std::min(n / 1024 + 1, kWideBlocks);
     hipLaunchKernelGGL(k_collapse_top, dim3(1), dim3(kCollapseThreads), 0, s, W, one ? n : 2048u, b.off, b.state);

@@ -689,7 +689,7 @@ struct Traverser {
     // (stack words, the culled-by-distance test, leaving an instance) inlined
     // behind each kind of visit is run by every subset of the wave in turn;
     // one copy after the leaves serves them together.  16 M closest rays on a
-    // triangle soup 9785 -> 9363 us, the 1080p frame loop 4325 -> 4282.  An
+    // triangle soup 9762 -> 9460 us, the 1080p frame loop 4313 -> 4268.  An
     // occlusion pop tests no distance and its lanes end at the first hit:
     // there the shared pop only adds a pass (3 M rays 1122 -> 1196 us), so
     // occlusion keeps the inlined one.

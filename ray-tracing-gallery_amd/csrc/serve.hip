@@ -304,9 +304,9 @@ extern "C" int rtg_server_create(rtg_ctx* ctx, const rtg_server_config* cfg, rtg
     RTG_REQUIRE(cfg->hbm_budget_bytes >= (64ull << 20), RTG_ERROR_INVALID_ARGUMENT,
                 "rtg_server_create: budget below 64 MiB");
     RTG_HIP(hipSetDevice(ctx->device));
-    // Every slot holds the spill area of the persistent traversal grid and a
-    // feed counter; the rest of its share of the budget is for the frame
-    // state and TLAS copies of its batches.
+    // Every slot holds the spill area of the persistent traversal grid (256
+    // bytes more are kept back); the rest of its share of the budget is for
+    // the frame state and TLAS copies of its batches.
     const uint64_t share = cfg->hbm_budget_bytes / cfg->max_inflight;
     const uint64_t fixed = spill_bytes(ctx, ctx->tune) + 256;
     const uint64_t smallest = frame_bytes(1, 1, 1);

@@ -8,7 +8,7 @@
 // Here each stage is a kernel over a queue of rays:
 //   raygen -> [trace closest -> shade] x max_traces -> trace occlusion -> resolve
 // Shade appends continuation rays (mirror, portal) and shadow rays to queues
-// with one atomic per wavefront (ballot/prefix-sum compaction). A path's
+// with one atomic per workgroup (ballot/prefix-sum compaction). A path's
 // result depends only on its own rays, so queue order never changes results.
 #include <algorithm>
 #include <atomic>
@@ -111,8 +111,8 @@ struct Frame {
     float2* hit_b;       // u, v
     float4* pair_o;      // shadow rays in pairs (slots 2j, 2j + 1) of one path: origin.xyz, path
     float4* pair_d;      // per slot: direction.xyz; of the first, 3 in w's bits, or 1 without a second
-    uint32_t* counts;    // [0..3] queue sizes per trace level, [4] shadow rays, [5] shadow
-                         // rays of level 0, [14] status bits
+    uint32_t* counts;    // [0..3] queue sizes per trace level, [4] shadow-queue slots of
+                         // level 0, [5] those of the bounce levels, [14] status bits
     uint32_t* feeds;     // feed counters of queue q: feeds[q + k * kFeedStride]
     uint64_t* counters;  // rtg_trace_counters
     uint2* spill;
@@ -655,6 +655,8 @@ __global__ __launch_bounds__(256) void k_shade(Frame F, int level, const uint32_
     const uint32_t n = min(count_ptr ? *count_ptr : fixed_count, F.path_cap);
     const Queue Q = F.q[level & 1];
     const Queue NQ = F.q[(level + 1) & 1];
+    // (level 3, the last, queues no rays: max_traces is at most 4, so the word
+    // after the level counts, which is kShadowFirst's, is never added to here)
     uint32_t* next_count = &F.counts[level + 1];
     const uint32_t stride = gridDim.x * blockDim.x;
     const uint32_t rounds = (n + stride - 1) / stride;
@@ -1285,8 +1287,9 @@ size_t frame_bytes(uint64_t paths, uint64_t shadow, uint32_t njobs) {
 }
 
 static int trace_grid(rtg_ctx* ctx, const Tuning& tune) {
-    // persistent grid: blocks_per_cu blocks of 256 lanes per CU (the LDS
-    // stack takes 32 KB per block, so at most 5 fit; registers allow 4)
+    // persistent grid: blocks_per_cu blocks of 256 lanes per CU (16 stack
+    // entries a lane take 32 KB of LDS per block, so 5 fit; the occlusion
+    // kernels' registers allow 4, the closest-hit ones' 5)
     return ctx->cu_count * tune.blocks_per_cu;
 }
 static int trace_grid(rtg_ctx* ctx) { return trace_grid(ctx, ctx->tune); }
